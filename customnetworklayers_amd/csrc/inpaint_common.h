@@ -60,6 +60,10 @@ struct Knobs {
   int tv_adj_rows = 0;
   int tv_fwd_split = -1;          // INPAINT_TV_FWD_SPLIT=0|1: forward pairs with one channel per wavefront (-1 = by the size of the launch)
   int tv_adj_split = -1;          // INPAINT_TV_ADJ_SPLIT=0|1: the same for the adjoint pairs of two channels
+  int tv_tile_rows = 0;           // INPAINT_TV_TILE=R,K: forward tiles of R rows per wavefront, K iterations per launch; =0: no tiles (not set: by the
+  int tv_tile_its = -1;           //   size of the problem; rows 0 and its -1 here)
+  int tv_atile_rows = 0;          // INPAINT_TV_ADJ_TILE=R,K: the same for the reverse sweep (one or two channels)
+  int tv_atile_its = -1;
   bool tgv_px_path = false;       // INPAINT_TGV_PATH=px: the per-pixel kernels
   bool tgv_fuse = true;           // INPAINT_TGV_FUSE=0
   bool tgv_fuse_adj = true;       // INPAINT_TGV_FUSE_ADJ=0
@@ -94,6 +98,16 @@ struct Knobs {
     tv_adj_rows = rows("INPAINT_TV_ADJ_ROWS");
     tv_fwd_split = is("INPAINT_TV_FWD_SPLIT", "1") ? 1 : (is("INPAINT_TV_FWD_SPLIT", "0") ? 0 : -1);
     tv_adj_split = is("INPAINT_TV_ADJ_SPLIT", "1") ? 1 : (is("INPAINT_TV_ADJ_SPLIT", "0") ? 0 : -1);
+    auto tile = [](const char* name, int& r_out, int& k_out) {
+      const char* e = getenv(name);
+      if (!e) return;
+      int r = 0, k = 0;
+      const bool both = sscanf(e, "%d,%d", &r, &k) == 2 && r > 0 && k > 0;
+      r_out = both ? r : 0;
+      k_out = both ? k : 0;
+    };
+    tile("INPAINT_TV_TILE", tv_tile_rows, tv_tile_its);
+    tile("INPAINT_TV_ADJ_TILE", tv_atile_rows, tv_atile_its);
     tgv_px_path = is("INPAINT_TGV_PATH", "px");
     tgv_fuse = !is("INPAINT_TGV_FUSE", "0");
     tgv_fuse_adj = !is("INPAINT_TGV_FUSE_ADJ", "0");

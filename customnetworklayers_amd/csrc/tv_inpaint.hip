@@ -18,6 +18,7 @@
 // ~5e-3 of their maximum, above the layer's 1e-3 tolerance.
 #include "inpaint_common.h"
 #include "tv_strip_kernels.h"
+#include "tv_tile_kernels.h"
 
 #include <cstddef>
 #include <cstdlib>
@@ -421,6 +422,76 @@ void launch_forward_pair(const Slot& s, hipStream_t stream, const float* dx, con
   }
 }
 
+// Iterations in register tiles (tv_tile_kernels.h): R rows per wavefront, K iterations per launch; R = 0: strips.
+struct TilePlan {
+  int R = 0, K = 0;
+};
+constexpr int kTileWaves = 4;
+
+// Workgroups on the fullest CU of a launch of `its` iterations in tiles of `cols` x `rows` pixels, halo included.
+long long tiles_per_cu(const Slot& s, int cols, int rows, int its, int channels) {
+  const long long tx = (s.iw + cols - 2 * its - 1) / (cols - 2 * its), ty = (s.ih + rows - 2 * its - 1) / (rows - 2 * its);
+  return (tx * ty * s.n * channels + compute_unit_count() - 1) / compute_unit_count();
+}
+
+// Tiles or strips, and which tile: the cheapest by a cost model fitted to both kernels' measured times.  A tile launch
+// costs 3.8 us however small it is, 3 us more for every further round of workgroups, and per iteration and row of a
+// wavefront 300 cycles where a SIMD holds one wavefront and 200 per wavefront where it holds several; keeping x05 rows adds
+// 0.5 us per iteration and million values, rebuilding the input iterate from them 100 cycles per row.  A strip launch
+// costs 4.3 us and 4.65 us per million values, for two iterations.  So tiles win while launches and latency dominate, and
+// strips, which have no halo columns to spare and stream their rows, on problems that fill the chip many times over.
+// Measured, forward pass, strips -> tiles: 1 x 2 x 64 x 128, 20 iterations 46 -> 27 us; 48 iterations of 2 x 2 x 112 x 256
+// 118 -> 76, 2 x 2 x 224 x 512 156 -> 122, 1 x 1 x 384 x 1248 158 -> 123, 1 x 2 x 384 x 1248 233 -> 192, 4 x 2 x 384 x
+// 1248 without rows 508 -> 477, with rows 536 (strips) against 567 (best tiles).
+TilePlan forward_tile_plan(const Slot& s, bool keeps_rows) {
+  TilePlan p;
+  if (!forward_pairs(s) || knobs().tv_fwd_rows > 0 || knobs().tv_fwd_split >= 0) return p;  // (a forced strip shape)
+  if (knobs().tv_tile_its >= 0) {
+    p.R = knobs().tv_tile_rows;
+    p.K = knobs().tv_tile_its;
+    const bool known = p.R == 4 || p.R == 8 || p.R == 16;
+    if (!known || p.K < 2 || p.K > tvtile::kMaxFwdSteps || kTileWaves * p.R <= 2 * p.K) p = TilePlan();
+    return p;
+  }
+  const int K = 2 * (s.its / 2);
+  const double mega = 1e-6 * s.n * s.ic * (double)s.ih * s.iw;
+  double best = 0.97 * (4.3 + 4.65 * mega) / 2;  // us per iteration
+  for (int R : {4, 8, 16}) {
+    for (int k = 2; k <= tvtile::kMaxFwdSteps && 2 * k < kTileWaves * R; k++) {
+      const int launches = (K + k - 1) / k, its = (K + launches - 1) / launches;
+      if (its != k) continue;  // (the same launches as a smaller k)
+      const long long on_cu = tiles_per_cu(s, 64, kTileWaves * R, its, s.ic);
+      const long long rounds = (on_cu + 32 / R - 1) / (32 / R);  // 8, 4 and 2 workgroups resident per CU
+      double us = (3.8 + 3.0 * (rounds - 1)) / its + on_cu * (R + 0.55) * (on_cu == 1 ? 300 : 200) / 2400.;
+      if (keeps_rows) us += 0.5 * mega + on_cu * R * 100 / 2400. / its;
+      if (us < best) { best = us; p.R = R; p.K = its; }
+    }
+  }
+  return p;
+}
+
+template <int R>
+void launch_forward_tile(const Slot& s, hipStream_t stream, const float* dx, const float* dy, const float* c, const float* b,
+                         const float* xin, const float* yin, const tvtile::FwdSteps& steps, int K, bool ring, float tP,
+                         float* keep_x, float* keep_y, bool rows) {
+  auto kern = rows ? tvtile::tv_forward_tile<R, kTileWaves, true> : tvtile::tv_forward_tile<R, kTileWaves, false>;
+  const int cols = 64 - 2 * K, trows = R * kTileWaves - 2 * K;
+  const int tx = (s.iw + cols - 1) / cols, ty = (s.ih + trows - 1) / trows;
+  const long long tiles = (long long)tx * ty * s.n * s.ic;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(64 * kTileWaves), 0, stream, dx, dy, c, b, xin, yin, steps, K,
+                     ring ? 1 : 0, tP, keep_x, keep_y, s.n, s.ic, s.ih, s.iw, tx, ty);
+}
+
+void launch_forward_tiles(const Slot& s, hipStream_t stream, int R, const float* dx, const float* dy, const float* c, const float* b,
+                          const float* xin, const float* yin, const tvtile::FwdSteps& steps, int K, bool ring, float tP,
+                          float* keep_x, float* keep_y, bool rows) {
+  switch (R) {
+    case 4: launch_forward_tile<4>(s, stream, dx, dy, c, b, xin, yin, steps, K, ring, tP, keep_x, keep_y, rows); break;
+    case 8: launch_forward_tile<8>(s, stream, dx, dy, c, b, xin, yin, steps, K, ring, tP, keep_x, keep_y, rows); break;
+    default: launch_forward_tile<16>(s, stream, dx, dy, c, b, xin, yin, steps, K, ring, tP, keep_x, keep_y, rows); break;
+  }
+}
+
 void launch_forward(const Slot& s, hipStream_t stream, const float* dx, const float* dy, const float* c,
                     const float* b, const float* xin, float* xout, const float* yin, float* yout, float* x05,
                     float t) {
@@ -659,6 +730,106 @@ bool adjoint_pairs(const Slot& s) {
   return forward_pairs(s) && s.ic <= kPairChannels;
 }
 
+// The reverse sweep in register tiles: one channel, or two in the two halves of a wavefront.  The same choice as
+// forward_tile_plan's: a tile launch costs 4.4 us, and per step and row 850 cycles with one wavefront per SIMD, 650 per
+// wavefront with more; strips cost 6.2 us and 11 us (one channel) or 15 us (two) per million values, for two steps.  A tile
+// has to be cheaper by a tenth: the reverse step is bound by the vector ALUs, and a tile of 16 rows does its halo's work
+// as well, so tiles win only where the chip is far from full.  (Taller tiles, 6 and 8 rows per wavefront, were measured:
+// 256 registers and one wavefront per SIMD, slower at every size.)  Measured, backward pass, strips -> tiles: 1 x 2 x 64 x
+// 128, 20 iterations 88 -> 70 us; 50 iterations of 1 x 1 x 112 x 256 186 -> 144, 2 x 2 x 112 x 256 232 -> 191, 1 x 2 x 187
+// x 621 322 -> 246; 2 x 2 x 224 x 512 327 (strips) against 365.
+TilePlan adjoint_tile_plan(const Slot& s) {
+  TilePlan p;
+  if (!adjoint_pairs(s) || s.ic > 2 || knobs().tv_adj_rows > 0 || knobs().tv_adj_split >= 0) return p;
+  constexpr int R = 4;
+  if (knobs().tv_atile_its >= 0) {
+    p.R = knobs().tv_atile_rows;
+    p.K = knobs().tv_atile_its;
+    if (p.R != R || p.K < 1 || p.K > tvtile::kMaxAdjSteps || kTileWaves * p.R <= 2 * p.K || 64 / s.ic <= 2 * p.K) p = TilePlan();
+    return p;
+  }
+  const int steps = 2 * (s.its / 2) - 1;
+  const double mega = 1e-6 * s.n * s.ic * (double)s.ih * s.iw;
+  double best = 0.9 * (6.2 + (s.ic == 1 ? 11 : 15) * mega) / 2;  // us per step
+  for (int k = 1; 2 * k < kTileWaves * R; k++) {
+    const int launches = (steps + k - 1) / k, its = (steps + launches - 1) / launches;
+    if (its != k) continue;
+    const long long on_cu = tiles_per_cu(s, 64 / s.ic, kTileWaves * R, its, 1);
+    if (on_cu > 2) continue;  // (all that is resident; further rounds: 2 x 2 x 224 x 512 and up, strips are faster)
+    const double us = 4.4 / its + on_cu * (R + 0.5) * (on_cu == 1 ? 850 : 650) / 2400.;
+    if (us < best) { best = us; p.R = R; p.K = its; }
+  }
+  return p;
+}
+
+template <int CL, int R, bool TRUE_ADJ>
+void launch_adjoint_tile(const Slot& s, hipStream_t stream, tvtile::AdjTileArgs a, const tvtile::AdjSteps& steps) {
+  const int cols = 64 / CL - 2 * a.K, trows = R * kTileWaves - 2 * a.K;
+  a.tiles_x = (s.iw + cols - 1) / cols;
+  a.tiles_y = (s.ih + trows - 1) / trows;
+  const long long tiles = (long long)a.tiles_x * a.tiles_y * s.n;
+  hipLaunchKernelGGL((tvtile::tv_adjoint_tile<CL, R, kTileWaves, TRUE_ADJ>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(64 * kTileWaves),
+                     0, stream, a, steps);
+}
+
+template <bool TRUE_ADJ>
+void launch_adjoint_tiles(const Slot& s, hipStream_t stream, const tvtile::AdjTileArgs& a, const tvtile::AdjSteps& steps) {
+  if (s.ic == 1) launch_adjoint_tile<1, 4, TRUE_ADJ>(s, stream, a, steps);
+  else launch_adjoint_tile<2, 4, TRUE_ADJ>(s, stream, a, steps);
+}
+
+// The whole reverse sweep (every x05 row kept): the sweep's first step rides on the first launch, then `plan.K` steps per
+// launch whatever the segments; a step that is a segment's first iteration leaves that segment's record.  Returns the half
+// of the g05 / g_x ping-pongs that holds the last launch's g05 and partial g_x (the corrected gradient reads them).
+int adjoint_sweep_tiles(Slot& s, hipStream_t stream, const TilePlan& plan, const float* dx, const float* dy, const float* c,
+                        const float* b, const float* gin, int its, bool corr) {
+  const size_t F = field_count(s);
+  const int K = 2 * (its / 2), steps_all = K - 1;
+  const int launches = (steps_all + plan.K - 1) / plan.K, per = (steps_all + launches - 1) / launches;
+  auto row = [&](int k) { return s.x05 + (size_t)k * F; };
+  auto segment_at = [&](int k) {
+    for (size_t i = 0; i < s.iterations.size(); i++)
+      if (s.iterations[i] == k) return (int)i;
+    return -1;
+  };
+  int src = 1, acc = 0;
+  bool fresh = true;  // the accumulators start at zero
+  for (int done = 0; done < steps_all;) {
+    const int len = std::min(per, steps_all - done), k_first = K - 2 - done;
+    const bool first = done == 0, last = done + len == steps_all;
+    tvtile::AdjSteps st{};
+    bool ended = false;
+    for (int j = 0; j < len; j++) {
+      const int k = k_first - j, seg = segment_at(k);
+      tvtile::AdjStep& f = st.step[j];
+      f.t = s.steps[k];
+      f.seg = seg;
+      f.xb = seg >= 0 ? (corr ? s.ckpt_x : s.ckpt_y) + (size_t)seg * F : row(k - 1);
+      f.xa_next = (seg >= 0 && k > 0) ? row(k - 1) : nullptr;
+      ended = seg >= 0;
+    }
+    tvtile::AdjTileArgs a{};
+    a.wx = dx; a.wy = dy; a.cf = c; a.b = b;
+    a.xa = row(k_first);
+    a.x_last = first ? row(K - 1) : nullptr;
+    a.g05_in = first ? gin : s.g05[src];
+    a.gx_in = first ? nullptr : s.gxk[src];
+    if (!fresh) { a.gc_in = s.acc_gc[acc]; a.gwx_in = s.acc_gx[acc]; a.gwy_in = s.acc_gy[acc]; a.gb_in = s.acc_gb[acc]; }
+    if (!last || corr) { a.g05_out = s.g05[1 - src]; a.gx_out = s.gxk[1 - src]; }
+    if (!ended) { a.gc_out = s.acc_gc[1 - acc]; a.gwx_out = s.acc_gx[1 - acc]; a.gwy_out = s.acc_gy[1 - acc]; a.gb_out = s.acc_gb[1 - acc]; }
+    a.gx_final = last ? s.gx_final : nullptr;  // the gradient wrt the starting point
+    a.seg_gc = s.seg_gc; a.seg_gwx = s.seg_gx; a.seg_gwy = s.seg_gy; a.seg_gb = s.seg_gb;
+    a.N = s.n; a.H = s.ih; a.W = s.iw; a.K = len;
+    if (corr) launch_adjoint_tiles<true>(s, stream, a, st);
+    else launch_adjoint_tiles<false>(s, stream, a, st);
+    src = 1 - src;
+    acc = 1 - acc;
+    fresh = ended;
+    done += len;
+  }
+  return src;
+}
+
 // -------------------------------------------------------------------------------------------------
 // Fixed scratch of tvinpaint_forward_noalloc: the y and x ping-pongs of a forward pass (4 fields) in a
 // device array that is part of the code object, so that the call allocates nothing.  Every GPU the
@@ -752,7 +923,47 @@ int tvinpaint_forward(const float* dx, const float* dy, const float* c, const fl
     // first iteration whose x05 row is kept, and the ring row of iteration k
     const int kl = s.iterations.empty() ? K : (keep == 2 ? 0 : (keep == 1 ? s.iterations.back() : K));
     auto ring_row = [&](int k) { return s.x05 + (size_t)(keep == 2 ? k : k - kl) * F; };
-    if (forward_pairs(s)) {
+    const TilePlan tile = forward_tile_plan(s, keep == 2);
+    if (tile.R > 0) {
+      // up to tile.K iterations per launch.  What an iteration leaves in memory: its x05 row where it is kept; the half (or
+      // both halves) of a checkpoint; the result; and at the end of a launch the iterate, unless the next launch rebuilds
+      // it from the x05 rows (keep mode 2).
+      const int launches = (K + tile.K - 1) / tile.K, per = (K + launches - 1) / launches;
+      for (int k = 0, li = 0; k < K; li++) {
+        const int len = std::min(per, K - k);
+        tvtile::FwdSteps st{};
+        for (int j = 0; j < len; j++) {
+          const int next = k + j + 1, ck = next < K ? ck_index(next) : -1;
+          const bool hand_on = j == len - 1 && next < K && keep != 2;
+          tvtile::FwdStep& f = st.step[j];
+          f.t = s.steps[k + j];
+          f.x05 = k + j >= kl ? ring_row(k + j) : nullptr;
+          if (ck >= 0) {
+            if (keep != 2 || want_y) f.y = s.ckpt_y + (size_t)ck * F;
+            if (keep != 2 || want_x) f.x = s.ckpt_x + (size_t)ck * F;
+          } else if (hand_on) {
+            f.y = s.ypp[li & 1];
+            f.x = s.xpp[li & 1];
+          }
+          if (next == K) f.x = out;
+        }
+        const bool rows = k + len > kl;
+        if (k == 0 && copy_in_pair) {
+          launch_forward_tiles(s, stream, tile.R, dx, dy, c, b, init, init, st, len, false, 0.f,
+                               (keep != 2 || want_x) ? s.ckpt_x : nullptr, s.ckpt_y, rows);
+        } else if (k == 0) {
+          launch_forward_tiles(s, stream, tile.R, dx, dy, c, b, s.ckpt_x, s.ckpt_y, st, len, false, 0.f, nullptr, nullptr, rows);
+        } else if (keep == 2) {
+          launch_forward_tiles(s, stream, tile.R, dx, dy, c, b, ring_row(k - 2), ring_row(k - 1), st, len, true, s.steps[k - 1],
+                               nullptr, nullptr, rows);
+        } else {
+          const int ck = ck_index(k);
+          launch_forward_tiles(s, stream, tile.R, dx, dy, c, b, ck >= 0 ? s.ckpt_x + (size_t)ck * F : s.xpp[(li & 1) ^ 1],
+                               ck >= 0 ? s.ckpt_y + (size_t)ck * F : s.ypp[(li & 1) ^ 1], st, len, false, 0.f, nullptr, nullptr, rows);
+        }
+        k += len;
+      }
+    } else if (forward_pairs(s)) {
       // two iterations per launch; K is even and so is every checkpoint index.  The intermediate
       // iterate k+1 stays in registers, so the ping-pong alternates per pair.
       auto Yp = [&](int k) { int i = ck_index(k); return (i >= 0 && k < K) ? s.ckpt_y + (size_t)i * F : s.ypp[(k >> 1) & 1]; };
@@ -829,10 +1040,11 @@ int tvinpaint_forward_noalloc(const float* dx, const float* dy, const float* c, 
     return 0;
   }
   // In place (out == init) a launch that both reads the starting point and stores the result would have strips read
-  // halo pixels that their neighbours have already overwritten: that is the single pair launch of its = 2 or 3.  It
+  // halo pixels that their neighbours have already overwritten: that is a forward pass of one launch.  It
   // then reads a copy of the starting point in the scratch (one copy kernel more, as tvinpaint_forward does in place).
   const float *x0 = init, *y0 = init;
-  if (out == init && K == 2 && forward_pairs(s)) {
+  const TilePlan tile = forward_tile_plan(s, false);
+  if (out == init && forward_pairs(s) && K <= std::max(tile.K, 2)) {
     hipLaunchKernelGGL(copy_twice_f32, dim3(grid_stride((long long)F)), dim3(256), 0, stream, init, xpp[0], ypp[0], (long long)F);
     x0 = xpp[0];
     y0 = ypp[0];
@@ -844,7 +1056,24 @@ int tvinpaint_forward_noalloc(const float* dx, const float* dy, const float* c, 
     t = (1. + std::sqrt(1. + 4. * t * t)) / 2.;
     return (float)std::max(0.0, (t_prev - 1.) / t);
   };
-  if (forward_pairs(s)) {
+  if (tile.R > 0) {
+    const int launches = (K + tile.K - 1) / tile.K, per = (K + launches - 1) / launches;
+    for (int k = 0, li = 0; k < K; li++) {
+      const int len = std::min(per, K - k), o = li & 1;
+      tvtile::FwdSteps st{};
+      for (int j = 0; j < len; j++) st.step[j].t = next_step();
+      tvtile::FwdStep& end = st.step[len - 1];
+      if (k + len == K) {
+        end.x = out;
+      } else {
+        end.x = xpp[o];
+        end.y = ypp[o];
+      }
+      launch_forward_tiles(s, stream, tile.R, dx, dy, c, b, k == 0 ? x0 : xpp[1 - o], k == 0 ? y0 : ypp[1 - o], st, len, false, 0.f,
+                           nullptr, nullptr, false);
+      k += len;
+    }
+  } else if (forward_pairs(s)) {
     for (int k = 0; k < K; k += 2) {
       const float tA = next_step(), tB = next_step();
       const int i = (k >> 1) & 1;
@@ -903,12 +1132,13 @@ int tvinpaint_backward(const float* dx, const float* dy, const float* c, const f
   // is then an inner step) and one launch holds every channel.  That launch starts from zero accumulators without
   // reading them, and every launch after it reads only what its predecessor wrote in full: nothing to clear.
   const int nseg = (int)s.iterations.size();
+  const TilePlan tile = (s.x05_valid && s.x05_mode == 2 && s.x05_from == 0 && nseg > 0) ? adjoint_tile_plan(s) : TilePlan();
   const bool first_two = adjoint_pairs(s) && s.ic <= kGroup && knobs().tv_fuse_first && nseg > 0 &&
                          2 * ((its - s.iterations[nseg - 1]) / 2) >= 4;
   {
     ZeroList z;
     int k = 0;
-    if (!first_two) {
+    if (!first_two && tile.R == 0) {
       for (float* p : {s.g05[0], s.g05[1], s.gxk[0], s.gxk[1], s.gx_final, s.acc_gb[0]}) { z.ptr[k] = p; z.bytes[k++] = (long long)F * 4; }
       for (float* p : {s.acc_gc[0], s.acc_gx[0], s.acc_gy[0]}) { z.ptr[k] = p; z.bytes[k++] = (long long)P * 4; }
     }
@@ -923,7 +1153,8 @@ int tvinpaint_backward(const float* dx, const float* dy, const float* c, const f
   // step (TV.cu:800 calls its store a debugging aid), so only that step stores it, into gx_final.
   int lastIt = its;
   int pp_src = 1;  // g05 / g_x buffer the next adjoint launch reads (pair path)
-  for (int outer = nseg - 1; outer >= 0; outer--) {
+  if (tile.R > 0) pp_src = adjoint_sweep_tiles(s, stream, tile, dx, dy, c, b, gin, its, corr);
+  for (int outer = tile.R > 0 ? -1 : nseg - 1; outer >= 0; outer--) {
     const int k0 = s.iterations[outer];
     const int len = 2 * ((lastIt - k0) / 2);
     bool flushed = false;
