@@ -217,7 +217,8 @@ __global__ __launch_bounds__(256) void quadfit_backward_kernel(const float* __re
 //                              pass B -- rare: it takes more than kSlots pixels landing on one position.
 // A tap that the image border clamps back onto the centre carries a zero coefficient (the axis is
 // not fitted at the border), so the gather leaves it out.
-// Workspace (caller provided): count[P] | overflow count, pad | slots[P*kSlots] | overflow list[P] | coef[5*P].
+// Workspace (caller provided): count[P] | overflow count, slow count, pad | slots[P*kSlots] | overflow list[P] | coef[5*P] |
+// slow list[P].
 // ---------------------------------------------------------------------------------------------
 constexpr int kSlots = 4;
 
@@ -225,18 +226,22 @@ struct QfWorkspace {
   int* count;      // sources per displaced position
   int* ovf_count;  // one counter
   int* slots;      // [P][kSlots] source pixel (index inside its sample)
+  int* slow_count; // one counter
   int* ovf;        // global index of the sources that did not fit
+  int* slow;       // global index of the target pixels that pass B leaves to pass C
   float* coef;     // [5][P]: taps 00, 0p, 0m, p0, m0
 };
-long long qf_workspace_bytes(long long P) { return (long long)sizeof(int) * (P * (7 + kSlots) + 64 + 4); }
+long long qf_workspace_bytes(long long P) { return (long long)sizeof(int) * (P * (8 + kSlots) + 64 + 4); }
 QfWorkspace qf_carve(void* base, long long P) {
   QfWorkspace w;
   int* p = reinterpret_cast<int*>(base);
   w.count = p;
   w.ovf_count = p + P;
+  w.slow_count = p + P + 1;
   w.slots = p + (P + 64 + 3) / 4 * 4;  // 16-byte aligned: a position's kSlots entries are read as one int4
   w.ovf = w.slots + P * kSlots;
   w.coef = reinterpret_cast<float*>(w.ovf + P);
+  w.slow = w.ovf + 6 * P;
   return w;
 }
 
@@ -392,13 +397,43 @@ __global__ __launch_bounds__(256) void quadfit_backward_gather(const float* __re
   }
 }
 
-// sources whose list was full: float atomics, after the gather has written g1
+// Pass C, after the gather has written g1: the sources whose list was full, one lane per (source, channel), and the target
+// pixels the gather has left at zero, one wavefront per pixel, one lane per list entry and then per channel.  Both add with
+// float atomics.
 __global__ __launch_bounds__(256) void quadfit_backward_overflow(const float* __restrict__ im0, const float* __restrict__ flow,
                                                                  float* __restrict__ g1, QfWorkspace ws, int N, int d, int H,
                                                                  int W, int fc) {
   const size_t HW = (size_t)H * W;
   const long long P = (long long)N * HW;
+  const int slow = *ws.slow_count;
   const long long total = (long long)*ws.ovf_count * d;
+  const int lane = threadIdx.x & 63;
+  for (long long r = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); r < slow; r += (long long)gridDim.x * 4) {
+    const int t = __builtin_amdgcn_readfirstlane(ws.slow[r]);
+    const int n = t / (int)HW;
+    const long long base = (long long)n * HW;
+    const unsigned p = (unsigned)(t - base);
+    const int y = p / W, x = p - y * W;
+    static_assert(kSlots == 4, "four entries per list");
+    const int k = lane >> 2, e = lane & 3;  // list (tap) and entry of lanes 0..19
+    const bool has = k == 0 || (k == 1 && x > 0) || (k == 2 && x < W - 1) || (k == 3 && y > 0) || (k == 4 && y < H - 1);
+    const long long ctr = base + (long long)p + (!has ? 0 : (k == 1 ? -1 : (k == 2 ? 1 : (k == 3 ? -W : (k == 4 ? W : 0)))));
+    const bool used = has && e < min(ws.count[ctr], kSlots);
+    const unsigned sp = used ? (unsigned)ws.slots[ctr * kSlots + e] : 0u;
+    const float c = used ? ws.coef[(long long)k * P + base + sp] : 0.f;
+    const unsigned long long mask = __ballot(used);
+    for (int cc = lane; cc < d; cc += 64) {
+      const float* ac = im0 + ((size_t)n * d + cc) * HW;
+      float v[5 * kSlots];
+#pragma unroll
+      for (int j = 0; j < 5 * kSlots; j++) v[j] = ac[(unsigned)__builtin_amdgcn_readlane((int)sp, j)];  // (unused: the plane's first value)
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < 5 * kSlots; j++)
+        if ((mask >> j) & 1) acc += v[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c), j));
+      unsafeAtomicAdd(g1 + ((size_t)n * d + cc) * HW + p, acc);
+    }
+  }
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
     const int e = (int)(i / d), cc = (int)(i - (long long)e * d);  // one lane per (source, channel)
     const long long t = ws.ovf[e];
@@ -515,11 +550,12 @@ __device__ __forceinline__ void place(TilePx& s, const Box& b, int W) {
 // past the last one re-read the last one -- so that the compiler can wait for exactly the loads a step needs instead of
 // for all loads in flight; `live` is false for the surplus step of an odd channel count (the same for the whole block):
 // the consumer must neither store nor accumulate then.
-template <int PX, typename Pre, typename Consume>
-__device__ __forceinline__ void window_pass(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
+// PER: elements per thread, at least window size / 256 (window_pass below picks it per block: windows of smooth flows hold
+// 900 to 1100 elements where the capacity is 2304, and nine loads per thread and channel for four took half the time again).
+template <int PX, int PER, typename Pre, typename Consume>
+__device__ __forceinline__ void window_pass_of(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
                                             float (*win)[TileCfg<PX>::ELEMS], Pre pre, Consume consume) {
-  constexpr int kElems = TileCfg<PX>::ELEMS, kPer = kElems / 256;
-  static_assert(kElems % 256 == 0, "every thread stores the same number of window elements");
+  constexpr int kPer = PER;
   const int count = box.w * box.h;
   // window elements of this thread: e = threadIdx.x + 256 k, row e / w, column e % w (exact in float for these sizes)
   unsigned goff[kPer];
@@ -569,6 +605,16 @@ __device__ __forceinline__ void window_pass(const float* __restrict__ q, int d, 
   }
 }
 
+template <int PX, typename Pre, typename Consume>
+__device__ __forceinline__ void window_pass(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
+                                            float (*win)[TileCfg<PX>::ELEMS], Pre pre, Consume consume) {
+  static_assert(TileCfg<PX>::ELEMS == 9 * 256, "loads per thread: 4 to 9");
+  const int count = __builtin_amdgcn_readfirstlane(box.w * box.h);
+  if (count <= 4 * 256) window_pass_of<PX, 4>(q, d, HW, W, box, win, pre, consume);
+  else if (count <= 6 * 256) window_pass_of<PX, 6>(q, d, HW, W, box, win, pre, consume);
+  else window_pass_of<PX, 9>(q, d, HW, W, box, win, pre, consume);
+}
+
 // The same stream with the windows loaded from memory straight into LDS (global_load_lds: no staging registers) through a
 // ring of kDmaStages buffers: while channel c is consumed, channels c+1 and c+2 are on their way and channel c+3 is asked
 // for as soon as c has been consumed -- three channels in flight per wavefront instead of two, one barrier per channel.
@@ -578,11 +624,10 @@ __device__ __forceinline__ void window_pass(const float* __restrict__ q, int d, 
 // consumption.  No `pre` values: for consumers that need the window only.
 // The four buffers are four separate __shared__ arrays, not one: the compiler waits, before a read of LDS, for every load
 // into LDS that may alias it, and it can tell loads into different variables apart, not into parts of one.
-template <int PX, typename Consume>
-__device__ __forceinline__ void window_pass_dma(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
+template <int PX, int PER, typename Consume>
+__device__ __forceinline__ void window_pass_dma_of(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
                                                 float* w0, float* w1, float* w2, float* w3, Consume consume) {
-  constexpr int kElems = TileCfg<PX>::ELEMS, kPer = kElems / 256;
-  static_assert(kElems % 256 == 0, "every thread loads the same number of window elements");
+  constexpr int kPer = PER;
   typedef const __attribute__((address_space(1))) void* GlobalPtr;
   typedef __attribute__((address_space(3))) void* LdsPtr;
   const int count = box.w * box.h;
@@ -621,6 +666,16 @@ __device__ __forceinline__ void window_pass_dma(const float* __restrict__ q, int
   }
   // (the loads still in flight at the end target LDS: they must have landed before the workgroup's LDS is handed on)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <int PX, typename Consume>
+__device__ __forceinline__ void window_pass_dma(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
+                                                float* w0, float* w1, float* w2, float* w3, Consume consume) {
+  static_assert(TileCfg<PX>::ELEMS == 9 * 256, "loads per thread: 4 to 9");
+  const int count = __builtin_amdgcn_readfirstlane(box.w * box.h);
+  if (count <= 4 * 256) window_pass_dma_of<PX, 4>(q, d, HW, W, box, w0, w1, w2, w3, consume);
+  else if (count <= 6 * 256) window_pass_dma_of<PX, 6>(q, d, HW, W, box, w0, w1, w2, w3, consume);
+  else window_pass_dma_of<PX, 9>(q, d, HW, W, box, w0, w1, w2, w3, consume);
 }
 
 // the five taps of every inside pixel of the lane, from the window or (far pixels) from the plane
@@ -916,6 +971,136 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// The same two passes for images with too few tiles to fill the chip.  On 64 x 96 x 312 the tiled kernels are 60 blocks
+// that walk 64 channels one barrier at a time (48 us forward, 98 us pass A).  Here a block owns 64 pixels of a row and its
+// four wavefronts share the CHANNELS: a wavefront reads the taps of eight of 32 channels straight from memory -- 48 loads in
+// flight per lane -- and leaves the five products of each in LDS; then the products are summed over the channels in the
+// reference's order (QF.cu:63-71: the sum is a chain, the products are not), one tap per wavefront.  NC > 0: d <= 32 NC
+// channels, whose taps the backward pass keeps in registers for the gradient wrt the first map; NC = 0: any d, read again.
+constexpr int kSplitChunk = 32, kSplitPer = kSplitChunk / 4;
+
+template <int MODE, int NC>
+__global__ __launch_bounds__(256) void quadfit_split(const float* __restrict__ im0, const float* __restrict__ im1,
+                                                     const float* __restrict__ flow, const float* __restrict__ gin,
+                                                     float* __restrict__ res, QfWorkspace ws, int N, int d, int H, int W,
+                                                     int fc, int tiles_x, int tiles_y) {
+  __shared__ float prod[kSplitChunk][5][64];
+  __shared__ float sums[5][64];
+  int n, tx, y;
+  if (!tile_of_block(N, tiles_x, tiles_y, n, tx, y)) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t HW = (size_t)H * W;
+  const float* a = im0 + (size_t)n * d * HW;
+  const float* q = im1 + (size_t)n * d * HW;
+  const int x = tx * 64 + lane;
+  const bool valid = x < W;
+  TilePx px;
+  int unused0 = 0, unused1 = 0, unused2 = 0, unused3 = 0;
+  locate(px, flow + (size_t)n * fc * HW, HW, H, W, x, y, valid, unused0, unused1, unused2, unused3);
+  const unsigned row = (unsigned)px.iy * W;  // (a pixel that is not inside reads the plane's first value; its sums are not used)
+  const unsigned o[5] = {row + px.ix, row + px.xp, row + px.xm, (unsigned)px.yp * W + px.ix, (unsigned)px.ym * W + px.ix};
+  float tap[NC > 0 ? NC * kSplitPer : kSplitPer][5];
+  float cost[2] = {0.f, 0.f};  // this wavefront's tap; wavefront 0 also sums tap 4
+  auto chunk = [&](int c0, float (*t)[5]) {
+    float v[kSplitPer];
+#pragma unroll
+    for (int j = 0; j < kSplitPer; j++) {
+      const size_t plane = (size_t)min(c0 + wave * kSplitPer + j, d - 1) * HW;
+      v[j] = a[plane + px.p];
+#pragma unroll
+      for (int k = 0; k < 5; k++) t[j][k] = q[plane + o[k]];
+    }
+#pragma unroll
+    for (int j = 0; j < kSplitPer; j++)
+#pragma unroll
+      for (int k = 0; k < 5; k++) prod[wave * kSplitPer + j][k][lane] = v[j] * t[j][k];
+    __syncthreads();
+    const int nc = min(kSplitChunk, d - c0);
+    for (int c = 0; c < nc; c++) cost[0] += prod[c][wave][lane];
+    if (wave == 0)
+      for (int c = 0; c < nc; c++) cost[1] += prod[c][4][lane];
+  };
+  if (NC > 0) {
+#pragma unroll
+    for (int b = 0; b < NC; b++) {
+      if (b * kSplitChunk < d) {
+        if (b > 0) __syncthreads();
+        chunk(b * kSplitChunk, tap + b * kSplitPer);
+      }
+    }
+  } else {
+    for (int c0 = 0; c0 < d; c0 += kSplitChunk) {
+      if (c0 > 0) __syncthreads();
+      chunk(c0, tap);
+    }
+  }
+  sums[wave][lane] = cost[0];
+  if (wave == 0) sums[4][lane] = cost[1];
+  __syncthreads();
+  Fit f;
+  f.inside = px.inside;
+  f.validX = f.validY = 0;
+  f.c00 = f.ax = f.ay = f.bx = f.by = f.fx = f.fy = 0.f;
+  if (px.inside) finish_fit(f, sums[0][lane], sums[1][lane], sums[3][lane], sums[2][lane], sums[4][lane], px.ix, px.iy, H, W);
+  if (MODE == 0) {
+    if (wave != 0 || !valid) return;
+    float* out = res + (size_t)n * 3 * HW + px.p;
+    float score = 0.f;
+    if (f.inside)  // QF.cu:136
+      score = f.ax * f.fx * f.fx + f.bx * f.fx + f.c00 + f.ay * f.fy * f.fy + f.by * f.fy;
+    out[0] = f.fx;
+    out[HW] = f.fy;
+    out[2 * HW] = score;
+    return;
+  }
+  if (!valid) return;
+  Factors kf{};
+  if (px.inside) kf = scatter_factors(f, gin, n, HW, px.p);
+  if (wave == 0 && px.inside) {
+    const long long P = (long long)N * HW, t = (long long)n * HW + px.p;
+    ws.coef[0 * P + t] = kf.any_valid ? (float)(0.5 * kf.k00) : kf.dFds;  // QF.cu:279-283,296
+    ws.coef[1 * P + t] = kf.any_valid ? 0.5f * kf.k0p : 0.f;
+    ws.coef[2 * P + t] = kf.any_valid ? 0.5f * kf.k0m : 0.f;
+    ws.coef[3 * P + t] = kf.any_valid ? 0.5f * kf.kp0 : 0.f;
+    ws.coef[4 * P + t] = kf.any_valid ? 0.5f * kf.km0 : 0.f;
+    const long long centre = (long long)n * HW + o[0];
+    const int pos = atomicAdd(ws.count + centre, 1);
+    if (pos < kSlots) ws.slots[centre * kSlots + pos] = (int)px.p;
+    else ws.ovf[atomicAdd(ws.ovf_count, 1)] = (int)t;
+  }
+  float* G0 = res + (size_t)n * d * HW;
+  auto gradient = [&](int c0, const float (*t)[5]) {
+#pragma unroll
+    for (int j = 0; j < kSplitPer; j++) {
+      const int c = c0 + wave * kSplitPer + j;
+      if (c < d) {
+        float g = 0.f;
+        if (px.inside) {
+          if (kf.any_valid)  // QF.cu:286-290
+            g = 0.5 * (t[j][0] * kf.k00 + t[j][1] * kf.k0p + t[j][2] * kf.k0m + t[j][3] * kf.kp0 + t[j][4] * kf.km0);
+          else  // QF.cu:295
+            g = t[j][0] * kf.dFds;
+        }
+        G0[(size_t)c * HW + px.p] = g;
+      }
+    }
+  };
+  if (NC > 0) {
+#pragma unroll
+    for (int b = 0; b < NC; b++) gradient(b * kSplitChunk, tap + b * kSplitPer);
+  } else {
+    for (int c0 = 0; c0 < d; c0 += kSplitChunk) {
+#pragma unroll
+      for (int j = 0; j < kSplitPer; j++) {
+        const size_t plane = (size_t)min(c0 + wave * kSplitPer + j, d - 1) * HW;
+#pragma unroll
+        for (int k = 0; k < 5; k++) tap[j][k] = q[plane + o[k]];
+      }
+      gradient(c0, tap);
+    }
+  }
+}
+
 // Pass B of the backward pass on tiles of target pixels: the (source, coefficient) pairs of every pixel are
 // collected once; per channel the window of the FIRST feature map that covers the tile's sources is
 // staged in LDS and the pairs are summed from it.
@@ -946,7 +1131,10 @@ __device__ __forceinline__ void lds_gather12(const float* buf, const unsigned (&
 
 template <int PX>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void quadfit_gather_tiles(const float* __restrict__ im0, float* __restrict__ g1, QfWorkspace ws,
-                                                            int N, int d, int H, int W, int tiles_x, int tiles_y) {
+                                                            int N, int d_all, int per_group, int H, int W, int tiles_x, int tiles_y) {
+  // blockIdx.y: this block's group of per_group channels (launches that would leave the chip short of blocks are split by
+  // channel; every group collects the tile's pairs for itself)
+  const int d_lo = (int)blockIdx.y * per_group, d = min(per_group, d_all - d_lo);
   constexpr int kTH = TileCfg<PX>::TH;
   __shared__ float win0[TileCfg<PX>::ELEMS], win1[TileCfg<PX>::ELEMS], win2[TileCfg<PX>::ELEMS], win3[TileCfg<PX>::ELEMS];
   __shared__ int red[16];
@@ -955,8 +1143,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const size_t HW = (size_t)H * W;
   const long long P = (long long)N * HW, base = (long long)n * HW;
-  const float* a = im0 + (size_t)n * d * HW;
-  float* G1 = g1 + (size_t)n * d * HW;
+  const float* a = im0 + ((size_t)n * d_all + d_lo) * HW;
+  float* G1 = g1 + ((size_t)n * d_all + d_lo) * HW;
   const int x = tx * kTW + lane;
   const float inv_w = 1.0f / (float)W;
   bool valid[PX];
@@ -970,6 +1158,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   // unconditionally and in batches (an absent list reads the pixel's own, an unused entry coefficient 0 of the sample):
   // lengths and lists of all pixels of the lane together, then the coefficients of one pixel at a time -- three round
   // trips to memory; behind `if (cnt > 0)` / `if (s < cnt)` each read waits for the one before it, some fifty in a row.
+  static_assert(TileCfg<PX>::ELEMS >= 2 * 64 * kPairs, "a window buffer holds the pairs of 64 pixels");
+  float2* const front = reinterpret_cast<float2*>(wave == 0 ? win0 : (wave == 1 ? win1 : (wave == 2 ? win2 : win3))) + lane;
   int cnt[PX][5];
   int4 sl[PX][5];
 #pragma unroll
@@ -978,11 +1168,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     valid[i] = x < W && y < H;
     pix[i] = valid[i] ? (unsigned)y * W + x : 0u;
     np[i] = 0;
-#pragma unroll
-    for (int j = 0; j < kPairs; j++) {
-      off[i][j] = 0u;
-      cf[i][j] = 0.f;
-    }
     const bool has[5] = {valid[i], valid[i] && x > 0, valid[i] && x < W - 1, valid[i] && y > 0, valid[i] && y < H - 1};
     const int step[5] = {0, -1, 1, -W, W};
 #pragma unroll
@@ -1014,33 +1199,39 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     for (int k = 0; k < 5; k++)
 #pragma unroll
       for (int s = 0; s < kSlots; s++) asm volatile("" : "+v"(cv[k][s]));
+    // The pairs that exist, moved to the front through the wavefront's own LDS (the windows' space, still unused): a
+    // write at a running index per entry.  (As selects between registers this took twelve compares and moves for each of
+    // the twenty entries: a third of the launch.)
 #pragma unroll
     for (int k = 0; k < 5; k++) {
 #pragma unroll
       for (int s = 0; s < kSlots; s++) {
         if (s < cnt[i][k]) {
-          const unsigned sp = spv[k][s];  // (below 2^24: the float quotient is off by one at most)
-          int sy = (int)((float)sp * inv_w), sx = (int)sp - sy * W;
-          if (sx < 0) { sy--; sx += W; }
-          if (sx >= W) { sy++; sx -= W; }
-          const float c = cv[k][s];
-#pragma unroll
-          for (int j = 0; j < kPairs; j++)
-            if (np[i] == j) {
-              off[i][j] = ((unsigned)sy << 16) | (unsigned)sx;
-              cf[i][j] = c;
-            }
-          if (np[i] < kPairs) {
-            minx = min(minx, sx); maxx = max(maxx, sx);
-            miny = min(miny, sy); maxy = max(maxy, sy);
-          }
+          if (np[i] < kPairs) front[np[i] * 64] = make_float2(__uint_as_float(spv[k][s]), cv[k][s]);
           np[i]++;
         }
       }
     }
+#pragma unroll
+    for (int j = 0; j < kPairs; j++) {
+      const float2 e = front[j * 64];
+      const bool used = j < np[i];
+      const unsigned sp = used ? __float_as_uint(e.x) : 0u;  // (below 2^24: the float quotient is off by one at most)
+      int sy = (int)((float)sp * inv_w), sx = (int)sp - sy * W;
+      if (sx < 0) { sy--; sx += W; }
+      if (sx >= W) { sy++; sx -= W; }
+      off[i][j] = ((unsigned)sy << 16) | (unsigned)sx;
+      cf[i][j] = used ? e.y : 0.f;
+      if (used) {
+        minx = min(minx, sx); maxx = max(maxx, sx);
+        miny = min(miny, sy); maxy = max(maxy, sy);
+      }
+    }
   }
   const Box box = block_box(minx, maxx, miny, maxy, red, TileCfg<PX>::ELEMS);
-  // a pixel with more pairs than registers, or with a source outside the window, walks its lists from memory instead
+  // A pixel with more pairs than registers, or with a source outside the window, is left to pass C.  (It used to walk its
+  // lists here, three dependent reads per entry and channel: eighteen such pixels in 479232 made the launch 290 us instead
+  // of 200 on 4 x 32 x 384 x 1248, and 581 us of 64 x 96 x 312, where one pixel in sixty-five is one.)
   bool slow[PX];
   unsigned need = 0;
 #pragma unroll
@@ -1061,6 +1252,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       }
       if (__ballot(!slow[i] && j < np[i]) != 0) need |= 1u << j;  // pairs nobody in the wavefront has are skipped by a uniform branch
     }
+    if (blockIdx.y == 0) {
+      const bool listed = valid[i] && slow[i];
+      const unsigned long long all = __ballot(listed);
+      if (all) {
+        int at = 0;
+        if (lane == __builtin_ctzll(all)) at = atomicAdd(ws.slow_count, __popcll(all));
+        at = __builtin_amdgcn_readlane(at, __builtin_ctzll(all));
+        if (listed) ws.slow[at + __popcll(all & ((1ull << lane) - 1))] = (int)(base + pix[i]);
+      }
+    }
   }
   window_pass_dma<PX>(a, d, HW, W, box, win0, win1, win2, win3, [&](int cc, const float* buf, const float* plane, int, bool live) {
     // all window reads of a pixel are issued before the first product: a read inside the branch that skips an unused pair
@@ -1073,32 +1274,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #pragma unroll
       for (int j = 0; j < kPairs; j++)
         if (need & (1u << j)) acc = __builtin_fmaf(v[j], cf[i][j], acc);
-      if (live && valid[i] && !slow[i]) __builtin_nontemporal_store(acc, &G1[(size_t)cc * HW + pix[i]]);
+      if (live && valid[i]) __builtin_nontemporal_store(slow[i] ? 0.f : acc, &G1[(size_t)cc * HW + pix[i]]);
     }
   });
-#pragma unroll
-  for (int i = 0; i < PX; i++) {
-    if (!valid[i] || !slow[i]) continue;
-    const int y = ty * kTH + wave * PX + i;
-    long long ctr[5];
-    ctr[0] = base + pix[i];
-    ctr[1] = x > 0 ? base + pix[i] - 1 : -1;
-    ctr[2] = x < W - 1 ? base + pix[i] + 1 : -1;
-    ctr[3] = y > 0 ? base + pix[i] - W : -1;
-    ctr[4] = y < H - 1 ? base + pix[i] + W : -1;
-    for (int cc = 0; cc < d; cc++) {
-      const float* ac = a + (size_t)cc * HW;
-      float acc = 0.f;
-      for (int k = 0; k < 5; k++) {
-        const int cnt = ctr[k] >= 0 ? min(ws.count[ctr[k]], kSlots) : 0;
-        for (int s = 0; s < cnt; s++) {
-          const unsigned sp = (unsigned)ws.slots[ctr[k] * kSlots + s];
-          acc += ac[sp] * ws.coef[(long long)k * P + base + sp];
-        }
-      }
-      G1[(size_t)cc * HW + pix[i]] = acc;
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1484,6 +1662,36 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 }  // namespace
 
+namespace {
+
+// Whether the per-pixel passes of the quadratic fit take the split kernels: too few tiles (64 x 8 pixels) to fill the chip.
+bool quadfit_few_tiles(long long tiles) {
+  if (inpaint::knobs().quadfit_split >= 0) return inpaint::knobs().quadfit_split == 1;
+  return tiles < 1ll * inpaint::compute_unit_count();
+}
+
+// Channels per block of the gather pass: all of them where the tiles fill the chip (four blocks resident per CU), else so
+// few that about that many blocks result, at least the four that the ring of windows holds.
+int gather_channels_per_block(long long tiles, int ic) {
+  const long long groups = std::max<long long>(1, 4ll * inpaint::compute_unit_count() / tiles);
+  return std::max<int>(4, (int)((ic + groups - 1) / groups + 3) / 4 * 4);
+}
+
+template <int MODE>
+void launch_quadfit_split(const float* im0, const float* im1, const float* flow, const float* gin, float* res, const QfWorkspace& ws,
+                          int n, int ic, int ih, int iw, int fc, hipStream_t st) {
+  const int tx = (iw + 63) / 64;
+  const dim3 grid((unsigned)(((long long)n * tx * ih + 7) / 8 * 8)), block(256);
+  if (ic <= kSplitChunk)
+    hipLaunchKernelGGL((quadfit_split<MODE, 1>), grid, block, 0, st, im0, im1, flow, gin, res, ws, n, ic, ih, iw, fc, tx, ih);
+  else if (ic <= 2 * kSplitChunk)
+    hipLaunchKernelGGL((quadfit_split<MODE, 2>), grid, block, 0, st, im0, im1, flow, gin, res, ws, n, ic, ih, iw, fc, tx, ih);
+  else
+    hipLaunchKernelGGL((quadfit_split<MODE, 0>), grid, block, 0, st, im0, im1, flow, gin, res, ws, n, ic, ih, iw, fc, tx, ih);
+}
+
+}  // namespace
+
 extern "C" {
 
 const char* flowaux_last_error(void) { return inpaint::error_buffer(); }
@@ -1510,6 +1718,8 @@ int quadfit_forward(const float* im0, const float* im1, const float* flow, float
   if (inpaint::knobs().quadfit_px_path)
     hipLaunchKernelGGL(quadfit_forward_kernel, banded_grid(P), dim3(256), 0, (hipStream_t)stream, im0, im1, flow, out, n,
                        ic, ih, iw, flow_channels);
+  else if (quadfit_few_tiles(tiles))
+    launch_quadfit_split<0>(im0, im1, flow, nullptr, out, QfWorkspace{}, n, ic, ih, iw, flow_channels, (hipStream_t)stream);
   else
     hipLaunchKernelGGL((quadfit_tiles<0, kPxForward>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, (hipStream_t)stream, im0, im1,
                        flow, nullptr, out, QfWorkspace{}, n, ic, ih, iw, flow_channels, tiles_x, tiles_y);
@@ -1552,7 +1762,9 @@ int quadfit_backward(const float* im0, const float* im1, const float* flow, cons
     hipLaunchKernelGGL(quadfit_backward_sources, grid, block, 0, st, im0, im1, flow, gin, g0, ws, n, ic, ih, iw, flow_channels);
   else {
     if (g_timed_pass == 1) g_timer.begin(st);
-    if (ic <= kResidentChannels && !inpaint::knobs().quadfit_reread) {
+    if (quadfit_few_tiles(tiles) && !inpaint::knobs().quadfit_reread) {
+      launch_quadfit_split<1>(im0, im1, flow, gin, g0, ws, n, ic, ih, iw, flow_channels, st);
+    } else if (ic <= kResidentChannels && !inpaint::knobs().quadfit_reread) {
       const int ry = (ih + kResidentRows - 1) / kResidentRows;
       const long long rt = (long long)n * tiles_x * ry;
       const dim3 rgrid((unsigned)((rt + 7) / 8 * 8));
@@ -1574,11 +1786,12 @@ int quadfit_backward(const float* im0, const float* im1, const float* flow, cons
     const int gy = (ih + TileCfg<kPxGather>::TH - 1) / TileCfg<kPxGather>::TH;
     const long long gt = (long long)n * tiles_x * gy;
     if (g_timed_pass == 2) g_timer.begin(st);
-    hipLaunchKernelGGL((quadfit_gather_tiles<kPxGather>), dim3((unsigned)((gt + 7) / 8 * 8)), block, 0, st, im0, g1, ws, n, ic,
-                       ih, iw, tiles_x, gy);
+    const int per = gather_channels_per_block(gt, ic);
+    hipLaunchKernelGGL((quadfit_gather_tiles<kPxGather>), dim3((unsigned)((gt + 7) / 8 * 8), (unsigned)((ic + per - 1) / per)), block, 0,
+                       st, im0, g1, ws, n, ic, per, ih, iw, tiles_x, gy);
     if (g_timed_pass == 2) g_timer.end(st, 1);
   }
-  hipLaunchKernelGGL(quadfit_backward_overflow, dim3(64), block, 0, st, im0, flow, g1, ws, n, ic, ih, iw, flow_channels);
+  hipLaunchKernelGGL(quadfit_backward_overflow, dim3((unsigned)std::min<long long>((P + 127) / 128, 512)), block, 0, st, im0, flow, g1, ws, n, ic, ih, iw, flow_channels);
   INPAINT_HIP(hipGetLastError());
   return 0;
 }

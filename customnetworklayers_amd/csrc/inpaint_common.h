@@ -76,6 +76,7 @@ struct Knobs {
   bool keep_gb_set = false;       // (the variable is set: the budget is the caller's, free device memory is not consulted)
   int stats_every = 0;            // INPAINT_STATS_EVERY=N: the guard's statistics on stderr every Nth backward pass of an id (a host wait; off by default)
   bool quadfit_px_path = false;   // INPAINT_QUADFIT_PATH=px: one pixel per lane, no LDS windows
+  int quadfit_split = -1;         // INPAINT_QUADFIT_PATH=split: the kernels for few tiles whatever the size; =tiles: never (-1 = by size)
   bool median_tile_per_wave = false;  // INPAINT_MEDIAN_PATH=tile: one tile of 64 pixels per wavefront for every bin count
   bool quadfit_reread = false;    // INPAINT_QUADFIT_PATH=reread: backward pass A reads the second map twice (any channel count)
   void load() {
@@ -123,6 +124,7 @@ struct Knobs {
     if (const char* e = getenv("INPAINT_KEEP_GB")) { keep_gb = atof(e); keep_gb_set = true; }
     if (const char* e = getenv("INPAINT_STATS_EVERY")) stats_every = std::max(0, atoi(e));
     quadfit_px_path = is("INPAINT_QUADFIT_PATH", "px");
+    quadfit_split = is("INPAINT_QUADFIT_PATH", "split") ? 1 : (is("INPAINT_QUADFIT_PATH", "tiles") ? 0 : -1);
     quadfit_reread = is("INPAINT_QUADFIT_PATH", "reread");
     median_tile_per_wave = is("INPAINT_MEDIAN_PATH", "tile");
   }

@@ -116,6 +116,30 @@ def test_quadfit_backward_that_reads_the_second_map_twice(qf, flowaux_oracle, n,
     check_quadfit(qf, flowaux_oracle, workloads.quadfit_inputs(n, c, h, w, seed=42), "reread warped")
 
 
+@pytest.mark.parametrize("path", ["split", "tiles"])
+@pytest.mark.parametrize("n,c,h,w,flow", [
+    (1, 1, 1, 1, "random"),      # one pixel
+    (1, 31, 3, 65, "random"),    # one column more than a block of the split kernels, a short chunk of channels
+    (2, 33, 9, 63, "random"),    # one channel in the second chunk
+    (1, 65, 9, 70, "random"),    # more channels than the split kernels keep taps of
+    (1, 20, 40, 130, "contracting"),  # up to twenty pairs per target pixel and full lists
+    (1, 8, 17, 140, "scattered"),     # sources outside every window
+])
+def test_quadfit_few_tiles_and_many(qf, flowaux_oracle, path, n, c, h, w, flow, monkeypatch):
+    # the kernels for images with few tiles and those for many, each forced; both meet target pixels with more sources than
+    # the gather pass holds
+    monkeypatch.setenv("INPAINT_QUADFIT_PATH", path)
+    from customnetworklayers_amd._lib import reload_env
+    reload_env()
+    d = random_quadfit(n, c, h, w, seed=51 + c, fc=3, amp=40.0 if flow == "scattered" else 3.0)
+    if flow == "contracting":  # every other column and row lands on its neighbour: four sources per position, some five
+        ys, xs = np.mgrid[0:h, 0:w]
+        rng = np.random.default_rng(7)
+        d["flow"][:, 0] = -0.5 * xs + 0.3 * rng.standard_normal((h, w))
+        d["flow"][:, 1] = -0.5 * ys + 0.3 * rng.standard_normal((h, w))
+    check_quadfit(qf, flowaux_oracle, d, "%s %s %dx%dx%dx%d" % (path, flow, n, c, h, w))
+
+
 def test_quadfit_non_finite_displacements_count_as_outside(qf, flowaux_oracle):
     d = random_quadfit(1, 3, 20, 70, seed=34)
     d["flow"][0, 0, 3, 5] = np.nan
