@@ -64,6 +64,8 @@ struct Knobs {
   int tv_tile_its = -1;           //   size of the problem; rows 0 and its -1 here)
   int tv_atile_rows = 0;          // INPAINT_TV_ADJ_TILE=R,K: the same for the reverse sweep (one or two channels)
   int tv_atile_its = -1;
+  int tgv_tile_rows = 0;          // INPAINT_TGV_TILE=rows,K: forward tiles of so many rows (12, 32, 40 or 80), K iterations per launch; =0: no tiles
+  int tgv_tile_its = -1;
   bool tgv_px_path = false;       // INPAINT_TGV_PATH=px: the per-pixel kernels
   bool tgv_fuse = true;           // INPAINT_TGV_FUSE=0
   bool tgv_fuse_adj = true;       // INPAINT_TGV_FUSE_ADJ=0
@@ -109,6 +111,7 @@ struct Knobs {
     };
     tile("INPAINT_TV_TILE", tv_tile_rows, tv_tile_its);
     tile("INPAINT_TV_ADJ_TILE", tv_atile_rows, tv_atile_its);
+    tile("INPAINT_TGV_TILE", tgv_tile_rows, tgv_tile_its);
     tgv_px_path = is("INPAINT_TGV_PATH", "px");
     tgv_fuse = !is("INPAINT_TGV_FUSE", "0");
     tgv_fuse_adj = !is("INPAINT_TGV_FUSE_ADJ", "0");

@@ -17,6 +17,7 @@
 // from the sources) is taken as 1.0f / sqrtf(x), both correctly rounded.
 #include "inpaint_common.h"
 #include "tgv_strip_kernels.h"
+#include "tgv_tile_kernels.h"
 #include "../../include/tgvinpaint.h"
 
 #include <cstddef>
@@ -772,6 +773,81 @@ void launch_forward_pair(const Slot& s, hipStream_t stream, const float* c, cons
   }
 }
 
+// Iterations in register tiles (tgv_tile_kernels.h): tiles of `rows` rows, halo included, K iterations per launch; rows = 0:
+// strips.  The four tiles there are: rows per wavefront x wavefronts.
+struct TilePlan {
+  int rows = 0, K = 0;
+};
+struct TileShape {
+  int R, waves;
+  int resident;   // workgroups a CU holds
+  int least;      // fewest iterations per launch (unless the pass has fewer)
+  double ns;      // per iteration, row and wavefront of a full SIMD
+};
+constexpr TileShape kTiles[] = {{3, 4, 5, 3, 40}, {4, 8, 2, 5, 100}, {5, 8, 2, 5, 95}, {5, 16, 1, 6, 116}};
+
+// Tiles or strips, and which tile: the cheapest by a cost model fitted to 570 measured forward passes (17 shapes from 1 x 1 x
+// 61 x 97 to 4 x 2 x 384 x 1248, all four tiles, 2 to 12 iterations per launch; 7% rms).  A tile launch costs 2.2 us and
+// 0.34 us per row of a SIMD's wavefronts for its loads; an iteration costs each of a tile's rows (and 0.45 of a row for the
+// triangles above) 297 ns on a SIMD that holds few wavefronts and `ns` per wavefront where that is more; keeping x05
+// states adds 1.8 us per iteration and million values.  A strip launch costs 5.1 us and 13.1 us per million values, for two
+// iterations.  The choice is within 2% of the best tile in the mean, 12% at most.  Few iterations per launch on the taller tiles
+// look better to the model than they measure, hence `least`.
+// Measured, forward pass, strips -> tiles, without and with x05 states: 1 x 1 x 61 x 97, 30 iterations 109 -> 78, 100 -> 87
+// us; 50 iterations of 1 x 2 x 112 x 256 163 -> 121, 167 -> 133; 1 x 2 x 187 x 621 (48) 222 -> 141, 233 -> 163; 1 x 2 x 375 x
+// 1241 446 -> 304, 435 -> 368 (397 chosen); 4 x 2 x 384 x 1248 1432 -> 993 (1040 chosen), 1538 -> 1307 (1374 chosen).
+TilePlan forward_tile_plan(const Slot& s, bool keeps_rows) {
+  TilePlan p;
+  if (!forward_pairs(s) || knobs().tgv_fwd_rows > 0 || knobs().tgv_fwd_split >= 0) return p;  // (a forced strip shape)
+  if (knobs().tgv_tile_its >= 0) {
+    p.rows = knobs().tgv_tile_rows;
+    p.K = knobs().tgv_tile_its;
+    bool known = false;
+    for (const TileShape& t : kTiles) known |= p.rows == t.R * t.waves;
+    if (!known || p.K < 2 || p.K > tgvtile::kMaxFwdSteps || p.rows <= 2 * p.K) p = TilePlan();
+    return p;
+  }
+  const int K = 2 * (s.its / 2), cus = compute_unit_count();
+  const double mega = 1e-6 * s.n * s.ic * (double)s.ih * s.iw;
+  double best = (5.1 + 13.1 * mega) / 2;  // us per iteration
+  for (const TileShape& t : kTiles) {
+    for (int k = std::min(t.least, K); k <= tgvtile::kMaxFwdSteps && 2 * k < t.R * t.waves - 1; k++) {
+      const int launches = (K + k - 1) / k;
+      if ((K + launches - 1) / launches != k) continue;  // (the same launches as a smaller k)
+      const int cols = 64 - 2 * k, rows = t.R * t.waves - 2 * k;
+      const long long tiles = (long long)((s.iw + cols - 1) / cols) * ((s.ih + rows - 1) / rows) * s.n * s.ic;
+      const long long on_cu = (tiles + cus - 1) / cus, full = on_cu / t.resident, rest = on_cu % t.resident;
+      auto round = [&](long long groups) { return groups ? std::max(297., t.ns * groups * t.waves / 4) * (t.R + 0.45) : 0.; };
+      double us = (2.2 + 0.338 * on_cu * t.R * t.waves / 4) / k + (full * round(t.resident) + round(rest)) / 1000.;
+      if (keeps_rows) us += 1.8 * mega;
+      if (us < best) { best = us; p.rows = t.R * t.waves; p.K = k; }
+    }
+  }
+  return p;
+}
+
+template <int R, int WAVES>
+void launch_forward_tile(const Slot& s, hipStream_t stream, const float* c, const float* b, const float* xin, const float* yin,
+                         const tgvtile::FwdSteps& steps, int K, bool ring, float tP, float* keep_x, float* keep_y, bool keeps_rows) {
+  auto kern = keeps_rows ? tgvtile::tgv_forward_tile<R, WAVES, true> : tgvtile::tgv_forward_tile<R, WAVES, false>;
+  const int cols = 64 - 2 * K, trows = R * WAVES - 2 * K;
+  const int tx = (s.iw + cols - 1) / cols, ty = (s.ih + trows - 1) / trows;
+  const long long tiles = (long long)tx * ty * s.n * s.ic;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(64 * WAVES), 0, stream, s.wx, s.wy, s.bx, s.by, c, b, xin,
+                     yin, steps, K, ring ? 1 : 0, tP, keep_x, keep_y, s.n, s.ic, s.ih, s.iw, tx, ty);
+}
+
+void launch_forward_tiles(const Slot& s, hipStream_t stream, int rows, const float* c, const float* b, const float* xin,
+                          const float* yin, const tgvtile::FwdSteps& steps, int K, bool ring, float tP, float* keep_x,
+                          float* keep_y, bool keeps_rows) {
+  switch (rows) {
+    case 12: launch_forward_tile<3, 4>(s, stream, c, b, xin, yin, steps, K, ring, tP, keep_x, keep_y, keeps_rows); break;
+    case 32: launch_forward_tile<4, 8>(s, stream, c, b, xin, yin, steps, K, ring, tP, keep_x, keep_y, keeps_rows); break;
+    case 40: launch_forward_tile<5, 8>(s, stream, c, b, xin, yin, steps, K, ring, tP, keep_x, keep_y, keeps_rows); break;
+    default: launch_forward_tile<5, 16>(s, stream, c, b, xin, yin, steps, K, ring, tP, keep_x, keep_y, keeps_rows); break;
+  }
+}
+
 // One group of a one-step adjoint launch.  Shared accumulators: set acc_cur in, the other out, flipped by the caller
 // after every launch; the per-channel accumulator gb: set accb_cur in, the other out, flipped once per step.
 template <int C, bool END, int ADJ, bool FIRST = false>
@@ -984,7 +1060,47 @@ int tgvinpaint_forward(const float* dx, const float* dy, const float* c, const f
     // first iteration whose x05 row is kept, and the ring row of iteration k
     const int kl = s.iterations.empty() ? K : (keep == 2 ? 0 : (keep == 1 ? s.iterations.back() : K));
     auto ring_row = [&](int k) { return s.x05 + (size_t)(keep == 2 ? k : k - kl) * S3; };
-    if (forward_pairs(s)) {
+    const TilePlan tile = forward_tile_plan(s, keep == 2);
+    if (tile.rows > 0) {
+      // up to tile.K iterations per launch.  What an iteration leaves in memory: its x05 state where it is kept; the half (or
+      // both halves) of a checkpoint; the result; and at the end of a launch the iterate, unless the next launch rebuilds
+      // it from the x05 states (keep mode 2).
+      const int launches = (K + tile.K - 1) / tile.K, per = (K + launches - 1) / launches;
+      for (int k = 0, li = 0; k < K; li++) {
+        const int len = std::min(per, K - k);
+        tgvtile::FwdSteps st{};
+        for (int j = 0; j < len; j++) {
+          const int next = k + j + 1, ck = next < K ? ck_index(next) : -1;
+          const bool hand_on = j == len - 1 && next < K && keep != 2;
+          tgvtile::FwdStep& f = st.step[j];
+          f.t = s.steps[k + j];
+          f.x05 = k + j >= kl ? ring_row(k + j) : nullptr;
+          if (ck >= 0) {
+            if (keep != 2 || want_y) f.y = s.ckpt_y + (size_t)ck * S3;
+            if (keep != 2 || want_x) f.x = s.ckpt_x + (size_t)ck * S3;
+          } else if (hand_on) {
+            f.y = s.ypp[li & 1];
+            f.x = s.xpp[li & 1];
+          }
+          if (next == K) f.x = out;
+        }
+        const bool rows = k + len > kl;
+        if (k == 0 && copy_in_pair) {
+          launch_forward_tiles(s, stream, tile.rows, c, b, init, init, st, len, false, 0.f, (keep != 2 || want_x) ? s.ckpt_x : nullptr,
+                               s.ckpt_y, rows);
+        } else if (k == 0) {
+          launch_forward_tiles(s, stream, tile.rows, c, b, s.ckpt_x, s.ckpt_y, st, len, false, 0.f, nullptr, nullptr, rows);
+        } else if (keep == 2) {
+          launch_forward_tiles(s, stream, tile.rows, c, b, ring_row(k - 2), ring_row(k - 1), st, len, true, s.steps[k - 1], nullptr,
+                               nullptr, rows);
+        } else {
+          const int ck = ck_index(k);
+          launch_forward_tiles(s, stream, tile.rows, c, b, ck >= 0 ? s.ckpt_x + (size_t)ck * S3 : s.xpp[(li & 1) ^ 1],
+                               ck >= 0 ? s.ckpt_y + (size_t)ck * S3 : s.ypp[(li & 1) ^ 1], st, len, false, 0.f, nullptr, nullptr, rows);
+        }
+        k += len;
+      }
+    } else if (forward_pairs(s)) {
       // two iterations per launch; K and every checkpoint index are even, the ping-pong alternates per pair
       auto Yp = [&](int k) { int i = ck_index(k); return (i >= 0 && k < K) ? s.ckpt_y + (size_t)i * S3 : s.ypp[(k >> 1) & 1]; };
       auto Xp = [&](int k) {
