@@ -407,8 +407,8 @@ __global__ __launch_bounds__(256) void quadfit_backward_overflow(const float* __
   const long long P = (long long)N * HW;
   const int slow = *ws.slow_count;
   const long long total = (long long)*ws.ovf_count * d;
-  const int lane = threadIdx.x & 63;
-  for (long long r = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); r < slow; r += (long long)gridDim.x * 4) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (long long r = (long long)blockIdx.x * 4 + wave; r < slow; r += (long long)gridDim.x * 4) {
     const int t = __builtin_amdgcn_readfirstlane(ws.slow[r]);
     const int n = t / (int)HW;
     const long long base = (long long)n * HW;
@@ -422,7 +422,9 @@ __global__ __launch_bounds__(256) void quadfit_backward_overflow(const float* __
     const unsigned sp = used ? (unsigned)ws.slots[ctr * kSlots + e] : 0u;
     const float c = used ? ws.coef[(long long)k * P + base + sp] : 0.f;
     const unsigned long long mask = __ballot(used);
-    for (int cc = lane; cc < d; cc += 64) {
+    // (all lanes stay in this loop, the ones past the last channel on that channel: lanes 0..19 hold the entries the others read)
+    for (int c0 = 0; c0 < d; c0 += 64) {
+      const int cc = min(c0 + lane, d - 1);
       const float* ac = im0 + ((size_t)n * d + cc) * HW;
       float v[5 * kSlots];
 #pragma unroll
@@ -431,7 +433,7 @@ __global__ __launch_bounds__(256) void quadfit_backward_overflow(const float* __
 #pragma unroll
       for (int j = 0; j < 5 * kSlots; j++)
         if ((mask >> j) & 1) acc += v[j] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c), j));
-      unsafeAtomicAdd(g1 + ((size_t)n * d + cc) * HW + p, acc);
+      if (c0 + lane < d) unsafeAtomicAdd(g1 + ((size_t)n * d + cc) * HW + p, acc);
     }
   }
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {

@@ -116,6 +116,15 @@ def test_quadfit_backward_that_reads_the_second_map_twice(qf, flowaux_oracle, n,
     check_quadfit(qf, flowaux_oracle, workloads.quadfit_inputs(n, c, h, w, seed=42), "reread warped")
 
 
+def contract(d):
+    """A flow under which every other column and row lands on its neighbour: four sources per position, some five."""
+    h, w = d["flow"].shape[2:]
+    ys, xs = np.mgrid[0:h, 0:w]
+    rng = np.random.default_rng(7)
+    d["flow"][:, 0] = -0.5 * xs + 0.3 * rng.standard_normal((h, w))
+    d["flow"][:, 1] = -0.5 * ys + 0.3 * rng.standard_normal((h, w))
+
+
 @pytest.mark.parametrize("path", ["split", "tiles"])
 @pytest.mark.parametrize("n,c,h,w,flow", [
     (1, 1, 1, 1, "random"),      # one pixel
@@ -132,12 +141,22 @@ def test_quadfit_few_tiles_and_many(qf, flowaux_oracle, path, n, c, h, w, flow, 
     from customnetworklayers_amd._lib import reload_env
     reload_env()
     d = random_quadfit(n, c, h, w, seed=51 + c, fc=3, amp=40.0 if flow == "scattered" else 3.0)
-    if flow == "contracting":  # every other column and row lands on its neighbour: four sources per position, some five
-        ys, xs = np.mgrid[0:h, 0:w]
-        rng = np.random.default_rng(7)
-        d["flow"][:, 0] = -0.5 * xs + 0.3 * rng.standard_normal((h, w))
-        d["flow"][:, 1] = -0.5 * ys + 0.3 * rng.standard_normal((h, w))
+    if flow == "contracting":
+        contract(d)
     check_quadfit(qf, flowaux_oracle, d, "%s %s %dx%dx%dx%d" % (path, flow, n, c, h, w))
+
+
+@pytest.mark.parametrize("path", ["split", "tiles"])
+@pytest.mark.parametrize("c", [1, 8, 19, 21, 64, 65, 84, 130])
+def test_quadfit_target_pixels_with_many_sources(qf, flowaux_oracle, path, c, monkeypatch):
+    # the pass that works off the target pixels the gather leaves out: fewer channels than a pixel has list entries (20), whole
+    # wavefronts of channels, and last trips with fewer channels than entries
+    monkeypatch.setenv("INPAINT_QUADFIT_PATH", path)
+    from customnetworklayers_amd._lib import reload_env
+    reload_env()
+    d = random_quadfit(1, c, 40, 130, seed=71 + c, fc=2)
+    contract(d)
+    check_quadfit(qf, flowaux_oracle, d, "%s contracting, %d channels" % (path, c))
 
 
 def test_quadfit_non_finite_displacements_count_as_outside(qf, flowaux_oracle):
