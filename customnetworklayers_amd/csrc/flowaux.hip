@@ -398,23 +398,31 @@ __global__ __launch_bounds__(256) void quadfit_backward_gather(const float* __re
 }
 
 // Pass C, after the gather has written g1: the sources whose list was full, one lane per (source, channel), and the target
-// pixels the gather has left at zero, one wavefront per pixel, one lane per list entry and then per channel.  Both add with
-// float atomics.
-__global__ __launch_bounds__(256) void quadfit_backward_overflow(const float* __restrict__ im0, const float* __restrict__ flow,
-                                                                 float* __restrict__ g1, QfWorkspace ws, int N, int d, int H,
-                                                                 int W, int fc) {
+// pixels the gather has left at zero.  Both add with float atomics.
+// Few such pixels -- up to 64 values to write per wavefront of the launch: one wavefront per pixel, one lane per list entry and
+// then per channel, so that all reads of a pixel are in flight at once; every read touches as many cache lines as there are
+// channels.
+// Many: one lane per pixel.  A wavefront takes 64 that follow each other in the list (the gather lists a row's pixels
+// together, so their sources are neighbours too) and a share of the channels, as small a share as gives every wavefront work;
+// each lane collects its pairs in LDS and sums four channels at a time.  Bound by the reads of the first map either way.
+// Backward pass, us, wavefront per pixel / lane per pixel (/ walked inside the gather, one lane per pixel and all channels):
+// 1 x 8 x 448 x 1000, a flow that scatters every tile 655 / 316 (/ 350); one that contracts by two 310 / 193 (/ 406);
+// 542 such pixels in the image 75 / 95 (/ 116), some 4500 92 / 97 (/ 158); 2 x 64 x 192 x 624, some 4500 of them 279 / 262
+// (/ 1076); 4 x 32 x 384 x 1248, 19384 of them 715 / 683 (/ 1436).
+constexpr int kEntries = 5 * kSlots, kQuad = 4;  // list entries a pixel can have, channels (and entries) in flight
+static_assert(kSlots == 4 && kEntries % kQuad == 0, "four entries per list");
+
+// (first: this wavefront's number in the launch of `waves`)
+__device__ __forceinline__ void add_one_pixel_per_wavefront(const float* __restrict__ im0, float* __restrict__ g1, const QfWorkspace& ws,
+                                                            int slow, int first, int waves, long long P, int d, int H, int W) {
   const size_t HW = (size_t)H * W;
-  const long long P = (long long)N * HW;
-  const int slow = *ws.slow_count;
-  const long long total = (long long)*ws.ovf_count * d;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (long long r = (long long)blockIdx.x * 4 + wave; r < slow; r += (long long)gridDim.x * 4) {
+  const int lane = threadIdx.x & 63;
+  for (int r = first; r < slow; r += waves) {
     const int t = __builtin_amdgcn_readfirstlane(ws.slow[r]);
     const int n = t / (int)HW;
     const long long base = (long long)n * HW;
     const unsigned p = (unsigned)(t - base);
     const int y = p / W, x = p - y * W;
-    static_assert(kSlots == 4, "four entries per list");
     const int k = lane >> 2, e = lane & 3;  // list (tap) and entry of lanes 0..19
     const bool has = k == 0 || (k == 1 && x > 0) || (k == 2 && x < W - 1) || (k == 3 && y > 0) || (k == 4 && y < H - 1);
     const long long ctr = base + (long long)p + (!has ? 0 : (k == 1 ? -1 : (k == 2 ? 1 : (k == 3 ? -W : (k == 4 ? W : 0)))));
@@ -436,6 +444,95 @@ __global__ __launch_bounds__(256) void quadfit_backward_overflow(const float* __
       if (c0 + lane < d) unsafeAtomicAdd(g1 + ((size_t)n * d + cc) * HW + p, acc);
     }
   }
+}
+
+__device__ __forceinline__ void add_one_pixel_per_lane(const float* __restrict__ im0, float* __restrict__ g1, const QfWorkspace& ws,
+                                                       float2 (*front)[64], int slow, int first, int waves, long long P, int d, int H,
+                                                       int W) {
+  const size_t HW = (size_t)H * W;
+  const int lane = threadIdx.x & 63;
+  const int groups = (int)((slow + 63ll) / 64), quads = (d + kQuad - 1) / kQuad;
+  const int shares = min(quads, max(1, waves / groups)), per = (quads + shares - 1) / shares;  // quads of channels per item
+  const long long items = (long long)groups * ((quads + per - 1) / per);
+  for (long long item = first; item < items; item += waves) {
+    const int share = (int)(item / groups), r = (int)(item - (long long)share * groups) * 64 + lane;
+    const bool live = r < slow;
+    const int t = ws.slow[min(r, slow - 1)];
+    const int n = t / (int)HW;
+    const long long base = (long long)n * HW;
+    const unsigned p = (unsigned)(t - base);
+    const int y = p / W, x = p - y * W;
+    const bool has[5] = {live, live && x > 0, live && x < W - 1, live && y > 0, live && y < H - 1};
+    const int step[5] = {0, -1, 1, -W, W};
+    int cnt[5];
+    int4 sl[5];
+#pragma unroll
+    for (int k = 0; k < 5; k++) {  // (an absent list reads the pixel's own)
+      const long long ctr = base + (long long)p + (has[k] ? step[k] : 0);
+      cnt[k] = ws.count[ctr];
+      sl[k] = *reinterpret_cast<const int4*>(ws.slots + ctr * kSlots);
+    }
+    float cv[5][kSlots];
+    unsigned spv[5][kSlots];
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+      cnt[k] = has[k] ? min(cnt[k], kSlots) : 0;
+      const int e[kSlots] = {sl[k].x, sl[k].y, sl[k].z, sl[k].w};
+#pragma unroll
+      for (int s = 0; s < kSlots; s++) {
+        spv[k][s] = s < cnt[k] ? (unsigned)e[s] : 0u;  // (an entry nobody filled: source 0, not used)
+        cv[k][s] = ws.coef[(long long)k * P + base + spv[k][s]];
+      }
+    }
+    // (computed here: all coefficients in one batch of loads, not each behind the branch of its entry)
+#pragma unroll
+    for (int k = 0; k < 5; k++)
+#pragma unroll
+      for (int s = 0; s < kSlots; s++) asm volatile("" : "+v"(cv[k][s]));
+    int np = 0;
+#pragma unroll
+    for (int k = 0; k < 5; k++)
+#pragma unroll
+      for (int s = 0; s < kSlots; s++)
+        if (s < cnt[k]) front[np++][lane] = make_float2(__uint_as_float(spv[k][s]), cv[k][s]);
+    const float* a = im0 + (size_t)n * d * HW;
+    float* G1 = g1 + (size_t)n * d * HW + p;
+    for (int c0 = share * per * kQuad; c0 < min((share + 1) * per * kQuad, d); c0 += kQuad) {
+      float acc[kQuad] = {0.f, 0.f, 0.f, 0.f};
+      for (int j0 = 0; __ballot(j0 < np) != 0; j0 += kQuad) {
+        float2 e[kQuad];
+        float v[kQuad][kQuad];
+#pragma unroll
+        for (int j = 0; j < kQuad; j++) e[j] = front[j0 + j][lane];
+#pragma unroll
+        for (int j = 0; j < kQuad; j++) {
+          const unsigned sp = j0 + j < np ? __float_as_uint(e[j].x) : 0u;  // (past a pixel's last entry: the plane's first value, not used)
+#pragma unroll
+          for (int q = 0; q < kQuad; q++) v[q][j] = a[(size_t)min(c0 + q, d - 1) * HW + sp];
+        }
+#pragma unroll
+        for (int j = 0; j < kQuad; j++)
+#pragma unroll
+          for (int q = 0; q < kQuad; q++) acc[q] = j0 + j < np ? acc[q] + v[q][j] * e[j].y : acc[q];
+      }
+#pragma unroll
+      for (int q = 0; q < kQuad; q++)
+        if (live && c0 + q < d) unsafeAtomicAdd(G1 + (size_t)(c0 + q) * HW, acc[q]);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void quadfit_backward_overflow(const float* __restrict__ im0, const float* __restrict__ flow,
+                                                                 float* __restrict__ g1, QfWorkspace ws, int N, int d, int H,
+                                                                 int W, int fc) {
+  __shared__ float2 front[4][kEntries][64];
+  const size_t HW = (size_t)H * W;
+  const long long P = (long long)N * HW;
+  const int slow = *ws.slow_count;
+  const long long total = (long long)*ws.ovf_count * d;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), first = (int)blockIdx.x * 4 + wave, waves = (int)gridDim.x * 4;
+  if ((long long)slow * d > 64ll * waves) add_one_pixel_per_lane(im0, g1, ws, front[wave], slow, first, waves, P, d, H, W);
+  else add_one_pixel_per_wavefront(im0, g1, ws, slow, first, waves, P, d, H, W);
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
     const int e = (int)(i / d), cc = (int)(i - (long long)e * d);  // one lane per (source, channel)
     const long long t = ws.ovf[e];

@@ -146,17 +146,23 @@ def test_quadfit_few_tiles_and_many(qf, flowaux_oracle, path, n, c, h, w, flow, 
     check_quadfit(qf, flowaux_oracle, d, "%s %s %dx%dx%dx%d" % (path, flow, n, c, h, w))
 
 
+@pytest.mark.parametrize("where", ["everywhere", "corner"])
 @pytest.mark.parametrize("path", ["split", "tiles"])
-@pytest.mark.parametrize("c", [1, 8, 19, 21, 64, 65, 84, 130])
-def test_quadfit_target_pixels_with_many_sources(qf, flowaux_oracle, path, c, monkeypatch):
+@pytest.mark.parametrize("c", [1, 9, 19, 21, 64, 65, 84, 130])
+def test_quadfit_target_pixels_with_many_sources(qf, flowaux_oracle, path, c, where, monkeypatch):
     # the pass that works off the target pixels the gather leaves out: fewer channels than a pixel has list entries (20), whole
-    # wavefronts of channels, and last trips with fewer channels than entries
+    # wavefronts of channels, and last trips with fewer channels than entries; a quarter of all pixels (one lane each from nine channels on), or those
+    # of a corner (one wavefront each)
     monkeypatch.setenv("INPAINT_QUADFIT_PATH", path)
     from customnetworklayers_amd._lib import reload_env
     reload_env()
     d = random_quadfit(1, c, 40, 130, seed=71 + c, fc=2)
+    still = d["flow"].copy()
     contract(d)
-    check_quadfit(qf, flowaux_oracle, d, "%s contracting, %d channels" % (path, c))
+    if where == "corner":
+        d["flow"][:, :, 16:] = still[:, :, 16:]
+        d["flow"][..., 16:] = still[..., 16:]
+    check_quadfit(qf, flowaux_oracle, d, "%s contracting %s, %d channels" % (path, where, c))
 
 
 def test_quadfit_non_finite_displacements_count_as_outside(qf, flowaux_oracle):
