@@ -1763,10 +1763,17 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 namespace {
 
-// Whether the per-pixel passes of the quadratic fit take the split kernels: too few tiles (64 x 8 pixels) to fill the chip.
-bool quadfit_few_tiles(long long tiles) {
+// Whether the per-pixel passes of the quadratic fit take the split kernels: too few tiles (64 x 8 pixels) to fill the chip.  The
+// split kernels work through whole chunks of 32 channels, so with fewer channels they pay up to fewer tiles only.  Measured, us,
+// split / tiled kernel, forward pass: 4 channels 6 tiles 6.0 / 7.2, 60 8.3 / 7.2; 8 channels 60 tiles 8.0 / 9.1, 104 12.2 / 9.5,
+// 248 23.5 / 10.2; 16 channels 104 tiles 12.1 / 13.4, 160 16.4 / 15.6; 20 channels 160 tiles 16.7 / 19.4, 192 19.7 / 16.8; 24
+// channels 248 tiles 23.0 / 24.7, 320 31.7 / 31.2; 32 channels 248 tiles 25.7 / 33.4; 64 channels 60 tiles 13.3 / 44.1, 248 44.9 /
+// 62.4; 65 channels (taps no longer kept in registers) 248 tiles 64.7 / 63.4; 128 channels 248 tiles 85 / 118.  Backward pass: the
+// lines cross at the same numbers of tiles up to 32 channels; 248 tiles: 64 channels 106 / 202, 65 176 / 203, 128 269 / 391.
+bool quadfit_few_tiles(long long tiles, int ic) {
   if (inpaint::knobs().quadfit_split >= 0) return inpaint::knobs().quadfit_split == 1;
-  return tiles < 1ll * inpaint::compute_unit_count();
+  const long long cus = inpaint::compute_unit_count();
+  return tiles <= (ic >= 24 ? cus - 1 : cus * ic / kSplitChunk);
 }
 
 // Channels per block of the gather pass: all of them where the tiles fill the chip (four blocks resident per CU), else so
@@ -1817,7 +1824,7 @@ int quadfit_forward(const float* im0, const float* im1, const float* flow, float
   if (inpaint::knobs().quadfit_px_path)
     hipLaunchKernelGGL(quadfit_forward_kernel, banded_grid(P), dim3(256), 0, (hipStream_t)stream, im0, im1, flow, out, n,
                        ic, ih, iw, flow_channels);
-  else if (quadfit_few_tiles(tiles))
+  else if (quadfit_few_tiles(tiles, ic))
     launch_quadfit_split<0>(im0, im1, flow, nullptr, out, QfWorkspace{}, n, ic, ih, iw, flow_channels, (hipStream_t)stream);
   else
     hipLaunchKernelGGL((quadfit_tiles<0, kPxForward>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, (hipStream_t)stream, im0, im1,
@@ -1861,7 +1868,7 @@ int quadfit_backward(const float* im0, const float* im1, const float* flow, cons
     hipLaunchKernelGGL(quadfit_backward_sources, grid, block, 0, st, im0, im1, flow, gin, g0, ws, n, ic, ih, iw, flow_channels);
   else {
     if (g_timed_pass == 1) g_timer.begin(st);
-    if (quadfit_few_tiles(tiles) && !inpaint::knobs().quadfit_reread) {
+    if (quadfit_few_tiles(tiles, ic) && !inpaint::knobs().quadfit_reread) {
       launch_quadfit_split<1>(im0, im1, flow, gin, g0, ws, n, ic, ih, iw, flow_channels, st);
     } else if (ic <= kResidentChannels && !inpaint::knobs().quadfit_reread) {
       const int ry = (ih + kResidentRows - 1) / kResidentRows;
