@@ -490,6 +490,9 @@ def bench_layer(config, steps, warmup, corrected=False, keep=None, detail=True):
     bpp = algorithmic_bytes_per_pixel(c, cfg["kind"])
     kernel_ms = tot_ms.value / max(launches.value, 1)
     steps_per_launch = 1 if kernel_name.split("<")[0].endswith("_strip") else 2  # the pair kernels run two adjoint steps
+    if cfg["kind"] == "tv" and keep in (None, 2) and launches.value and lib.tvinpaint_adjoint_tile_steps(n, c, h, w, its):
+        kernel_name = "tvtile::tv_adjoint_tile<%d,4,4,%s>" % (c, "true" if corrected else "false")
+        steps_per_launch = round((2 * (its // 2) - 1) * min(steps, 5) / launches.value, 2)
     cnt = load_counters(config) if not corrected and keep is None else None  # the counters were read on the default path
     kernel_bytes = steps_per_launch * bpp["adjoint"] * n * h * w
     model_gbs = bpp["total"] * pxit / sec / 1e9

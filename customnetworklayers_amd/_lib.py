@@ -38,6 +38,7 @@ def _load():
     lib.tvinpaint_guard_decide.argtypes = [_int, ctypes.c_double, ctypes.c_double,
                                            ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_double)]
     lib.tvinpaint_profile.argtypes = [_int]
+    lib.tvinpaint_adjoint_tile_steps.argtypes = [_int] * 5
     lib.tvinpaint_profile_read.argtypes = [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_int)]
     lib.inpaint_selftest_math.argtypes = [ctypes.POINTER(ctypes.c_ulonglong), ctypes.c_uint]
     lib.inpaint_selftest_division_pairs.argtypes = [ctypes.c_uint, ctypes.c_uint, ctypes.POINTER(ctypes.c_ulonglong)]

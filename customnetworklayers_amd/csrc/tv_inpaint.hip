@@ -792,9 +792,10 @@ int adjoint_sweep_tiles(Slot& s, hipStream_t stream, const TilePlan& plan, const
       if (s.iterations[i] == k) return (int)i;
     return -1;
   };
-  int src = 1, acc = 0;
+  int src = 1, acc = 0, launched = 0;
   bool fresh = true;  // the accumulators start at zero
-  for (int done = 0; done < steps_all;) {
+  g_timer.begin(stream);
+  for (int done = 0; done < steps_all; launched++) {
     const int len = std::min(per, steps_all - done), k_first = K - 2 - done;
     const bool first = done == 0, last = done + len == steps_all;
     tvtile::AdjSteps st{};
@@ -827,6 +828,7 @@ int adjoint_sweep_tiles(Slot& s, hipStream_t stream, const TilePlan& plan, const
     fresh = ended;
     done += len;
   }
+  g_timer.end(stream, launched);  // one event pair around the sweep's launches
   return src;
 }
 
@@ -1460,6 +1462,13 @@ int tvinpaint_profile(int enable) {
 }
 
 int tvinpaint_profile_read(double* total_ms, int* launches) { return g_timer.read(total_ms, launches); }
+
+int tvinpaint_adjoint_tile_steps(int n, int ic, int ih, int iw, int its) {
+  if (check_common(nullptr, 0, n, ic, ih, iw, its, 0) || its < 2) return 0;
+  Slot s;  // shape only, as in tvinpaint_forward_noalloc
+  s.n = n; s.ic = ic; s.ih = ih; s.iw = iw; s.its = its;
+  return adjoint_tile_plan(s).K;
+}
 
 const char* tvinpaint_last_error(void) { return error_buffer(); }
 

@@ -22,10 +22,15 @@ int tvinpaint_selftest_guard(const void* values, long long n, int is_f32, int ru
                              double* result7);
 
 /* Timing of the main adjoint kernel (the dominant one) with HIP events recorded on the launch
- * stream around every launch.  profile(1) starts collecting, profile_read waits for the recorded
- * events, returns their summed duration and count and clears the collection. */
+ * stream around every run of its launches.  profile(1) starts collecting, profile_read waits for the recorded
+ * events, returns their summed duration and the number of launches and clears the collection.  The kernel is the strip
+ * kernel of inner steps, or the register-tile kernel where the reverse sweep runs in tiles. */
 int tvinpaint_profile(int enable);
 int tvinpaint_profile_read(double* total_ms, int* launches);
+
+/* The most reverse-sweep steps one register-tile launch takes in the backward pass of such a problem, when its forward pass
+ * kept every x05 row; 0: the sweep runs in strips (or the shape is refused). */
+int tvinpaint_adjoint_tile_steps(int n, int ic, int ih, int iw, int its);
 
 /* Compares the library's cheap correctly-rounded division / square root with the
  * compiler's IEEE expansions on the GPU (exhaustively over single floats, on `pair_rounds` hashed

@@ -35,7 +35,8 @@ def check(ext, oracle, d, its, pid, **forward):
         np.testing.assert_array_equal(a.cpu().numpy(), r)
 
 
-@pytest.mark.parametrize("fwd,adj", [("4,2", "4,1"), ("4,5", "4,3"), ("4,7", "4,7"), ("8,6", "4,5"), ("16,12", "4,6")])
+@pytest.mark.parametrize("fwd,adj", [("4,2", "4,1"), ("4,5", "4,3"), ("4,7", "4,7"), ("8,6", "4,5"), ("16,12", "4,6"),
+                                     ("0", "0")])  # strips
 @pytest.mark.parametrize("n,c,h,w,its", [
     (1, 1, 1, 1, 4),        # one pixel
     (1, 2, 5, 3, 7),        # smaller than any tile, odd its
@@ -87,6 +88,31 @@ def test_allocation_free_forward_in_place(ext, monkeypatch, tile, its):
     x = t["di"].clone()
     ext.forward_noalloc(*args, x, its, x)
     assert torch.equal(x, want)
+
+
+@pytest.mark.parametrize("n,c,h,w,its", [(1, 2, 64, 128, 20), (1, 1, 40, 70, 9), (1, 2, 30, 50, 2), (4, 2, 384, 1248, 8)])
+def test_profile_times_the_reverse_sweep_that_ran(ext, n, c, h, w, its):
+    # tiles (the first two), a single launch that is not an inner strip launch, strips
+    import ctypes
+
+    from customnetworklayers_amd._lib import lib
+
+    t = tensors(tv_inputs(n, c, h, w, seed=9))
+    ext.reset_id(4)
+    steps = lib.tvinpaint_adjoint_tile_steps(n, c, h, w, its)
+    lib.tvinpaint_profile(1)
+    ext.forward(t["dx"], t["dy"], t["dc"], t["db"], t["di"], its, 4)
+    ext.backward(t["grad"], t["dx"], t["dy"], t["dc"], t["db"], its, 4)
+    ms, launches = ctypes.c_double(0), ctypes.c_int(0)
+    lib.tvinpaint_profile_read(ctypes.byref(ms), ctypes.byref(launches))
+    lib.tvinpaint_profile(0)
+    ext.reset_id(4)
+    all_steps = 2 * (its // 2) - 1
+    if steps:
+        assert launches.value == -(-all_steps // steps) and 0 < ms.value < 1000
+    else:
+        assert launches.value <= all_steps // 2  # inner pair launches only
+    assert bool(steps) == (n == 1 and its > 2)
 
 
 @pytest.mark.parametrize("n,c,h,w,its", [(1, 2, 64, 128, 20), (2, 2, 112, 256, 24), (1, 1, 187, 621, 20), (1, 2, 384, 1248, 20)])
