@@ -740,7 +740,7 @@ bool adjoint_pairs(const Slot& s) {
 // x 621 322 -> 246; 2 x 2 x 224 x 512 327 (strips) against 365.
 TilePlan adjoint_tile_plan(const Slot& s) {
   TilePlan p;
-  if (!adjoint_pairs(s) || s.ic > 2 || knobs().tv_adj_rows > 0 || knobs().tv_adj_split >= 0) return p;
+  if (!adjoint_pairs(s) || s.ic > 2 || knobs().tv_adj_rows > 0 || knobs().tv_adj_split >= 0 || !knobs().tv_fuse_first) return p;
   constexpr int R = 4;
   if (knobs().tv_atile_its >= 0) {
     p.R = knobs().tv_atile_rows;

@@ -7,6 +7,7 @@ import os
 import re
 
 import numpy as np
+import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -74,3 +75,15 @@ def test_flow_layers_reject_bad_arguments_before_any_gpu_work():
     assert b"null pointer" in lib.flowaux_last_error()
     assert lib.quadfit_backward_workspace_bytes(4, 384, 1248) >= 4 * 384 * 1248 * 4 * 11
     assert lib.quadfit_backward_workspace_bytes(0, 384, 1248) == 0
+
+
+@pytest.mark.parametrize("switch", ["INPAINT_TV_FUSE=0", "INPAINT_TV_FUSE_ADJ=0", "INPAINT_TV_FUSE_FIRST=0", "INPAINT_TV_ADJ_ROWS=8",
+                                    "INPAINT_TV_ADJ_SPLIT=1", "INPAINT_TV_ADJ_TILE=0"])
+def test_a_forced_strip_kernel_keeps_the_reverse_sweep_out_of_tiles(monkeypatch, switch):
+    from customnetworklayers_amd._lib import lib, reload_env
+
+    shape = (1, 2, 64, 128, 20)
+    assert lib.tvinpaint_adjoint_tile_steps(*shape) > 0
+    monkeypatch.setenv(*switch.split("="))
+    reload_env()
+    assert lib.tvinpaint_adjoint_tile_steps(*shape) == 0

@@ -291,11 +291,14 @@ def test_every_pairing_of_the_reverse_sweep(ext, tv_oracle, its):
 def test_first_step_of_the_sweep_rides_on_the_second(ext, tv_oracle, c, its, monkeypatch):
     # up to four channels, a last segment of at least four iterations: one launch does the sweep's first two steps
     # (its = 4, 5: the last segment has two iterations, so the two steps stay apart; c = 5 always keeps them apart);
-    # INPAINT_TV_FUSE_FIRST=0 keeps the separate launches covered
+    # INPAINT_TV_FUSE_FIRST=0 keeps the separate launches covered.  (Register tiles take the first step along whatever the
+    # segments: switched off here; the second setting switches them off by itself.)
+    monkeypatch.setenv("INPAINT_TV_ADJ_TILE", "0")
     d = tv_inputs(2, c, 37, 130, seed=500 + 10 * c + its, conf_density=0.4)
     ref = run_oracle(tv_oracle, d, its, 2)
     a = run_gpu(ext, d, its, 2)
     compare("first two steps in one launch c=%d its=%d" % (c, its), a, ref)
+    monkeypatch.delenv("INPAINT_TV_ADJ_TILE")
     monkeypatch.setenv("INPAINT_TV_FUSE_FIRST", "0")
     b = run_gpu(ext, d, its, 2)
     compare("first step in its own launch c=%d its=%d" % (c, its), b, ref)
