@@ -22,6 +22,19 @@ def fresh_environment_switches():
     yield
 
 
+@pytest.fixture(params=["by size", "strips"])
+def kernels(request, monkeypatch):
+    """A test that asks for this runs twice: with the kernels the library picks for the problem's size (register tiles for
+    most small ones), and with the strip kernels, which large problems run."""
+    from customnetworklayers_amd._lib import reload_env
+
+    if request.param == "strips":
+        for name in ("INPAINT_TV_TILE", "INPAINT_TV_ADJ_TILE", "INPAINT_TGV_TILE"):
+            monkeypatch.setenv(name, "0")
+        reload_env()
+    return request.param
+
+
 @pytest.fixture(scope="session")
 def tv_oracle():
     from oracle.oracle_lib import TVOracle

@@ -76,7 +76,11 @@ def check_quadfit(qf, o, d, name):
     (2, 2, 12, 70, 2),
     (1, 6, 20, 66, 2),      # a channel count that ends in the middle of the ring
 ])
-def test_quadfit_random_inputs_match_oracle(qf, flowaux_oracle, n, c, h, w, fc):
+@pytest.mark.parametrize("path", ["split", "tiles"])
+def test_quadfit_random_inputs_match_oracle(qf, flowaux_oracle, n, c, h, w, fc, path, monkeypatch):
+    monkeypatch.setenv("INPAINT_QUADFIT_PATH", path)  # (by size all of these take the split kernels)
+    from customnetworklayers_amd._lib import reload_env
+    reload_env()
     d = random_quadfit(n, c, h, w, seed=n * 100 + c + h + w, fc=fc)
     check_quadfit(qf, flowaux_oracle, d, "random %dx%dx%dx%d fc=%d" % (n, c, h, w, fc))
 
@@ -99,9 +103,13 @@ def test_quadfit_one_pixel_per_lane_kernels(qf, flowaux_oracle, n, c, h, w, monk
     check_quadfit(qf, flowaux_oracle, workloads.quadfit_inputs(n, c, h, w, seed=32), "px path warped")
 
 
+@pytest.mark.parametrize("path", ["split", "tiles"])
 @pytest.mark.parametrize("c", [4, 32, 40])
-def test_quadfit_flow_that_scatters_the_tile(qf, flowaux_oracle, c):
-    # a flow that varies by tens of pixels inside one tile: most taps fall outside the LDS window
+def test_quadfit_flow_that_scatters_the_tile(qf, flowaux_oracle, c, path, monkeypatch):
+    # a flow that varies by tens of pixels inside one tile: most taps fall outside the LDS window (the split kernels have none)
+    monkeypatch.setenv("INPAINT_QUADFIT_PATH", path)
+    from customnetworklayers_amd._lib import reload_env
+    reload_env()
     d = random_quadfit(1, c, 64, 256, seed=33, amp=40.0)
     check_quadfit(qf, flowaux_oracle, d, "scattered, %d channels" % c)
 

@@ -94,7 +94,7 @@ def compare(name, got, ref):
     (1, 2, 21, 64, 6),      # exactly one wavefront wide
     (1, 2, 19, 65, 6),      # one column more
 ])
-def test_forward_backward_match_oracle(ext, tgv_oracle, n, c, h, w, its):
+def test_forward_backward_match_oracle(ext, tgv_oracle, kernels, n, c, h, w, its):
     d = tgv_inputs(n, c, h, w, seed=n * 1000 + h + w + its, conf_density=0.3)
     print("case n=%d c=%d h=%d w=%d its=%d" % (n, c, h, w, its), flush=True)
     compare("%dx%dx%dx%d its=%d" % (n, c, h, w, its), run_gpu(ext, d, its, 2), run_oracle(tgv_oracle, d, its, 2))
@@ -106,7 +106,7 @@ def test_forward_backward_match_oracle(ext, tgv_oracle, n, c, h, w, its):
     (1, 5, 19, 126, 20),    # three groups, several segments
     (1, 3, 45, 130, 12),
 ])
-def test_more_than_two_channels_run_in_channel_groups(ext, tgv_oracle, n, c, h, w, its):
+def test_more_than_two_channels_run_in_channel_groups(ext, tgv_oracle, kernels, n, c, h, w, its):
     # the strip kernels hold up to two flow channels; more run as launches over groups of channels, whose shared
     # accumulators (confidence and weight gradients) are summed group after group in the reference's order
     d = varying_inputs(n, c, h, w, seed=300 + c)
@@ -141,7 +141,7 @@ def test_removed_kernel_path_is_refused(ext, monkeypatch):
     (1, 2, 40, 125, 10),    # two strips and a column
     (3, 1, 130, 200, 50),   # several segments of unequal length
 ])
-def test_strip_edges(ext, tgv_oracle, n, c, h, w, its):
+def test_strip_edges(ext, tgv_oracle, kernels, n, c, h, w, its):
     d = varying_inputs(n, c, h, w, seed=n * 100 + h + w)
     compare("%dx%dx%dx%d its=%d" % (n, c, h, w, its), run_gpu(ext, d, its, 2), run_oracle(tgv_oracle, d, its, 2))
 
@@ -163,7 +163,7 @@ def test_single_iteration_strip_kernels(ext, tgv_oracle, n, c, h, w, its, monkey
     (1, 2, 2, 59, 4),
     (2, 2, 18, 121, 12),    # two fused strips and a column
 ])
-def test_fused_forward_strip_edges(ext, tgv_oracle, n, c, h, w, its):
+def test_fused_forward_strip_edges(ext, tgv_oracle, kernels, n, c, h, w, its):
     d = varying_inputs(n, c, h, w, seed=n * 100 + h + w)
     compare("%dx%dx%dx%d its=%d" % (n, c, h, w, its), run_gpu(ext, d, its, 2), run_oracle(tgv_oracle, d, its, 2))
 

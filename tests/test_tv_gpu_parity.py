@@ -78,7 +78,7 @@ def compare(name, got, ref):
     (1, 4, 19, 126, 6),     # four channels, two forward strips
     (1, 3, 40, 125, 10),    # three channels, ragged
 ])
-def test_forward_backward_match_oracle(ext, tv_oracle, n, c, h, w, its):
+def test_forward_backward_match_oracle(ext, tv_oracle, kernels, n, c, h, w, its):
     d = tv_inputs(n, c, h, w, seed=n * 1000 + h + w + its, conf_density=0.3)
     print("case n=%d c=%d h=%d w=%d its=%d" % (n, c, h, w, its), flush=True)
     compare("%dx%dx%dx%d its=%d" % (n, c, h, w, its), run_gpu(ext, d, its, 2), run_oracle(tv_oracle, d, its, 2))
@@ -91,7 +91,7 @@ def test_forward_backward_match_oracle(ext, tv_oracle, n, c, h, w, its):
     (2, 8, 45, 130, 12),    # 4 + 4
     (1, 9, 11, 62, 8),      # three groups
 ])
-def test_more_than_four_channels_run_in_channel_groups(ext, tv_oracle, n, c, h, w, its):
+def test_more_than_four_channels_run_in_channel_groups(ext, tv_oracle, kernels, n, c, h, w, its):
     # the strip kernels hold up to four channels; more run as launches over groups of channels, whose shared
     # accumulators (confidence and edge-weight gradients) are summed group after group in the reference's order
     d = tv_inputs(n, c, h, w, seed=300 + c, conf_density=0.3)
@@ -279,7 +279,7 @@ def test_single_step_adjoint_strip_kernels(ext, tv_oracle, n, c, h, w, its, monk
 
 
 @pytest.mark.parametrize("its", [2, 3, 4, 5, 6, 8, 16, 17, 26])
-def test_every_pairing_of_the_reverse_sweep(ext, tv_oracle, its):
+def test_every_pairing_of_the_reverse_sweep(ext, tv_oracle, kernels, its):
     # its decides how the sweep splits into the first step, an optional single step and pairs:
     # one segment of 2 (first step + single segment-start step), segments of even and odd remainder
     d = tv_inputs(1, 2, 23, 75, seed=300 + its, conf_density=0.4)
@@ -313,7 +313,7 @@ def test_first_step_of_the_sweep_rides_on_the_second(ext, tv_oracle, c, its, mon
     (1, 2, 2, 59, 4),
     (2, 4, 18, 121, 12),    # four channels, two fused strips and a column
 ])
-def test_fused_forward_strip_edges(ext, tv_oracle, n, c, h, w, its):
+def test_fused_forward_strip_edges(ext, tv_oracle, kernels, n, c, h, w, its):
     d = tv_inputs(n, c, h, w, seed=n * 100 + h + w, conf_density=0.3)
     compare("%dx%dx%dx%d its=%d" % (n, c, h, w, its), run_gpu(ext, d, its, 2), run_oracle(tv_oracle, d, its, 2))
 
