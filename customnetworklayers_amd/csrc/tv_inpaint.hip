@@ -434,15 +434,27 @@ long long tiles_per_cu(const Slot& s, int cols, int rows, int its, int channels)
   return (tx * ty * s.n * channels + compute_unit_count() - 1) / compute_unit_count();
 }
 
-// Tiles or strips, and which tile: the cheapest by a cost model fitted to both kernels' measured times.  A tile launch
-// costs 3.8 us however small it is, 3 us more for every further round of workgroups, and per iteration and row of a
-// wavefront 300 cycles where a SIMD holds one wavefront and 200 per wavefront where it holds several; keeping x05 rows adds
-// 0.5 us per iteration and million values, rebuilding the input iterate from them 100 cycles per row.  A strip launch
-// costs 4.3 us and 4.65 us per million values, for two iterations.  So tiles win while launches and latency dominate, and
-// strips, which have no halo columns to spare and stream their rows, on problems that fill the chip many times over.
-// Measured, forward pass, strips -> tiles: 1 x 2 x 64 x 128, 20 iterations 46 -> 27 us; 48 iterations of 2 x 2 x 112 x 256
-// 118 -> 76, 2 x 2 x 224 x 512 156 -> 122, 1 x 1 x 384 x 1248 158 -> 123, 1 x 2 x 384 x 1248 233 -> 192, 4 x 2 x 384 x
-// 1248 without rows 508 -> 477, with rows 536 (strips) against 567 (best tiles).
+// Tiles or strips, and which tile: the cheapest by a cost model fitted to 1846 measured forward passes (47 shapes from 1 x 1 x 48
+// x 64 to 8 x 2 x 448 x 1280, 1 to 8 channels, with and without x05 rows, 2 to 12 iterations per launch; 8, 6 and 6% rms for R = 4,
+// 8, 16).  A tile launch costs `launch` us, and for the loads and stores of its ends `io` us per row and workgroup of the fullest
+// CU; an iteration costs each of a wavefront's rows (and 0.55 of a row for the triangles above) `lone` us, and `share` us more per
+// workgroup on the CU.  Keeping x05 rows adds `keep` us per iteration and million values, rebuilding the input iterate from them
+// `rebuild` us per row and workgroup.  A strip launch costs 4.8 us per group of four channels and 5 us per million values, for two
+// iterations.  With x05 rows tiles have to be cheaper by 3%: there the two are level on problems that fill the chip.  4, 8 and 12
+// iterations (output columns that start on 16-byte boundaries) take 3% less.  Two and three iterations per launch are left out: they
+// read and write nearly as much as strips, and look better to the model than they are.
+// As committed, this picks the fastest tile or strips within 0.5% in the mean, 7.4% at most (its = 2, 11 us: 11%).  (A first fit, to ten
+// shapes up to 4 x 2 x 384 x 1248, charged full chips for rounds of workgroups that overlap: 4 x 4 x 384 x 1248 without rows took 547 us
+// for 24 iterations in tiles of 64 rows, 478 in strips.)
+// Measured, forward pass, strips -> tiles: 1 x 2 x 64 x 128, 20 iterations 41 -> 23 us; 48 iterations of 1 x 2 x 112 x 256 97 -> 61;
+// 24 iterations of 1 x 2 x 187 x 621 68 -> 44, 1 x 2 x 384 x 1248 118 -> 86, 4 x 2 x 384 x 1248 without rows 274 -> 238, with rows 272
+// (strips) against 284, 4 x 4 x 384 x 1248 478 -> 428, with rows 525 (strips) against 545.
+struct TileCost {
+  int R;
+  double launch, io, lone, share, keep, rebuild;
+};
+constexpr TileCost kTileCosts[] = {{4, 2.5, .139, .097, .052, .19, .022}, {8, 3.0, .109, .063, .061, .29, .030}, {16, 3.2, .140, .044, .0666, .70, .032}};
+
 TilePlan forward_tile_plan(const Slot& s, bool keeps_rows) {
   TilePlan p;
   if (!forward_pairs(s) || knobs().tv_fwd_rows > 0 || knobs().tv_fwd_split >= 0) return p;  // (a forced strip shape)
@@ -455,16 +467,16 @@ TilePlan forward_tile_plan(const Slot& s, bool keeps_rows) {
   }
   const int K = 2 * (s.its / 2);
   const double mega = 1e-6 * s.n * s.ic * (double)s.ih * s.iw;
-  double best = 0.97 * (4.3 + 4.65 * mega) / 2;  // us per iteration
-  for (int R : {4, 8, 16}) {
-    for (int k = 2; k <= tvtile::kMaxFwdSteps && 2 * k < kTileWaves * R; k++) {
+  double best = (keeps_rows ? 0.97 : 1.) * (4.8 * ((s.ic + kGroup - 1) / kGroup) + 5.0 * mega) / 2;  // us per iteration
+  for (const TileCost& t : kTileCosts) {
+    for (int k = 4; k <= tvtile::kMaxFwdSteps && 2 * k < kTileWaves * t.R; k++) {
       const int launches = (K + k - 1) / k, its = (K + launches - 1) / launches;
       if (its != k) continue;  // (the same launches as a smaller k)
-      const long long on_cu = tiles_per_cu(s, 64, kTileWaves * R, its, s.ic);
-      const long long rounds = (on_cu + 32 / R - 1) / (32 / R);  // 8, 4 and 2 workgroups resident per CU
-      double us = (3.8 + 3.0 * (rounds - 1)) / its + on_cu * (R + 0.55) * (on_cu == 1 ? 300 : 200) / 2400.;
-      if (keeps_rows) us += 0.5 * mega + on_cu * R * 100 / 2400. / its;
-      if (us < best) { best = us; p.R = R; p.K = its; }
+      const long long on_cu = tiles_per_cu(s, 64, kTileWaves * t.R, its, s.ic);
+      double us = (t.launch + t.io * on_cu * t.R) / its + (t.R + 0.55) * (t.lone + t.share * on_cu);
+      if (keeps_rows) us += t.keep * mega + t.rebuild * on_cu * t.R / its;
+      if (its % 4 == 0) us *= 0.97;
+      if (us < best) { best = us; p.R = t.R; p.K = its; }
     }
   }
   return p;
