@@ -97,3 +97,19 @@ def test_default_choice_of_kernels_matches_the_oracle(ext, tgv_oracle, n, c, h, 
     ext.reset_id(4)
     check(ext, tgv_oracle, tgv_inputs(n, c, h, w, seed=8), its, 4)
     ext.reset_id(4)
+
+
+@pytest.mark.parametrize("pixel", [(30, 64), (0, 20), (59, 129), (17, 0)])  # inside, and on the image's edges
+@pytest.mark.parametrize("name,value", [("dx", np.nan), ("dy", np.inf), ("dc", np.inf), ("db", np.inf), ("di", -np.inf), ("di", np.nan)])
+def test_non_finite_inputs_spread_as_in_strips(ext, monkeypatch, name, value, pixel):
+    d = tgv_inputs(1, 2, 60, 130, seed=9)
+    d[name][0, -1, pixel[0], pixel[1]] = value
+    t = {k: torch.from_numpy(v).to(DEV) for k, v in d.items()}
+    out = []
+    for tile in ("0", "12,3", "40,5"):
+        monkeypatch.setenv("INPAINT_TGV_TILE", tile)
+        ext.reset_id(4)
+        out.append(ext.forward(t["dx"], t["dy"], t["dc"], t["db"], t["di"], 10, 4)[0].cpu().numpy())
+    ext.reset_id(4)
+    for got in out[1:]:
+        np.testing.assert_array_equal(got, out[0])

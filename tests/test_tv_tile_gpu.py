@@ -120,3 +120,25 @@ def test_default_choice_of_kernels_matches_the_oracle(ext, tv_oracle, n, c, h, w
     ext.reset_id(4)
     check(ext, tv_oracle, tv_inputs(n, c, h, w, seed=8), its, 4)
     ext.reset_id(4)
+
+
+@pytest.mark.parametrize("pixel", [(30, 64), (0, 20), (59, 129), (17, 0)])  # inside, and on the image's edges
+@pytest.mark.parametrize("name,value", [("dx", np.inf), ("dy", np.nan), ("dc", np.inf), ("db", np.inf), ("di", -np.inf), ("di", np.nan)])
+def test_non_finite_inputs_spread_as_in_strips(ext, monkeypatch, name, value, pixel):
+    # What a pixel outside the image takes on from a neighbour inside must not come back sooner than it spreads inside; the
+    # reverse sweep's clip turns NaN into a number, outside the image too.
+    d = tv_inputs(1, 2, 60, 130, seed=9)
+    d[name][0, -1, pixel[0], pixel[1]] = value
+    t = tensors(d)
+    out = []
+    for fwd, adj in (("0", "0"), ("4,3", "4,3"), ("8,6", "4,7")):
+        monkeypatch.setenv("INPAINT_TV_TILE", fwd)
+        monkeypatch.setenv("INPAINT_TV_ADJ_TILE", adj)
+        ext.reset_id(4)
+        (sol,) = ext.forward(t["dx"], t["dy"], t["dc"], t["db"], t["di"], 12, 4)
+        out.append([sol] + ext.backward(t["grad"].clone(), t["dx"], t["dy"], t["dc"], t["db"], 12, 4))
+    ext.reset_id(4)
+    assert name != "di" or not torch.isfinite(out[0][0]).all()
+    for got in out[1:]:
+        for a, b in zip(out[0], got):
+            np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
