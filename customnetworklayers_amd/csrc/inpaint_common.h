@@ -175,6 +175,22 @@ inline void make_step_sizes(int its, std::vector<float>& s) {
   }
 }
 
+// Waits for the stream of an id's last call on `device` (a null stream is the current device's); where that stream no longer
+// exists, for the whole device.
+inline int wait_for_last_call(hipStream_t last, int device) {
+  int cur = -1;
+  (void)hipGetDevice(&cur);
+  if (device >= 0 && cur != device) (void)hipSetDevice(device);
+  hipError_t e = hipStreamSynchronize(last);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    e = hipDeviceSynchronize();
+  }
+  if (device >= 0 && cur >= 0 && cur != device) (void)hipSetDevice(cur);
+  if (e != hipSuccess) return fail(INPAINT_ERR_HIP, "waiting for the id's last call failed: %s", hipGetErrorString(e));
+  return 0;
+}
+
 // ---------------------------------------------------------------------------------------------
 // device arena: one hipMalloc per slot, re-made only when the shape changes
 // ---------------------------------------------------------------------------------------------

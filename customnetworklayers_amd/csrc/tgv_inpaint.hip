@@ -526,7 +526,8 @@ int fetch_running_means(Slot& s, unsigned int* skipped = nullptr) {
   if (skipped) *skipped = 0;
   if (s.guard) {
     GuardState host;
-    INPAINT_HIP(hipStreamSynchronize(s.stream));
+    const int rc = wait_for_last_call(s.stream, s.arena.device);
+    if (rc) return rc;
     INPAINT_HIP(hipMemcpy(&host, s.guard, kGuardHeaderBytes, hipMemcpyDeviceToHost));
     for (int k = 0; k < 5; k++) s.pending_av[k] = host.av[k];
     if (skipped) *skipped = host.skipped;
@@ -543,11 +544,15 @@ int prepare_slot(Slot& s, int n, int ic, int ih, int iw, int its, int keep_mode,
   const int ring_rows = keep_mode == 2 ? std::max(its, 1) : std::max(max_inter_its, 1);
   const bool same = s.arena.base && s.arena.device == dev && s.n == n && s.ic == ic && s.ih == ih &&
                     s.iw == iw && s.its == its && s.ring_rows >= ring_rows;  // the ring only grows
-  s.stream = stream;
-  if (same) return 0;
+  if (same) {
+    s.stream = stream;
+    return 0;
+  }
+  // the running means survive a change of shape; the block goes back only when the last call, on whatever stream, is done with it
   unsigned int skipped = 0;
   int rc = fetch_running_means(s, &skipped);
   if (rc) return rc;
+  s.stream = stream;
   s.run -= (int)skipped;  // the new guard state starts counting refused passes from zero
   s.guard = nullptr;  // the arena is about to be released; the means live in pending_av until the new one exists
   s.n = n; s.ic = ic; s.ih = ih; s.iw = iw; s.its = its;
@@ -1465,7 +1470,7 @@ int tgvinpaint_reset_id(int id) {
   if (id < 0 || id >= kUniqueIds) return fail(INPAINT_ERR_ID, "bad id %d", id);
   reload_knobs();
   Slot& s = g_slots[id];
-  if (s.arena.base) (void)hipStreamSynchronize(s.stream);
+  if (s.arena.base) (void)wait_for_last_call(s.stream, s.arena.device);
   int rc = s.arena.release();
   s = Slot();
   return rc;

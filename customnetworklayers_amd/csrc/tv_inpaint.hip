@@ -236,7 +236,8 @@ size_t plane_count(const Slot& s) { return (size_t)s.n * s.ih * s.iw; }
 int fetch_running_means(Slot& s) {
   if (s.guard) {
     GuardState host;
-    INPAINT_HIP(hipStreamSynchronize(s.stream));
+    const int rc = wait_for_last_call(s.stream, s.arena.device);
+    if (rc) return rc;
     INPAINT_HIP(hipMemcpy(&host, s.guard, kGuardHeaderBytes, hipMemcpyDeviceToHost));
     for (int k = 0; k < 5; k++) s.pending_av[k] = host.av[k];
   }
@@ -252,10 +253,14 @@ int prepare_slot(Slot& s, int n, int ic, int ih, int iw, int its, int keep_mode,
   const int ring_rows = keep_mode == 2 ? std::max(its, 1) : std::max(max_inter_its, 1);
   const bool same = s.arena.base && s.arena.device == dev && s.n == n && s.ic == ic && s.ih == ih &&
                     s.iw == iw && s.its == its && s.ring_rows >= ring_rows;  // the ring only grows
-  s.stream = stream;
-  if (same) return 0;
-  int rc = fetch_running_means(s);  // the running means survive a change of shape
+  if (same) {
+    s.stream = stream;
+    return 0;
+  }
+  // the running means survive a change of shape; the block goes back only when the last call, on whatever stream, is done with it
+  int rc = fetch_running_means(s);
   if (rc) return rc;
+  s.stream = stream;
   s.guard = nullptr;  // the arena is about to be released; the means live in pending_av until the new one exists
   s.n = n; s.ic = ic; s.ih = ih; s.iw = iw; s.its = its;
   make_schedule(its, s.iterations, s.max_inter_its);
@@ -1396,7 +1401,7 @@ int tvinpaint_reset_id(int id) {
   if (id < 0 || id >= kUniqueIds) return fail(INPAINT_ERR_ID, "bad id %d", id);
   reload_knobs();
   Slot& s = g_slots[id];
-  if (s.arena.base) (void)hipStreamSynchronize(s.stream);
+  if (s.arena.base) (void)wait_for_last_call(s.stream, s.arena.device);
   int rc = s.arena.release();
   s = Slot();
   return rc;

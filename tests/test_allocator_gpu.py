@@ -90,3 +90,41 @@ def test_allocator_callbacks_come_in_pairs_and_may_refuse():
     torch.cuda.synchronize()
     assert bool(torch.isfinite(sol).all())
     ext.reset_id(6)
+
+
+@pytest.mark.parametrize("layer", ["tv", "tgv"])
+def test_a_block_goes_back_only_when_the_last_call_is_done_with_it(layer):
+    # the id's last call ran on another stream than the one that changes its shape; the callbacks keep every block until the end,
+    # so that nothing is ever handed on while it is in use
+    if layer == "tv":
+        from customnetworklayers_amd.cudaTV import tvInpaint_cuda_ext as ext
+        make, lib_set = tv_inputs, _lib.lib.tvinpaint_set_allocator
+    else:
+        from customnetworklayers_amd.cudaTGV import tgvInpaint_cuda_ext as ext
+        make, lib_set = tgv_inputs, _lib.lib.tgvinpaint_set_allocator
+    large = {k: torch.from_numpy(v).to(DEV) for k, v in make(2, 2, 384, 1248, seed=4).items()}
+    small = {k: torch.from_numpy(v).to(DEV) for k, v in make(1, 1, 16, 64, seed=4).items()}
+    kept, idle, other = [], [], torch.cuda.Stream()
+
+    def alloc(nbytes, device, stream, user):
+        kept.append(torch.empty(int(nbytes) + 256, dtype=torch.uint8, device=DEV))
+        return (kept[-1].data_ptr() + 255) // 256 * 256
+
+    alloc_c, release_c = _lib._ALLOC_FN(alloc), _lib._RELEASE_FN(lambda ptr, user: idle.append(other.query()))
+    ext.reset_id(5)
+    torch.cuda.synchronize()
+    try:
+        assert lib_set(ctypes.cast(alloc_c, ctypes.c_void_p), ctypes.cast(release_c, ctypes.c_void_p), None) == 0
+        with torch.cuda.stream(other):
+            ext.forward(large["dx"], large["dy"], large["dc"], large["db"], large["di"], 100, 5)
+            ext.backward(large["grad"], large["dx"], large["dy"], large["dc"], large["db"], 100, 5)
+        assert not other.query()  # milliseconds of work
+        ext.forward(small["dx"], small["dy"], small["dc"], small["db"], small["di"], 4, 5)
+        assert idle == [True]
+        torch.cuda.synchronize()
+        ext.reset_id(5)
+        assert len(idle) == 2
+    finally:
+        torch.cuda.synchronize()
+        ext.reset_id(5)
+        _lib.use_torch_allocator(True)
