@@ -213,8 +213,11 @@ __global__ __launch_bounds__(256) void quadfit_backward_kernel(const float* __re
 //   pass B (per target pixel)  gathers, per channel, I1 * coefficient from the sources listed at the
 //                              target and at its four neighbours (a source centred on the left
 //                              neighbour reaches the target with its right tap, and so on);
-//   pass C (overflow list)     sources that found their list full scatter with float atomics after
-//                              pass B -- rare: it takes more than kSlots pixels landing on one position.
+//   pass C (two lists)         after pass B, with float atomics: the sources that found their list full (it takes more
+//                              than kSlots pixels landing on one position), and the target pixels that pass B has listed
+//                              and left at zero: more sources than it holds in registers, or one outside its window.  A
+//                              few pixels in a hundred on a smooth flow, a quarter on one that contracts by two, nearly
+//                              all on one that scatters every tile.
 // A tap that the image border clamps back onto the centre carries a zero coefficient (the axis is
 // not fitted at the border), so the gather leaves it out.
 // Workspace (caller provided): count[P] | overflow count, slow count, pad | slots[P*kSlots] | overflow list[P] | coef[5*P] |

@@ -792,15 +792,18 @@ struct TileShape {
 constexpr TileShape kTiles[] = {{3, 4, 5, 3, 40}, {4, 8, 2, 5, 100}, {5, 8, 2, 5, 95}, {5, 16, 1, 6, 116}};
 
 // Tiles or strips, and which tile: the cheapest by a cost model fitted to 570 measured forward passes (17 shapes from 1 x 1 x
-// 61 x 97 to 4 x 2 x 384 x 1248, all four tiles, 2 to 12 iterations per launch; 7% rms).  A tile launch costs 2.2 us and
+// 61 x 97 to 4 x 2 x 384 x 1248, all four tiles, 2 to 12 iterations per launch; against a second sweep of these shapes 15% rms, 8% of
+// it a common factor).  A tile launch costs 2.2 us and
 // 0.34 us per row of a SIMD's wavefronts for its loads; an iteration costs each of a tile's rows (and 0.45 of a row for the
 // triangles above) 297 ns on a SIMD that holds few wavefronts and `ns` per wavefront where that is more; keeping x05
 // states adds 1.8 us per iteration and million values.  A strip launch costs 5.1 us and 13.1 us per million values, for two
-// iterations.  The choice is within 2% of the best tile in the mean, 12% at most.  Few iterations per launch on the taller tiles
-// look better to the model than they measure, hence `least`.
-// Measured, forward pass, strips -> tiles, without and with x05 states: 1 x 1 x 61 x 97, 30 iterations 109 -> 78, 100 -> 87
-// us; 50 iterations of 1 x 2 x 112 x 256 163 -> 121, 167 -> 133; 1 x 2 x 187 x 621 (48) 222 -> 141, 233 -> 163; 1 x 2 x 375 x
-// 1241 446 -> 304, 435 -> 368 (397 chosen); 4 x 2 x 384 x 1248 1432 -> 993 (1040 chosen), 1538 -> 1307 (1374 chosen).
+// iterations.  Few iterations per launch on the taller tiles look better to the model than they measure, hence `least`.
+// With these constants the choice is always faster than strips, and within 2.0% of the fastest tile in the mean, 8.5% at most but for
+// one shape: full batches without x05 states (4 x 2 x 384 x 1248) get 80 rows, 1188 us for 50 iterations, where 40 rows, 7
+// iterations per launch, take 986; the same constants pick 80 rows with x05 states, where they are the fastest.
+// Measured, forward pass, strips -> chosen, without and with x05 states: 1 x 1 x 61 x 97, 30 iterations 90 -> 59, 93 -> 62 us (12
+// rows, 5 per launch); 50 iterations of 1 x 2 x 112 x 256 148 -> 111, 166 -> 129; 1 x 2 x 187 x 621 (48) 218 -> 135, 223 -> 154; 1 x
+// 2 x 375 x 1241 440 -> 299, 437 -> 365; 4 x 2 x 384 x 1248 1407 -> 1188, 1538 -> 1297.
 TilePlan forward_tile_plan(const Slot& s, bool keeps_rows) {
   TilePlan p;
   if (!forward_pairs(s) || knobs().tgv_fwd_rows > 0 || knobs().tgv_fwd_split >= 0) return p;  // (a forced strip shape)

@@ -46,8 +46,9 @@ struct FwdSteps {
 // Bound by instruction issue: about 80 vector instructions per pixel and iteration where the Huber terms of a row are quiet,
 // 120 where none is, on two to five wavefronts per SIMD (the strips issue as many, but wait for memory every second
 // iteration and read 19 planes for it).  Taller tiles waste less on the halo; 5 rows per wavefront are what fits 128 registers.
-// 50 iterations of 1 x 2 x 375 x 1241: 446 us in strips, 304 in tiles of 40 rows, 7 iterations per launch; 4 x 2 x 384 x 1248:
-// 1432 -> 993, with every x05 state kept 1538 -> 1307 (80 rows, 8 per launch); 30 iterations of 1 x 1 x 61 x 97: 109 -> 78.
+// 50 iterations of 1 x 2 x 375 x 1241: 440 us in strips, 299 in tiles of 40 rows, 7 iterations per launch; 4 x 2 x 384 x 1248:
+// 1407 -> 986 in such tiles, with every x05 state kept 1538 -> 1297 (80 rows, 8 per launch); 30 iterations of 1 x 1 x 61 x 97:
+// 90 -> 59 (12 rows, 5 per launch).
 //
 // xin, yin: the iterate, or, with `ring`, the x05 states of the two iterations before (as in tgv_forward_strip2).  keep_x,
 // keep_y (optional): a copy of the input iterate.

@@ -753,8 +753,8 @@ bool adjoint_pairs(const Slot& s) {
 // has to be cheaper by a tenth: the reverse step is bound by the vector ALUs, and a tile of 16 rows does its halo's work
 // as well, so tiles win only where the chip is far from full.  (Taller tiles, 6 and 8 rows per wavefront, were measured:
 // 256 registers and one wavefront per SIMD, slower at every size.)  Measured, backward pass, strips -> tiles: 1 x 2 x 64 x
-// 128, 20 iterations 88 -> 70 us; 50 iterations of 1 x 1 x 112 x 256 186 -> 144, 2 x 2 x 112 x 256 232 -> 191, 1 x 2 x 187
-// x 621 322 -> 246; 2 x 2 x 224 x 512 327 (strips) against 365.
+// 128, 20 iterations 86 -> 66 us; 50 iterations of 2 x 2 x 112 x 256 231 -> 188, 1 x 2 x 187 x 621 325 -> 244, 1 x 1 x 187 x 621 224
+// -> 183; 2 x 2 x 224 x 512 327 (strips) against 365.
 TilePlan adjoint_tile_plan(const Slot& s) {
   TilePlan p;
   if (!adjoint_pairs(s) || s.ic > 2 || knobs().tv_adj_rows > 0 || knobs().tv_adj_split >= 0 || !knobs().tv_fuse_first) return p;

@@ -43,8 +43,8 @@ struct FwdSteps {
 // channels of a tile are neighbours in the grid and share c and the weights in the XCD's L2).  xin, yin: the iterate, or,
 // with `ring`, the x05 rows of the two iterations before (as in tv_forward_strip2).  keep_x, keep_y (optional): a copy of
 // the input iterate.  48 vector instructions per pixel and iteration; bound by launch and load latency (about 4 us) and
-// instruction issue on one or two wavefronts per SIMD.  1 x 2 x 64 x 128, 20 iterations: 46 us in ten strip launches, 27 us
-// in four launches of 5 iterations with R = 4; 48 iterations of 1 x 2 x 187 x 621: 135 -> 80 us (R = 8, 6 per launch).
+// instruction issue on one or two wavefronts per SIMD.  1 x 2 x 64 x 128, 20 iterations: 41 us in ten strip launches, 23 us
+// in three launches of 6 to 7 iterations with R = 4; 48 iterations of 1 x 2 x 187 x 621: 130 -> 82 us (R = 8, 6 per launch).
 template <int R, int WAVES, bool X05>
 __global__ __launch_bounds__(64 * WAVES) void tv_forward_tile(
     const float* __restrict__ wx, const float* __restrict__ wy, const float* __restrict__ cf,
@@ -247,7 +247,7 @@ struct AdjTileArgs {
 // them, so launches need not follow the segments.  FIRST (x_last given): the sweep's first step (TV.cu:222-287) on the way
 // in.  The x05 row of the next step is loaded while this one computes.  About 150 vector instructions per pixel, channel
 // and step, 20 more for the extra triangle of a wavefront; bound by their issue on one wavefront per SIMD (1.5 us per step)
-// and by the launch (4.4 us).  1 x 2 x 64 x 128, 20 iterations: backward pass 88 us in strips, 70 us in four launches.
+// and by the launch (4.4 us).  1 x 2 x 64 x 128, 20 iterations: backward pass 86 us in strips, 66 us in three launches.
 template <int CL, int R, int WAVES, bool TRUE_ADJ>
 __global__ __launch_bounds__(64 * WAVES) void tv_adjoint_tile(AdjTileArgs a, AdjSteps steps) {
   static_assert(CL == 1 || CL == 2, "one channel, or two in the two halves of a wavefront");

@@ -37,7 +37,8 @@ int quadfit_forward(const float* im0, const float* im1, const float* flow, float
  *            (quadFit.h:11-12).
  *   workspace, workspace_bytes : device scratch of at least quadfit_backward_workspace_bytes(n,ih,iw)
  *            bytes, 16-byte aligned, contents irrelevant on entry.  With it g1 is GATHERED through a
- *            per-call inverse map (no float atomics unless more than 4 pixels land on one position).
+ *            per-call inverse map; float atomics add what does not fit it: the fifth and further pixels that land on
+ *            one position, and targets with more than twelve sources or with sources far from their neighbours'.
  *            workspace == NULL selects the reference's scatter with float atomics (quadFit.cu:279-283,
  *            296), which this GPU executes far below memory speed.  Either way the sums that form g1 are
  *            order dependent at the rounding level, as they are in the reference.
