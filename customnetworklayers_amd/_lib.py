@@ -71,6 +71,8 @@ def _load():
     lib.quadfit_backward_workspace_bytes.restype = ctypes.c_longlong
     lib.medimax_forward.argtypes = [_f32p] * 2 + [_int] * 4 + [ctypes.c_void_p]
     lib.medimax_backward.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_void_p]
+    lib.medimax_forward_saving.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_void_p]
+    lib.medimax_backward_saved.argtypes = [_f32p] * 4 + [_int] * 4 + [ctypes.c_void_p]
     lib.flowaux_last_error.restype = ctypes.c_char_p
     lib.hierarchy_next_level_forward.argtypes = [_f32p] * 5 + [_int] * 4 + [ctypes.c_float, ctypes.c_float, ctypes.c_void_p]
     lib.hierarchy_next_level_backward.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_float, ctypes.c_void_p]

@@ -1459,26 +1459,18 @@ __global__ __launch_bounds__(256) void median_forward_kernel(const float* __rest
   }
 }
 
-// MM.cu:46-93.  Pass 1 finds each pixel's crossing, pass 2 writes every bin's gradient.
-__global__ __launch_bounds__(256) void median_backward_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
-                                                              float* __restrict__ gvol, long long P, long long HW, int D) {
-  __shared__ float tiles[4][64][kPitch];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const long long p0 = ((long long)blockIdx.x * 4 + wave) * 64;
+// MM.cu:46-93 for the 64 pixels from p0 on.  Pass 1 finds each pixel's crossing, pass 2 writes every bin's gradient.  (All
+// wavefronts of the block, each with a tile and 64 pixels of its own.)
+__device__ __forceinline__ void backward_from_bins(const float* __restrict__ vol, float* __restrict__ gvol, float (*tile)[kPitch],
+                                                   long long p0, long long P, int D, int lane, float g0v, float g1v) {
   const long long p = p0 + lane;
   Crossing s{false, 0, 0.f, 1.f, 0.f};
   for (int c0 = 0; c0 < D; c0 += kBins) {
     const int nb = min(kBins, D - c0);
-    stage_in(vol, tiles[wave], p0, P, D, c0, nb, lane);
+    stage_in(vol, tile, p0, P, D, c0, nb, lane);
     __syncthreads();
-    walk(s, tiles[wave][lane], c0, nb);
+    walk(s, tile[lane], c0, nb);
     if (__syncthreads_and(s.found || p >= P)) break;
-  }
-  float g0v = 0.f, g1v = 0.f;
-  if (p < P) {
-    const long long n = p / HW, q = p - n * HW;
-    g0v = gin[n * 2 * HW + q];
-    g1v = gin[n * 2 * HW + HW + q];
   }
   const float cross = g0v * s.alpha / (-s.pmid) + g1v;  // MM.cu:69
   const float neg = -g0v / (2. * s.pmid);               // MM.cu:85
@@ -1487,9 +1479,9 @@ __global__ __launch_bounds__(256) void median_backward_kernel(const float* __res
   for (int c0 = 0; c0 < D; c0 += kBins) {
     const int nb = min(kBins, D - c0);
     __syncthreads();
-    stage_in(vol, tiles[wave], p0, P, D, c0, nb, lane);
+    stage_in(vol, tile, p0, P, D, c0, nb, lane);
     __syncthreads();
-    float* row = tiles[wave][lane];
+    float* row = tile[lane];
     for (int j = 0; j < nb; j++) {  // MM.cu:77-92; the crossing bin keeps the value of MM.cu:69
       const float cScore = row[j];
       float g = (s.found && c0 + j == s.c) ? cross : 0.f;
@@ -1499,8 +1491,23 @@ __global__ __launch_bounds__(256) void median_backward_kernel(const float* __res
       score = score + cScore;
     }
     __syncthreads();
-    stage_out(gvol, tiles[wave], p0, P, D, c0, nb, lane);
+    stage_out(gvol, tile, p0, P, D, c0, nb, lane);
   }
+}
+
+__global__ __launch_bounds__(256) void median_backward_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
+                                                              float* __restrict__ gvol, long long P, long long HW, int D) {
+  __shared__ float tiles[4][64][kPitch];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const long long p0 = ((long long)blockIdx.x * 4 + wave) * 64;
+  const long long p = p0 + lane;
+  float g0v = 0.f, g1v = 0.f;
+  if (p < P) {
+    const long long n = p / HW, q = p - n * HW;
+    g0v = gin[n * 2 * HW + q];
+    g1v = gin[n * 2 * HW + HW + q];
+  }
+  backward_from_bins(vol, gvol, tiles[wave], p0, P, D, lane, g0v, g1v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1585,10 +1592,50 @@ __device__ __forceinline__ void stage_rows(const float* __restrict__ src, float*
   }
 }
 
-template <int VEC, bool BACKWARD>
+// The walk of MM.cu:26-43 == MM.cu:59-75 over a whole histogram, without the early exit.  The crossing bin's interpolation (a
+// double division) is formed once, after the walk: inside the loop it would run in every iteration in which ANY lane of the
+// wavefront crosses.  The comparisons against 0.5 are the reference's (a float promoted to double compares as the float does);
+// in front of the crossing the running sum is below one half or a NaN, so the bin that brings it there is the crossing.
+struct Walked {
+  bool found;
+  bool regular;  // every sum from the crossing on is at least one half (no crossing: no sum is a NaN)
+  int cidx;
+  float before, pmid;  // sum in front of the crossing bin, its mass
+};
+template <bool CHECK>
+__device__ __forceinline__ Walked walk_histogram(const float* row, int D) {
+  Walked s{false, true, 0, 0.f, 1.f};
+  float run = 0.f;
+#pragma unroll 4
+  for (int c = 0; c < D; c++) {
+    const float cScore = row[c];
+    const float sum = run + cScore;
+    const bool half = sum >= 0.5f, hit = half && !s.found;
+    s.pmid = hit ? cScore : s.pmid;
+    s.cidx = hit ? c : s.cidx;
+    s.before = hit ? run : s.before;
+    if (CHECK) s.regular = s.regular && (half || !s.found);
+    s.found = s.found || half;
+    run = sum;
+  }
+  if (CHECK) s.regular = s.regular && (s.found || run == run);
+  return s;
+}
+__device__ __forceinline__ float crossing_offset(float before, float pmid) {
+  return (1. - 2. * before - pmid) / (2. * pmid);  // MM.cu:34
+}
+// What the backward pass takes from the forward pass, one plane each: the crossing's offset, its mass, and its bin -- num_disp
+// where there is none, -1 where the running sum falls below one half again (or becomes a NaN) and the bins alone decide.
+__device__ __forceinline__ void save_crossing(float* __restrict__ saved, long long P, long long p, const Walked& s, float alpha, int D) {
+  saved[p] = alpha;
+  saved[P + p] = s.pmid;
+  saved[2 * P + p] = !s.regular ? -1.f : (float)(s.found ? s.cidx : D);
+}
+
+template <int VEC, bool BACKWARD, bool SAVE>
 __global__ __launch_bounds__(64) void median_rows_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
-                                                         float* __restrict__ res, long long P, long long HW, int D, int Dp,
-                                                         long long first_tile) {
+                                                         float* __restrict__ res, float* __restrict__ saved, long long P,
+                                                         long long HW, int D, int Dp, long long first_tile) {
   extern __shared__ __align__(16) float tile[];  // 64 rows of pitch Dp
   const int lane = threadIdx.x;
   const long long p0 = (first_tile + blockIdx.x) * 64;
@@ -1597,46 +1644,30 @@ __global__ __launch_bounds__(64) void median_rows_kernel(const float* __restrict
   stage_rows<VEC, false>(vol + p0 * D, nullptr, tile, total, D, Dp, lane);
   __syncthreads();
   float* row = tile + lane * Dp;
-  // the walk of MM.cu:26-43 == MM.cu:59-75, without the early exit (the bins past the crossing are skipped by `found`)
-  // The crossing bin's interpolation (a double division) is formed once, after the walk: inside the loop it would run in
-  // every iteration in which ANY lane of the wavefront crosses.  The comparisons against 0.5 are the reference's
-  // (a float promoted to double compares as the float does).
-  bool found = false;
-  int cidx = 0;
-  float score = 0.f, pmid = 1.f, alpha = 0.f;
-  if (lane < npx) {
-#pragma unroll 4
-    for (int c = 0; c < D; c++) {
-      const float cScore = row[c];
-      const float sum = score + cScore;
-      const bool hit = !found && score < 0.5f && sum >= 0.5f;
-      pmid = hit ? cScore : pmid;
-      cidx = hit ? c : cidx;
-      found = found || hit;
-      score = found ? score : sum;  // (the running sum stops in front of the crossing bin)
-    }
-    if (found) alpha = (1. - 2. * score - pmid) / (2. * pmid);  // MM.cu:34
-  }
+  Walked s{false, true, 0, 0.f, 1.f};
+  if (lane < npx) s = walk_histogram<SAVE>(row, D);
+  const float alpha = s.found ? crossing_offset(s.before, s.pmid) : 0.f;
   const long long p = p0 + lane;
   const long long n = p / HW, q = p - n * HW;
   if (!BACKWARD) {
     if (lane < npx) {
-      res[n * 2 * HW + q] = found ? (float)cidx - 0.f + alpha : 0.f;  // MM.cu:35
-      res[n * 2 * HW + HW + q] = found ? pmid : 0.f;
+      res[n * 2 * HW + q] = s.found ? (float)s.cidx - 0.f + alpha : 0.f;  // MM.cu:35
+      res[n * 2 * HW + HW + q] = s.found ? s.pmid : 0.f;
+      if (SAVE) save_crossing(saved, P, p, s, alpha, D);
     }
     return;
   }
   if (lane < npx) {
     const float g0v = gin[n * 2 * HW + q], g1v = gin[n * 2 * HW + HW + q];
-    const float cross = g0v * alpha / (-pmid) + g1v;  // MM.cu:69
-    const float neg = -g0v / (2. * pmid);             // MM.cu:85
-    const float pos = +g0v / (2. * pmid);             // MM.cu:88
-    score = 0.f;
+    const float cross = g0v * alpha / (-s.pmid) + g1v;  // MM.cu:69
+    const float neg = -g0v / (2. * s.pmid);             // MM.cu:85
+    const float pos = +g0v / (2. * s.pmid);             // MM.cu:88
+    float score = 0.f;
 #pragma unroll 4
     for (int c = 0; c < D; c++) {  // MM.cu:77-92; the crossing bin keeps the value of MM.cu:69
       const float cScore = row[c];
       const float sum = score + cScore;
-      float g = (found && c == cidx) ? cross : 0.f;
+      float g = (s.found && c == s.cidx) ? cross : 0.f;
       g = (sum < 0.5f) ? neg : ((score >= 0.5f) ? pos : g);
       row[c] = g;
       score = sum;
@@ -1657,9 +1688,10 @@ __device__ __forceinline__ void lds_only_barrier() {
 // copy of the run), as a loop: a wavefront keeps the next tile's run in flight (NV 16-byte loads per lane, held in registers)
 // while it walks the current one.  With one tile per wavefront only a quarter of the resident wavefronts have loads in
 // flight at any time (the rest walk, store or are being launched), and the pass runs at half the rate memory allows.
-template <int NV, bool BACKWARD>
+template <int NV, bool BACKWARD, bool SAVE>
 __global__ __launch_bounds__(64) void median_stream_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
-                                                           float* __restrict__ res, long long tiles, long long HW, int D) {
+                                                           float* __restrict__ res, float* __restrict__ saved, long long tiles,
+                                                           long long P, long long HW, int D) {
   extern __shared__ __align__(16) float tile[];  // 64 rows of D floats
   const int lane = threadIdx.x;
   const int per = 16 * D;  // 16-byte elements of a tile
@@ -1692,35 +1724,24 @@ __global__ __launch_bounds__(64) void median_stream_kernel(const float* __restri
     const long long tn = t + gridDim.x;
     fetch(tn < tiles ? tn : t, tn < tiles);
     lds_only_barrier();  // (a full barrier would also wait for the loads just issued)
-    bool found = false;
-    int cidx = 0;
-    float score = 0.f, pmid = 1.f, alpha = 0.f;
-#pragma unroll 4
-    for (int c = 0; c < D; c++) {  // the walk of median_rows_kernel
-      const float cScore = row[c];
-      const float sum = score + cScore;
-      const bool hit = !found && score < 0.5f && sum >= 0.5f;
-      pmid = hit ? cScore : pmid;
-      cidx = hit ? c : cidx;
-      found = found || hit;
-      score = found ? score : sum;
-    }
-    if (found) alpha = (1. - 2. * score - pmid) / (2. * pmid);  // MM.cu:34
+    const Walked s = walk_histogram<SAVE>(row, D);
+    const float alpha = s.found ? crossing_offset(s.before, s.pmid) : 0.f;
     if (!BACKWARD) {
       const long long p = t * 64 + lane, n = p / HW, q = p - n * HW;
-      res[n * 2 * HW + q] = found ? (float)cidx - 0.f + alpha : 0.f;  // MM.cu:35
-      res[n * 2 * HW + HW + q] = found ? pmid : 0.f;
+      res[n * 2 * HW + q] = s.found ? (float)s.cidx - 0.f + alpha : 0.f;  // MM.cu:35
+      res[n * 2 * HW + HW + q] = s.found ? s.pmid : 0.f;
+      if (SAVE) save_crossing(saved, P, p, s, alpha, D);
     } else {
-      const float cross = g0v * alpha / (-pmid) + g1v;  // MM.cu:69
-      const float neg = -g0v / (2. * pmid);             // MM.cu:85
-      const float pos = +g0v / (2. * pmid);             // MM.cu:88
+      const float cross = g0v * alpha / (-s.pmid) + g1v;  // MM.cu:69
+      const float neg = -g0v / (2. * s.pmid);             // MM.cu:85
+      const float pos = +g0v / (2. * s.pmid);             // MM.cu:88
       float* wrow = tile + lane * D;
-      score = 0.f;
+      float score = 0.f;
 #pragma unroll 4
       for (int c = 0; c < D; c++) {  // MM.cu:77-92; the crossing bin keeps the value of MM.cu:69
         const float cScore = wrow[c];
         const float sum = score + cScore;
-        float g = (found && c == cidx) ? cross : 0.f;
+        float g = (s.found && c == s.cidx) ? cross : 0.f;
         g = (sum < 0.5f) ? neg : ((score >= 0.5f) ? pos : g);
         wrow[c] = g;
         score = sum;
@@ -1735,8 +1756,71 @@ __global__ __launch_bounds__(64) void median_stream_kernel(const float* __restri
   }
 }
 
-template <bool BACKWARD>
-void launch_median_rows(const float* vol, const float* gin, float* res, long long P, long long HW, int D, bool aligned,
+// Gradient of a histogram from the crossing that the forward pass saved (save_crossing): bins in front of it, the crossing
+// bin, bins behind it -- the volume is not read again, the pass writes it and little else.  One wavefront per 64 pixels, whose
+// gradients are one contiguous run; the three values of a pixel are handed out through LDS and every lane stores 16 bytes at a
+// time.  A run with a pixel whose bins alone decide goes through the reference's two walks.
+// Bound by the stores: 4 x 384 x 1248 x 33 42.6 us, 291 MB at 6.8 TB/s (from the volume: 88 us; plain stores instead of
+// non-temporal ones: 61.7), 2 x 187 x 621 x 64 13.1 us.
+template <int VEC>
+__global__ __launch_bounds__(64) void median_backward_saved_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
+                                                                   const float* __restrict__ saved, float* __restrict__ gvol,
+                                                                   long long P, long long HW, int D) {
+  __shared__ float tile[64][kPitch];
+  __shared__ float4 bins[64];  // value in front of the crossing, at it, its bin
+  typedef float vec4 __attribute__((ext_vector_type(4)));
+  const int lane = threadIdx.x;
+  const long long p0 = (long long)blockIdx.x * 64, p = p0 + lane;
+  const int npx = (int)min((long long)64, P - p0);
+  float g0v = 0.f, g1v = 0.f, alpha = 0.f, pmid = 1.f, at = 0.f;
+  if (lane < npx) {
+    const long long n = p / HW, q = p - n * HW;
+    g0v = gin[n * 2 * HW + q];
+    g1v = gin[n * 2 * HW + HW + q];
+    alpha = saved[p];
+    pmid = saved[P + p];
+    at = saved[2 * P + p];
+  }
+  if (__ballot(at < 0.f) != 0) {
+    backward_from_bins(vol, gvol, tile, p0, P, D, lane, g0v, g1v);
+    return;
+  }
+  const float cross = g0v * alpha / (-pmid) + g1v;  // MM.cu:69
+  const float neg = -g0v / (2. * pmid);             // MM.cu:85 (and MM.cu:88 with its sign turned)
+  bins[lane] = make_float4(neg, cross, at, 0.f);
+  __syncthreads();
+  const int total = npx * D;
+  float* dst = gvol + p0 * D;
+  constexpr int kStep = 64 * VEC;
+  const int qs = kStep / D, rs = kStep - qs * D;
+  int i = lane * VEC, px = i / D, b = i - px * D;
+  auto value = [&](const float4& v, int bin) {
+    const float f = (float)bin;
+    return f < v.z ? v.x : (f == v.z ? v.y : -v.x);
+  };
+  for (; i < total; i += kStep) {
+    const float4 v0 = bins[px];
+    if (VEC == 4) {  // (four bins of one pixel, or the last of one and the first of the next: at least four bins each)
+      const float4 v1 = bins[min(px + 1, 63)];
+      vec4 g;
+#pragma unroll
+      for (int k = 0; k < 4; k++) g[k] = b + k < D ? value(v0, b + k) : value(v1, b + k - D);
+      if (i + 3 < total) {
+        __builtin_nontemporal_store(g, reinterpret_cast<vec4*>(dst + i));
+      } else {
+        for (int k = 0; k < 4 && i + k < total; k++) dst[i + k] = g[k];
+      }
+    } else {
+      dst[i] = value(v0, b);
+    }
+    b += rs;
+    px += qs;
+    if (b >= D) { b -= D; px++; }
+  }
+}
+
+template <bool BACKWARD, bool SAVE>
+void launch_median_rows(const float* vol, const float* gin, float* res, float* saved, long long P, long long HW, int D, bool aligned,
                         hipStream_t stream) {
   const int Dp = D | 1;
   constexpr int kStreamNV = 10;
@@ -1744,20 +1828,20 @@ void launch_median_rows(const float* vol, const float* gin, float* res, long lon
     // full tiles in the streaming loop, the last partial tile (if any) below
     const long long tiles = P / 64;
     const long long waves = std::min<long long>(tiles, 16ll * inpaint::compute_unit_count());
-    hipLaunchKernelGGL((median_stream_kernel<kStreamNV, BACKWARD>), dim3((unsigned)waves), dim3(64), (size_t)64 * D * sizeof(float), stream,
-                       vol, gin, res, tiles, HW, D);
+    hipLaunchKernelGGL((median_stream_kernel<kStreamNV, BACKWARD, SAVE>), dim3((unsigned)waves), dim3(64), (size_t)64 * D * sizeof(float),
+                       stream, vol, gin, res, saved, tiles, P, HW, D);
     if (P % 64 == 0) return;
     // (the kernel below takes its pixels from P and blockIdx: give it the last tile only)
-    hipLaunchKernelGGL((median_rows_kernel<4, BACKWARD>), dim3(1), dim3(64), (size_t)64 * Dp * sizeof(float), stream, vol, gin, res, P, HW, D,
-                       Dp, tiles);
+    hipLaunchKernelGGL((median_rows_kernel<4, BACKWARD, SAVE>), dim3(1), dim3(64), (size_t)64 * Dp * sizeof(float), stream, vol, gin, res,
+                       saved, P, HW, D, Dp, tiles);
     return;
   }
   const dim3 grid((unsigned)((P + 63) / 64)), block(64);
   const size_t lds = (size_t)64 * Dp * sizeof(float);
   if (aligned && D >= 4)
-    hipLaunchKernelGGL((median_rows_kernel<4, BACKWARD>), grid, block, lds, stream, vol, gin, res, P, HW, D, Dp, 0ll);
+    hipLaunchKernelGGL((median_rows_kernel<4, BACKWARD, SAVE>), grid, block, lds, stream, vol, gin, res, saved, P, HW, D, Dp, 0ll);
   else
-    hipLaunchKernelGGL((median_rows_kernel<1, BACKWARD>), grid, block, lds, stream, vol, gin, res, P, HW, D, Dp, 0ll);
+    hipLaunchKernelGGL((median_rows_kernel<1, BACKWARD, SAVE>), grid, block, lds, stream, vol, gin, res, saved, P, HW, D, Dp, 0ll);
 }
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -1911,7 +1995,7 @@ int medimax_forward(const float* vol, float* out, int n, int ih, int iw, int num
     return fail(INPAINT_ERR_ARG, "medimax_forward: bad shape %dx%dx%dx%d", n, ih, iw, num_disp);
   const long long HW = (long long)ih * iw, P = n * HW;
   if (num_disp <= kMaxRowBins)
-    launch_median_rows<false>(vol, nullptr, out, P, HW, num_disp, aligned16(vol), (hipStream_t)stream);
+    launch_median_rows<false, false>(vol, nullptr, out, nullptr, P, HW, num_disp, aligned16(vol), (hipStream_t)stream);
   else
     hipLaunchKernelGGL(median_forward_kernel, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, (hipStream_t)stream, vol, out, P,
                      HW, num_disp);
@@ -1926,11 +2010,38 @@ int medimax_backward(const float* vol, const float* gin, float* gvol, int n, int
   const long long HW = (long long)ih * iw, P = n * HW;
   if (num_disp <= kMaxRowBins) {
     g_timer.begin((hipStream_t)stream);
-    launch_median_rows<true>(vol, gin, gvol, P, HW, num_disp, aligned16(vol) && aligned16(gvol), (hipStream_t)stream);
+    launch_median_rows<true, false>(vol, gin, gvol, nullptr, P, HW, num_disp, aligned16(vol) && aligned16(gvol), (hipStream_t)stream);
     g_timer.end((hipStream_t)stream, 1);
   } else
     hipLaunchKernelGGL(median_backward_kernel, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, (hipStream_t)stream, vol, gin,
                      gvol, P, HW, num_disp);
+  INPAINT_HIP(hipGetLastError());
+  return 0;
+}
+
+int medimax_forward_saving(const float* vol, float* out, float* saved, int n, int ih, int iw, int num_disp, void* stream) {
+  if (!vol || !out || !saved) return fail(INPAINT_ERR_ARG, "medimax_forward_saving: null pointer");
+  if (n < 1 || ih < 1 || iw < 1 || num_disp < 1 || num_disp > kMaxRowBins)
+    return fail(INPAINT_ERR_ARG, "medimax_forward_saving: bad shape %dx%dx%dx%d", n, ih, iw, num_disp);
+  const long long HW = (long long)ih * iw;
+  launch_median_rows<false, true>(vol, nullptr, out, saved, n * HW, HW, num_disp, aligned16(vol), (hipStream_t)stream);
+  INPAINT_HIP(hipGetLastError());
+  return 0;
+}
+
+int medimax_backward_saved(const float* vol, const float* gin, const float* saved, float* gvol, int n, int ih, int iw, int num_disp,
+                           void* stream) {
+  if (!vol || !gin || !saved || !gvol) return fail(INPAINT_ERR_ARG, "medimax_backward_saved: null pointer");
+  if (n < 1 || ih < 1 || iw < 1 || num_disp < 1 || num_disp > kMaxRowBins)
+    return fail(INPAINT_ERR_ARG, "medimax_backward_saved: bad shape %dx%dx%dx%d", n, ih, iw, num_disp);
+  const long long HW = (long long)ih * iw, P = n * HW;
+  const dim3 grid((unsigned)((P + 63) / 64)), block(64);
+  g_timer.begin((hipStream_t)stream);
+  if (aligned16(gvol) && num_disp >= 4)
+    hipLaunchKernelGGL((median_backward_saved_kernel<4>), grid, block, 0, (hipStream_t)stream, vol, gin, saved, gvol, P, HW, num_disp);
+  else
+    hipLaunchKernelGGL((median_backward_saved_kernel<1>), grid, block, 0, (hipStream_t)stream, vol, gin, saved, gvol, P, HW, num_disp);
+  g_timer.end((hipStream_t)stream, 1);
   INPAINT_HIP(hipGetLastError());
   return 0;
 }

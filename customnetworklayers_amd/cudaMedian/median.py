@@ -9,14 +9,19 @@ from . import median_cuda_ext
 class MedianFunction(Function):
     @staticmethod
     def forward(ctx, in_vol):  # median.py:18-44
-        outputs = median_cuda_ext.forward(in_vol.contiguous())
+        vol = in_vol.contiguous()
+        if ctx.needs_input_grad[0] and vol.dim() == 4 and vol.shape[3] <= median_cuda_ext.MAX_SAVED_BINS:
+            solution, saved = median_cuda_ext.forward_saving(vol)
+            ctx.save_for_backward(in_vol, saved)
+            return solution
+        outputs = median_cuda_ext.forward(vol)
         ctx.save_for_backward(in_vol)
         return outputs[0]
 
     @staticmethod
     def backward(ctx, grad_sol):  # median.py:47-56
-        (in_vol,) = ctx.saved_tensors
-        outputs = median_cuda_ext.backward(grad_sol.contiguous(), in_vol.contiguous())
+        in_vol, *saved = ctx.saved_tensors
+        outputs = median_cuda_ext.backward(grad_sol.contiguous(), in_vol.contiguous(), *saved)
         return outputs[0]
 
 

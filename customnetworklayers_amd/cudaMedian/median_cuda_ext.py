@@ -33,13 +33,20 @@ def _stream(t):
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
 
 
-def forward(in_vol):
-    """in_vol: (n,h,w,d), the d histogram bins innermost (median_cuda.cpp:43-46).  Returns [(n,2,h,w)]:
-    the median's position in bins and the mass of the bin that holds it."""
+MAX_SAVED_BINS = 255  # most bins forward_saving takes
+
+
+def _check_volume(in_vol):
     _check_input(in_vol, "in_vol")
     if in_vol.dim() != 4:
         raise ValueError("in_vol must be (n, h, w, d)")
-    n, h, w, d = in_vol.shape
+    return in_vol.shape
+
+
+def forward(in_vol):
+    """in_vol: (n,h,w,d), the d histogram bins innermost (median_cuda.cpp:43-46).  Returns [(n,2,h,w)]:
+    the median's position in bins and the mass of the bin that holds it."""
+    n, h, w, d = _check_volume(in_vol)
     solution = torch.empty((n, 2, h, w), dtype=torch.float32, device=in_vol.device)
     with torch.cuda.device(in_vol.device):
         rc = lib.medimax_forward(in_vol.data_ptr(), solution.data_ptr(), n, h, w, d, _stream(in_vol))
@@ -48,20 +55,40 @@ def forward(in_vol):
     return [solution]
 
 
-def backward(d_iGf, in_vol):
-    """d_iGf: (n,2,h,w) gradient wrt the result.  Returns [gradient wrt in_vol]."""
-    _check_input(in_vol, "in_vol")
+def forward_saving(in_vol):
+    """forward (at most MAX_SAVED_BINS bins) that also returns what backward takes as `saved`: [solution, saved (3,n,h,w)]."""
+    n, h, w, d = _check_volume(in_vol)
+    solution = torch.empty((n, 2, h, w), dtype=torch.float32, device=in_vol.device)
+    saved = torch.empty((3, n, h, w), dtype=torch.float32, device=in_vol.device)
+    with torch.cuda.device(in_vol.device):
+        rc = lib.medimax_forward_saving(in_vol.data_ptr(), solution.data_ptr(), saved.data_ptr(), n, h, w, d, _stream(in_vol))
+    if rc:
+        raise _ERRORS.get(rc, RuntimeError)("MediMax::forward failed: %s" % _last_error())
+    return [solution, saved]
+
+
+def backward(d_iGf, in_vol, saved=None):
+    """d_iGf: (n,2,h,w) gradient wrt the result.  Returns [gradient wrt in_vol].  `saved`: the second result of
+    forward_saving(in_vol); the gradient is the same without it, at the cost of a second read of the volume."""
+    n, h, w, d = _check_volume(in_vol)
     _check_input(d_iGf, "d_iGf")
-    if in_vol.dim() != 4:
-        raise ValueError("in_vol must be (n, h, w, d)")
-    n, h, w, d = in_vol.shape
     if tuple(d_iGf.shape) != (n, 2, h, w):
         raise ValueError("d_iGf must have shape (%d, 2, %d, %d), got %s" % (n, h, w, tuple(d_iGf.shape)))
     if d_iGf.device != in_vol.device:
         raise RuntimeError("all tensors must live on one device")
     outGrad = torch.empty_like(in_vol)
+    if saved is not None:
+        _check_input(saved, "saved")
+        if tuple(saved.shape) != (3, n, h, w):
+            raise ValueError("saved must have shape (3, %d, %d, %d), got %s" % (n, h, w, tuple(saved.shape)))
+        if saved.device != in_vol.device:
+            raise RuntimeError("all tensors must live on one device")
     with torch.cuda.device(in_vol.device):
-        rc = lib.medimax_backward(in_vol.data_ptr(), d_iGf.data_ptr(), outGrad.data_ptr(), n, h, w, d, _stream(in_vol))
+        if saved is None:
+            rc = lib.medimax_backward(in_vol.data_ptr(), d_iGf.data_ptr(), outGrad.data_ptr(), n, h, w, d, _stream(in_vol))
+        else:
+            rc = lib.medimax_backward_saved(in_vol.data_ptr(), d_iGf.data_ptr(), saved.data_ptr(), outGrad.data_ptr(), n, h, w, d,
+                                            _stream(in_vol))
     if rc:
         raise _ERRORS.get(rc, RuntimeError)("MediMax::backward failed: %s" % _last_error())
     return [outGrad]

@@ -64,6 +64,18 @@ int medimax_forward(const float* vol, float* out, int n, int ih, int iw, int num
 int medimax_backward(const float* vol, const float* gin, float* gvol, int n, int ih, int iw, int num_disp,
                      void* stream);
 
+/* The same two passes with the crossing handed from one to the other (no counterpart in the reference, whose backward pass walks
+ * the histogram again): the gradient of the backward pass is what medimax_backward computes from the same volume, bit for bit,
+ * without a second read of the volume.
+ *   saved : 3*n*ih*iw floats, written by medimax_forward_saving and read by medimax_backward_saved
+ *   vol   : the volume of the forward pass; the backward pass reads it where a running sum that has reached one half falls
+ *           below it again, or is not a number
+ * num_disp is at most 255.
+ */
+int medimax_forward_saving(const float* vol, float* out, float* saved, int n, int ih, int iw, int num_disp, void* stream);
+int medimax_backward_saved(const float* vol, const float* gin, const float* saved, float* gvol, int n, int ih, int iw,
+                           int num_disp, void* stream);
+
 /* Measurement hooks, as tvinpaint_profile / tvinpaint_profile_read: with profiling on, every backward
  * call brackets one kernel with a HIP event pair on the caller's stream; _read waits for them and returns their
  * total.  enable = 1: the per-source pass of the quadratic fit, the whole-histogram kernel of the median;
