@@ -198,7 +198,7 @@ def bench_flowaux(args, cfg, d):
         bwd = lambda: ext.backward(t["grad"], t["vol"])  # noqa: E731
         # forward reads the histogram once (it may stop early) and writes 2; backward reads it, the upstream and writes it
         bpp = dict(forward=4 * (dd + 2), backward=4 * (2 * dd + 2), kernel=4 * (2 * dd + 2))
-        kernel = "median_stream_kernel<10,true> (backward)"
+        kernel = "median_backward_stream_kernel<10> (backward)"
         shape = "histograms %dx%dx%d" % (h, w, dd)
     bpp["total"] = bpp["forward"] + bpp["backward"]  # "kernel": the dominant kernel alone
     for _ in range(args.warmup):

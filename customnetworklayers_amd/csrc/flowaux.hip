@@ -1517,6 +1517,7 @@ __global__ __launch_bounds__(256) void median_backward_kernel(const float* __res
 // HBM sees the histogram once per pass.
 // ---------------------------------------------------------------------------------------------
 constexpr int kMaxRowBins = 255;
+constexpr int kWalkAhead = 8;  // LDS reads in flight in the forward walk
 
 // In: kBatch loads per lane are issued before the first of them is stored to LDS (a loop that stores each value right
 // after its load waits for memory once per element: 9 round trips per wavefront at 33 bins where one or two suffice).
@@ -1602,22 +1603,24 @@ struct Walked {
   int cidx;
   float before, pmid;  // sum in front of the crossing bin, its mass
 };
+// What the walk does with one bin
+template <bool CHECK>
+__device__ __forceinline__ void walk_bin(Walked& s, float& run, float mass, int c) {
+  const float sum = run + mass;
+  const bool half = sum >= 0.5f, hit = half && !s.found;
+  s.pmid = hit ? mass : s.pmid;
+  s.cidx = hit ? c : s.cidx;
+  s.before = hit ? run : s.before;
+  if (CHECK) s.regular = s.regular && (half || !s.found);
+  s.found = s.found || half;
+  run = sum;
+}
 template <bool CHECK>
 __device__ __forceinline__ Walked walk_histogram(const float* row, int D) {
   Walked s{false, true, 0, 0.f, 1.f};
   float run = 0.f;
 #pragma unroll 4
-  for (int c = 0; c < D; c++) {
-    const float cScore = row[c];
-    const float sum = run + cScore;
-    const bool half = sum >= 0.5f, hit = half && !s.found;
-    s.pmid = hit ? cScore : s.pmid;
-    s.cidx = hit ? c : s.cidx;
-    s.before = hit ? run : s.before;
-    if (CHECK) s.regular = s.regular && (half || !s.found);
-    s.found = s.found || half;
-    run = sum;
-  }
+  for (int c = 0; c < D; c++) walk_bin<CHECK>(s, run, row[c], c);
   if (CHECK) s.regular = s.regular && (s.found || run == run);
   return s;
 }
@@ -1677,6 +1680,81 @@ __global__ __launch_bounds__(64) void median_rows_kernel(const float* __restrict
   stage_rows<VEC, true>(nullptr, res + p0 * D, tile, total, D, Dp, lane);
 }
 
+// The forward pass with the run of 64 histograms going from memory straight into LDS (global_load_lds, 16 bytes a lane): all
+// loads of a tile are in flight at once, where staging through registers had eight a lane and then waited.  The run stands in
+// LDS as in memory and a lane reads RD bins of its row at a time: one where the bin count is odd, two where it is twice an odd
+// number, four where it is a multiple of four.  In the last case rows whose pitch would put neighbours into the same banks
+// have their 16-byte pieces rotated, row by row, on the way in (the loads pick the piece, LDS takes them in lane order).
+// Bound by memory; behind it the walk, where long rows leave room for few wavefronts in LDS (100 bins: six a CU).  us, staged
+// through registers / so: 4 x 384 x 1248 x 33 51.9 / 44.3 (6.1 TB/s), x 16 25.9 / 23.0, x 22 33.9 / 31.1; 384 x 1248 x 65 49.5 /
+// 26.3, x 64 32.2 / 24.9; 2 x 384 x 1248 x 128 187 / 120; 2 x 187 x 621 x 64 19.6 / 15.6; 100 x 140 x 33 7.7 / 4.4.  Without the
+// non-temporal hint 47.1 at 33 bins; four reads ahead instead of eight 123 at 128 bins.
+template <int RD, bool SAVE>
+__global__ __launch_bounds__(64) void median_forward_run_kernel(const float* __restrict__ vol, float* __restrict__ res,
+                                                                float* __restrict__ saved, long long P, long long HW, int D) {
+  extern __shared__ __align__(16) float tile[];  // 64 rows of D floats
+  typedef const __attribute__((address_space(1))) void* GlobalPtr;
+  typedef __attribute__((address_space(3))) void* LdsPtr;
+  typedef float vec __attribute__((ext_vector_type(RD)));
+  constexpr int kReadOnce = 2;  // the instruction's non-temporal bit
+  const int lane = threadIdx.x;
+  const long long p0 = (long long)blockIdx.x * 64, p = p0 + lane;
+  const int npx = (int)min((long long)64, P - p0);
+  const int total = npx * D, pieces = total >> 2;  // (at least one: npx * D >= 4)
+  const float* const src = vol + p0 * D;
+  // rotation of a row, RD == 4: a row is D4 pieces long; banks repeat every 16 pieces, so of each 16 / g rows, g the common
+  // factors of 16 and D4, the pieces j already lie in different banks, and the next 16 / g rows are turned by one more piece
+  const int D4 = D >> 2, shift = RD == 4 ? max(0, 4 - (__ffs(D4) - 1)) : 0, turns = RD == 4 ? min(16, D4 & -D4) - 1 : 0;
+  auto rotation = [&](int px) { return (px >> shift) & turns; };
+  if (RD == 4) {
+    const int qs = 64 / D4, rs = 64 - qs * D4;
+    int px = lane / D4, slot = lane - px * D4;
+    for (int i = 0; i < total; i += 256) {  // (lane l writes piece i / 4 + l)
+      int j = slot - rotation(px);
+      j += j < 0 ? D4 : 0;
+      const int piece = px < npx ? px * D4 + j : 0;
+      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + 4 * piece), (LdsPtr)(tile + i), 16, 0, kReadOnce);
+      slot += rs;
+      px += qs;
+      if (slot >= D4) { slot -= D4; px++; }
+    }
+  } else {
+    for (int i = 0; i < total; i += 256)
+      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + 4 * min((i >> 2) + lane, pieces - 1)), (LdsPtr)(tile + i), 16, 0, kReadOnce);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (RD != 4 && lane < (total & 3)) tile[4 * pieces + lane] = src[4 * pieces + lane];
+  __syncthreads();
+  Walked s{false, true, 0, 0.f, 1.f};
+  float run = 0.f;
+  if (lane < npx) {
+    const vec* const row = reinterpret_cast<const vec*>(tile) + lane * (D / RD);
+    const int per = D / RD, r = RD == 4 ? rotation(lane) : 0;
+    for (int j0 = 0; j0 < per; j0 += kWalkAhead) {
+      vec v[kWalkAhead];
+#pragma unroll
+      for (int u = 0; u < kWalkAhead; u++) {
+        int slot = min(j0 + u, per - 1) + r;
+        if (RD == 4) slot -= slot >= per ? per : 0;
+        v[u] = row[slot];
+      }
+#pragma unroll
+      for (int u = 0; u < kWalkAhead; u++)
+        if (j0 + u < per) {
+#pragma unroll
+          for (int k = 0; k < RD; k++) walk_bin<SAVE>(s, run, v[u][k], (j0 + u) * RD + k);
+        }
+      if (!SAVE && __ballot(!s.found) == 0) break;
+    }
+    if (SAVE) s.regular = s.regular && (s.found || run == run);
+    const float alpha = s.found ? crossing_offset(s.before, s.pmid) : 0.f;
+    const long long n = p / HW, q = p - n * HW;
+    res[n * 2 * HW + q] = s.found ? (float)s.cidx - 0.f + alpha : 0.f;  // MM.cu:35
+    res[n * 2 * HW + HW + q] = s.found ? s.pmid : 0.f;
+    if (SAVE) save_crossing(saved, P, p, s, alpha, D);
+  }
+}
+
 // Workgroup barrier that orders LDS traffic only: global loads issued before it stay in flight.
 __device__ __forceinline__ void lds_only_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -1684,14 +1762,13 @@ __device__ __forceinline__ void lds_only_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The same pass over FULL tiles of 64 pixels for odd bin counts up to 4 * NV - 1 (no padding: the tile in LDS is a plain
+// The backward pass over FULL tiles of 64 pixels for odd bin counts up to 4 * NV - 1 (no padding: the tile in LDS is a plain
 // copy of the run), as a loop: a wavefront keeps the next tile's run in flight (NV 16-byte loads per lane, held in registers)
 // while it walks the current one.  With one tile per wavefront only a quarter of the resident wavefronts have loads in
 // flight at any time (the rest walk, store or are being launched), and the pass runs at half the rate memory allows.
-template <int NV, bool BACKWARD, bool SAVE>
-__global__ __launch_bounds__(64) void median_stream_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
-                                                           float* __restrict__ res, float* __restrict__ saved, long long tiles,
-                                                           long long P, long long HW, int D) {
+template <int NV>
+__global__ __launch_bounds__(64) void median_backward_stream_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
+                                                                    float* __restrict__ res, long long tiles, long long HW, int D) {
   extern __shared__ __align__(16) float tile[];  // 64 rows of D floats
   const int lane = threadIdx.x;
   const int per = 16 * D;  // 16-byte elements of a tile
@@ -1706,11 +1783,9 @@ __global__ __launch_bounds__(64) void median_stream_kernel(const float* __restri
     const int last = live ? per : 0;
 #pragma unroll
     for (int u = 0; u < NV; u++) v[u] = __builtin_nontemporal_load(src + (lane + 64 * u < last ? lane + 64 * u : lane));  // read once
-    if (BACKWARD) {
-      const long long p = t * 64 + lane, n = p / HW, q = p - n * HW;
-      gn0 = gin[n * 2 * HW + q];
-      gn1 = gin[n * 2 * HW + HW + q];
-    }
+    const long long p = t * 64 + lane, n = p / HW, q = p - n * HW;
+    gn0 = gin[n * 2 * HW + q];
+    gn1 = gin[n * 2 * HW + HW + q];
   };
   long long t = blockIdx.x;
   if (t >= tiles) return;
@@ -1724,34 +1799,27 @@ __global__ __launch_bounds__(64) void median_stream_kernel(const float* __restri
     const long long tn = t + gridDim.x;
     fetch(tn < tiles ? tn : t, tn < tiles);
     lds_only_barrier();  // (a full barrier would also wait for the loads just issued)
-    const Walked s = walk_histogram<SAVE>(row, D);
+    const Walked s = walk_histogram<false>(row, D);
     const float alpha = s.found ? crossing_offset(s.before, s.pmid) : 0.f;
-    if (!BACKWARD) {
-      const long long p = t * 64 + lane, n = p / HW, q = p - n * HW;
-      res[n * 2 * HW + q] = s.found ? (float)s.cidx - 0.f + alpha : 0.f;  // MM.cu:35
-      res[n * 2 * HW + HW + q] = s.found ? s.pmid : 0.f;
-      if (SAVE) save_crossing(saved, P, p, s, alpha, D);
-    } else {
-      const float cross = g0v * alpha / (-s.pmid) + g1v;  // MM.cu:69
-      const float neg = -g0v / (2. * s.pmid);             // MM.cu:85
-      const float pos = +g0v / (2. * s.pmid);             // MM.cu:88
-      float* wrow = tile + lane * D;
-      float score = 0.f;
+    const float cross = g0v * alpha / (-s.pmid) + g1v;  // MM.cu:69
+    const float neg = -g0v / (2. * s.pmid);             // MM.cu:85
+    const float pos = +g0v / (2. * s.pmid);             // MM.cu:88
+    float* wrow = tile + lane * D;
+    float score = 0.f;
 #pragma unroll 4
-      for (int c = 0; c < D; c++) {  // MM.cu:77-92; the crossing bin keeps the value of MM.cu:69
-        const float cScore = wrow[c];
-        const float sum = score + cScore;
-        float g = (s.found && c == s.cidx) ? cross : 0.f;
-        g = (sum < 0.5f) ? neg : ((score >= 0.5f) ? pos : g);
-        wrow[c] = g;
-        score = sum;
-      }
-      lds_only_barrier();
-      vec4* dst = reinterpret_cast<vec4*>(res) + t * per;
-#pragma unroll
-      for (int u = 0; u < NV; u++)
-        if (lane + 64 * u < per) dst[lane + 64 * u] = tile4[lane + 64 * u];  // (plain stores: the non-temporal hint costs this pass 7%)
+    for (int c = 0; c < D; c++) {  // MM.cu:77-92; the crossing bin keeps the value of MM.cu:69
+      const float cScore = wrow[c];
+      const float sum = score + cScore;
+      float g = (s.found && c == s.cidx) ? cross : 0.f;
+      g = (sum < 0.5f) ? neg : ((score >= 0.5f) ? pos : g);
+      wrow[c] = g;
+      score = sum;
     }
+    lds_only_barrier();
+    vec4* dst = reinterpret_cast<vec4*>(res) + t * per;
+#pragma unroll
+    for (int u = 0; u < NV; u++)
+      if (lane + 64 * u < per) dst[lane + 64 * u] = tile4[lane + 64 * u];  // (plain stores: the non-temporal hint costs this pass 7%)
     lds_only_barrier();  // the next tile overwrites the rows
   }
 }
@@ -1824,12 +1892,20 @@ void launch_median_rows(const float* vol, const float* gin, float* res, float* s
                         hipStream_t stream) {
   const int Dp = D | 1;
   constexpr int kStreamNV = 10;
-  if (aligned && (D & 1) && D >= 5 && D < 4 * kStreamNV && P >= 64 && !inpaint::knobs().median_tile_per_wave) {
+  if (!BACKWARD && aligned && D >= 4 && !inpaint::knobs().median_tile_per_wave) {
+    const dim3 grid((unsigned)((P + 63) / 64)), block(64);
+    const size_t lds = (size_t)64 * D * sizeof(float);
+    if (D % 4 == 0) hipLaunchKernelGGL((median_forward_run_kernel<4, SAVE>), grid, block, lds, stream, vol, res, saved, P, HW, D);
+    else if (D % 2 == 0) hipLaunchKernelGGL((median_forward_run_kernel<2, SAVE>), grid, block, lds, stream, vol, res, saved, P, HW, D);
+    else hipLaunchKernelGGL((median_forward_run_kernel<1, SAVE>), grid, block, lds, stream, vol, res, saved, P, HW, D);
+    return;
+  }
+  if (BACKWARD && aligned && (D & 1) && D >= 5 && D < 4 * kStreamNV && P >= 64 && !inpaint::knobs().median_tile_per_wave) {
     // full tiles in the streaming loop, the last partial tile (if any) below
     const long long tiles = P / 64;
     const long long waves = std::min<long long>(tiles, 16ll * inpaint::compute_unit_count());
-    hipLaunchKernelGGL((median_stream_kernel<kStreamNV, BACKWARD, SAVE>), dim3((unsigned)waves), dim3(64), (size_t)64 * D * sizeof(float),
-                       stream, vol, gin, res, saved, tiles, P, HW, D);
+    hipLaunchKernelGGL((median_backward_stream_kernel<kStreamNV>), dim3((unsigned)waves), dim3(64), (size_t)64 * D * sizeof(float),
+                       stream, vol, gin, res, tiles, HW, D);
     if (P % 64 == 0) return;
     // (the kernel below takes its pixels from P and blockIdx: give it the last tile only)
     hipLaunchKernelGGL((median_rows_kernel<4, BACKWARD, SAVE>), dim3(1), dim3(64), (size_t)64 * Dp * sizeof(float), stream, vol, gin, res,
