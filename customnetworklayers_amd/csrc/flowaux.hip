@@ -280,6 +280,21 @@ __device__ __forceinline__ Factors scatter_factors(const Fit& f, const float* __
   return k;
 }
 
+// a source's scatter coefficients (contribution to g1 at a tap = I1 * coefficient, QF.cu:279-283,296) and its entry in the list
+// of the position it lands on
+__device__ __forceinline__ void store_source(const QfWorkspace& ws, const Factors& k, long long P, long long base, long long t,
+                                             long long landing, unsigned p) {
+  ws.coef[0 * P + t] = k.any_valid ? (float)(0.5 * k.k00) : k.dFds;
+  ws.coef[1 * P + t] = k.any_valid ? 0.5f * k.k0p : 0.f;
+  ws.coef[2 * P + t] = k.any_valid ? 0.5f * k.k0m : 0.f;
+  ws.coef[3 * P + t] = k.any_valid ? 0.5f * k.kp0 : 0.f;
+  ws.coef[4 * P + t] = k.any_valid ? 0.5f * k.km0 : 0.f;
+  const long long centre = base + landing;
+  const int pos = atomicAdd(ws.count + centre, 1);
+  if (pos < kSlots) ws.slots[centre * kSlots + pos] = (int)p;
+  else ws.ovf[atomicAdd(ws.ovf_count, 1)] = (int)t;
+}
+
 __global__ __launch_bounds__(256) void quadfit_backward_sources(const float* __restrict__ im0, const float* __restrict__ im1,
                                                                 const float* __restrict__ flow, const float* __restrict__ gin,
                                                                 float* __restrict__ g0, QfWorkspace ws, int N, int d, int H,
@@ -300,16 +315,7 @@ __global__ __launch_bounds__(256) void quadfit_backward_sources(const float* __r
     return;
   }
   const Factors k = scatter_factors(f, gin, n, HW, p);
-  // scatter coefficients: contribution to g1 at a tap = I1 * coefficient (QF.cu:279-283,296)
-  ws.coef[0 * P + t] = k.any_valid ? (float)(0.5 * k.k00) : k.dFds;
-  ws.coef[1 * P + t] = k.any_valid ? 0.5f * k.k0p : 0.f;
-  ws.coef[2 * P + t] = k.any_valid ? 0.5f * k.k0m : 0.f;
-  ws.coef[3 * P + t] = k.any_valid ? 0.5f * k.kp0 : 0.f;
-  ws.coef[4 * P + t] = k.any_valid ? 0.5f * k.km0 : 0.f;
-  const long long centre = (long long)n * HW + f.o00;
-  const int pos = atomicAdd(ws.count + centre, 1);
-  if (pos < kSlots) ws.slots[centre * kSlots + pos] = (int)p;
-  else ws.ovf[atomicAdd(ws.ovf_count, 1)] = (int)t;
+  store_source(ws, k, P, (long long)n * HW, t, f.o00, p);
   if (k.any_valid) {
 #pragma unroll 4
     for (int cc = 0; cc < d; cc++) {  // QF.cu:286-290
@@ -573,7 +579,7 @@ template <int PX>              // PX pixels per lane (rows PX * wave + i): tile 
 struct TileCfg {
   static constexpr int TH = 4 * PX, ELEMS = (96 * (4 * PX + 16) + 255) / 256 * 256;
 };
-constexpr int kPxForward = 2, kPxSources = 2;
+constexpr int kPxTile = 2;
 
 struct Box {
   int x0, y0, w, h;
@@ -812,12 +818,12 @@ __device__ __forceinline__ bool tile_of_block(int N, int tiles_x, int tiles_y, i
   return true;
 }
 
-// MODE 0: the forward pass (QF.cu:14-139).  MODE 1: pass A of the backward pass (fit, g0, coefficients, lists).
-template <int MODE, int PX>
-__global__ __launch_bounds__(256) void quadfit_tiles(const float* __restrict__ im0, const float* __restrict__ im1,
-                                                     const float* __restrict__ flow, const float* __restrict__ gin,
-                                                     float* __restrict__ res, QfWorkspace ws, int N, int d, int H, int W,
-                                                     int fc, int tiles_x, int tiles_y) {
+// Pass A of the backward pass (fit, g0, coefficients, lists), the second map read twice.
+__global__ __launch_bounds__(256) void quadfit_sources_tiles(const float* __restrict__ im0, const float* __restrict__ im1,
+                                                             const float* __restrict__ flow, const float* __restrict__ gin,
+                                                             float* __restrict__ res, QfWorkspace ws, int N, int d, int H, int W,
+                                                             int fc, int tiles_x, int tiles_y) {
+  constexpr int PX = kPxTile;
   constexpr int kPX = PX, kTH = TileCfg<PX>::TH;
   __shared__ float win[2][TileCfg<PX>::ELEMS];
   __shared__ int red[16];
@@ -874,20 +880,6 @@ __global__ __launch_bounds__(256) void quadfit_tiles(const float* __restrict__ i
     f[i].c00 = f[i].ax = f[i].ay = f[i].bx = f[i].by = f[i].fx = f[i].fy = 0.f;
     if (px[i].inside) finish_fit(f[i], cost[i][0], cost[i][1], cost[i][3], cost[i][2], cost[i][4], px[i].ix, px[i].iy, H, W);
   }
-  if (MODE == 0) {
-#pragma unroll
-    for (int i = 0; i < kPX; i++) {
-      if (!valid[i]) continue;
-      float* o = res + (size_t)n * 3 * HW + px[i].p;
-      float score = 0.f;
-      if (f[i].inside)  // QF.cu:136
-        score = f[i].ax * f[i].fx * f[i].fx + f[i].bx * f[i].fx + f[i].c00 + f[i].ay * f[i].fy * f[i].fy + f[i].by * f[i].fy;
-      o[0] = f[i].fx;
-      o[HW] = f[i].fy;
-      o[2 * HW] = score;
-    }
-    return;
-  }
   float* G0 = res + (size_t)n * d * HW;
   Factors k[kPX];
 #pragma unroll
@@ -900,15 +892,7 @@ __global__ __launch_bounds__(256) void quadfit_tiles(const float* __restrict__ i
     if (!px[i].inside) continue;
     k[i] = scatter_factors(f[i], gin, n, HW, px[i].p);
     const long long t = (long long)n * HW + px[i].p;
-    ws.coef[0 * P + t] = k[i].any_valid ? (float)(0.5 * k[i].k00) : k[i].dFds;  // QF.cu:279-283,296
-    ws.coef[1 * P + t] = k[i].any_valid ? 0.5f * k[i].k0p : 0.f;
-    ws.coef[2 * P + t] = k[i].any_valid ? 0.5f * k[i].k0m : 0.f;
-    ws.coef[3 * P + t] = k[i].any_valid ? 0.5f * k[i].kp0 : 0.f;
-    ws.coef[4 * P + t] = k[i].any_valid ? 0.5f * k[i].km0 : 0.f;
-    const long long centre = (long long)n * HW + (long long)px[i].iy * W + px[i].ix;
-    const int pos = atomicAdd(ws.count + centre, 1);
-    if (pos < kSlots) ws.slots[centre * kSlots + pos] = (int)px[i].p;
-    else ws.ovf[atomicAdd(ws.ovf_count, 1)] = (int)t;
+    store_source(ws, k[i], P, (long long)n * HW, t, (long long)px[i].iy * W + px[i].ix, px[i].p);
   }
   auto nothing = [](int) { return 0; };
   window_pass<PX>(q, d, HW, W, box, win, nothing, [&](int cc, const float* buf, const float* plane, int, bool live) {
@@ -926,8 +910,8 @@ __global__ __launch_bounds__(256) void quadfit_tiles(const float* __restrict__ i
 // Pass A of the backward pass with one read of the second feature map.  The gradient wrt the first map needs
 // the finished fit (all channels) and then the five taps of every channel again.  Here a lane owns ONE pixel and
 // keeps its taps of up to DMAX channels in registers (5 * DMAX floats) while the windows stream through LDS, so
-// the second sweep over the channels is arithmetic and stores only.  Same sums in the same order as MODE 1 of
-// quadfit_tiles (QF.cu:63-71 for the costs, QF.cu:279-297 for the gradient).
+// the second sweep over the channels is arithmetic and stores only.  Same sums in the same order as
+// quadfit_sources_tiles (QF.cu:63-71 for the costs, QF.cu:279-297 for the gradient).
 constexpr int kResidentChannels = 32;
 constexpr int kResidentRows = 4;      // tile height: one row per wavefront
 constexpr int kResidentElems = 1024;  // window capacity in floats (a 64 x 4 tile with +-3 pixels of spread needs ~800)
@@ -1051,15 +1035,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   finish_fit(f, cost[0], cost[1], cost[3], cost[2], cost[4], px.ix, px.iy, H, W);
   const Factors kf = scatter_factors(f, gin, n, HW, px.p);
   const long long t = (long long)n * HW + px.p;
-  ws.coef[0 * P + t] = kf.any_valid ? (float)(0.5 * kf.k00) : kf.dFds;  // QF.cu:279-283,296
-  ws.coef[1 * P + t] = kf.any_valid ? 0.5f * kf.k0p : 0.f;
-  ws.coef[2 * P + t] = kf.any_valid ? 0.5f * kf.k0m : 0.f;
-  ws.coef[3 * P + t] = kf.any_valid ? 0.5f * kf.kp0 : 0.f;
-  ws.coef[4 * P + t] = kf.any_valid ? 0.5f * kf.km0 : 0.f;
-  const long long centre = (long long)n * HW + (long long)px.iy * W + px.ix;
-  const int pos = atomicAdd(ws.count + centre, 1);
-  if (pos < kSlots) ws.slots[centre * kSlots + pos] = (int)px.p;
-  else ws.ovf[atomicAdd(ws.ovf_count, 1)] = (int)t;
+  store_source(ws, kf, P, (long long)n * HW, t, (long long)px.iy * W + px.ix, px.p);
 #pragma unroll
   for (int c = 0; c < DMAX; c++) {
     if (c < d) {
@@ -1071,6 +1047,302 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       __builtin_nontemporal_store(g, &G0[(size_t)c * HW + px.p]);  // (the caller reads it, later: kept out of the caches, it leaves them to the windows)
     }
   }
+}
+
+// Reads of LDS issued together and waited for once, as one block the compiler does not look into: before an LDS read that it
+// sees, it waits for the loads into LDS that may alias it, and with the buffers of a ring it takes that to be all of them -- the
+// whole prefetch queue.  The caller has waited for the buffer's own loads.
+constexpr int kPairs = 12;
+__device__ __forceinline__ void lds_read12(const unsigned (&a)[kPairs], float (&v)[kPairs]) {  // (byte addresses)
+  asm volatile(
+      "ds_read_b32 %0, %12\n\tds_read_b32 %1, %13\n\tds_read_b32 %2, %14\n\tds_read_b32 %3, %15\n\t"
+      "ds_read_b32 %4, %16\n\tds_read_b32 %5, %17\n\tds_read_b32 %6, %18\n\tds_read_b32 %7, %19\n\t"
+      "ds_read_b32 %8, %20\n\tds_read_b32 %9, %21\n\tds_read_b32 %10, %22\n\tds_read_b32 %11, %23\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]),
+        "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9]), "v"(a[10]),
+        "v"(a[11])
+      : "memory");
+}
+__device__ __forceinline__ void lds_read10(const unsigned (&a)[10], float (&v)[10]) {
+  asm volatile(
+      "ds_read_b32 %0, %10\n\tds_read_b32 %1, %11\n\tds_read_b32 %2, %12\n\tds_read_b32 %3, %13\n\tds_read_b32 %4, %14\n\t"
+      "ds_read_b32 %5, %15\n\tds_read_b32 %6, %16\n\tds_read_b32 %7, %17\n\tds_read_b32 %8, %18\n\tds_read_b32 %9, %19\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]),
+        "=&v"(v[9])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9])
+      : "memory");
+}
+// (element offsets into one buffer)
+__device__ __forceinline__ void lds_gather12(const float* buf, const unsigned (&off)[kPairs], float (&v)[kPairs]) {
+  const unsigned b = (unsigned)(size_t)(const __attribute__((address_space(3))) float*)buf;
+  unsigned a[kPairs];
+#pragma unroll
+  for (int j = 0; j < kPairs; j++) a[j] = b + 4u * off[j];
+  lds_read12(a, v);
+}
+
+// The forward pass, and pass A of the backward pass when the forward pass has left its five costs per pixel, with everything
+// the channel loop reads coming from memory straight into LDS (global_load_lds): the window of the second map and, forward, the
+// tile's own pixels of the first.  No load of the loop has a register as its target, so nothing but the ring's own count is
+// waited for, and one barrier per channel is all the synchronisation.  With the costs at hand pass A streams the second map
+// once and keeps no taps: resident in registers they allow two wavefronts per SIMD and every map is read twice.
+// A pixel whose taps leave the window's capacity is worked out from memory behind the loop.
+// Bound by memory.  4 x 32 x 384 x 1248, us: forward 153 -> 121 (590 MB at 4.9 TB/s), with the costs stored 127; pass A 268 -> 160;
+// 2 x 64 x 192 x 624 forward + backward 222 -> 134, 2 x 48 x 448 x 1280 660 -> 422.  With 4 pixels of noise on the flow (a fifth of
+// the pixels outside the window) 1230 -> 1020, with 12 (nearly all) as before.
+constexpr int kRingElems = 8448;  // floats of LDS for the ring: four blocks per CU
+constexpr int kFarThreads = 128;
+
+// Streams the windows of planes q[0 .. d) (and, FIRST, the tile's pixels of planes a[0 .. d)) through STAGES buffers: while
+// channel c is consumed, STAGES - 1 more are on their way.  Loads return in order: when at most the loads of STAGES - 2
+// channels are outstanding, channel c has landed (a wavefront's stores in between make the wait longer, never shorter).  A
+// buffer is refilled one barrier after its consumption.
+template <int PX, int PER, int STAGES, bool FIRST, typename Consume>
+__device__ __forceinline__ void ring_pass_of(const float* __restrict__ q, const float* __restrict__ a, const unsigned (&pix)[PX], int d,
+                                             size_t HW, int W, const Box& box, float* ring, Consume consume) {
+  typedef const __attribute__((address_space(1))) void* GlobalPtr;
+  typedef __attribute__((address_space(3))) void* LdsPtr;
+  constexpr int kLoads = PER + (FIRST ? PX : 0), kStage = 256 * kLoads;
+  static_assert(kStage * STAGES <= kRingElems && (STAGES - 2) * kLoads < 63, "the ring's space; the counter's range");
+  const int count = box.w * box.h;
+  unsigned goff[PER];
+  const float inv_w = 1.0f / (float)max(box.w, 1);
+#pragma unroll
+  for (int k = 0; k < PER; k++) {  // (row e / w, column e % w, exact in float for these sizes; past the window: its first element)
+    const int e = threadIdx.x + 256 * k;
+    const int r = (int)(((float)e + 0.5f) * inv_w);
+    goff[k] = e < count ? (unsigned)(r * W + (e - r * box.w)) : 0u;
+  }
+  const float* corner = q + (size_t)box.y0 * W + box.x0;
+  const int wave_first = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
+  auto fetch = [&](int c, float* buf) {
+    const float* src = corner + (size_t)c * HW;
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + goff[k]), (LdsPtr)(buf + 256 * k + wave_first), 4, 0, 0);
+    if (FIRST) {
+      const float* own = a + (size_t)c * HW;
+#pragma unroll
+      for (int i = 0; i < PX; i++)
+        __builtin_amdgcn_global_load_lds((GlobalPtr)(own + pix[i]), (LdsPtr)(buf + 256 * (PER + i) + wave_first), 4, 0, 0);
+    }
+  };
+  // (what the wavefront has in flight already is not the ring's: the count starts from nothing)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int c = 0; c < STAGES - 1; c++)
+    if (c < d) fetch(c, ring + c * kStage);
+  int at = 0, refill = STAGES - 1;
+  for (int c = 0; c < d; c++) {
+    if (c + STAGES - 2 < d) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((STAGES - 2) * kLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (c + STAGES - 1 < d) fetch(c + STAGES - 1, ring + refill * kStage);
+    consume(c, (unsigned)(size_t)(const __attribute__((address_space(3))) float*)(ring + at * kStage), 256u * PER);
+    at = at + 1 == STAGES ? 0 : at + 1;
+    refill = refill + 1 == STAGES ? 0 : refill + 1;
+  }
+}
+template <int PX, bool FIRST, typename Consume>
+__device__ __forceinline__ void ring_pass(const float* __restrict__ q, const float* __restrict__ a, const unsigned (&pix)[PX], int d,
+                                          size_t HW, int W, const Box& box, float* ring, Consume consume) {
+  static_assert(PX == 2 && TileCfg<PX>::ELEMS == 9 * 256, "loads per thread: 4 to 9");
+  const int count = __builtin_amdgcn_readfirstlane(box.w * box.h);
+  if (count <= 4 * 256) ring_pass_of<PX, 4, 5, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
+  else if (count <= 6 * 256) ring_pass_of<PX, 6, 4, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
+  else ring_pass_of<PX, 9, 3, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
+}
+
+// MODE 0: the forward pass (costs: its five sums per pixel, a plane of N * H * W each, or null).  MODE 1: pass A from the costs.
+template <int MODE>
+__global__ __launch_bounds__(256) void quadfit_ring_tiles(const float* __restrict__ im0, const float* __restrict__ im1,
+                                                          const float* __restrict__ flow, const float* __restrict__ gin,
+                                                          float* __restrict__ costs, float* __restrict__ res, QfWorkspace ws, int N,
+                                                          int d, int H, int W, int fc, int tiles_x, int tiles_y) {
+  constexpr int PX = kPxTile, kTH = TileCfg<PX>::TH;
+  __shared__ __align__(16) float ring[kRingElems];
+  __shared__ int red[16];
+  int n, tx, ty;
+  if (!tile_of_block(N, tiles_x, tiles_y, n, tx, ty)) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const size_t HW = (size_t)H * W;
+  const long long P = (long long)N * HW, base = (long long)n * HW;
+  const float* a = im0 + (size_t)n * d * HW;
+  const float* q = im1 + (size_t)n * d * HW;
+  const float* fl = flow + (size_t)n * fc * HW;
+  const int x = tx * kTW + lane;
+  TilePx px[PX];
+  bool valid[PX];
+  unsigned pix[PX];
+  int minx = INT_MAX, maxx = INT_MIN, miny = INT_MAX, maxy = INT_MIN;
+#pragma unroll
+  for (int i = 0; i < PX; i++) {
+    const int y = ty * kTH + wave * PX + i;
+    valid[i] = x < W && y < H;
+    locate(px[i], fl, HW, H, W, x, y, valid[i], minx, maxx, miny, maxy);
+    pix[i] = px[i].p;
+  }
+  Factors k[PX];
+  auto factors = [&](int i, const float (&c)[5]) {  // finished fit of pixel i
+    Fit f;
+    f.inside = px[i].inside;
+    f.validX = f.validY = 0;
+    f.c00 = f.ax = f.ay = f.bx = f.by = f.fx = f.fy = 0.f;
+    if (px[i].inside) finish_fit(f, c[0], c[1], c[3], c[2], c[4], px[i].ix, px[i].iy, H, W);
+    return f;
+  };
+  if (MODE == 1) {
+#pragma unroll
+    for (int i = 0; i < PX; i++) {
+      k[i] = Factors{};
+      if (!px[i].inside) continue;
+      const long long t = base + pix[i];
+      float c[5];
+#pragma unroll
+      for (int j = 0; j < 5; j++) c[j] = costs[j * P + t];
+      k[i] = scatter_factors(factors(i, c), gin, n, HW, pix[i]);
+      store_source(ws, k[i], P, base, t, (long long)px[i].iy * W + px[i].ix, pix[i]);
+    }
+  }
+  const Box box = block_box(minx, maxx, miny, maxy, red, TileCfg<PX>::ELEMS);
+  unsigned lo[PX][5];
+  bool far[PX], any_far = false;
+#pragma unroll
+  for (int i = 0; i < PX; i++) {
+    place(px[i], box, W);
+    far[i] = px[i].far;
+    any_far = any_far || far[i];
+#pragma unroll
+    for (int j = 0; j < 5; j++) lo[i][j] = px[i].inside && !far[i] ? 4u * px[i].o[j] : 0u;
+  }
+  // where the window holds few pixels of the tile it is not worth its loads: all of them from memory then
+  const bool windowless = __syncthreads_count(any_far) > kFarThreads;
+  any_far = __ballot(any_far) != 0;
+  // taps from memory, both pixels of the lane together; use(cc, first map, taps) per channel.  Few pixels: four channels in flight;
+  // a whole tile of scattered taps: one, the lines of a channel's taps then stay in the cache until they have been used
+  // (4 x 32 x 384 x 1248, 12 pixels of noise on the flow: 630 us with one, 655 with two, 766 with four; 4 pixels: 211, 214, 205).
+  auto from_memory_of = [&](auto ahead, auto use) {
+    constexpr int kFarAhead = decltype(ahead)::value;
+    unsigned o[PX][5];
+#pragma unroll
+    for (int i = 0; i < PX; i++) {
+      far[i] = far[i] || (windowless && px[i].inside);
+      const int ix = far[i] ? px[i].ix : 0, iy = far[i] ? px[i].iy : 0;  // (other pixels read the plane's first corner)
+      o[i][0] = (unsigned)iy * W + ix;
+      o[i][1] = (unsigned)iy * W + min(ix + 1, W - 1);
+      o[i][2] = (unsigned)iy * W + max(ix - 1, 0);
+      o[i][3] = (unsigned)min(iy + 1, H - 1) * W + ix;
+      o[i][4] = (unsigned)max(iy - 1, 0) * W + ix;
+    }
+    for (int c0 = 0; c0 < d; c0 += kFarAhead) {
+      float v[kFarAhead][PX], t[kFarAhead][PX][5];
+#pragma unroll
+      for (int u = 0; u < kFarAhead; u++) {
+        const size_t plane = (size_t)min(c0 + u, d - 1) * HW;
+#pragma unroll
+        for (int i = 0; i < PX; i++) {
+          if (MODE == 0) v[u][i] = a[plane + pix[i]];
+#pragma unroll
+          for (int j = 0; j < 5; j++) t[u][i][j] = q[plane + o[i][j]];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kFarAhead; u++)
+        if (c0 + u < d) use(c0 + u, v[u], t[u]);
+    }
+  };
+  auto from_memory = [&](auto use) {
+    if (windowless) from_memory_of(std::integral_constant<int, 1>{}, use);
+    else if (any_far) from_memory_of(std::integral_constant<int, 4>{}, use);
+  };
+  if (MODE == 0) {
+    float cost[PX][5];
+#pragma unroll
+    for (int i = 0; i < PX; i++)
+#pragma unroll
+      for (int j = 0; j < 5; j++) cost[i][j] = 0.f;
+    if (!windowless)
+      ring_pass<PX, true>(q, a, pix, d, HW, W, box, ring, [&](int, unsigned buf, unsigned own) {
+        unsigned addr[kPairs];
+        float v[kPairs];
+#pragma unroll
+        for (int i = 0; i < PX; i++) {
+#pragma unroll
+          for (int j = 0; j < 5; j++) addr[5 * i + j] = buf + lo[i][j];
+          addr[10 + i] = buf + 4u * (own + 256u * i + threadIdx.x);
+        }
+        lds_read12(addr, v);
+#pragma unroll
+        for (int i = 0; i < PX; i++)
+#pragma unroll
+          for (int j = 0; j < 5; j++) cost[i][j] += v[10 + i] * v[5 * i + j];  // QF.cu:63-71
+      });
+    if (any_far || windowless) {
+      float sum[PX][5];
+#pragma unroll
+      for (int i = 0; i < PX; i++)
+#pragma unroll
+        for (int j = 0; j < 5; j++) sum[i][j] = 0.f;
+      from_memory([&](int, const float (&v)[PX], const float (&t)[PX][5]) {
+#pragma unroll
+        for (int i = 0; i < PX; i++)
+#pragma unroll
+          for (int j = 0; j < 5; j++) sum[i][j] += v[i] * t[i][j];
+      });
+#pragma unroll
+      for (int i = 0; i < PX; i++)
+#pragma unroll
+        for (int j = 0; j < 5; j++) cost[i][j] = far[i] ? sum[i][j] : cost[i][j];
+    }
+#pragma unroll
+    for (int i = 0; i < PX; i++) {
+      if (!valid[i]) continue;
+      const Fit f = factors(i, cost[i]);
+      float* o = res + (size_t)n * 3 * HW + pix[i];
+      float score = 0.f;
+      if (f.inside)  // QF.cu:136
+        score = f.ax * f.fx * f.fx + f.bx * f.fx + f.c00 + f.ay * f.fy * f.fy + f.by * f.fy;
+      o[0] = f.fx;
+      o[HW] = f.fy;
+      o[2 * HW] = score;
+      if (costs) {
+#pragma unroll
+        for (int j = 0; j < 5; j++) __builtin_nontemporal_store(cost[i][j], &costs[j * P + base + pix[i]]);
+      }
+    }
+    return;
+  }
+  float* G0 = res + (size_t)n * d * HW;
+  auto gradient = [&](int i, const float* t) -> float {
+    if (!px[i].inside) return 0.f;
+    if (k[i].any_valid)  // QF.cu:286-290
+      return 0.5 * (t[0] * k[i].k00 + t[1] * k[i].k0p + t[2] * k[i].k0m + t[3] * k[i].kp0 + t[4] * k[i].km0);
+    return t[0] * k[i].dFds;  // QF.cu:295
+  };
+  if (!windowless)
+    ring_pass<PX, false>(q, nullptr, pix, d, HW, W, box, ring, [&](int cc, unsigned buf, unsigned) {
+      unsigned addr[10];
+      float v[10];
+#pragma unroll
+      for (int i = 0; i < PX; i++)
+#pragma unroll
+        for (int j = 0; j < 5; j++) addr[5 * i + j] = buf + lo[i][j];
+      lds_read10(addr, v);
+#pragma unroll
+      for (int i = 0; i < PX; i++) {
+        const float g = gradient(i, v + 5 * i);
+        if (valid[i] && !far[i]) __builtin_nontemporal_store(g, &G0[(size_t)cc * HW + pix[i]]);
+      }
+    });
+  from_memory([&](int cc, const float (&)[PX], const float (&t)[PX][5]) {
+#pragma unroll
+    for (int i = 0; i < PX; i++) {
+      const float g = gradient(i, t[i]);
+      if (far[i] || (windowless && valid[i])) __builtin_nontemporal_store(g, &G0[(size_t)cc * HW + pix[i]]);
+    }
+  });
 }
 
 // The same two passes for images with too few tiles to fill the chip.  On 64 x 96 x 312 the tiled kernels are 60 blocks
@@ -1160,15 +1432,7 @@ __global__ __launch_bounds__(256) void quadfit_split(const float* __restrict__ i
   if (px.inside) kf = scatter_factors(f, gin, n, HW, px.p);
   if (wave == 0 && px.inside) {
     const long long P = (long long)N * HW, t = (long long)n * HW + px.p;
-    ws.coef[0 * P + t] = kf.any_valid ? (float)(0.5 * kf.k00) : kf.dFds;  // QF.cu:279-283,296
-    ws.coef[1 * P + t] = kf.any_valid ? 0.5f * kf.k0p : 0.f;
-    ws.coef[2 * P + t] = kf.any_valid ? 0.5f * kf.k0m : 0.f;
-    ws.coef[3 * P + t] = kf.any_valid ? 0.5f * kf.kp0 : 0.f;
-    ws.coef[4 * P + t] = kf.any_valid ? 0.5f * kf.km0 : 0.f;
-    const long long centre = (long long)n * HW + o[0];
-    const int pos = atomicAdd(ws.count + centre, 1);
-    if (pos < kSlots) ws.slots[centre * kSlots + pos] = (int)px.p;
-    else ws.ovf[atomicAdd(ws.ovf_count, 1)] = (int)t;
+    store_source(ws, kf, P, (long long)n * HW, t, o[0], px.p);
   }
   float* G0 = res + (size_t)n * d * HW;
   auto gradient = [&](int c0, const float (*t)[5]) {
@@ -1206,30 +1470,7 @@ __global__ __launch_bounds__(256) void quadfit_split(const float* __restrict__ i
 // Pass B of the backward pass on tiles of target pixels: the (source, coefficient) pairs of every pixel are
 // collected once; per channel the window of the FIRST feature map that covers the tile's sources is
 // staged in LDS and the pairs are summed from it.
-constexpr int kPairs = 12;
 constexpr int kPxGather = 2;
-
-// Twelve reads of one LDS buffer at per-lane element offsets, issued together and waited for once, as one block the
-// compiler does not look into: before an LDS read that it sees, it waits for the loads into LDS that may alias it, and
-// with four buffers in a ring it takes that to be all of them -- the whole prefetch queue.  The caller has waited for the
-// buffer's own loads (window_pass_dma).
-static_assert(kPairs == 12, "lds_gather12 reads twelve elements");
-__device__ __forceinline__ void lds_gather12(const float* buf, const unsigned (&off)[kPairs], float (&v)[kPairs]) {
-  const unsigned b = (unsigned)(size_t)(const __attribute__((address_space(3))) float*)buf;
-  unsigned a[kPairs];
-#pragma unroll
-  for (int j = 0; j < kPairs; j++) a[j] = b + 4u * off[j];
-  asm volatile(
-      "ds_read_b32 %0, %12\n\tds_read_b32 %1, %13\n\tds_read_b32 %2, %14\n\tds_read_b32 %3, %15\n\t"
-      "ds_read_b32 %4, %16\n\tds_read_b32 %5, %17\n\tds_read_b32 %6, %18\n\tds_read_b32 %7, %19\n\t"
-      "ds_read_b32 %8, %20\n\tds_read_b32 %9, %21\n\tds_read_b32 %10, %22\n\tds_read_b32 %11, %23\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]),
-        "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11])
-      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9]), "v"(a[10]),
-        "v"(a[11])
-      : "memory");
-}
 
 template <int PX>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void quadfit_gather_tiles(const float* __restrict__ im0, float* __restrict__ g1, QfWorkspace ws,
@@ -1974,26 +2215,44 @@ int flowaux_profile(int enable) {
 
 int flowaux_profile_read(double* total_ms, int* launches) { return g_timer.read(total_ms, launches); }
 
-int quadfit_forward(const float* im0, const float* im1, const float* flow, float* out, int n, int ic, int ih, int iw,
-                    int flow_channels, void* stream) {
-  if (!im0 || !im1 || !flow || !out) return fail(INPAINT_ERR_ARG, "quadfit_forward: null pointer");
-  if (n < 1 || ic < 1 || ih < 1 || iw < 1) return fail(INPAINT_ERR_ARG, "quadfit_forward: bad shape %dx%dx%dx%d", n, ic, ih, iw);
-  if (flow_channels < 2) return fail(INPAINT_ERR_ARG, "quadfit_forward: the flow needs at least 2 channels, got %d", flow_channels);
-  if ((long long)ih * iw >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "quadfit_forward: image too large");
+static int forward_of(const char* name, const float* im0, const float* im1, const float* flow, float* out, float* costs, int n, int ic,
+                      int ih, int iw, int flow_channels, void* stream) {
+  if (!im0 || !im1 || !flow || !out) return fail(INPAINT_ERR_ARG, "%s: null pointer", name);
+  if (n < 1 || ic < 1 || ih < 1 || iw < 1) return fail(INPAINT_ERR_ARG, "%s: bad shape %dx%dx%dx%d", name, n, ic, ih, iw);
+  if (flow_channels < 2) return fail(INPAINT_ERR_ARG, "%s: the flow needs at least 2 channels, got %d", name, flow_channels);
+  if ((long long)ih * iw >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "%s: image too large", name);
   const long long P = (long long)n * ih * iw;
-  const int tiles_x = (iw + kTW - 1) / kTW, tiles_y = (ih + TileCfg<kPxForward>::TH - 1) / TileCfg<kPxForward>::TH;
+  const int tiles_x = (iw + kTW - 1) / kTW, tiles_y = (ih + TileCfg<kPxTile>::TH - 1) / TileCfg<kPxTile>::TH;
   const long long tiles = (long long)n * tiles_x * tiles_y;
-  if (tiles >= (1ll << 31) - 8) return fail(INPAINT_ERR_ARG, "quadfit_forward: too many tiles");
-  if (inpaint::knobs().quadfit_px_path)
+  if (tiles >= (1ll << 31) - 8) return fail(INPAINT_ERR_ARG, "%s: too many tiles", name);
+  if (!costs && inpaint::knobs().quadfit_px_path)
     hipLaunchKernelGGL(quadfit_forward_kernel, banded_grid(P), dim3(256), 0, (hipStream_t)stream, im0, im1, flow, out, n,
                        ic, ih, iw, flow_channels);
-  else if (quadfit_few_tiles(tiles, ic))
+  else if (!costs && quadfit_few_tiles(tiles, ic))
     launch_quadfit_split<0>(im0, im1, flow, nullptr, out, QfWorkspace{}, n, ic, ih, iw, flow_channels, (hipStream_t)stream);
   else
-    hipLaunchKernelGGL((quadfit_tiles<0, kPxForward>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, (hipStream_t)stream, im0, im1,
-                       flow, nullptr, out, QfWorkspace{}, n, ic, ih, iw, flow_channels, tiles_x, tiles_y);
+    hipLaunchKernelGGL((quadfit_ring_tiles<0>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), 0, (hipStream_t)stream, im0, im1,
+                       flow, nullptr, costs, out, QfWorkspace{}, n, ic, ih, iw, flow_channels, tiles_x, tiles_y);
   INPAINT_HIP(hipGetLastError());
   return 0;
+}
+
+int quadfit_forward(const float* im0, const float* im1, const float* flow, float* out, int n, int ic, int ih, int iw,
+                    int flow_channels, void* stream) {
+  return forward_of("quadfit_forward", im0, im1, flow, out, nullptr, n, ic, ih, iw, flow_channels, stream);
+}
+
+int quadfit_forward_saving(const float* im0, const float* im1, const float* flow, float* out, float* costs, int n, int ic, int ih,
+                           int iw, int flow_channels, void* stream) {
+  if (!costs) return fail(INPAINT_ERR_ARG, "quadfit_forward_saving: null pointer");
+  return forward_of("quadfit_forward_saving", im0, im1, flow, out, costs, n, ic, ih, iw, flow_channels, stream);
+}
+
+// Images that the split kernels take have nothing to gain: their backward pass keeps all taps in registers and is bound by latency.
+int quadfit_saving_pays(int n, int ic, int ih, int iw) {
+  if (n < 1 || ic < 1 || ih < 1 || iw < 1 || inpaint::knobs().quadfit_px_path || inpaint::knobs().quadfit_reread) return 0;
+  const long long tiles = (long long)n * ((iw + kTW - 1) / kTW) * ((ih + TileCfg<kPxTile>::TH - 1) / TileCfg<kPxTile>::TH);
+  return !quadfit_few_tiles(tiles, ic);
 }
 
 long long quadfit_backward_workspace_bytes(int n, int ih, int iw) {
@@ -2001,12 +2260,13 @@ long long quadfit_backward_workspace_bytes(int n, int ih, int iw) {
   return qf_workspace_bytes((long long)n * ih * iw);
 }
 
-int quadfit_backward(const float* im0, const float* im1, const float* flow, const float* gin, float* g0, float* g1, int n,
-                     int ic, int ih, int iw, int flow_channels, void* workspace, long long workspace_bytes, void* stream) {
-  if (!im0 || !im1 || !flow || !gin || !g0 || !g1) return fail(INPAINT_ERR_ARG, "quadfit_backward: null pointer");
-  if (n < 1 || ic < 1 || ih < 1 || iw < 1) return fail(INPAINT_ERR_ARG, "quadfit_backward: bad shape %dx%dx%dx%d", n, ic, ih, iw);
-  if (flow_channels < 2) return fail(INPAINT_ERR_ARG, "quadfit_backward: the flow needs at least 2 channels, got %d", flow_channels);
-  if ((long long)ih * iw >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "quadfit_backward: image too large");
+static int backward_of(const char* name, const float* im0, const float* im1, const float* flow, const float* gin, const float* costs,
+                       float* g0, float* g1, int n, int ic, int ih, int iw, int flow_channels, void* workspace, long long workspace_bytes,
+                       void* stream) {
+  if (!im0 || !im1 || !flow || !gin || !g0 || !g1) return fail(INPAINT_ERR_ARG, "%s: null pointer", name);
+  if (n < 1 || ic < 1 || ih < 1 || iw < 1) return fail(INPAINT_ERR_ARG, "%s: bad shape %dx%dx%dx%d", name, n, ic, ih, iw);
+  if (flow_channels < 2) return fail(INPAINT_ERR_ARG, "%s: the flow needs at least 2 channels, got %d", name, flow_channels);
+  if ((long long)ih * iw >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "%s: image too large", name);
   const long long P = (long long)n * ih * iw, total = P * ic;
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid = banded_grid(P), block(256);
@@ -2017,21 +2277,24 @@ int quadfit_backward(const float* im0, const float* im1, const float* flow, cons
     return 0;
   }
   if (workspace_bytes < qf_workspace_bytes(P))
-    return fail(INPAINT_ERR_ARG, "quadfit_backward: workspace of %lld bytes, %lld needed", workspace_bytes, qf_workspace_bytes(P));
-  if (((uintptr_t)workspace & 15) != 0) return fail(INPAINT_ERR_ARG, "quadfit_backward: workspace must be 16-byte aligned");
-  if (P >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "quadfit_backward: too many pixels for the inverse map");
+    return fail(INPAINT_ERR_ARG, "%s: workspace of %lld bytes, %lld needed", name, workspace_bytes, qf_workspace_bytes(P));
+  if (((uintptr_t)workspace & 15) != 0) return fail(INPAINT_ERR_ARG, "%s: workspace must be 16-byte aligned", name);
+  if (P >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "%s: too many pixels for the inverse map", name);
   const QfWorkspace ws = qf_carve(workspace, P);
   // the counters start at zero (a fill kernel, so that the call can be captured into a graph)
   hipLaunchKernelGGL(inpaint::fill_zero_f32, dim3(inpaint::grid_stride(P + 64)), dim3(256), 0, st,
                      reinterpret_cast<float*>(ws.count), P + 64);
-  const int tiles_x = (iw + kTW - 1) / kTW, tiles_y = (ih + TileCfg<kPxSources>::TH - 1) / TileCfg<kPxSources>::TH;
+  const int tiles_x = (iw + kTW - 1) / kTW, tiles_y = (ih + TileCfg<kPxTile>::TH - 1) / TileCfg<kPxTile>::TH;
   const long long tiles = (long long)n * tiles_x * tiles_y;
-  const bool px_path = inpaint::knobs().quadfit_px_path;
+  const bool px_path = !costs && inpaint::knobs().quadfit_px_path;
   if (px_path)
     hipLaunchKernelGGL(quadfit_backward_sources, grid, block, 0, st, im0, im1, flow, gin, g0, ws, n, ic, ih, iw, flow_channels);
   else {
     if (g_timed_pass == 1) g_timer.begin(st);
-    if (quadfit_few_tiles(tiles, ic) && !inpaint::knobs().quadfit_reread) {
+    if (costs) {
+      hipLaunchKernelGGL((quadfit_ring_tiles<1>), dim3((unsigned)((tiles + 7) / 8 * 8)), block, 0, st, im0, im1, flow, gin,
+                         const_cast<float*>(costs), g0, ws, n, ic, ih, iw, flow_channels, tiles_x, tiles_y);
+    } else if (quadfit_few_tiles(tiles, ic) && !inpaint::knobs().quadfit_reread) {
       launch_quadfit_split<1>(im0, im1, flow, gin, g0, ws, n, ic, ih, iw, flow_channels, st);
     } else if (ic <= kResidentChannels && !inpaint::knobs().quadfit_reread) {
       const int ry = (ih + kResidentRows - 1) / kResidentRows;
@@ -2044,7 +2307,7 @@ int quadfit_backward(const float* im0, const float* im1, const float* flow, cons
         hipLaunchKernelGGL((quadfit_sources_resident<kResidentChannels, false>), rgrid, block, 0, st, im0, im1, flow, gin, g0, ws, n,
                            ic, ih, iw, flow_channels, tiles_x, ry);
     } else {
-      hipLaunchKernelGGL((quadfit_tiles<1, kPxSources>), dim3((unsigned)((tiles + 7) / 8 * 8)), block, 0, st, im0, im1, flow, gin, g0,
+      hipLaunchKernelGGL(quadfit_sources_tiles, dim3((unsigned)((tiles + 7) / 8 * 8)), block, 0, st, im0, im1, flow, gin, g0,
                          ws, n, ic, ih, iw, flow_channels, tiles_x, tiles_y);
     }
     if (g_timed_pass == 1) g_timer.end(st, 1);
@@ -2063,6 +2326,20 @@ int quadfit_backward(const float* im0, const float* im1, const float* flow, cons
   hipLaunchKernelGGL(quadfit_backward_overflow, dim3((unsigned)std::min<long long>((P + 127) / 128, 512)), block, 0, st, im0, flow, g1, ws, n, ic, ih, iw, flow_channels);
   INPAINT_HIP(hipGetLastError());
   return 0;
+}
+
+int quadfit_backward(const float* im0, const float* im1, const float* flow, const float* gin, float* g0, float* g1, int n,
+                     int ic, int ih, int iw, int flow_channels, void* workspace, long long workspace_bytes, void* stream) {
+  return backward_of("quadfit_backward", im0, im1, flow, gin, nullptr, g0, g1, n, ic, ih, iw, flow_channels, workspace, workspace_bytes,
+                     stream);
+}
+
+int quadfit_backward_saved(const float* im0, const float* im1, const float* flow, const float* gin, const float* costs, float* g0,
+                           float* g1, int n, int ic, int ih, int iw, int flow_channels, void* workspace, long long workspace_bytes,
+                           void* stream) {
+  if (!costs || !workspace) return fail(INPAINT_ERR_ARG, "quadfit_backward_saved: null pointer");
+  return backward_of("quadfit_backward_saved", im0, im1, flow, gin, costs, g0, g1, n, ic, ih, iw, flow_channels, workspace,
+                     workspace_bytes, stream);
 }
 
 int medimax_forward(const float* vol, float* out, int n, int ih, int iw, int num_disp, void* stream) {

@@ -49,13 +49,17 @@ def _stream(t):
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
 
 
-def forward(featureImage0, featureImage1, flow):
-    """featureImage0/1: (n,c,h,w) feature maps; flow: (n,>=2,h,w).  Returns [(n,3,h,w)]: the offsets of the
-    fitted maximum in x and y (to be added to the rounded displaced position) and the fitted score."""
+def _check_maps(featureImage0, featureImage1, flow):
     for t, name in ((featureImage0, "featureImage0"), (featureImage1, "featureImage1"), (flow, "flow")):
         _check_input(t, name)
     _check_shapes(featureImage0, featureImage1, flow)
-    n, c, h, w = featureImage0.shape
+    return featureImage0.shape
+
+
+def forward(featureImage0, featureImage1, flow):
+    """featureImage0/1: (n,c,h,w) feature maps; flow: (n,>=2,h,w).  Returns [(n,3,h,w)]: the offsets of the
+    fitted maximum in x and y (to be added to the rounded displaced position) and the fitted score."""
+    n, c, h, w = _check_maps(featureImage0, featureImage1, flow)
     flowUpdate = torch.empty((n, 3, h, w), dtype=torch.float32, device=flow.device)
     with torch.cuda.device(flow.device):
         rc = lib.quadfit_forward(featureImage0.data_ptr(), featureImage1.data_ptr(), flow.data_ptr(),
@@ -65,23 +69,48 @@ def forward(featureImage0, featureImage1, flow):
     return [flowUpdate]
 
 
-def backward(d_iGf, featureImage0, featureImage1, flow, use_atomics=False):
+def saving_pays(featureImage0):
+    """Whether forward_saving followed by backward(costs=...) is the faster pair at this shape (not at small ones)."""
+    return featureImage0.dim() == 4 and bool(lib.quadfit_saving_pays(*featureImage0.shape))
+
+
+def forward_saving(featureImage0, featureImage1, flow):
+    """forward that also returns what backward takes as `costs`: [flowUpdate, costs (5,n,h,w)]."""
+    n, c, h, w = _check_maps(featureImage0, featureImage1, flow)
+    flowUpdate = torch.empty((n, 3, h, w), dtype=torch.float32, device=flow.device)
+    costs = torch.empty((5, n, h, w), dtype=torch.float32, device=flow.device)
+    with torch.cuda.device(flow.device):
+        rc = lib.quadfit_forward_saving(featureImage0.data_ptr(), featureImage1.data_ptr(), flow.data_ptr(), flowUpdate.data_ptr(),
+                                        costs.data_ptr(), n, c, h, w, flow.shape[1], _stream(flow))
+    if rc:
+        raise _ERRORS.get(rc, RuntimeError)("FlowQuadFitting::forward failed: %s" % _last_error())
+    return [flowUpdate, costs]
+
+
+def backward(d_iGf, featureImage0, featureImage1, flow, use_atomics=False, costs=None):
     """d_iGf: (n,3,h,w) gradient wrt the result.  Returns [d_oFeat0, d_oFeat1].  `use_atomics` selects the
-    reference's scatter with float atomics instead of the gather through a scratch buffer."""
-    for t, name in ((featureImage0, "featureImage0"), (featureImage1, "featureImage1"), (flow, "flow"),
-                    (d_iGf, "d_iGf")):
-        _check_input(t, name)
-    _check_shapes(featureImage0, featureImage1, flow)
-    n, c, h, w = featureImage0.shape
+    reference's scatter with float atomics instead of the gather through a scratch buffer.  `costs`: the second result of
+    forward_saving on the same inputs; without it they are formed again."""
+    n, c, h, w = _check_maps(featureImage0, featureImage1, flow)
+    _check_input(d_iGf, "d_iGf")
     if tuple(d_iGf.shape) != (n, 3, h, w):
         raise ValueError("d_iGf must have shape (%d, 3, %d, %d), got %s" % (n, h, w, tuple(d_iGf.shape)))
+    if costs is not None:
+        _check_input(costs, "costs")
+        if tuple(costs.shape) != (5, n, h, w):
+            raise ValueError("costs must have shape (5, %d, %d, %d), got %s" % (n, h, w, tuple(costs.shape)))
+        if costs.device != flow.device:
+            raise RuntimeError("all tensors must live on one device")
+        if use_atomics:
+            raise ValueError("the scatter with float atomics takes no costs")
     d_oFeat0, d_oFeat1 = torch.empty_like(featureImage0), torch.empty_like(featureImage1)
     ws_bytes = 0 if use_atomics else lib.quadfit_backward_workspace_bytes(n, h, w)
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=flow.device) if ws_bytes else None
+    maps = (featureImage0.data_ptr(), featureImage1.data_ptr(), flow.data_ptr(), d_iGf.data_ptr())
+    rest = (d_oFeat0.data_ptr(), d_oFeat1.data_ptr(), n, c, h, w, flow.shape[1], workspace.data_ptr() if ws_bytes else None, ws_bytes,
+            _stream(flow))
     with torch.cuda.device(flow.device):
-        rc = lib.quadfit_backward(featureImage0.data_ptr(), featureImage1.data_ptr(), flow.data_ptr(),
-                                  d_iGf.data_ptr(), d_oFeat0.data_ptr(), d_oFeat1.data_ptr(), n, c, h, w,
-                                  flow.shape[1], workspace.data_ptr() if ws_bytes else None, ws_bytes, _stream(flow))
+        rc = lib.quadfit_backward(*maps, *rest) if costs is None else lib.quadfit_backward_saved(*maps, costs.data_ptr(), *rest)
     if rc:
         raise _ERRORS.get(rc, RuntimeError)("FlowQuadFitting::backward failed: %s" % _last_error())
     return [d_oFeat0, d_oFeat1]

@@ -13,15 +13,20 @@ class QuadFittingFromFlowFunction(Function):
 
     @staticmethod
     def forward(ctx, feat0, feat1, flow):  # QuadFitting.py:20-30
-        outputs = QuadFit_cuda_ext.forward(feat0.contiguous(), feat1.contiguous(), flow.contiguous())
+        maps = feat0.contiguous(), feat1.contiguous(), flow.contiguous()
+        if any(ctx.needs_input_grad[:2]) and QuadFit_cuda_ext.saving_pays(maps[0]):
+            sol, costs = QuadFit_cuda_ext.forward_saving(*maps)
+            ctx.save_for_backward(feat0, feat1, flow, costs)
+            return sol
+        outputs = QuadFit_cuda_ext.forward(*maps)
         ctx.save_for_backward(feat0, feat1, flow)
         return outputs[0]
 
     @staticmethod
     def backward(ctx, grad_sol):  # QuadFitting.py:33-40 (which returns two values for three inputs)
-        feat0, feat1, flow = ctx.saved_tensors
-        d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.backward(grad_sol.contiguous(), feat0.contiguous(),
-                                                         feat1.contiguous(), flow.contiguous())
+        feat0, feat1, flow, *costs = ctx.saved_tensors
+        d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.backward(grad_sol.contiguous(), feat0.contiguous(), feat1.contiguous(),
+                                                         flow.contiguous(), costs=costs[0] if costs else None)
         return d_oGfeat0, d_oGfeat1, None
 
 

@@ -48,6 +48,19 @@ int quadfit_backward(const float* im0, const float* im1, const float* flow, cons
                      float* g1, int n, int ic, int ih, int iw, int flow_channels, void* workspace,
                      long long workspace_bytes, void* stream);
 
+/* The same two passes with the five matching costs of every pixel handed from one to the other (no counterpart in the reference,
+ * whose backward pass forms them again): the same results, the gradient wrt im0 bit for bit, with one read of im1 less and, in the
+ * pass over the sources, none of im0.
+ *   costs : 5*n*ih*iw floats, written by quadfit_forward_saving and read by quadfit_backward_saved (workspace required)
+ * quadfit_saving_pays returns 1 for the shapes at which the pair is the faster one (small images are not).
+ */
+int quadfit_forward_saving(const float* im0, const float* im1, const float* flow, float* out, float* costs, int n, int ic, int ih,
+                           int iw, int flow_channels, void* stream);
+int quadfit_backward_saved(const float* im0, const float* im1, const float* flow, const float* gin, const float* costs, float* g0,
+                           float* g1, int n, int ic, int ih, int iw, int flow_channels, void* workspace, long long workspace_bytes,
+                           void* stream);
+int quadfit_saving_pays(int n, int ic, int ih, int iw);
+
 /* Replaces MediMax::forward (cudaMedian/cudaCode/medimax.h:13, cudaMedian/cudaCode/medimax.cu:17-44,
  * 131-168), bound by cudaMedian/median_cuda.cpp:36-70.
  *   vol : (n,ih,iw,num_disp) histogram over num_disp displacement bins, bins innermost
