@@ -723,69 +723,6 @@ __device__ __forceinline__ void window_pass(const float* __restrict__ q, int d, 
   else window_pass_of<PX, 9>(q, d, HW, W, box, win, pre, consume);
 }
 
-// The same stream with the windows loaded from memory straight into LDS (global_load_lds: no staging registers) through a
-// ring of kDmaStages buffers: while channel c is consumed, channels c+1 and c+2 are on their way and channel c+3 is asked
-// for as soon as c has been consumed -- three channels in flight per wavefront instead of two, one barrier per channel.
-// Loads return in order, so "at most two channels' worth of loads outstanding" means channel c has arrived (a wavefront's
-// stores in between make the wait a little longer, never shorter); the barrier then makes every wavefront's part of the
-// window visible.  A buffer is overwritten two barriers after its last reader has passed the barrier that follows its
-// consumption.  No `pre` values: for consumers that need the window only.
-// The four buffers are four separate __shared__ arrays, not one: the compiler waits, before a read of LDS, for every load
-// into LDS that may alias it, and it can tell loads into different variables apart, not into parts of one.
-template <int PX, int PER, typename Consume>
-__device__ __forceinline__ void window_pass_dma_of(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
-                                                float* w0, float* w1, float* w2, float* w3, Consume consume) {
-  constexpr int kPer = PER;
-  typedef const __attribute__((address_space(1))) void* GlobalPtr;
-  typedef __attribute__((address_space(3))) void* LdsPtr;
-  const int count = box.w * box.h;
-  unsigned goff[kPer];
-  const float inv_w = 1.0f / (float)max(box.w, 1);
-#pragma unroll
-  for (int k = 0; k < kPer; k++) {
-    const int e = threadIdx.x + 256 * k;
-    const int r = (int)(((float)e + 0.5f) * inv_w);
-    goff[k] = e < count ? (unsigned)(r * W + (e - r * box.w)) : 0u;
-  }
-  const float* corner = q + (size_t)box.y0 * W + box.x0;
-  const int wave_first = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));  // lane l of the wavefront writes element wave_first + l
-  auto fetch = [&](int c, float* buf) {
-    const float* src = corner + (size_t)c * HW;
-#pragma unroll
-    for (int k = 0; k < kPer; k++)
-      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + goff[k]), (LdsPtr)(buf + 256 * k + wave_first), 4, 0, 0);
-  };
-  const int last = d - 1;
-  auto phase = [&](int c, float* buf, float* refill) {
-    // channel c's loads have landed when at most the two younger channels' loads are outstanding
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * kPer) : "memory");
-    const int cc = min(c, last);
-    consume(cc, buf, q + (size_t)cc * HW, 0, c < d);
-    fetch(min(c + 3, last), refill);
-  };
-  fetch(0, w0);
-  fetch(min(1, last), w1);
-  fetch(min(2, last), w2);
-  for (int c0 = 0; c0 < d; c0 += 4) {
-    phase(c0, w0, w3);
-    phase(c0 + 1, w1, w0);
-    phase(c0 + 2, w2, w1);
-    phase(c0 + 3, w3, w2);
-  }
-  // (the loads still in flight at the end target LDS: they must have landed before the workgroup's LDS is handed on)
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-
-template <int PX, typename Consume>
-__device__ __forceinline__ void window_pass_dma(const float* __restrict__ q, int d, size_t HW, int W, const Box& box,
-                                                float* w0, float* w1, float* w2, float* w3, Consume consume) {
-  static_assert(TileCfg<PX>::ELEMS == 9 * 256, "loads per thread: 4 to 9");
-  const int count = __builtin_amdgcn_readfirstlane(box.w * box.h);
-  if (count <= 4 * 256) window_pass_dma_of<PX, 4>(q, d, HW, W, box, w0, w1, w2, w3, consume);
-  else if (count <= 6 * 256) window_pass_dma_of<PX, 6>(q, d, HW, W, box, w0, w1, w2, w3, consume);
-  else window_pass_dma_of<PX, 9>(q, d, HW, W, box, w0, w1, w2, w3, consume);
-}
-
 // the five taps of every inside pixel of the lane, from the window or (far pixels) from the plane
 template <int PX, typename Body>
 __device__ __forceinline__ void each_pixel_taps(const TilePx (&px)[PX], const float* buf, const float* plane, Body body) {
@@ -1049,64 +986,103 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
+// The forward pass, and pass A of the backward pass when the forward pass has left its five costs per pixel, with everything
+// the channel loop reads coming from memory straight into LDS (global_load_lds): the window of the second map and, forward, the
+// tile's own pixels of the first.  No load of the loop has a register as its target, so nothing but the ring's own count is
+// waited for, and one barrier per two channels is all the synchronisation.  With the costs at hand pass A streams the second map
+// once and keeps no taps: resident in registers they allow two wavefronts per SIMD and every map is read twice.
+// A pixel whose taps leave the window's capacity is worked out from memory behind the loop.
+// Bound by memory.  4 x 32 x 384 x 1248, us: forward 153 -> 121 (590 MB at 4.9 TB/s), with the costs stored 129; pass A 268 -> 158;
+// 2 x 64 x 192 x 624 forward + backward 222 -> 131, 2 x 48 x 448 x 1280 660 -> 413.  With 4 pixels of noise on the flow (a fifth of
+// the pixels outside the window) 1230 -> 1015, with 12 (nearly all) as before.
+constexpr int kRingElems = 9216;   // floats of LDS for the ring: four blocks per CU
+constexpr int kFarThreads = 128;
+
 // Reads of LDS issued together and waited for once, as one block the compiler does not look into: before an LDS read that it
 // sees, it waits for the loads into LDS that may alias it, and with the buffers of a ring it takes that to be all of them -- the
 // whole prefetch queue.  The caller has waited for the buffer's own loads.
 constexpr int kPairs = 12;
 __device__ __forceinline__ void lds_read12(const unsigned (&a)[kPairs], float (&v)[kPairs]) {  // (byte addresses)
   asm volatile(
-      "ds_read_b32 %0, %12\n\tds_read_b32 %1, %13\n\tds_read_b32 %2, %14\n\tds_read_b32 %3, %15\n\t"
-      "ds_read_b32 %4, %16\n\tds_read_b32 %5, %17\n\tds_read_b32 %6, %18\n\tds_read_b32 %7, %19\n\t"
-      "ds_read_b32 %8, %20\n\tds_read_b32 %9, %21\n\tds_read_b32 %10, %22\n\tds_read_b32 %11, %23\n\t"
+      "ds_read_b32 %0, %12\n\t"
+      "ds_read_b32 %1, %13\n\t"
+      "ds_read_b32 %2, %14\n\t"
+      "ds_read_b32 %3, %15\n\t"
+      "ds_read_b32 %4, %16\n\t"
+      "ds_read_b32 %5, %17\n\t"
+      "ds_read_b32 %6, %18\n\t"
+      "ds_read_b32 %7, %19\n\t"
+      "ds_read_b32 %8, %20\n\t"
+      "ds_read_b32 %9, %21\n\t"
+      "ds_read_b32 %10, %22\n\t"
+      "ds_read_b32 %11, %23\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]),
-        "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11])
-      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9]), "v"(a[10]),
-        "v"(a[11])
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]),
+        "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9]),
+        "v"(a[10]), "v"(a[11])
       : "memory");
 }
-__device__ __forceinline__ void lds_read10(const unsigned (&a)[10], float (&v)[10]) {
+// the same from two channels' windows, STRIDE x 64 floats apart: each read fetches an element of both
+typedef float float2v __attribute__((ext_vector_type(2)));
+template <int STRIDE>
+__device__ __forceinline__ void lds_read12(const unsigned (&a)[12], float2v (&v)[12]) {  // (byte addresses)
+  static_assert(STRIDE < 256, "the offset is eight bits wide");
   asm volatile(
-      "ds_read_b32 %0, %10\n\tds_read_b32 %1, %11\n\tds_read_b32 %2, %12\n\tds_read_b32 %3, %13\n\tds_read_b32 %4, %14\n\t"
-      "ds_read_b32 %5, %15\n\tds_read_b32 %6, %16\n\tds_read_b32 %7, %17\n\tds_read_b32 %8, %18\n\tds_read_b32 %9, %19\n\t"
+      "ds_read2st64_b32 %0, %12 offset1:%24\n\t"
+      "ds_read2st64_b32 %1, %13 offset1:%24\n\t"
+      "ds_read2st64_b32 %2, %14 offset1:%24\n\t"
+      "ds_read2st64_b32 %3, %15 offset1:%24\n\t"
+      "ds_read2st64_b32 %4, %16 offset1:%24\n\t"
+      "ds_read2st64_b32 %5, %17 offset1:%24\n\t"
+      "ds_read2st64_b32 %6, %18 offset1:%24\n\t"
+      "ds_read2st64_b32 %7, %19 offset1:%24\n\t"
+      "ds_read2st64_b32 %8, %20 offset1:%24\n\t"
+      "ds_read2st64_b32 %9, %21 offset1:%24\n\t"
+      "ds_read2st64_b32 %10, %22 offset1:%24\n\t"
+      "ds_read2st64_b32 %11, %23 offset1:%24\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]),
-        "=&v"(v[9])
-      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9])
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]),
+        "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9]),
+        "v"(a[10]), "v"(a[11]), "n"(STRIDE)
       : "memory");
 }
-// (element offsets into one buffer)
-__device__ __forceinline__ void lds_gather12(const float* buf, const unsigned (&off)[kPairs], float (&v)[kPairs]) {
-  const unsigned b = (unsigned)(size_t)(const __attribute__((address_space(3))) float*)buf;
-  unsigned a[kPairs];
-#pragma unroll
-  for (int j = 0; j < kPairs; j++) a[j] = b + 4u * off[j];
-  lds_read12(a, v);
+template <int STRIDE>
+__device__ __forceinline__ void lds_read10(const unsigned (&a)[10], float2v (&v)[10]) {  // (byte addresses)
+  static_assert(STRIDE < 256, "the offset is eight bits wide");
+  asm volatile(
+      "ds_read2st64_b32 %0, %10 offset1:%20\n\t"
+      "ds_read2st64_b32 %1, %11 offset1:%20\n\t"
+      "ds_read2st64_b32 %2, %12 offset1:%20\n\t"
+      "ds_read2st64_b32 %3, %13 offset1:%20\n\t"
+      "ds_read2st64_b32 %4, %14 offset1:%20\n\t"
+      "ds_read2st64_b32 %5, %15 offset1:%20\n\t"
+      "ds_read2st64_b32 %6, %16 offset1:%20\n\t"
+      "ds_read2st64_b32 %7, %17 offset1:%20\n\t"
+      "ds_read2st64_b32 %8, %18 offset1:%20\n\t"
+      "ds_read2st64_b32 %9, %19 offset1:%20\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]),
+        "=&v"(v[8]), "=&v"(v[9])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]), "v"(a[8]), "v"(a[9]), "n"(STRIDE)
+      : "memory");
 }
 
-// The forward pass, and pass A of the backward pass when the forward pass has left its five costs per pixel, with everything
-// the channel loop reads coming from memory straight into LDS (global_load_lds): the window of the second map and, forward, the
-// tile's own pixels of the first.  No load of the loop has a register as its target, so nothing but the ring's own count is
-// waited for, and one barrier per channel is all the synchronisation.  With the costs at hand pass A streams the second map
-// once and keeps no taps: resident in registers they allow two wavefronts per SIMD and every map is read twice.
-// A pixel whose taps leave the window's capacity is worked out from memory behind the loop.
-// Bound by memory.  4 x 32 x 384 x 1248, us: forward 153 -> 121 (590 MB at 4.9 TB/s), with the costs stored 127; pass A 268 -> 160;
-// 2 x 64 x 192 x 624 forward + backward 222 -> 134, 2 x 48 x 448 x 1280 660 -> 422.  With 4 pixels of noise on the flow (a fifth of
-// the pixels outside the window) 1230 -> 1020, with 12 (nearly all) as before.
-constexpr int kRingElems = 8448;  // floats of LDS for the ring: four blocks per CU
-constexpr int kFarThreads = 128;
-
-// Streams the windows of planes q[0 .. d) (and, FIRST, the tile's pixels of planes a[0 .. d)) through STAGES buffers: while
-// channel c is consumed, STAGES - 1 more are on their way.  Loads return in order: when at most the loads of STAGES - 2
-// channels are outstanding, channel c has landed (a wavefront's stores in between make the wait longer, never shorter).  A
-// buffer is refilled one barrier after its consumption.
-template <int PX, int PER, int STAGES, bool FIRST, typename Consume>
+// Streams the windows of planes q[0 .. d) (and, FIRST, the tile's pixels of planes a[0 .. d)) through STAGES buffers of CH
+// channels each: while one is consumed, STAGES - 1 more are on their way.  Loads return in order: when at most the loads of
+// STAGES - 2 buffers are outstanding, the one at hand has landed (a wavefront's stores in between make the wait longer, never
+// shorter).  A buffer is refilled one barrier after its consumption.  consume(c, two, buffer's byte address, own pixels' offset in
+// floats, distance of the channels / 64): channel c and, CH = 2 and `two`, c + 1 (else the second is the last channel once more).
+// Two channels at a time halve the reads and the barriers; with the first map in the ring as well they leave it too few buffers
+// (forward 4 x 32 x 384 x 1248 121 / 126 us; pass A 160 / 158, gather pass 168 / 160).
+template <int PX, int PER, int STAGES, int CH, bool FIRST, typename Consume>
 __device__ __forceinline__ void ring_pass_of(const float* __restrict__ q, const float* __restrict__ a, const unsigned (&pix)[PX], int d,
                                              size_t HW, int W, const Box& box, float* ring, Consume consume) {
   typedef const __attribute__((address_space(1))) void* GlobalPtr;
   typedef __attribute__((address_space(3))) void* LdsPtr;
-  constexpr int kLoads = PER + (FIRST ? PX : 0), kStage = 256 * kLoads;
-  static_assert(kStage * STAGES <= kRingElems && (STAGES - 2) * kLoads < 63, "the ring's space; the counter's range");
+  constexpr int kLoads = PER + (FIRST ? PX : 0), kChannel = 256 * kLoads, kStage = CH * kChannel;
+  static_assert(kStage * STAGES <= kRingElems && STAGES >= 2 && (STAGES - 2) * CH * kLoads < 63, "the ring's space; the counter's range");
   const int count = box.w * box.h;
   unsigned goff[PER];
   const float inv_w = 1.0f / (float)max(box.w, 1);
@@ -1118,29 +1094,35 @@ __device__ __forceinline__ void ring_pass_of(const float* __restrict__ q, const 
   }
   const float* corner = q + (size_t)box.y0 * W + box.x0;
   const int wave_first = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
-  auto fetch = [&](int c, float* buf) {
-    const float* src = corner + (size_t)c * HW;
+  auto fetch = [&](int group, float* buf) {
 #pragma unroll
-    for (int k = 0; k < PER; k++)
-      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + goff[k]), (LdsPtr)(buf + 256 * k + wave_first), 4, 0, 0);
-    if (FIRST) {
-      const float* own = a + (size_t)c * HW;
+    for (int u = 0; u < CH; u++) {
+      const int c = min(CH * group + u, d - 1);
+      const float* src = corner + (size_t)c * HW;
+      float* to = buf + u * kChannel + wave_first;
 #pragma unroll
-      for (int i = 0; i < PX; i++)
-        __builtin_amdgcn_global_load_lds((GlobalPtr)(own + pix[i]), (LdsPtr)(buf + 256 * (PER + i) + wave_first), 4, 0, 0);
+      for (int k = 0; k < PER; k++) __builtin_amdgcn_global_load_lds((GlobalPtr)(src + goff[k]), (LdsPtr)(to + 256 * k), 4, 0, 0);
+      if (FIRST) {
+        const float* own = a + (size_t)c * HW;
+#pragma unroll
+        for (int i = 0; i < PX; i++)
+          __builtin_amdgcn_global_load_lds((GlobalPtr)(own + pix[i]), (LdsPtr)(to + 256 * (PER + i)), 4, 0, 0);
+      }
     }
   };
   // (what the wavefront has in flight already is not the ring's: the count starts from nothing)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int groups = (d + CH - 1) / CH;
 #pragma unroll
   for (int c = 0; c < STAGES - 1; c++)
-    if (c < d) fetch(c, ring + c * kStage);
+    if (c < groups) fetch(c, ring + c * kStage);
   int at = 0, refill = STAGES - 1;
-  for (int c = 0; c < d; c++) {
-    if (c + STAGES - 2 < d) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((STAGES - 2) * kLoads) : "memory");
+  for (int c = 0; c < groups; c++) {
+    if (c + STAGES - 2 < groups) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((STAGES - 2) * CH * kLoads) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    if (c + STAGES - 1 < d) fetch(c + STAGES - 1, ring + refill * kStage);
-    consume(c, (unsigned)(size_t)(const __attribute__((address_space(3))) float*)(ring + at * kStage), 256u * PER);
+    if (c + STAGES - 1 < groups) fetch(c + STAGES - 1, ring + refill * kStage);
+    consume(CH * c, CH * c + 1 < d, (unsigned)(size_t)(const __attribute__((address_space(3))) float*)(ring + at * kStage), 256u * PER,
+            std::integral_constant<int, kChannel / 64>{});
     at = at + 1 == STAGES ? 0 : at + 1;
     refill = refill + 1 == STAGES ? 0 : refill + 1;
   }
@@ -1150,9 +1132,10 @@ __device__ __forceinline__ void ring_pass(const float* __restrict__ q, const flo
                                           size_t HW, int W, const Box& box, float* ring, Consume consume) {
   static_assert(PX == 2 && TileCfg<PX>::ELEMS == 9 * 256, "loads per thread: 4 to 9");
   const int count = __builtin_amdgcn_readfirstlane(box.w * box.h);
-  if (count <= 4 * 256) ring_pass_of<PX, 4, 5, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
-  else if (count <= 6 * 256) ring_pass_of<PX, 6, 4, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
-  else ring_pass_of<PX, 9, 3, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
+  constexpr int CH = FIRST ? 1 : 2;
+  if (count <= 4 * 256) ring_pass_of<PX, 4, FIRST ? 5 : 4, CH, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
+  else if (count <= 6 * 256) ring_pass_of<PX, 6, FIRST ? 4 : 3, CH, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
+  else ring_pass_of<PX, 9, FIRST ? 3 : 2, CH, FIRST>(q, a, pix, d, HW, W, box, ring, consume);
 }
 
 // MODE 0: the forward pass (costs: its five sums per pixel, a plane of N * H * W each, or null).  MODE 1: pass A from the costs.
@@ -1264,7 +1247,7 @@ __global__ __launch_bounds__(256) void quadfit_ring_tiles(const float* __restric
 #pragma unroll
       for (int j = 0; j < 5; j++) cost[i][j] = 0.f;
     if (!windowless)
-      ring_pass<PX, true>(q, a, pix, d, HW, W, box, ring, [&](int, unsigned buf, unsigned own) {
+      ring_pass<PX, true>(q, a, pix, d, HW, W, box, ring, [&](int, bool, unsigned buf, unsigned own, auto) {
         unsigned addr[kPairs];
         float v[kPairs];
 #pragma unroll
@@ -1322,18 +1305,23 @@ __global__ __launch_bounds__(256) void quadfit_ring_tiles(const float* __restric
     return t[0] * k[i].dFds;  // QF.cu:295
   };
   if (!windowless)
-    ring_pass<PX, false>(q, nullptr, pix, d, HW, W, box, ring, [&](int cc, unsigned buf, unsigned) {
+    ring_pass<PX, false>(q, nullptr, pix, d, HW, W, box, ring, [&](int cc, bool two, unsigned buf, unsigned, auto stride) {
       unsigned addr[10];
-      float v[10];
+      float2v v[10];
 #pragma unroll
       for (int i = 0; i < PX; i++)
 #pragma unroll
         for (int j = 0; j < 5; j++) addr[5 * i + j] = buf + lo[i][j];
-      lds_read10(addr, v);
+      lds_read10<decltype(stride)::value>(addr, v);
 #pragma unroll
-      for (int i = 0; i < PX; i++) {
-        const float g = gradient(i, v + 5 * i);
-        if (valid[i] && !far[i]) __builtin_nontemporal_store(g, &G0[(size_t)cc * HW + pix[i]]);
+      for (int u = 0; u < 2; u++) {
+        if (u == 1 && !two) break;
+#pragma unroll
+        for (int i = 0; i < PX; i++) {
+          const float t[5] = {v[5 * i][u], v[5 * i + 1][u], v[5 * i + 2][u], v[5 * i + 3][u], v[5 * i + 4][u]};
+          const float g = gradient(i, t);
+          if (valid[i] && !far[i]) __builtin_nontemporal_store(g, &G0[(size_t)(cc + u) * HW + pix[i]]);
+        }
       }
     });
   from_memory([&](int cc, const float (&)[PX], const float (&t)[PX][5]) {
@@ -1479,7 +1467,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   // channel; every group collects the tile's pairs for itself)
   const int d_lo = (int)blockIdx.y * per_group, d = min(per_group, d_all - d_lo);
   constexpr int kTH = TileCfg<PX>::TH;
-  __shared__ float win0[TileCfg<PX>::ELEMS], win1[TileCfg<PX>::ELEMS], win2[TileCfg<PX>::ELEMS], win3[TileCfg<PX>::ELEMS];
+  __shared__ __align__(16) float ring[kRingElems];
   __shared__ int red[16];
   int n, tx, ty;
   if (!tile_of_block(N, tiles_x, tiles_y, n, tx, ty)) return;
@@ -1501,8 +1489,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   // unconditionally and in batches (an absent list reads the pixel's own, an unused entry coefficient 0 of the sample):
   // lengths and lists of all pixels of the lane together, then the coefficients of one pixel at a time -- three round
   // trips to memory; behind `if (cnt > 0)` / `if (s < cnt)` each read waits for the one before it, some fifty in a row.
-  static_assert(TileCfg<PX>::ELEMS >= 2 * 64 * kPairs, "a window buffer holds the pairs of 64 pixels");
-  float2* const front = reinterpret_cast<float2*>(wave == 0 ? win0 : (wave == 1 ? win1 : (wave == 2 ? win2 : win3))) + lane;
+  static_assert(kRingElems >= 4 * 2 * 64 * kPairs, "the ring holds the pairs of 64 pixels per wavefront");
+  float2* const front = reinterpret_cast<float2*>(ring) + 64 * kPairs * wave + lane;
   int cnt[PX][5];
   int4 sl[PX][5];
 #pragma unroll
@@ -1585,7 +1573,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       const int sx = off[i][j] & 0xffff, sy = off[i][j] >> 16;
       const bool used = j < np[i];
       if (used && !(sx - box.x0 < box.w && sy - box.y0 < box.h)) slow[i] = true;
-      off[i][j] = used ? (unsigned)((sy - box.y0) * box.w + (sx - box.x0)) : 0u;
+      off[i][j] = used ? 4u * (unsigned)((sy - box.y0) * box.w + (sx - box.x0)) : 0u;
     }
 #pragma unroll
     for (int j = 0; j < kPairs; j++) {
@@ -1606,18 +1594,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
       }
     }
   }
-  window_pass_dma<PX>(a, d, HW, W, box, win0, win1, win2, win3, [&](int cc, const float* buf, const float* plane, int, bool live) {
+  const unsigned none[PX] = {};
+  ring_pass<PX, false>(a, nullptr, none, d, HW, W, box, ring, [&](int cc, bool two, unsigned buf, unsigned, auto stride) {
     // all window reads of a pixel are issued before the first product: a read inside the branch that skips an unused pair
     // is waited for on the spot, one LDS round trip after the other (an unused pair reads element 0, a broadcast)
 #pragma unroll
     for (int i = 0; i < PX; i++) {
-      float v[kPairs];
-      lds_gather12(buf, off[i], v);
-      float acc = 0.f;
+      unsigned addr[kPairs];
+      float2v v[kPairs];
+#pragma unroll
+      for (int j = 0; j < kPairs; j++) addr[j] = buf + off[i][j];
+      lds_read12<decltype(stride)::value>(addr, v);
+      float acc[2] = {0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < kPairs; j++)
-        if (need & (1u << j)) acc = __builtin_fmaf(v[j], cf[i][j], acc);
-      if (live && valid[i]) __builtin_nontemporal_store(slow[i] ? 0.f : acc, &G1[(size_t)cc * HW + pix[i]]);
+        if (need & (1u << j)) {
+          acc[0] = __builtin_fmaf(v[j][0], cf[i][j], acc[0]);
+          acc[1] = __builtin_fmaf(v[j][1], cf[i][j], acc[1]);
+        }
+      if (valid[i]) {
+        __builtin_nontemporal_store(slow[i] ? 0.f : acc[0], &G1[(size_t)cc * HW + pix[i]]);
+        if (two) __builtin_nontemporal_store(slow[i] ? 0.f : acc[1], &G1[(size_t)(cc + 1) * HW + pix[i]]);
+      }
     }
   });
 }
@@ -2169,15 +2167,14 @@ namespace {
 
 // Whether the per-pixel passes of the quadratic fit take the split kernels: too few tiles (64 x 8 pixels) to fill the chip.  The
 // split kernels work through whole chunks of 32 channels, so with fewer channels they pay up to fewer tiles only.  Measured, us,
-// split / tiled kernel, forward pass: 4 channels 6 tiles 6.0 / 7.2, 60 8.3 / 7.2; 8 channels 60 tiles 8.0 / 9.1, 104 12.2 / 9.5,
-// 248 23.5 / 10.2; 16 channels 104 tiles 12.1 / 13.4, 160 16.4 / 15.6; 20 channels 160 tiles 16.7 / 19.4, 192 19.7 / 16.8; 24
-// channels 248 tiles 23.0 / 24.7, 320 31.7 / 31.2; 32 channels 248 tiles 25.7 / 33.4; 64 channels 60 tiles 13.3 / 44.1, 248 44.9 /
-// 62.4; 65 channels (taps no longer kept in registers) 248 tiles 64.7 / 63.4; 128 channels 248 tiles 85 / 118.  Backward pass: the
-// lines cross at the same numbers of tiles up to 32 channels; 248 tiles: 64 channels 106 / 202, 65 176 / 203, 128 269 / 391.
+// split / ring, forward pass: 4 channels 40 tiles 7.4 / 8.9, 128 10.7 / 8.9; 8 channels 60 tiles 7.2 / 9.8, 91 9.5 / 10.0, 128
+// 11.0 / 10.3; 16 channels 128 tiles 11.0 / 11.5, 195 17.0 / 11.0; 24 channels 128 tiles 10.9 / 13.8, 195 16.9 / 14.0; 32 channels
+// 128 tiles 10.8 / 16.5, 195 17.8 / 17.3, 248 19.2 / 17.7; 64 channels 60 tiles 11.7 / 28.4, 195 31.5 / 28.8; 96 channels 128 tiles
+// 27.8 / 41.1, 195 45.9 / 40.1.  Backward pass (split / the faster of the others): 32 channels 128 tiles 51 / 50, 195 61 / 55; 64
+// channels 128 tiles 64 / 78, 195 82 / 83; 96 channels 195 tiles 147 / 115.
 bool quadfit_few_tiles(long long tiles, int ic) {
   if (inpaint::knobs().quadfit_split >= 0) return inpaint::knobs().quadfit_split == 1;
-  const long long cus = inpaint::compute_unit_count();
-  return tiles <= (ic >= 24 ? cus - 1 : cus * ic / kSplitChunk);
+  return tiles <= (long long)inpaint::compute_unit_count() * std::min(ic, 24) / kSplitChunk;
 }
 
 // Channels per block of the gather pass: all of them where the tiles fill the chip (four blocks resident per CU), else so
@@ -2248,11 +2245,13 @@ int quadfit_forward_saving(const float* im0, const float* im1, const float* flow
   return forward_of("quadfit_forward_saving", im0, im1, flow, out, costs, n, ic, ih, iw, flow_channels, stream);
 }
 
-// Images that the split kernels take have nothing to gain: their backward pass keeps all taps in registers and is bound by latency.
+// Not where the split kernels run, whose backward pass keeps all taps in registers and is bound by latency, and up to 32 channels
+// not before every CU has a tile: the resident pass A has twice as many (forward + backward, us, with / without the costs: 32
+// channels 195 tiles 80 / 72, 250 81 / 73, 300 84 / 85, 480 89 / 92, 960 124 / 140; 64 channels 195 tiles 112 / 178).
 int quadfit_saving_pays(int n, int ic, int ih, int iw) {
   if (n < 1 || ic < 1 || ih < 1 || iw < 1 || inpaint::knobs().quadfit_px_path || inpaint::knobs().quadfit_reread) return 0;
   const long long tiles = (long long)n * ((iw + kTW - 1) / kTW) * ((ih + TileCfg<kPxTile>::TH - 1) / TileCfg<kPxTile>::TH);
-  return !quadfit_few_tiles(tiles, ic);
+  return !quadfit_few_tiles(tiles, ic) && (ic > kResidentChannels || tiles > inpaint::compute_unit_count());
 }
 
 long long quadfit_backward_workspace_bytes(int n, int ih, int iw) {

@@ -59,7 +59,7 @@ def test_windows_of_every_size(qf, flowaux_oracle, spread):
 def test_autograd_saves_the_costs_where_it_pays(qf, flowaux_oracle):
     from customnetworklayers_amd import QuadFittingFromFlowFunction
 
-    for (n, c, h, w), kept_tensors in (((1, 8, 192, 640), 4), ((1, 32, 40, 64), 3)):
+    for (n, c, h, w), kept_tensors in (((1, 8, 200, 704), 4), ((1, 33, 192, 640), 4), ((1, 8, 192, 640), 3), ((1, 33, 40, 64), 3)):
         f0, f1, flow, grad = inputs(n, c, h, w, 1.0)
         a, b = dev(f0).requires_grad_(True), dev(f1).requires_grad_(True)
         kept = []
