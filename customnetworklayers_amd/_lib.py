@@ -72,6 +72,9 @@ def _load():
     lib.quadfit_forward_saving.argtypes = [_f32p] * 5 + [_int] * 5 + [ctypes.c_void_p]
     lib.quadfit_backward_saved.argtypes = [_f32p] * 7 + [_int] * 5 + [ctypes.c_void_p, ctypes.c_longlong, ctypes.c_void_p]
     lib.quadfit_saving_pays.argtypes = [_int] * 4
+    lib.quadfit_image_forward.argtypes = [_f32p] * 5 + [_int] * 3 + [ctypes.c_longlong] * 2 + [ctypes.c_void_p]
+    lib.quadfit_image_backward.argtypes = ([_f32p] * 7 + [_int] * 3 + [ctypes.c_longlong] * 2 + [ctypes.c_void_p, ctypes.c_longlong]
+                                           + [ctypes.c_void_p])
     lib.medimax_forward.argtypes = [_f32p] * 2 + [_int] * 4 + [ctypes.c_void_p]
     lib.medimax_backward.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_void_p]
     lib.medimax_forward_saving.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_void_p]

@@ -254,7 +254,7 @@ struct Factors {
   double k00;
   float k0p, k0m, kp0, km0, dFds;
 };
-__device__ __forceinline__ Factors scatter_factors(const Fit& f, const float* __restrict__ gin, size_t n, size_t HW, unsigned p) {
+__device__ __forceinline__ Factors scatter_factors(const Fit& f, float dFdfx, float dFdfy, float dFds) {
   Factors k;
   const int validX = f.validX, validY = f.validY;
   const float ax = f.ax, ay = f.ay, fx = f.fx, fy = f.fy;
@@ -267,9 +267,6 @@ __device__ __forceinline__ Factors scatter_factors(const Fit& f, const float* __
   const float ds_dc = (validX || validY) ? 1. : 0.;
   const float ds_day = validY ? fy * fy : 0.;
   const float ds_dby = validY ? fy : 0.;
-  const float dFdfx = gin[n * 3 * HW + p];  // QF.cu:261-263
-  const float dFdfy = gin[n * 3 * HW + HW + p];
-  const float dFds = gin[n * 3 * HW + 2 * HW + p];
   k.any_valid = validX || validY;
   k.dFds = dFds;
   k.k00 = -2. * dFdfx * dfx_dax - 2. * dFdfy * dfy_day - 2. * dFds * ds_dax - 2. * dFds * ds_day + 2. * dFds * ds_dc;
@@ -278,6 +275,10 @@ __device__ __forceinline__ Factors scatter_factors(const Fit& f, const float* __
   k.kp0 = dFdfy * dfy_day + dFdfy * dfy_dby + dFds * ds_day + dFds * ds_dby;
   k.km0 = dFdfy * dfy_day - dFdfy * dfy_dby + dFds * ds_day - dFds * ds_dby;
   return k;
+}
+
+__device__ __forceinline__ Factors scatter_factors(const Fit& f, const float* __restrict__ gin, size_t n, size_t HW, unsigned p) {
+  return scatter_factors(f, gin[n * 3 * HW + p], gin[n * 3 * HW + HW + p], gin[n * 3 * HW + 2 * HW + p]);  // QF.cu:261-263
 }
 
 // a source's scatter coefficients (contribution to g1 at a tap = I1 * coefficient, QF.cu:279-283,296) and its entry in the list
@@ -591,15 +592,15 @@ struct TilePx {
   unsigned o[5];  // taps 00, 0p, 0m, p0, m0: offsets into the window, or into the plane when far
 };
 
-// QF.cu:31-53: displaced position and tap coordinates of pixel (x, y); widens the tile's bounding box
-__device__ __forceinline__ void locate(TilePx& s, const float* __restrict__ fl, size_t HW, int H, int W, int x, int y,
-                                       bool valid, int& minx, int& maxx, int& miny, int& maxy) {
+// QF.cu:31-53: displaced position and tap coordinates of pixel (x, y), displacement (u, v); widens the tile's bounding box
+__device__ __forceinline__ void locate_at(TilePx& s, float u, float v, int H, int W, int x, int y, bool valid, int& minx, int& maxx,
+                                          int& miny, int& maxy) {
   s.inside = s.far = false;
   s.ix = s.iy = s.xm = s.xp = s.ym = s.yp = 0;
   s.p = valid ? (unsigned)y * W + x : 0u;
   if (!valid) return;
-  const float idx = x + fl[s.p];
-  const float idy = y + fl[HW + s.p];
+  const float idx = x + u;
+  const float idy = y + v;
   if (!(idx <= W - 1 && idx >= 0 && idy <= H - 1 && idy >= 0)) return;  // QF.cu:35; NaN counts as outside
   s.inside = true;
   s.ix = (int)floor(idx + 0.5);
@@ -608,6 +609,11 @@ __device__ __forceinline__ void locate(TilePx& s, const float* __restrict__ fl, 
   s.xp = min(s.ix + 1, W - 1); s.yp = min(s.iy + 1, H - 1);
   minx = min(minx, s.xm); maxx = max(maxx, s.xp);
   miny = min(miny, s.ym); maxy = max(maxy, s.yp);
+}
+__device__ __forceinline__ void locate(TilePx& s, const float* __restrict__ fl, size_t HW, int H, int W, int x, int y,
+                                       bool valid, int& minx, int& maxx, int& miny, int& maxy) {
+  const unsigned p = valid ? (unsigned)y * W + x : 0u;
+  locate_at(s, fl[p], fl[HW + p], H, W, x, y, valid, minx, maxx, miny, maxy);
 }
 
 __device__ __forceinline__ Box block_box(int minx, int maxx, int miny, int maxy, int* red, int capacity) {
@@ -1620,6 +1626,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
   });
 }
 
+// Workgroup barrier that orders LDS traffic only: global loads issued before it stay in flight.
+__device__ __forceinline__ void lds_only_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+#include "quadfit_image_kernels.h"
+
 // ---------------------------------------------------------------------------------------------
 // median
 // ---------------------------------------------------------------------------------------------
@@ -1994,13 +2009,6 @@ __global__ __launch_bounds__(64) void median_forward_run_kernel(const float* __r
   }
 }
 
-// Workgroup barrier that orders LDS traffic only: global loads issued before it stay in flight.
-__device__ __forceinline__ void lds_only_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // The backward pass over FULL tiles of 64 pixels for odd bin counts up to 4 * NV - 1 (no padding: the tile in LDS is a plain
 // copy of the run), as a loop: a wavefront keeps the next tile's run in flight (NV 16-byte loads per lane, held in registers)
 // while it walks the current one.  With one tile per wavefront only a quarter of the resident wavefronts have loads in
@@ -2339,6 +2347,60 @@ int quadfit_backward_saved(const float* im0, const float* im1, const float* flow
   if (!costs || !workspace) return fail(INPAINT_ERR_ARG, "quadfit_backward_saved: null pointer");
   return backward_of("quadfit_backward_saved", im0, im1, flow, gin, costs, g0, g1, n, ic, ih, iw, flow_channels, workspace,
                      workspace_bytes, stream);
+}
+
+static int image_args(const char* name, bool pointers, int ic, int ih, int iw, long long flow_pixel_stride, long long flow_channel_stride) {
+  if (!pointers) return fail(INPAINT_ERR_ARG, "%s: null pointer", name);
+  if (ic < 1 || ih < 1 || iw < 1) return fail(INPAINT_ERR_ARG, "%s: bad shape %dx%dx%d", name, ih, iw, ic);
+  if ((long long)ih * iw * ic >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "%s: image too large", name);
+  if (flow_pixel_stride < 1 || flow_channel_stride < 1) return fail(INPAINT_ERR_ARG, "%s: bad strides of the flow", name);
+  return 0;
+}
+static dim3 image_grid(long long P) { return dim3((unsigned)(((P + quadfit_image::kPixels - 1) / quadfit_image::kPixels + 7) / 8 * 8)); }
+
+int quadfit_image_forward(const float* im0, const float* im1, const float* flow, float* out, float* costs, int ic, int ih, int iw,
+                          long long flow_pixel_stride, long long flow_channel_stride, void* stream) {
+  if (const int rc = image_args("quadfit_image_forward", im0 && im1 && flow && out, ic, ih, iw, flow_pixel_stride, flow_channel_stride))
+    return rc;
+  const quadfit_image::FlowStrides fs{flow_pixel_stride, flow_channel_stride};
+  const dim3 grid = image_grid((long long)ih * iw), block(256);
+  if (ic % 4 == 0 && aligned16(im0) && aligned16(im1))
+    hipLaunchKernelGGL((quadfit_image::forward<4>), grid, block, 0, (hipStream_t)stream, im0, im1, flow, fs, out, costs, ic, ih, iw);
+  else
+    hipLaunchKernelGGL((quadfit_image::forward<1>), grid, block, 0, (hipStream_t)stream, im0, im1, flow, fs, out, costs, ic, ih, iw);
+  INPAINT_HIP(hipGetLastError());
+  return 0;
+}
+
+int quadfit_image_backward(const float* im0, const float* im1, const float* flow, const float* gin, const float* costs, float* g0,
+                           float* g1, int ic, int ih, int iw, long long flow_pixel_stride, long long flow_channel_stride,
+                           void* workspace, long long workspace_bytes, void* stream) {
+  if (const int rc = image_args("quadfit_image_backward", im0 && im1 && flow && gin && costs && g0 && g1 && workspace, ic, ih, iw,
+                                flow_pixel_stride, flow_channel_stride))
+    return rc;
+  const long long P = (long long)ih * iw;
+  if (workspace_bytes < qf_workspace_bytes(P))
+    return fail(INPAINT_ERR_ARG, "quadfit_image_backward: workspace of %lld bytes, %lld needed", workspace_bytes, qf_workspace_bytes(P));
+  if (((uintptr_t)workspace & 15) != 0) return fail(INPAINT_ERR_ARG, "quadfit_image_backward: workspace must be 16-byte aligned");
+  const QfWorkspace ws = qf_carve(workspace, P);
+  const quadfit_image::FlowStrides fs{flow_pixel_stride, flow_channel_stride};
+  const dim3 grid = image_grid(P), block(256);
+  hipStream_t st = (hipStream_t)stream;
+  // the counters start at zero (a fill kernel, so that the call can be captured into a graph)
+  hipLaunchKernelGGL(inpaint::fill_zero_f32, dim3(inpaint::grid_stride(P + 64)), dim3(256), 0, st, reinterpret_cast<float*>(ws.count),
+                     P + 64);
+  const bool wide = ic % 4 == 0 && aligned16(im0) && aligned16(im1) && aligned16(g0) && aligned16(g1);
+  if (wide) {
+    hipLaunchKernelGGL((quadfit_image::sources<4>), grid, block, 0, st, im1, flow, fs, gin, costs, g0, ws, ic, ih, iw);
+    hipLaunchKernelGGL((quadfit_image::gather<4>), grid, block, 0, st, im0, g1, ws, ic, ih, iw);
+  } else {
+    hipLaunchKernelGGL((quadfit_image::sources<1>), grid, block, 0, st, im1, flow, fs, gin, costs, g0, ws, ic, ih, iw);
+    hipLaunchKernelGGL((quadfit_image::gather<1>), grid, block, 0, st, im0, g1, ws, ic, ih, iw);
+  }
+  hipLaunchKernelGGL(quadfit_image::overflow, dim3((unsigned)std::min<long long>((P + 127) / 128, 512)), block, 0, st, im0, flow, fs, g1,
+                     ws, ic, ih, iw);
+  INPAINT_HIP(hipGetLastError());
+  return 0;
 }
 
 int medimax_forward(const float* vol, float* out, int n, int ih, int iw, int num_disp, void* stream) {

@@ -116,6 +116,57 @@ def backward(d_iGf, featureImage0, featureImage1, flow, use_atomics=False, costs
     return [d_oFeat0, d_oFeat1]
 
 
+def takes_image(feat0, feat1, flow):
+    """Whether image_forward / image_backward take these H x W x C maps and H x W x 3 flow as they are: both maps contiguous with
+    more than one channel innermost.  (Maps that are views of channel planes, and everything that is to be refused, go through
+    forward / backward.)"""
+    if not (feat0.dim() == 3 and flow.dim() == 3 and feat0.shape == feat1.shape and feat0.shape[:2] == flow.shape[:2]):
+        return False
+    if not all(t.is_cuda and t.dtype == torch.float32 and t.device == flow.device for t in (feat0, feat1, flow)):
+        return False
+    h, w, c = feat0.shape
+    return (feat0.is_contiguous() and feat1.is_contiguous() and c > 1 and h * w > 1 and h * w * c < 2 ** 31)
+
+
+def _flow_strides(flow):
+    """flow with its pixels a fixed distance apart, that distance and the one between its channels"""
+    if flow.stride(0) != flow.shape[1] * flow.stride(1) or min(flow.stride()) < 1:
+        flow = flow.contiguous()
+    return flow, flow.stride(1), flow.stride(2)
+
+
+def image_forward(feat0, feat1, flow, want_costs):
+    """The fit of one image, feat0, feat1 H x W x C, flow H x W x 3 (takes_image).  Returns [H x W x 3, costs (5,H,W) or None]."""
+    h, w, c = feat0.shape
+    flow, pixel, channel = _flow_strides(flow)
+    out = torch.empty((h, w, 3), dtype=torch.float32, device=flow.device)
+    costs = torch.empty((5, h, w), dtype=torch.float32, device=flow.device) if want_costs else None
+    with torch.cuda.device(flow.device):
+        rc = lib.quadfit_image_forward(feat0.data_ptr(), feat1.data_ptr(), flow.data_ptr(), out.data_ptr(),
+                                       costs.data_ptr() if want_costs else None, c, h, w, pixel, channel, _stream(flow))
+    if rc:
+        raise _ERRORS.get(rc, RuntimeError)("FlowQuadFitting::forward failed: %s" % _last_error())
+    return [out, costs]
+
+
+def image_backward(d_iGf, feat0, feat1, flow, costs):
+    """d_iGf: H x W x 3 gradient wrt the result, costs: the second result of image_forward.  Returns the two maps' gradients."""
+    for t, name in ((d_iGf, "d_iGf"), (feat0, "featureImage0"), (feat1, "featureImage1"), (costs, "costs")):
+        _check_input(t, name)
+    h, w, c = feat0.shape
+    flow, pixel, channel = _flow_strides(flow)
+    g0, g1 = torch.empty_like(feat0), torch.empty_like(feat1)
+    ws_bytes = lib.quadfit_backward_workspace_bytes(1, h, w)
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=flow.device)
+    with torch.cuda.device(flow.device):
+        rc = lib.quadfit_image_backward(feat0.data_ptr(), feat1.data_ptr(), flow.data_ptr(), d_iGf.data_ptr(), costs.data_ptr(),
+                                        g0.data_ptr(), g1.data_ptr(), c, h, w, pixel, channel, workspace.data_ptr(), ws_bytes,
+                                        _stream(flow))
+    if rc:
+        raise _ERRORS.get(rc, RuntimeError)("FlowQuadFitting::backward failed: %s" % _last_error())
+    return [g0, g1]
+
+
 def dummy():
     print("Input: not present just dummy:")
     return []

@@ -30,6 +30,23 @@ class QuadFittingFromFlowFunction(Function):
         return d_oGfeat0, d_oGfeat1, None
 
 
+class _QuadFittingImage(Function):
+    """QuadFittingFromFlowFunction of one image with its channels innermost, no permutations around it."""
+
+    @staticmethod
+    def forward(ctx, feat0, feat1, flow):
+        sol, costs = QuadFit_cuda_ext.image_forward(feat0, feat1, flow, any(ctx.needs_input_grad))
+        ctx.save_for_backward(feat0, feat1, flow, costs)
+        return sol
+
+    @staticmethod
+    def backward(ctx, grad_sol):
+        feat0, feat1, flow, costs = ctx.saved_tensors
+        d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.image_backward(grad_sol.contiguous(), feat0.contiguous(), feat1.contiguous(), flow,
+                                                               costs.contiguous())
+        return d_oGfeat0, d_oGfeat1, None
+
+
 class QuadFittingFromFlow(nn.Module):
     def __init__(self, device):
         super(QuadFittingFromFlow, self).__init__()
@@ -40,6 +57,8 @@ class QuadFittingFromFlow(nn.Module):
         only the first two, the x and y displacement, are read).  Returns H x W x 3."""
         Yi, Xi, Li = t_flow.shape
         assert Li == 3, "flow should have 3 channels: the displacement in X and Y direction and one more\n"
+        if QuadFit_cuda_ext.takes_image(t_feat0, t_feat1, t_flow):
+            return _QuadFittingImage.apply(t_feat0, t_feat1, t_flow)
         t_feat0_in = t_feat0.permute(2, 0, 1).unsqueeze(0)
         t_feat1_in = t_feat1.permute(2, 0, 1).unsqueeze(0)
         t_flow_in = t_flow.permute(2, 0, 1).unsqueeze(0)

@@ -61,6 +61,19 @@ int quadfit_backward_saved(const float* im0, const float* im1, const float* flow
                            void* stream);
 int quadfit_saving_pays(int n, int ic, int ih, int iw);
 
+/* The fit of one image with its channels innermost, the layout of the reference's Python module (QuadFitting.py:43-62, which
+ * permutes on the way in and out): the same numbers as quadfit_forward / quadfit_backward on the permuted planes, without the copies.
+ *   im0, im1, g0, g1 : (ih,iw,ic)      out, gin : (ih,iw,3)
+ *   flow : element (pixel p in row order, channel c) lies at p*flow_pixel_stride + c*flow_channel_stride; two channels are read
+ *   costs : 5*ih*iw floats, written by the forward pass (NULL: not wanted) and read by the backward pass
+ *   workspace : as for quadfit_backward(1, ih, iw), required
+ * ih*iw*ic is below 2^31. */
+int quadfit_image_forward(const float* im0, const float* im1, const float* flow, float* out, float* costs, int ic, int ih, int iw,
+                          long long flow_pixel_stride, long long flow_channel_stride, void* stream);
+int quadfit_image_backward(const float* im0, const float* im1, const float* flow, const float* gin, const float* costs, float* g0,
+                           float* g1, int ic, int ih, int iw, long long flow_pixel_stride, long long flow_channel_stride,
+                           void* workspace, long long workspace_bytes, void* stream);
+
 /* Replaces MediMax::forward (cudaMedian/cudaCode/medimax.h:13, cudaMedian/cudaCode/medimax.cu:17-44,
  * 131-168), bound by cudaMedian/median_cuda.cpp:36-70.
  *   vol : (n,ih,iw,num_disp) histogram over num_disp displacement bins, bins innermost
