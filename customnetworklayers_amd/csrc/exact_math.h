@@ -62,6 +62,43 @@ __device__ __forceinline__ float exact_sqrt(float x) {
   return __builtin_fmaf(e, 0.5f * y, s);
 }
 
+// What the TV layer's Huber norm is needed for, from its square A, with the one transcendental instruction that the root takes.
+// v_rsq_f32 of A is the reciprocal of the root to an ulp or two: refined once against the rounded root it serves as the reciprocal
+// that a division needs, and its square as the one of A.  A = 0 gives a NaN for the root, which counts as below the threshold.
+//
+// Forward: m = max(1, sqrt(A) / 0.1f) and rm with div_by(w, m, rm) = w / m, correctly rounded for every w: rm is the correctly
+// rounded reciprocal for all but 271 values of A, and for those the quotients are right for all 2^23 mantissas of w.
+// Adjoint: active = sqrt(A) > 0.1f, nom = 0.1f / sqrt(A) and twice = 2 * (nom / (2 sqrt(A)^2)) where it is active, 1 and 0 where not.
+// The same bits as the divisions one by one up to A = 2^80 (twice is below the smallest normal number from there on).
+// (All three checked for every float: inpaint_selftest_huber.)  35 -> 25 issue slots in the adjoint (reciprocals take four),
+// 24 -> 21 in the forward pass.  With the regime test in one comparison (regime_threshold), us, before / after: forward pass at
+// inference 4 x 2 x 384 x 1248, 100 iterations 973 / 936, backward 2659 / 2635 (231 -> 206 registers); 1 x 1 x 384 x 1248 659 / 638.
+struct HuberForward {
+  float m, rm;
+};
+__device__ __forceinline__ HuberForward huber_forward(float A) {
+  const float y = __builtin_amdgcn_rsqf(A);
+  const float s = A * y;
+  const float hub = __builtin_fmaf(__builtin_fmaf(-s, s, A), 0.5f * y, s);
+  const float m = fmaxf(1.f, div_by_tenth(hub));
+  const float r = fminf(1.f, 0.1f * y);
+  return {m, __builtin_fmaf(__builtin_fmaf(-m, r, 1.f), r, r)};
+}
+struct HuberAdjoint {
+  bool active;
+  float nom, twice;
+};
+__device__ __forceinline__ HuberAdjoint huber_adjoint(float A) {
+  const float y = __builtin_amdgcn_rsqf(A);
+  const float s = A * y;
+  const float hub = __builtin_fmaf(__builtin_fmaf(-s, s, A), 0.5f * y, s);
+  const bool active = hub > 0.1f;
+  const float nom = div_by(0.1f, hub, __builtin_fmaf(__builtin_fmaf(-hub, y, 1.f), y, y));
+  const float square = hub * hub, z = y * y;
+  const float twice = div_by(nom, square, __builtin_fmaf(__builtin_fmaf(-square, z, 1.f), z, z));
+  return {active, active ? nom : 1.f, active ? twice : 0.f};
+}
+
 // Values of lanes outside the image read as +0: inside(v) is v where `ok` held and +0 elsewhere, bit for bit what
 // `ok ? v : 0.f` gives.  The loaded bits are ANDed with an all-ones / all-zeros word whose origin the empty asm hides
 // from the optimizer; written as a conditional, a group of such values is compiled into a branch that zeroes all of

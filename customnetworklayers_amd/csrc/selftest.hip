@@ -142,6 +142,43 @@ __global__ __launch_bounds__(256) void selftest_pairs_kernel(unsigned long long*
   if (bad1) atomicAdd(&counts[1], (unsigned long long)bad1);
 }
 
+// The Huber norm's forms against the compiler's IEEE root and divisions, over A = 0 and every float in [2^-96, 2^80].
+// counts[0]: the forward factor m; counts[1]: active, nom or twice of the adjoint; counts[2]: values of A whose rm is not the
+// correctly rounded reciprocal of m, listed for the second kernel.
+constexpr unsigned kHuberList = 4096;
+__global__ __launch_bounds__(256) void selftest_huber_kernel(unsigned long long* counts, unsigned* list) {
+  unsigned bad0 = 0, bad1 = 0;
+  for (unsigned long long i = blockIdx.x * 256ull + threadIdx.x; i < 0x7f800000ull; i += gridDim.x * 256ull) {
+    const float A = __uint_as_float((unsigned)i);
+    if (!(A == 0.f || (A >= 1.2621774e-29f && A <= 1.2089258e24f))) continue;
+    const float root = sqrtf(A);
+    const HuberForward f = huber_forward(A);
+    bad0 += !same_bits(f.m, fmaxf(1.f, root / 0.1f));
+    if (!same_bits(f.rm, 1.f / f.m)) {
+      const unsigned long long at = atomicAdd(&counts[2], 1ull);
+      if (at < kHuberList) list[at] = (unsigned)i;
+    }
+    const HuberAdjoint a = huber_adjoint(A);
+    const bool active = root > 0.1f;
+    const float nom = active ? 0.1f / root : 1.f;
+    const float twice = active ? 2.f * (nom / (2.f * root * root)) : 0.f;
+    bad1 += a.active != active || !same_bits(a.nom, nom) || !same_bits(a.twice, twice);
+  }
+  if (bad0) atomicAdd(&counts[0], (unsigned long long)bad0);
+  if (bad1) atomicAdd(&counts[1], (unsigned long long)bad1);
+}
+// counts[3]: wrong quotients w / m over all mantissas of w, one listed A per block
+__global__ __launch_bounds__(256) void selftest_huber_quotients(unsigned long long* counts, const unsigned* list) {
+  if (blockIdx.x >= counts[2]) return;
+  const HuberForward f = huber_forward(__uint_as_float(list[blockIdx.x]));
+  unsigned bad = 0;
+  for (unsigned w = threadIdx.x; w < 0x800000u; w += 256) {
+    const float x = __uint_as_float(0x3f800000u | w);
+    bad += !same_bits(div_by(x, f.m, f.rm), x / f.m);
+  }
+  if (bad) atomicAdd(&counts[3], (unsigned long long)bad);
+}
+
 int run_selftest(void (*kernel)(unsigned long long*, unsigned int), unsigned long long* host4, unsigned int rounds) {
   unsigned long long* dev = nullptr;
   INPAINT_HIP(hipMalloc((void**)&dev, 4 * sizeof(unsigned long long)));
@@ -157,6 +194,21 @@ int run_selftest(void (*kernel)(unsigned long long*, unsigned int), unsigned lon
 
 extern "C" int inpaint_selftest_rsqrt(unsigned long long* mismatches4_host, unsigned int pair_rounds) {
   return run_selftest(selftest_rsqrt_kernel, mismatches4_host, pair_rounds);
+}
+
+extern "C" int inpaint_selftest_huber(unsigned long long* counts4_host) {
+  if (!counts4_host) return inpaint::fail(INPAINT_ERR_ARG, "inpaint_selftest_huber: null pointer");
+  unsigned long long* dev = nullptr;
+  const size_t bytes = 4 * sizeof(unsigned long long) + kHuberList * sizeof(unsigned);
+  INPAINT_HIP(hipMalloc((void**)&dev, bytes));
+  INPAINT_HIP(hipMemset(dev, 0, bytes));
+  unsigned* list = reinterpret_cast<unsigned*>(dev + 4);
+  hipLaunchKernelGGL(selftest_huber_kernel, dim3(4096), dim3(256), 0, 0, dev, list);
+  hipLaunchKernelGGL(selftest_huber_quotients, dim3(kHuberList), dim3(256), 0, 0, dev, list);
+  INPAINT_HIP(hipGetLastError());
+  INPAINT_HIP(hipMemcpy(counts4_host, dev, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+  INPAINT_HIP(hipFree(dev));
+  return 0;
 }
 
 // Slices first_slice .. first_slice + slices - 1 of the 64 slices of 2^17 denominator mantissas each (all 2^23

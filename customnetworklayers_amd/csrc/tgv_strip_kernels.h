@@ -570,6 +570,23 @@ __global__ __launch_bounds__(256) void tgv_forward_strip2(
   }
 }
 
+// u of y_{k+1} by the TV layer's rule from x05[k] (xa) and x05[k-1] (xb), TV.cu:1149-1165; rc = rcp_refined(1 + conf)
+__device__ __forceinline__ float rebuild_u(float bb, float xa, float xb, float conf, float rc, double opc_d,
+                                           float t) {
+  float diff = bb - xa;
+  float sign = (diff < 0) ? -1.f : 1.f;
+  const bool quad = (opc_d >= (double)(sign * diff));  // opc_d = 1. + (double)conf
+  const float cb = conf * bb;
+  const float xk_q = div_by(cb + xa, 1.f + conf, rc);
+  const float xkm_q = div_by(cb + xb, 1.f + conf, rc);
+  const float y_q = xk_q + t * (xk_q - xkm_q);
+  const float xk_l = (conf <= sign * diff) ? bb - diff + sign * conf : bb;
+  diff = bb - xb;
+  sign = (diff < 0) ? -1.f : 1.f;
+  const float y_l = xk_l + t * (xk_l - ((conf <= sign * diff) ? bb - diff + sign * conf : bb));
+  return quad ? y_q : y_l;
+}
+
 // -------------------------------------------------------------------------------------------------
 // Adjoint iteration with the y rebuild fused in: TGV.cu:224-644 (+1478-1541); END = the
 // segment-start variant TGV.cu:1061-1472 that reads y from the checkpoint and writes the Huber
@@ -713,7 +730,7 @@ __global__ __launch_bounds__(256) void tgv_adjoint_strip(
           o.y[v][ch] = xv + t * (xv - xp);  // TGV.cu:1686-1690
         }
       } else {
-        o.y[0][ch] = END ? xb : tvstrip::rebuild_y_fast(bv, xa, xb, o.c, o.rc1, o.opc_d, t);
+        o.y[0][ch] = END ? xb : rebuild_u(bv, xa, xb, o.c, o.rc1, o.opc_d, t);
         o.y[1][ch] = inside(o.y[1][ch]);
         o.y[2][ch] = inside(o.y[2][ch]);
       }
@@ -1113,8 +1130,8 @@ __global__ __launch_bounds__(256) void tgv_adjoint_strip2(
 #pragma unroll
     for (int ch = 0; ch < C; ch++) {
       const float xa = inside(o.xa0[ch]), xb = inside(o.xb0[ch]), xc = inside(o.yB[0][ch]), bv = inside(o.bb[ch]);
-      o.yA[0][ch] = tvstrip::rebuild_y_fast(bv, xa, xb, o.c, rc1, opc_d, tA);
-      o.yB[0][ch] = BEND ? xc : tvstrip::rebuild_y_fast(bv, xb, xc, o.c, rc1, opc_d, tB);
+      o.yA[0][ch] = rebuild_u(bv, xa, xb, o.c, rc1, opc_d, tA);
+      o.yB[0][ch] = BEND ? xc : rebuild_u(bv, xb, xc, o.c, rc1, opc_d, tB);
       o.xa0[ch] = xa;
       o.xb0[ch] = xb;
       o.bb[ch] = bv;
@@ -1798,7 +1815,7 @@ __global__ __launch_bounds__(128) void tgv_adjoint_strip2w(
           const float pa = tvstrip::prox_huber1(xa, o.c, rc1, bv), pb = tvstrip::prox_huber1(xb, o.c, rc1, bv);
           o.yA[0][ch] = pa + tA * (pa - pb);  // TGV.cu:1773
         } else {
-          o.yA[0][ch] = tvstrip::rebuild_y_fast(bv, xa, xb, o.c, rc1, opc_d, tA);
+          o.yA[0][ch] = rebuild_u(bv, xa, xb, o.c, rc1, opc_d, tA);
         }
         o.xa0[ch] = xa;
         o.xb0[ch] = xb;
@@ -1951,7 +1968,7 @@ __global__ __launch_bounds__(128) void tgv_adjoint_strip2w(
           const float pc = BEND ? xc : tvstrip::prox_huber1(xc, o.c, rc1, bv);
           o.yB[0][ch] = pb + tB * (pb - pc);
         } else {
-          o.yB[0][ch] = BEND ? xc : tvstrip::rebuild_y_fast(bv, xb, xc, o.c, rc1, opc_d, tB);
+          o.yB[0][ch] = BEND ? xc : rebuild_u(bv, xb, xc, o.c, rc1, opc_d, tB);
         }
         o.xb0[ch] = xb;
         o.bb[ch] = bv;
@@ -2440,7 +2457,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           const float pa = tvstrip::prox_huber1(xa, o.c, rc1, bv), pb = tvstrip::prox_huber1(xb, o.c, rc1, bv);
           o.yA[0][ch] = pa + tA * (pa - pb);  // TGV.cu:1773
         } else {
-          o.yA[0][ch] = tvstrip::rebuild_y_fast(bv, xa, xb, o.c, rc1, opc_d, tA);
+          o.yA[0][ch] = rebuild_u(bv, xa, xb, o.c, rc1, opc_d, tA);
         }
         o.xa0[ch] = xa;
         o.bb[ch] = bv;
@@ -2617,7 +2634,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           const float pc = BEND ? xc : tvstrip::prox_huber1(xc, o.c, rc1, bv);
           o.yB[0][ch] = pb + tB * (pb - pc);
         } else {
-          o.yB[0][ch] = BEND ? xc : tvstrip::rebuild_y_fast(bv, xb, xc, o.c, rc1, opc_d, tB);
+          o.yB[0][ch] = BEND ? xc : rebuild_u(bv, xb, xc, o.c, rc1, opc_d, tB);
         }
         o.xb0[ch] = xb;
         o.bb[ch] = bv;

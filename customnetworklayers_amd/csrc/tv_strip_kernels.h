@@ -28,7 +28,6 @@
 namespace tvstrip {
 
 using inpaint::div_by;
-using inpaint::exact_sqrt;
 using inpaint::rcp_refined;
 
 constexpr int kFwdCols = 63;      // output columns per wavefront, forward (lane 0 is the apron)
@@ -224,11 +223,9 @@ __global__ __launch_bounds__(256) void tv_forward_strip(
       const float yc = cur.y[ch];
       const float d1 = yc - nxt.y[ch];
       const float d2 = yc - cur.yr[ch];
-      const float hub = exact_sqrt(d1 * d1 * cur.wys + d2 * d2 * cur.wxs);
-      const float m = fmaxf(1.f, inpaint::div_by_tenth(hub));
-      const float rm = rcp_refined(m);
-      const float e1 = d1 * div_by(cur.wys, m, rm);
-      const float e2 = d2 * div_by(cur.wxs, m, rm);
+      const inpaint::HuberForward hub = inpaint::huber_forward(d1 * d1 * cur.wys + d2 * d2 * cur.wxs);
+      const float e1 = d1 * div_by(cur.wys, hub.m, hub.rm);
+      const float e2 = d2 * div_by(cur.wxs, hub.m, hub.rm);
       const float e1_above = e1_up[ch];
       e1_up[ch] = e1;
       if (first.value) continue;
@@ -396,11 +393,9 @@ __global__ __launch_bounds__(256) void tv_forward_strip2(
   auto triangle = [&](float yc, float yd, float wxs, float wys, float& e1, float& e2) {
     const float d1 = yc - yd;
     const float d2 = yc - from_right_lane(yc);
-    const float hub = exact_sqrt(d1 * d1 * wys + d2 * d2 * wxs);
-    const float m = fmaxf(1.f, inpaint::div_by_tenth(hub));
-    const float rm = rcp_refined(m);
-    e1 = d1 * div_by(wys, m, rm);
-    e2 = d2 * div_by(wxs, m, rm);
+    const inpaint::HuberForward hub = inpaint::huber_forward(d1 * d1 * wys + d2 * d2 * wxs);
+    e1 = d1 * div_by(wys, hub.m, hub.rm);
+    e2 = d2 * div_by(wxs, hub.m, hub.rm);
   };
   // gradient step + Huber-1 prox + extrapolation of one pixel (TV.cu:1258-1316)
   auto update = [&](float yc, float e1_above, float e2_left, float e1, float e2, float c, float rc1, float bv,
@@ -528,44 +523,52 @@ __global__ __launch_bounds__(256) void tv_forward_strip2(
 // with nom = 1, denom = 0, which reproduces the inactive branch exactly.
 // -------------------------------------------------------------------------------------------------
 
-// y_{k+1} from x05[k] (xa) and x05[k-1] (xb), TV.cu:1149-1165; rc = rcp_refined(1 + conf)
-__device__ __forceinline__ float rebuild_y_fast(float bb, float xa, float xb, float conf, float rc, double opc_d,
-                                                float t) {
-  float diff = bb - xa;
-  float sign = (diff < 0) ? -1.f : 1.f;
-  const bool quad = (opc_d >= (double)(sign * diff));  // opc_d = 1. + (double)conf
-  const float cb = conf * bb;
-  const float xk_q = div_by(cb + xa, 1.f + conf, rc);
-  const float xkm_q = div_by(cb + xb, 1.f + conf, rc);
-  const float y_q = xk_q + t * (xk_q - xkm_q);
-  const float xk_l = (conf <= sign * diff) ? bb - diff + sign * conf : bb;
-  diff = bb - xb;
-  sign = (diff < 0) ? -1.f : 1.f;
-  const float y_l = xk_l + t * (xk_l - ((conf <= sign * diff) ? bb - diff + sign * conf : bb));
-  return quad ? y_q : y_l;
+// The largest float that is not above 1. + (double)c: the reference's regime test compares a float with that double
+// (TV.cu:806, 1154), which is the same as comparing it with this float.
+__device__ __forceinline__ float regime_threshold(float c) {
+  const double d = 1. + (double)c;
+  const float f = (float)d;
+  if (!((double)f > d)) return f;
+  return __uint_as_float(__float_as_uint(f) + (f > 0.f ? -1 : 1));
 }
 
-// The pieces of that rebuild for one half-step value v: q = the quadratic branch's iterate (TV.cu:1156-1157),
-// l = the other branch's (TV.cu:1162-1164), quad = the regime test on v (TV.cu:1154).  rebuild_y_fast(bb, xa, xb, ...)
-// is quad(xa) ? q(xa) + t (q(xa) - q(xb)) : l(xa) + t (l(xa) - l(xb)); a kernel that rebuilds two consecutive y
-// evaluates the pieces of the shared middle value once.
-struct RebuildPieces {
-  float q, l;
-  bool quad;
-};
-__device__ __forceinline__ RebuildPieces rebuild_pieces(float bb, float v, float conf, float rc, double opc_d) {
-  RebuildPieces r;
-  const float diff = bb - v;
-  const float sign = (diff < 0) ? -1.f : 1.f;
-  r.quad = (opc_d >= (double)(sign * diff));
-  r.q = div_by(conf * bb + v, 1.f + conf, rc);
-  r.l = (conf <= sign * diff) ? bb - diff + sign * conf : bb;
-  return r;
+// Prox adjoint of one pixel at the half-step value xh (TV.cu:806-828): the incoming adjoint df becomes g05; gc_add and
+// gb_add are the confidence's and the right-hand side's share.  rc1, rc2: refined reciprocals of 1 + conf and its square.
+// The reference has a third regime between the two (TV.cu:818-822: conf >= |b - xh| > 1. + (double)conf); no number is in
+// it, so it is left out.  Its sign * diff (sign: -1 where diff < 0, else 1) is |diff|.
+template <bool TRUE_ADJ>
+__device__ __forceinline__ void prox_adjoint(float df, float bv, float xh, float conf, float rc1, float rc2, float thr,
+                                             float& g05v, float& gc_add, float& gb_add) {
+  constexpr float kGC = TRUE_ADJ ? 1.f : kLocalGCMult;
+  const float diff = bv - xh;
+  const bool quad = thr >= fabsf(diff);
+  const float opc = 1.f + conf;
+  const float gc_q = df * (div_by(bv, opc, rc1) - div_by(conf * bv + xh, opc * opc, rc2)) * kGC;
+  const float g05_q = div_by(df, opc, rc1);
+  const float gb_q = div_by(df * conf, opc, rc1) * 1.0f;
+  g05v = quad ? g05_q : df;
+  gc_add = quad ? gc_q : (diff < 0 ? -df : df) * kGC;
+  gb_add = quad ? gb_q : 0.f;  // (adding +0 where the reference adds nothing leaves an accumulator unchanged)
 }
-__device__ __forceinline__ float rebuild_from(const RebuildPieces& a, const RebuildPieces& b, float t) {
+
+// What the y rebuild of TV.cu:1149-1165 takes from one half-step value v: the iterate by the quadratic rule (q) and by the
+// other rule (l).  Every x05 row serves two steps, as the later and as the earlier value, so a step keeps them for the next.
+struct Rebuild {
+  float q, l;
+};
+__device__ __forceinline__ Rebuild rebuild_of(float v, float bv, float conf, float rc1) {
+  const float diff = bv - v;
+  return {div_by(conf * bv + v, 1.f + conf, rc1), conf <= fabsf(diff) ? bv - diff + (diff < 0 ? -conf : conf) : bv};
+}
+
+// y_{k+1} from the half-step values x05[k] (a its pieces, xa the value) and x05[k-1], thr = regime_threshold(conf)
+__device__ __forceinline__ float rebuild_from(const Rebuild& a, const Rebuild& b, float bv, float xa, float thr, float t) {
   const float y_q = a.q + t * (a.q - b.q);
   const float y_l = a.l + t * (a.l - b.l);
-  return a.quad ? y_q : y_l;
+  return thr >= fabsf(bv - xa) ? y_q : y_l;
+}
+__device__ __forceinline__ float rebuild_y(float bv, float xa, float xb, float conf, float rc1, float thr, float t) {
+  return rebuild_from(rebuild_of(xa, bv, conf, rc1), rebuild_of(xb, bv, conf, rc1), bv, xa, thr, t);
 }
 
 // y_{k+1} exactly as the forward pass made it: x_{k+1} = prox(x05[k]) (TV.cu:1286-1292), y_{k+1} = x_{k+1} +
@@ -583,7 +586,7 @@ struct AdjRow {
   float c, rc1, wxs, wys, xa[C], y[C], bb[C], g[C];  // y is loaded as x05[k-1] (or the checkpoint y) and rebuilt in place
   float xl[C];                                       // FIRST only: the last x05 row, which the first step linearises at
   float gc_i, gwx_i, gwy_i, gx_i[C], gb_i[C];        // accumulators and partial g_x the row's pixel update continues
-  double opc_d;                                      // 1. + (double)c, the left side of the prox regime test
+  float thr;  // regime_threshold(c)
 };
 
 // TRUE_ADJ selects the corrected gradient (not the reference's): y is the forward pass's own y (see prox_huber1;
@@ -667,7 +670,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip(
     const inpaint::LaneMask inside(ok);
     o.c = inside(o.c);
     o.rc1 = rcp_refined(1.f + o.c);
-    o.opc_d = 1. + (double)o.c;
+    o.thr = regime_threshold(o.c);
     o.wxs = (ok && wx_ok) ? kL * o.wxs : 0.f;
     o.wys = (ok && h < H - 1) ? kL * o.wys : 0.f;
 #pragma unroll
@@ -678,7 +681,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip(
         const float xo = END ? xb : prox_huber1(xb, o.c, o.rc1, bv);
         o.y[ch] = xn + t * (xn - xo);
       } else {
-        o.y[ch] = END ? xb : rebuild_y_fast(bv, xa, xb, o.c, o.rc1, o.opc_d, t);
+        o.y[ch] = END ? xb : rebuild_y(bv, xa, xb, o.c, o.rc1, o.thr, t);
       }
       o.g[ch] = inside(o.g[ch]);
       o.xa[ch] = xa;
@@ -694,12 +697,11 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip(
       for (int ch = 0; ch < C; ch++) {
         const float df = o.g[ch], bv = o.bb[ch], xh = inside(o.xl[ch]);
         const float diff = bv - xh;
-        const float sign = (diff < 0) ? -1.f : 1.f;
-        const bool quad = (o.opc_d >= (double)(sign * diff));
+        const bool quad = o.thr >= fabsf(diff);
         const float gc_q = df * (div_by(bv, opc, o.rc1) - div_by(o.c * bv + xh, opc * opc, rc2)) * kGC;
         const float gb_q = div_by(df * o.c, opc, o.rc1) * 1.0f;
         o.g[ch] = quad ? div_by(df, opc, o.rc1) : df;
-        gcv += quad ? gc_q : sign * df * kGC;
+        gcv += quad ? gc_q : (diff < 0 ? -df : df) * kGC;
         o.gb_i[ch] = quad ? o.gb_i[ch] + gb_q : 0.f;  // (TV.cu:254 writes zero outside the quadratic regime)
       }
       o.gc_i = gcv;
@@ -727,18 +729,14 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip(
       const float d1 = yk - yd, d2 = yk - yrt;
       const float a1 = d1 * d1 * wyv;  // wy_nyy2
       const float a2 = d2 * d2 * wxv;  // wx_nyx2
-      const float hub = exact_sqrt(a2 + a1);
-      const bool act = hub > kDelta;
-      float nom = inpaint::exact_div(kDelta, hub);
-      float denom = inpaint::exact_div(nom, 2.f * hub * hub);
-      nom = act ? nom : 1.f;
-      denom = act ? denom : 0.f;
+      const inpaint::HuberAdjoint hub = inpaint::huber_adjoint(a2 + a1);
+      const bool act = hub.active;
+      const float nom = hub.nom, dd = hub.twice, denom = 0.5f * dd;
       const float gpd = gk - gd, gpr = gk - grt;
       const float O1 = gpd * (wyv * nom);
       const float O2 = gpr * (wxv * nom);
       const float P1 = gpd * wyv * d1;
       const float P2 = gpr * wxv * d2;
-      const float dd = denom * 2.0f;
       const float tp = dd * ((yd - yk) * wyv + (yrt - yk) * wxv);
       const float tu = dd * d1 * wyv;
       const float tl = dd * d2 * wxv;
@@ -774,25 +772,16 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip(
         tt -= O2;        // TV.cu:733 / 764
         tt -= O3;        // TV.cu:741
         tt -= O4;        // TV.cu:743
-        // momentum adjoint, TV.cu:796-801
-        float df = (float)((double)gxv + opt * (double)tt);
+        // momentum adjoint, TV.cu:796-801.  (The product is exact in 53 bits -- t is 0 or at least 1/4, so 1 + t has 27 -- and
+        // the fused form rounds once where the reference rounds once.)
+        float df = (float)__builtin_fma(opt, (double)tt, (double)gxv);
         df = fmaxf(-kClipLocalGrad, fminf(df, kClipLocalGrad));
         const float gxm = -t * tt;
         // prox adjoint, TV.cu:806-828
-        const float conf = cur.c, bv = cur.bb[ch], xh = cur.xa[ch];
-        const float diff = bv - xh;
-        const float sign = (diff < 0) ? -1.f : 1.f;
-        const bool quad = (cur.opc_d >= (double)(sign * diff));
-        const float opc = 1.f + conf;
-        const float gc_q = df * (div_by(bv, opc, cur.rc1) - div_by(conf * bv + xh, opc * opc, rc2)) * kGC;
-        const float g05_q = div_by(df, opc, cur.rc1);
-        const float gb_q = div_by(df * conf, opc, cur.rc1) * 1.0f;
-        // three regimes (quadratic / TV.cu:818-822, unreachable for c >= 0 / linear) as selects;
-        // adding +0 where the reference adds nothing leaves the accumulators unchanged
-        const bool mid = !quad && (conf >= sign * diff);
-        const float g05v = quad ? g05_q : (mid ? 0.f : df);
-        gcv += quad ? gc_q : (mid ? 0.f : sign * df * kGC);
-        gbv += quad ? gb_q : (mid ? df * 1.0f : 0.f);
+        float g05v, gc_add, gb_add;
+        prox_adjoint<TRUE_ADJ>(df, cur.bb[ch], cur.xa[ch], cur.c, cur.rc1, rc2, cur.thr, g05v, gc_add, gb_add);
+        gcv += gc_add;
+        gbv += gb_add;
         if (store_lane) {  // a block this small is predicated, not branched around
           if (FINAL) stg(gxf_p[ch], roff, df);  // only the last step's g_x is read again (TV.cu:800,1785)
           stg(gxm_p[ch], roff, gxm);
@@ -881,7 +870,7 @@ struct Adj2Row {
   float yA[C];         // loaded as nothing, rebuilt from xa, xb
   float yB[C];         // loaded as x05[j-2] (or the checkpoint y), rebuilt from xb and itself
   float bb[C], g[C], gx_i[C], gb_i[C], gc_i, gwx_i, gwy_i;
-  double opc_d;
+  float thr;  // regime_threshold(c)
 };
 
 // TRUE_ADJ: the corrected gradient, as in tv_adjoint_strip (with BEND, x05c is the checkpointed x of the segment start).
@@ -955,7 +944,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
     const std::conditional_t<BEND, inpaint::LaneSelect, inpaint::LaneMask> inside(ok);  // (the segment-end pair is short of registers)
     o.c = inside(o.c);
     o.rc1 = rcp_refined(1.f + o.c);
-    o.opc_d = 1. + (double)o.c;
+    o.thr = regime_threshold(o.c);
     o.wxs = (ok && wx_ok) ? kL * o.wxs : 0.f;
     o.wys = (ok && h < H - 1) ? kL * o.wys : 0.f;
 #pragma unroll
@@ -967,10 +956,10 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
         o.yA[ch] = pa + tA * (pa - pb);
         o.yB[ch] = pb + tB * (pb - pc);
       } else {
-        // rebuild_y_fast(bv, xa, xb, ..., tA) and rebuild_y_fast(bv, xb, xc, ..., tB) with the pieces of xb formed once
-        const RebuildPieces ra = rebuild_pieces(bv, xa, o.c, o.rc1, o.opc_d), rb = rebuild_pieces(bv, xb, o.c, o.rc1, o.opc_d);
-        o.yA[ch] = rebuild_from(ra, rb, tA);
-        o.yB[ch] = BEND ? xc : rebuild_from(rb, rebuild_pieces(bv, xc, o.c, o.rc1, o.opc_d), tB);
+        // rebuild_y(bv, xa, xb, ..., tA) and rebuild_y(bv, xb, xc, ..., tB) with the pieces of xb formed once
+        const Rebuild ra = rebuild_of(xa, bv, o.c, o.rc1), rb = rebuild_of(xb, bv, o.c, o.rc1);
+        o.yA[ch] = rebuild_from(ra, rb, bv, xa, o.thr, tA);
+        o.yB[ch] = BEND ? xc : rebuild_from(rb, rebuild_of(xc, bv, o.c, o.rc1), bv, xb, o.thr, tB);
       }
       o.g[ch] = inside(o.g[ch]);
       o.xa[ch] = xa;
@@ -979,7 +968,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
     }
   };
 
-  constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult, kGC = TRUE_ADJ ? 1.f : kLocalGCMult;
+  constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult;
   struct Tri {  // everything one triangle contributes (see tv_adjoint_strip)
     float O1, O2, O3, O4, n3, n4, l1, l3, l4, ux, uy;
   };
@@ -990,18 +979,14 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
     const float d1 = yk - yd, d2 = yk - yrt;
     const float a1 = d1 * d1 * wyv;
     const float a2 = d2 * d2 * wxv;
-    const float hub = exact_sqrt(a2 + a1);
-    const bool act = hub > kDelta;
-    float nom = inpaint::exact_div(kDelta, hub);
-    float denom = inpaint::exact_div(nom, 2.f * hub * hub);
-    nom = act ? nom : 1.f;
-    denom = act ? denom : 0.f;
+    const inpaint::HuberAdjoint hub = inpaint::huber_adjoint(a2 + a1);
+    const bool act = hub.active;
+    const float nom = hub.nom, dd = hub.twice, denom = 0.5f * dd;
     const float gpd = gk - gd, gpr = gk - grt;
     r.O1 = gpd * (wyv * nom);
     r.O2 = gpr * (wxv * nom);
     const float P1 = gpd * wyv * d1;
     const float P2 = gpr * wxv * d2;
-    const float dd = denom * 2.0f;
     // the reference's factor dd * ((yd - yk) * wyv + (yrt - yk) * wxv) is minus this one, exactly: a - b = -(b - a),
     // (-a) * w = -(a * w) and (-a) + (-b) = -(a + b) in IEEE arithmetic; O3, O4 carry the sign
     const float tp = dd * (d1 * wyv + d2 * wxv);
@@ -1027,7 +1012,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
   };
   // pixel update: J^T assembly, momentum adjoint, prox adjoint (TV.cu:668-743, 796-828)
   auto update = [&](float gk, const Tri& t, float a1_, float a3_, float a4_, float gxv, double opt, float tmom,
-                    float conf, float rc1, float rc2, double opc_d, float bv, float xh, float& df, float& gxm,
+                    float conf, float rc1, float rc2, float thr, float bv, float xh, float& df, float& gxm,
                     float& g05v, float& gc_add, float& gb_add) {
     float tt = gk;
     tt -= -a1_;
@@ -1040,27 +1025,17 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
     tt -= t.O2;
     tt -= t.O3;
     tt -= t.O4;
-    df = (float)((double)gxv + opt * (double)tt);
+    df = (float)__builtin_fma(opt, (double)tt, (double)gxv);
     df = fmaxf(-kClipLocalGrad, fminf(df, kClipLocalGrad));
     gxm = -tmom * tt;
-    const float diff = bv - xh;
-    const float sign = (diff < 0) ? -1.f : 1.f;
-    const bool quad = (opc_d >= (double)(sign * diff));
-    const float opc = 1.f + conf;
-    const float gc_q = df * (div_by(bv, opc, rc1) - div_by(conf * bv + xh, opc * opc, rc2)) * kGC;
-    const float g05_q = div_by(df, opc, rc1);
-    const float gb_q = div_by(df * conf, opc, rc1) * 1.0f;
-    const bool mid = !quad && (conf >= sign * diff);
-    g05v = quad ? g05_q : (mid ? 0.f : df);
-    gc_add = quad ? gc_q : (mid ? 0.f : sign * df * kGC);
-    gb_add = quad ? gb_q : (mid ? df * 1.0f : 0.f);
+    prox_adjoint<TRUE_ADJ>(df, bv, xh, conf, rc1, rc2, thr, g05v, gc_add, gb_add);
   };
 
   float dA1[C], dA3[C], dA4[C], dB1[C], dB3[C], dB4[C];  // terms handed down, per step
   // row k-1 as step B sees it
   float pG[C], pgxm[C], pyB[C], pxb[C], pbb[C], pgb[C], pgc = 0.f, pgwx = 0.f, pgwy = 0.f;
   float pc = 0.f, prc1 = 1.f, prc2 = 1.f, pwxs = 0.f, pwys = 0.f;
-  double popc_d = 1.;
+  float pthr = 1.f;
 #pragma unroll
   for (int ch = 0; ch < C; ch++) {
     dA1[ch] = dA3[ch] = dA4[ch] = dB1[ch] = dB3[ch] = dB4[ch] = 0.f;
@@ -1087,7 +1062,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
         if (g.w < W - 1) gwxv = gwxv - t.ux;
         if (h < H - 1) gwyv = gwyv - t.uy;
         float df, gxm, g05v, gc_add, gb_add;
-        update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.opc_d, cur.bb[ch],
+        update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.thr, cur.bb[ch],
                cur.xa[ch], df, gxm, g05v, gc_add, gb_add);
         gcv += gc_add;
         ngb[ch] += gb_add;
@@ -1107,7 +1082,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
           if (g.w < W - 1) gwxB = gwxB - t.ux;
           if (h - 1 < H - 1) gwyB = gwyB - t.uy;
           float df, gxm, g05v, gc_add, gb_add;
-          update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, popc_d, pbb[ch], pxb[ch], df, gxm, g05v,
+          update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, pthr, pbb[ch], pxb[ch], df, gxm, g05v,
                  gc_add, gb_add);
           gcB += gc_add;
           const float gbv = pgb[ch] + gb_add;
@@ -1137,7 +1112,7 @@ __global__ __launch_bounds__(256) void tv_adjoint_strip2(
       }
     }
     pgc = gcv; pgwx = gwxv; pgwy = gwyv;
-    pc = cur.c; prc1 = cur.rc1; prc2 = rc2A; popc_d = cur.opc_d; pwxs = cur.wxs; pwys = cur.wys;
+    pc = cur.c; prc1 = cur.rc1; prc2 = rc2A; pthr = cur.thr; pwxs = cur.wxs; pwys = cur.wys;
 #pragma unroll
     for (int ch = 0; ch < C; ch++) {
       pG[ch] = nG[ch]; pgxm[ch] = ngxm[ch]; pgb[ch] = ngb[ch];
@@ -1264,7 +1239,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
       const std::conditional_t<BEND, inpaint::LaneSelect, inpaint::LaneMask> inside(ok);  // (the segment-end pair is short of registers)
       o.c = inside(o.c);
       o.rc1 = rcp_refined(1.f + o.c);
-      o.opc_d = 1. + (double)o.c;
+      o.thr = regime_threshold(o.c);
       o.wxs = (ok && wx_ok) ? kL * o.wxs : 0.f;
       o.wys = (ok && h < H - 1) ? kL * o.wys : 0.f;
   #pragma unroll
@@ -1276,10 +1251,10 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
           o.yA[ch] = pa + tA * (pa - pb);
           o.yB[ch] = pb + tB * (pb - pc);
         } else {
-          // rebuild_y_fast(bv, xa, xb, ..., tA) and rebuild_y_fast(bv, xb, xc, ..., tB) with the pieces of xb formed once
-          const RebuildPieces ra = rebuild_pieces(bv, xa, o.c, o.rc1, o.opc_d), rb = rebuild_pieces(bv, xb, o.c, o.rc1, o.opc_d);
-          o.yA[ch] = rebuild_from(ra, rb, tA);
-          o.yB[ch] = BEND ? xc : rebuild_from(rb, rebuild_pieces(bv, xc, o.c, o.rc1, o.opc_d), tB);
+          // rebuild_y(bv, xa, xb, ..., tA) and rebuild_y(bv, xb, xc, ..., tB) with the pieces of xb formed once
+          const Rebuild ra = rebuild_of(xa, bv, o.c, o.rc1), rb = rebuild_of(xb, bv, o.c, o.rc1);
+          o.yA[ch] = rebuild_from(ra, rb, bv, xa, o.thr, tA);
+          o.yB[ch] = BEND ? xc : rebuild_from(rb, rebuild_of(xc, bv, o.c, o.rc1), bv, xb, o.thr, tB);
         }
         o.g[ch] = inside(o.g[ch]);
         o.xa[ch] = xa;
@@ -1288,7 +1263,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
       }
     };
 
-    constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult, kGC = TRUE_ADJ ? 1.f : kLocalGCMult;
+    constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult;
     struct Tri {  // everything one triangle contributes (see tv_adjoint_strip)
       float O1, O2, O3, O4, n3, n4, l1, l3, l4, ux, uy;
     };
@@ -1299,18 +1274,14 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
       const float d1 = yk - yd, d2 = yk - yrt;
       const float a1 = d1 * d1 * wyv;
       const float a2 = d2 * d2 * wxv;
-      const float hub = exact_sqrt(a2 + a1);
-      const bool act = hub > kDelta;
-      float nom = inpaint::exact_div(kDelta, hub);
-      float denom = inpaint::exact_div(nom, 2.f * hub * hub);
-      nom = act ? nom : 1.f;
-      denom = act ? denom : 0.f;
+      const inpaint::HuberAdjoint hub = inpaint::huber_adjoint(a2 + a1);
+      const bool act = hub.active;
+      const float nom = hub.nom, dd = hub.twice, denom = 0.5f * dd;
       const float gpd = gk - gd, gpr = gk - grt;
       r.O1 = gpd * (wyv * nom);
       r.O2 = gpr * (wxv * nom);
       const float P1 = gpd * wyv * d1;
       const float P2 = gpr * wxv * d2;
-      const float dd = denom * 2.0f;
       // the reference's factor dd * ((yd - yk) * wyv + (yrt - yk) * wxv) is minus this one, exactly: a - b = -(b - a),
       // (-a) * w = -(a * w) and (-a) + (-b) = -(a + b) in IEEE arithmetic; O3, O4 carry the sign
       const float tp = dd * (d1 * wyv + d2 * wxv);
@@ -1336,7 +1307,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
     };
     // pixel update: J^T assembly, momentum adjoint, prox adjoint (TV.cu:668-743, 796-828)
     auto update = [&](float gk, const Tri& t, float a1_, float a3_, float a4_, float gxv, double opt, float tmom,
-                      float conf, float rc1, float rc2, double opc_d, float bv, float xh, float& df, float& gxm,
+                      float conf, float rc1, float rc2, float thr, float bv, float xh, float& df, float& gxm,
                       float& g05v, float& gc_add, float& gb_add) {
       float tt = gk;
       tt -= -a1_;
@@ -1349,27 +1320,17 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
       tt -= t.O2;
       tt -= t.O3;
       tt -= t.O4;
-      df = (float)((double)gxv + opt * (double)tt);
+      df = (float)__builtin_fma(opt, (double)tt, (double)gxv);
       df = fmaxf(-kClipLocalGrad, fminf(df, kClipLocalGrad));
       gxm = -tmom * tt;
-      const float diff = bv - xh;
-      const float sign = (diff < 0) ? -1.f : 1.f;
-      const bool quad = (opc_d >= (double)(sign * diff));
-      const float opc = 1.f + conf;
-      const float gc_q = df * (div_by(bv, opc, rc1) - div_by(conf * bv + xh, opc * opc, rc2)) * kGC;
-      const float g05_q = div_by(df, opc, rc1);
-      const float gb_q = div_by(df * conf, opc, rc1) * 1.0f;
-      const bool mid = !quad && (conf >= sign * diff);
-      g05v = quad ? g05_q : (mid ? 0.f : df);
-      gc_add = quad ? gc_q : (mid ? 0.f : sign * df * kGC);
-      gb_add = quad ? gb_q : (mid ? df * 1.0f : 0.f);
+      prox_adjoint<TRUE_ADJ>(df, bv, xh, conf, rc1, rc2, thr, g05v, gc_add, gb_add);
     };
 
     float dA1[C], dA3[C], dA4[C], dB1[C], dB3[C], dB4[C];  // terms handed down, per step
     // row k-1 as step B sees it
     float pG[C], pgxm[C], pyB[C], pxb[C], pbb[C], pgb[C], pgc = 0.f, pgwx = 0.f, pgwy = 0.f;
     float pc = 0.f, prc1 = 1.f, prc2 = 1.f, pwxs = 0.f, pwys = 0.f;
-    double popc_d = 1.;
+    float pthr = 1.f;
   #pragma unroll
     for (int ch = 0; ch < C; ch++) {
       dA1[ch] = dA3[ch] = dA4[ch] = dB1[ch] = dB3[ch] = dB4[ch] = 0.f;
@@ -1400,7 +1361,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
         nG[ch] = 0.f; ngxm[ch] = 0.f; ngb[ch] = cur.gb_i[ch];
         if (do_a.value) {
           float df, gxm, g05v, gc_add, gb_add;
-          update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.opc_d, cur.bb[ch],
+          update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.thr, cur.bb[ch],
                  cur.xa[ch], df, gxm, g05v, gc_add, gb_add);
           if (ROLE == 1) {
             if (g.w < W - 1) gwxv = gwxv - t.ux;
@@ -1431,7 +1392,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
           dB1[ch] = t.O1; dB3[ch] = t.n3; dB4[ch] = t.n4;
           if (do_b.value) {
             float df, gxm, g05v, gc_add, gb_add;
-            update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, popc_d, pbb[ch], pxb[ch], df, gxm, g05v,
+            update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, pthr, pbb[ch], pxb[ch], df, gxm, g05v,
                    gc_add, gb_add);
             if (ROLE == 1) {
               if (g.w < W - 1) gwxB = gwxB - t.ux;
@@ -1469,7 +1430,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2c(
         }
       }
       pgc = gcv; pgwx = gwxv; pgwy = gwyv;
-      pc = cur.c; prc1 = cur.rc1; prc2 = rc2A; popc_d = cur.opc_d; pwxs = cur.wxs; pwys = cur.wys;
+      pc = cur.c; prc1 = cur.rc1; prc2 = rc2A; pthr = cur.thr; pwxs = cur.wxs; pwys = cur.wys;
   #pragma unroll
       for (int ch = 0; ch < C; ch++) {
         pG[ch] = nG[ch]; pgxm[ch] = ngxm[ch]; pgb[ch] = ngb[ch];
@@ -1540,7 +1501,7 @@ template <int C>
 struct Adj2wRow {
   float c, rc1, wxs, wys;
   float xa[C], xb[C], yA[C], bb[C], g[C], gx_i[C], gb_i[C], gc_i, gwx_i, gwy_i;
-  double opc_d;
+  float thr;  // regime_threshold(c)
 };
 
 template <int C, bool BEND, bool FINAL, bool TRUE_ADJ = false>
@@ -1576,7 +1537,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
   const int h_lo = max(g.hs - 1, 0), h_hi = min(g.hs + Reff, H - 1);  // rows A updates
   const int o_lo = g.hs, o_hi = g.hs + Reff - 1;                       // output rows
 
-  constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult, kGC = TRUE_ADJ ? 1.f : kLocalGCMult;
+  constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult;
   struct Tri {  // everything one triangle contributes (see tv_adjoint_strip)
     float O1, O2, O3, O4, n3, n4, l1, l3, l4, ux, uy;
   };
@@ -1587,18 +1548,14 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
     const float d1 = yk - yd, d2 = yk - yrt;
     const float a1 = d1 * d1 * wyv;
     const float a2 = d2 * d2 * wxv;
-    const float hub = exact_sqrt(a2 + a1);
-    const bool act = hub > kDelta;
-    float nom = inpaint::exact_div(kDelta, hub);
-    float denom = inpaint::exact_div(nom, 2.f * hub * hub);
-    nom = act ? nom : 1.f;
-    denom = act ? denom : 0.f;
+    const inpaint::HuberAdjoint hub = inpaint::huber_adjoint(a2 + a1);
+    const bool act = hub.active;
+    const float nom = hub.nom, dd = hub.twice, denom = 0.5f * dd;
     const float gpd = gk - gd, gpr = gk - grt;
     r.O1 = gpd * (wyv * nom);
     r.O2 = gpr * (wxv * nom);
     const float P1 = gpd * wyv * d1;
     const float P2 = gpr * wxv * d2;
-    const float dd = denom * 2.0f;
     const float tp = dd * (d1 * wyv + d2 * wxv);  // minus the reference's factor, exactly; O3, O4 carry the sign
     const float tu = dd * d1 * wyv;
     const float tl = dd * d2 * wxv;
@@ -1622,7 +1579,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
   };
   // pixel update: J^T assembly, momentum adjoint, prox adjoint (TV.cu:668-743, 796-828)
   auto update = [&](float gk, const Tri& t, float a1_, float a3_, float a4_, float gxv, double opt, float tmom,
-                    float conf, float rc1, float rc2, double opc_d, float bv, float xh, float& df, float& gxm,
+                    float conf, float rc1, float rc2, float thr, float bv, float xh, float& df, float& gxm,
                     float& g05v, float& gc_add, float& gb_add) {
     float tt = gk;
     tt -= -a1_;
@@ -1635,20 +1592,10 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
     tt -= t.O2;
     tt -= t.O3;
     tt -= t.O4;
-    df = (float)((double)gxv + opt * (double)tt);
+    df = (float)__builtin_fma(opt, (double)tt, (double)gxv);
     df = fmaxf(-kClipLocalGrad, fminf(df, kClipLocalGrad));
     gxm = -tmom * tt;
-    const float diff = bv - xh;
-    const float sign = (diff < 0) ? -1.f : 1.f;
-    const bool quad = (opc_d >= (double)(sign * diff));
-    const float opc = 1.f + conf;
-    const float gc_q = df * (div_by(bv, opc, rc1) - div_by(conf * bv + xh, opc * opc, rc2)) * kGC;
-    const float g05_q = div_by(df, opc, rc1);
-    const float gb_q = div_by(df * conf, opc, rc1) * 1.0f;
-    const bool mid = !quad && (conf >= sign * diff);
-    g05v = quad ? g05_q : (mid ? 0.f : df);
-    gc_add = quad ? gc_q : (mid ? 0.f : sign * df * kGC);
-    gb_add = quad ? gb_q : (mid ? df * 1.0f : 0.f);
+    prox_adjoint<TRUE_ADJ>(df, bv, xh, conf, rc1, rc2, thr, g05v, gc_add, gb_add);
   };
   const std::true_type kYes{};
   const std::false_type kNo{};
@@ -1689,7 +1636,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
       const inpaint::LaneMask inside(ok);
       o.c = inside(o.c);
       o.rc1 = rcp_refined(1.f + o.c);
-      o.opc_d = 1. + (double)o.c;
+      o.thr = regime_threshold(o.c);
       o.wxs = (ok && wx_ok) ? kL * o.wxs : 0.f;
       o.wys = (ok && h < H - 1) ? kL * o.wys : 0.f;
 #pragma unroll
@@ -1699,7 +1646,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
           const float pa = prox_huber1(xa, o.c, o.rc1, bv), pb = prox_huber1(xb, o.c, o.rc1, bv);
           o.yA[ch] = pa + tA * (pa - pb);
         } else {
-          o.yA[ch] = rebuild_y_fast(bv, xa, xb, o.c, o.rc1, o.opc_d, tA);
+          o.yA[ch] = rebuild_y(bv, xa, xb, o.c, o.rc1, o.thr, tA);
         }
         o.g[ch] = inside(o.g[ch]);
         o.xa[ch] = xa;
@@ -1727,7 +1674,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
           if (g.w < W - 1) gwxv = gwxv - t.ux;
           if (h < H - 1) gwyv = gwyv - t.uy;
           float df, gxm, g05v, gc_add, gb_add;
-          update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.opc_d, cur.bb[ch],
+          update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.thr, cur.bb[ch],
                  cur.xa[ch], df, gxm, g05v, gc_add, gb_add);
           gcv += gc_add;
           ngb += gb_add;
@@ -1823,7 +1770,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
       const float gcv = slot[5 * C + 0][g.lane], gwxv = slot[5 * C + 1][g.lane], gwyv = slot[5 * C + 2][g.lane];
       const float cc = slot[5 * C + 3][g.lane], rc1 = slot[5 * C + 4][g.lane];
       const float wxs = slot[5 * C + 5][g.lane], wys = slot[5 * C + 6][g.lane];
-      const double opc_d = 1. + (double)cc;
+      const float thr = regime_threshold(cc);
 #pragma unroll
       for (int ch = 0; ch < C; ch++) {  // y of iteration j-1 on row k (the row below B's)
         const float xc = inside(in.xc[ch]);
@@ -1832,13 +1779,13 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
           const float pcv = BEND ? xc : prox_huber1(xc, cc, rc1, bbv[ch]);
           yB[ch] = pb + tB * (pb - pcv);
         } else {
-          yB[ch] = BEND ? xc : rebuild_y_fast(bbv[ch], xbv[ch], xc, cc, rc1, opc_d, tB);
+          yB[ch] = BEND ? xc : rebuild_y(bbv[ch], xbv[ch], xc, cc, rc1, thr, tB);
         }
       }
       if (tri_b.value) {
         float gcB = pgc, gwxB = pgwx, gwyB = pgwy;
         const float rc2B = rcp_refined((1.f + pc) * (1.f + pc));
-        const double popc_d = 1. + (double)pc;
+        const float pthr = regime_threshold(pc);
 #pragma unroll
         for (int ch = 0; ch < C; ch++) {
           const Tri t = triangle(pyB[ch], yB[ch], pG[ch], nG[ch], pwxs, pwys, kBEnd);
@@ -1848,7 +1795,7 @@ __global__ __launch_bounds__(128) void tv_adjoint_strip2w(
             if (g.w < W - 1) gwxB = gwxB - t.ux;
             if (h - 1 < H - 1) gwyB = gwyB - t.uy;
             float df, gxm, g05v, gc_add, gb_add;
-            update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, popc_d, pbb[ch], pxb[ch], df, gxm, g05v,
+            update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, pthr, pbb[ch], pxb[ch], df, gxm, g05v,
                    gc_add, gb_add);
             gcB += gc_add;
             const float gbv = pgb[ch] + gb_add;
@@ -1965,7 +1912,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int h_lo = max(g.hs - 1, 0), h_hi = min(g.hs + Reff, H - 1);  // rows A updates
   const int o_lo = g.hs, o_hi = g.hs + Reff - 1;                       // output rows
 
-  constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult, kGC = TRUE_ADJ ? 1.f : kLocalGCMult;
+  constexpr float kGX = TRUE_ADJ ? 1.f : kLocalGXMult;
   struct Tri {  // everything one triangle contributes (see tv_adjoint_strip)
     float O1, O2, O3, O4, n3, n4, l1, l3, l4, ux, uy;
   };
@@ -1976,18 +1923,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const float d1 = yk - yd, d2 = yk - yrt;
     const float a1 = d1 * d1 * wyv;
     const float a2 = d2 * d2 * wxv;
-    const float hub = exact_sqrt(a2 + a1);
-    const bool act = hub > kDelta;
-    float nom = inpaint::exact_div(kDelta, hub);
-    float denom = inpaint::exact_div(nom, 2.f * hub * hub);
-    nom = act ? nom : 1.f;
-    denom = act ? denom : 0.f;
+    const inpaint::HuberAdjoint hub = inpaint::huber_adjoint(a2 + a1);
+    const bool act = hub.active;
+    const float nom = hub.nom, dd = hub.twice, denom = 0.5f * dd;
     const float gpd = gk - gd, gpr = gk - grt;
     r.O1 = gpd * (wyv * nom);
     r.O2 = gpr * (wxv * nom);
     const float P1 = gpd * wyv * d1;
     const float P2 = gpr * wxv * d2;
-    const float dd = denom * 2.0f;
     const float tp = dd * (d1 * wyv + d2 * wxv);  // minus the reference's factor, exactly; O3, O4 carry the sign
     const float tu = dd * d1 * wyv;
     const float tl = dd * d2 * wxv;
@@ -2011,7 +1954,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
   // pixel update: J^T assembly, momentum adjoint, prox adjoint (TV.cu:668-743, 796-828)
   auto update = [&](float gk, const Tri& t, float a1_, float a3_, float a4_, float gxv, double opt, float tmom,
-                    float conf, float rc1, float rc2, double opc_d, float bv, float xh, float& df, float& gxm,
+                    float conf, float rc1, float rc2, float thr, float bv, float xh, float& df, float& gxm,
                     float& g05v, float& gc_add, float& gb_add) {
     float tt = gk;
     tt -= -a1_;
@@ -2024,20 +1967,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     tt -= t.O2;
     tt -= t.O3;
     tt -= t.O4;
-    df = (float)((double)gxv + opt * (double)tt);
+    df = (float)__builtin_fma(opt, (double)tt, (double)gxv);
     df = fmaxf(-kClipLocalGrad, fminf(df, kClipLocalGrad));
     gxm = -tmom * tt;
-    const float diff = bv - xh;
-    const float sign = (diff < 0) ? -1.f : 1.f;
-    const bool quad = (opc_d >= (double)(sign * diff));
-    const float opc = 1.f + conf;
-    const float gc_q = df * (div_by(bv, opc, rc1) - div_by(conf * bv + xh, opc * opc, rc2)) * kGC;
-    const float g05_q = div_by(df, opc, rc1);
-    const float gb_q = div_by(df * conf, opc, rc1) * 1.0f;
-    const bool mid = !quad && (conf >= sign * diff);
-    g05v = quad ? g05_q : (mid ? 0.f : df);
-    gc_add = quad ? gc_q : (mid ? 0.f : sign * df * kGC);
-    gb_add = quad ? gb_q : (mid ? df * 1.0f : 0.f);
+    prox_adjoint<TRUE_ADJ>(df, bv, xh, conf, rc1, rc2, thr, g05v, gc_add, gb_add);
   };
   const std::true_type kYes{};
   const std::false_type kNo{};
@@ -2053,7 +1986,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     struct Row {
       float c, rc1, wxs, wys;
       float xa[C], xb[C], yA[C], bb[C], g[C], gx_i[C], gb_i[C], gc_i, gwx_i, gwy_i;
-      double opc_d;
+      float thr;  // regime_threshold(c)
     };
     auto load_row = [&](int k, Row& in) {
       const int kk = min(k, klast + 1);
@@ -2088,7 +2021,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const inpaint::LaneMask inside(ok);
       o.c = inside(o.c);
       o.rc1 = rcp_refined(1.f + o.c);
-      o.opc_d = 1. + (double)o.c;
+      o.thr = regime_threshold(o.c);
       o.wxs = (ok && wx_ok) ? kL * o.wxs : 0.f;
       o.wys = (ok && h < H - 1) ? kL * o.wys : 0.f;
 #pragma unroll
@@ -2098,7 +2031,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           const float pa = prox_huber1(xa, o.c, o.rc1, bv), pb = prox_huber1(xb, o.c, o.rc1, bv);
           o.yA[ch] = pa + tA * (pa - pb);
         } else {
-          o.yA[ch] = rebuild_y_fast(bv, xa, xb, o.c, o.rc1, o.opc_d, tA);
+          o.yA[ch] = rebuild_y(bv, xa, xb, o.c, o.rc1, o.thr, tA);
         }
         o.g[ch] = inside(o.g[ch]);
         o.xa[ch] = xa;
@@ -2131,7 +2064,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           if (g.w < W - 1) gwxv = gwxv - t.ux;
           if (h < H - 1) gwyv = gwyv - t.uy;
           float df, gxm, g05v, gc_add, gb_add;
-          update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.opc_d, cur.bb[ch],
+          update(cur.g[ch], t, a1_, a3_, a4_, cur.gx_i[ch], optA, tA, cur.c, cur.rc1, rc2A, cur.thr, cur.bb[ch],
                  cur.xa[ch], df, gxm, g05v, gc_add, gb_add);
           gcv += gc_add;
           ngb += gb_add;
@@ -2217,7 +2150,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const inpaint::LaneMask inside(ok);
       o.c = inside(o.c);
       o.rc1 = rcp_refined(1.f + o.c);
-      const double opc_d = 1. + (double)o.c;
+      const float thr = regime_threshold(o.c);
       o.wxs = (ok && wx_ok) ? kL * o.wxs : 0.f;
       o.wys = (ok && h < H - 1) ? kL * o.wys : 0.f;
 #pragma unroll
@@ -2228,7 +2161,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           const float pcv = BEND ? xc : prox_huber1(xc, o.c, o.rc1, bv);
           o.yB[ch] = pb + tB * (pb - pcv);
         } else {
-          o.yB[ch] = BEND ? xc : rebuild_y_fast(bv, xb, xc, o.c, o.rc1, opc_d, tB);
+          o.yB[ch] = BEND ? xc : rebuild_y(bv, xb, xc, o.c, o.rc1, thr, tB);
         }
         o.xb[ch] = xb;
         o.bb[ch] = bv;
@@ -2272,7 +2205,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           }
         }
         const float rc2B = rcp_refined((1.f + pc) * (1.f + pc));
-        const double popc_d = 1. + (double)pc;
+        const float pthr = regime_threshold(pc);
 #pragma unroll
         for (int ch = 0; ch < C; ch++) {
           const Tri t = triangle(pyB[ch], cur.yB[ch], pG[ch], nG[ch], pwxs, pwys, kBEnd);
@@ -2280,7 +2213,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
           dB1[ch] = t.O1; dB3[ch] = t.n3; dB4[ch] = t.n4;
           if (do_b.value) {
             float df, gxm, g05v, gc_add, gb_add;
-            update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, popc_d, pbb[ch], pxb[ch], df, gxm, g05v,
+            update(pG[ch], t, a1_, a3_, a4_, pgxm[ch], optB, tB, pc, prc1, rc2B, pthr, pbb[ch], pxb[ch], df, gxm, g05v,
                    gc_add, gb_add);
             if (G == 0) {
               terms[ch][g.lane] = gc_add;

@@ -20,13 +20,16 @@
 namespace tvtile {
 
 using inpaint::div_by;
-using inpaint::exact_sqrt;
 using inpaint::rcp_refined;
+using tvstrip::Rebuild;
 using tvstrip::from_left_lane;
 using tvstrip::from_right_lane;
 using tvstrip::kL;
 using tvstrip::ldg;
 using tvstrip::lds_barrier;
+using tvstrip::prox_adjoint;
+using tvstrip::rebuild_of;
+using tvstrip::regime_threshold;
 using tvstrip::stg;
 
 constexpr int kMaxFwdSteps = 12;  // forward iterations one launch can hold
@@ -140,11 +143,9 @@ __global__ __launch_bounds__(64 * WAVES) void tv_forward_tile(
   auto triangle = [&](float yc, float yd, float wxv, float wyv, float& e1, float& e2) {
     const float d1 = yc - yd;
     const float d2 = yc - from_right_lane(yc);
-    const float hub = exact_sqrt(d1 * d1 * wyv + d2 * d2 * wxv);
-    const float m = fmaxf(1.f, inpaint::div_by_tenth(hub));
-    const float rm = rcp_refined(m);
-    e1 = d1 * div_by(wyv, m, rm);
-    e2 = d2 * div_by(wxv, m, rm);
+    const inpaint::HuberForward hub = inpaint::huber_forward(d1 * d1 * wyv + d2 * d2 * wxv);
+    e1 = d1 * div_by(wyv, hub.m, hub.rm);
+    e2 = d2 * div_by(wxv, hub.m, hub.rm);
   };
 
   for (int it = 0; it < K; it++) {
@@ -179,44 +180,6 @@ __global__ __launch_bounds__(64 * WAVES) void tv_forward_tile(
   }
 }
 
-
-// The largest float that is not above 1. + (double)c: the reference's regime test compares a float with that double
-// (TV.cu:806, 1154), which is the same as comparing it with this float.
-__device__ __forceinline__ float regime_threshold(float c) {
-  const double d = 1. + (double)c;
-  const float f = (float)d;
-  if (!((double)f > d)) return f;
-  return __uint_as_float(__float_as_uint(f) + (f > 0.f ? -1 : 1));
-}
-
-// Prox adjoint of one pixel at the half-step value xh (TV.cu:806-828): the incoming adjoint df becomes g05; gc_add and
-// gb_add are the confidence's and the right-hand side's share.  rc1, rc2: refined reciprocals of 1 + conf and its square.
-// The reference has a third regime between the two (TV.cu:818-822: conf >= |b - xh| > 1. + (double)conf); no number is in
-// it, so it is left out.  Its sign * diff (sign: -1 where diff < 0, else 1) is |diff|.
-template <bool TRUE_ADJ>
-__device__ __forceinline__ void prox_adjoint(float df, float bv, float xh, float conf, float rc1, float rc2, float thr,
-                                             float& g05v, float& gc_add, float& gb_add) {
-  constexpr float kGC = TRUE_ADJ ? 1.f : tvstrip::kLocalGCMult;
-  const float diff = bv - xh;
-  const bool quad = thr >= fabsf(diff);
-  const float opc = 1.f + conf;
-  const float gc_q = df * (div_by(bv, opc, rc1) - div_by(conf * bv + xh, opc * opc, rc2)) * kGC;
-  const float g05_q = div_by(df, opc, rc1);
-  const float gb_q = div_by(df * conf, opc, rc1) * 1.0f;
-  g05v = quad ? g05_q : df;
-  gc_add = quad ? gc_q : (diff < 0 ? -df : df) * kGC;
-  gb_add = quad ? gb_q : 0.f;  // (adding +0 where the reference adds nothing leaves an accumulator unchanged)
-}
-
-// What the y rebuild of TV.cu:1149-1165 takes from one half-step value v: the iterate by the quadratic rule (q) and by the
-// other rule (l).  Every x05 row serves two steps, as the later and as the earlier value, so a step keeps them for the next.
-struct Rebuild {
-  float q, l;
-};
-__device__ __forceinline__ Rebuild rebuild_of(float v, float bv, float conf, float rc1) {
-  const float diff = bv - v;
-  return {div_by(conf * bv + v, 1.f + conf, rc1), conf <= fabsf(diff) ? bv - diff + (diff < 0 ? -conf : conf) : bv};
-}
 
 constexpr int kMaxAdjSteps = 12;  // reverse-sweep steps one launch can hold
 
@@ -441,16 +404,12 @@ __global__ __launch_bounds__(64 * WAVES) void tv_adjoint_tile(AdjTileArgs a, Adj
         const float yrt = from_right_lane(yk), grt = from_right_lane(gk);
         const float d1 = yk - yd, d2 = yk - yrt;
         const float a1 = d1 * d1 * wyv, a2 = d2 * d2 * wxv;
-        const float hub = exact_sqrt(a2 + a1);
-        const bool act = hub > tvstrip::kDelta;
-        float nom = inpaint::exact_div(tvstrip::kDelta, hub);
-        float denom = inpaint::exact_div(nom, 2.f * hub * hub);
-        nom = act ? nom : 1.f;
-        denom = act ? denom : 0.f;
+        const inpaint::HuberAdjoint hub = inpaint::huber_adjoint(a2 + a1);
+        const bool act = hub.active;
+        const float nom = hub.nom, dd = hub.twice, denom = 0.5f * dd;
         const float gpd = gk - gd, gpr = gk - grt;
         const float O1 = gpd * (wyv * nom), O2 = gpr * (wxv * nom);
         const float P1 = gpd * wyv * d1, P2 = gpr * wxv * d2;
-        const float dd = denom * 2.0f;
         const float tu = dd * d1 * wyv;
         const float n3 = P1 * tu, n4 = P2 * tu;
         if (i >= 0) {
@@ -483,7 +442,7 @@ __global__ __launch_bounds__(64 * WAVES) void tv_adjoint_tile(AdjTileArgs a, Adj
           tt -= O3;    // TV.cu:741
           tt -= O4;    // TV.cu:743
           // momentum adjoint, TV.cu:796-801
-          float df = (float)((double)gx[i] + (1. + (double)t) * (double)tt);
+          float df = (float)__builtin_fma(1. + (double)t, (double)tt, (double)gx[i]);  // (see tv_adjoint_strip)
           df = fmaxf(-tvstrip::kClipLocalGrad, fminf(df, tvstrip::kClipLocalGrad));
           gx[i] = -t * tt;
           const float rc2 = rcp_refined((1.f + c[i]) * (1.f + c[i]));

@@ -59,6 +59,12 @@ int tgvinpaint_profile_read(double* total_ms, int* launches);
  * against the compiler's IEEE expansions on the GPU (host array of four mismatch counts, all 0). */
 int inpaint_selftest_rsqrt(unsigned long long* mismatches4_host, unsigned int pair_rounds);
 
+/* The TV layer's Huber terms, formed with one transcendental instruction, against the compiler's IEEE root and divisions over
+ * A = 0 and every float in [2^-96, 2^80] (host array of four counts): mismatches of the forward factor, mismatches of the
+ * adjoint's, values of A whose reciprocal of the forward factor is not the correctly rounded one (some 270), and wrong quotients
+ * by those over all mantissas.  All but the third are 0. */
+int inpaint_selftest_huber(unsigned long long* counts4_host);
+
 /* The rate a plain device-to-device copy kernel reaches on the current GPU (bytes read + bytes written per
  * second, in GB/s, host pointer), to quote beside the published HBM peak.  Allocates and frees two buffers of `bytes`,
  * copies `repeats` times after a warm-up launch, timed with HIP events on `stream`; waits for the result. */
