@@ -43,6 +43,9 @@ struct FwdSteps {
   FwdStep step[kMaxFwdSteps];
 };
 
+// Rows of the halo that neither a later iteration nor the output needs are skipped (a row more at either end with every iteration):
+// 1 to 5% of a pass (4 x 2 x 384 x 1248 2508 -> 2484 us, 1 x 2 x 375 x 1241 at inference 589 -> 577, 2 x 2 x 224 x 512 199 -> 191); the
+// wavefronts in the middle of a tile have none, and set its pace.
 // Bound by instruction issue: about 80 vector instructions per pixel and iteration where the Huber terms of a row are quiet,
 // 120 where none is, on two to five wavefronts per SIMD (the strips issue as many, but wait for memory every second
 // iteration and read 19 planes for it).  Taller tiles waste less on the halo; 5 rows per wavefront are what fits 128 registers.
@@ -214,13 +217,21 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(fwd_
         yu[v] = edge[par][max(wave - 1, 0)][1][v][lane];
         yb[v] = edge[par][min(wave + 1, WAVES - 1)][0][v][lane];
       }
-      Tri above = triangle(yu[0], yu[1], yu[2], y[0][0], y[1][0], y[2][0], wxu, wyu, bxu, byu, h0 - 1 >= 0 && h0 - 1 < H - 1);
+      // rows of this wavefront that a later iteration or the output still needs
+      const int lo = max(it + 1 - wave * R, 0), hi = min(TR - 2 - it - wave * R, R - 1);
+      Tri above{};
+      if (lo == 0) above = triangle(yu[0], yu[1], yu[2], y[0][0], y[1][0], y[2][0], wxu, wyu, bxu, byu, h0 - 1 >= 0 && h0 - 1 < H - 1);
       float xh[R];
 #pragma unroll
       for (int i = 0; i < R; i++) {
+        if (i + 1 < lo || i > hi) continue;
         const int j = i + 1 < R ? i + 1 : i;
         const Tri t = triangle(y[0][i], y[1][i], y[2][i], i + 1 < R ? y[0][j] : yb[0], i + 1 < R ? y[1][j] : yb[1],
                                i + 1 < R ? y[2][j] : yb[2], wxs[i], wys[i], bxs[i], bys[i], h0 + i >= 0 && h0 + i < H - 1);
+        if (i < lo) {
+          above = t;
+          continue;
+        }
         float yt = y[0][i], y1n = y[1][i], y2n = y[2][i];
         yt -= -above.Fa;               // TGV.cu:1637
         y1n -= -above.G1y;             // TGV.cu:1638
