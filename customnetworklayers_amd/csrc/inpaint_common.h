@@ -72,7 +72,7 @@ struct Knobs {
   int tgv_fwd_rows = 0;           // INPAINT_TGV_FWD_ROWS / INPAINT_TGV_ADJ_ROWS
   int tgv_adj_rows = 0;
   int tgv_fwd_split = -1;         // INPAINT_TGV_FWD_SPLIT=0|1: forward pairs with one channel per wavefront (-1 = by the size of the launch)
-  int tgv_pair_waves = 0;         // INPAINT_TGV_PAIR_WAVES=1|2 (0 = by channel count)
+  int tgv_pair_waves = 0;         // INPAINT_TGV_PAIR_WAVES=1|2|4 (0 = by size; 4: two channels only)
   int keep = -1;                  // INPAINT_KEEP=0|1|2 (INPAINT_KEEP_LAST=0 is INPAINT_KEEP=0); -1 = the id's own mode
   double keep_gb = 32.0;          // INPAINT_KEEP_GB: budget of keep mode 2
   bool keep_gb_set = false;       // (the variable is set: the budget is the caller's, free device memory is not consulted)
@@ -118,7 +118,7 @@ struct Knobs {
     tgv_fwd_rows = rows("INPAINT_TGV_FWD_ROWS");
     tgv_adj_rows = rows("INPAINT_TGV_ADJ_ROWS");
     tgv_fwd_split = is("INPAINT_TGV_FWD_SPLIT", "1") ? 1 : (is("INPAINT_TGV_FWD_SPLIT", "0") ? 0 : -1);
-    tgv_pair_waves = is("INPAINT_TGV_PAIR_WAVES", "1") ? 1 : (is("INPAINT_TGV_PAIR_WAVES", "2") ? 2 : (getenv("INPAINT_TGV_PAIR_WAVES") ? 1 : 0));
+    tgv_pair_waves = is("INPAINT_TGV_PAIR_WAVES", "1") ? 1 : (is("INPAINT_TGV_PAIR_WAVES", "2") ? 2 : (is("INPAINT_TGV_PAIR_WAVES", "4") ? 4 : (getenv("INPAINT_TGV_PAIR_WAVES") ? 1 : 0)));
     if (is("INPAINT_KEEP_LAST", "0")) keep = 0;
     if (const char* e = getenv("INPAINT_KEEP")) {
       const int v = atoi(e);
@@ -291,6 +291,9 @@ inline int compute_unit_count() {
 // Measured: 4 x 2 x 384 x 1248, pair kernels: 16 rows (504 workgroups, two per CU) beat 8, 17, 18 and 24;
 // 16 x 2 x 256 x 512: 19 rows (504 workgroups) 9.8 ms, 16 rows (576: three on some CUs) 12.0 ms.
 inline int choose_strip_rows(long long strips, int ih, int waves_per_block, int lag) {
+  // (asked before every launch of a sweep, with the same numbers: the last answer is kept, 30 pairs of divisions otherwise)
+  static thread_local struct { long long strips; int ih, waves, lag, R; } last = {-1, 0, 0, 0, 0};
+  if (last.strips == strips && last.ih == ih && last.waves == waves_per_block && last.lag == lag) return last.R;
   const long long cus = compute_unit_count();
   int best = 0;
   long long best_cost = 0;
@@ -305,7 +308,8 @@ inline int choose_strip_rows(long long strips, int ih, int waves_per_block, int 
       best_cost = cost;
     }
   }
-  return best > 0 ? best : 2;
+  last = {strips, ih, waves_per_block, lag, best > 0 ? best : 2};
+  return last.R;
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -463,6 +463,11 @@ __global__ __launch_bounds__(256) void tgv_finalize_init(const float* __restrict
 // -------------------------------------------------------------------------------------------------
 // per-id state (idStructBs, TGVInpaintFista.h:7-50)
 // -------------------------------------------------------------------------------------------------
+// wavefronts per strip of the reverse sweep's pair launches, and rows per strip
+struct PairShape {
+  int waves = 2, R = 1;
+};
+
 struct Slot {
   // backward passes so far, INCLUDING those whose upstream gradient was refused: the device counts those in
   // GuardState::skipped, and the reference's `run` is the difference (run_count())
@@ -503,6 +508,7 @@ struct Slot {
         *acc_gb[2] = {nullptr, nullptr};
   int acc_cur = 0;   // set of the shared accumulators (gc, gx, gy) the next adjoint launch reads
   int accb_cur = 0;  // set of the per-channel accumulator (gb) the next adjoint step reads
+  PairShape pair;    // of the backward pass under way
   double *tot_gc = nullptr, *tot_gx = nullptr, *tot_gy = nullptr, *tot_gb = nullptr;
   // strip path: one fp32 record per segment and tensor, added into the totals after the last segment
   float *seg_gc = nullptr, *seg_gx = nullptr, *seg_gy = nullptr, *seg_gb = nullptr;
@@ -673,22 +679,17 @@ int strip_rows(int n, int ih, int iw, int cols, int forced_rows, int lag) {
 
 // Rows per strip of the two-wavefront pair kernel.  Its workgroups (one strip each) are resident four per CU, so a
 // launch runs in ceil(workgroups / (4 * CUs)) rounds of (R + 3 pipeline rows + start-up) row steps each; the
-// strip height that minimises rounds x steps is taken (on 4 x 384 x 1248: 32 rows, 1008 workgroups, one round).
+// strip height that minimises rounds x steps is taken (on 4 x 384 x 1248: 32 rows, 1008 workgroups, one round), down to a
+// single row: a launch that does not fill the chip lasts as long as one strip.  Backward pass, us, at least 8 rows / as few as
+// fill a round: 1 x 2 x 200 x 640, 50 iterations 784 / 517 (3 rows), 2 x 2 x 224 x 512 840 / 623 (4), 4 x 2 x 100 x 150 660 / 401 (2);
+// the best of all heights on each of 17 shapes with two channels, 0.7% from it in the mean on 13 with one.
 int pair_split_rows(int n, int ih, int iw) {
   if (knobs().tgv_adj_rows > 0) return knobs().tgv_adj_rows;
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    hipDeviceProp_t prop;
-    cus = (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess && prop.multiProcessorCount > 0)
-              ? prop.multiProcessorCount
-              : 256;
-  }
-  const long long cap = 4ll * cus;
+  const long long cap = 4ll * compute_unit_count();
   const long long sx = (iw + tgvstrip::kCols2 - 1) / tgvstrip::kCols2;
-  int best = 16;
+  int best = 1;
   long long best_cost = -1;
-  for (int R = 8; R <= 64; R++) {
+  for (int R = 1; R <= 64; R++) {
     const long long wg = sx * ((ih + R - 1) / R) * n;
     const long long cost = ((wg + cap - 1) / cap) * (R + 7);
     if (best_cost < 0 || cost < best_cost) {
@@ -906,23 +907,42 @@ void launch_adjoint(Slot& s, hipStream_t stream, const float* c, const float* b,
   s.accb_cur = 1 - s.accb_cur;
 }
 
+int pair_quad_rows(int n, int ih, int iw);
+
 // Two adjoint steps in one launch (strip path): A = local iteration j (x05 slots xa = j, xb = j-1), B = j-1
 // (xc = slot j-2, or the checkpoint y when B is the segment's first iteration).
-// Whether the pair kernel runs its two steps in two wavefronts (the default with two channels).
-bool pair_split(int channels) { return knobs().tgv_pair_waves ? knobs().tgv_pair_waves == 2 : channels >= 2; }
+// Wavefronts per strip of such a launch with one or two channels, and rows per strip: two (a step each), but where strips of
+// one row fit a round -- the launch then lasts as long as one strip's few rows -- one wavefront for one channel and four (a
+// step of one channel each) for two.  One channel: up to a strip per CU two are still the faster ones (backward pass, us, one
+// / two: 61 x 97 152 / 148, 100 x 200 228 / 237, 147 x 286 238 / 251, 200 x 640 340 / 321, 384 x 1248 594 / 576).  Two channels, two / four:
+// 61 x 97 208 / 182, 100 x 200 348 / 316, 147 x 286 368 / 350, 4 x 60 x 80 222 / 202, but 2 x 147 x 286 (strips of 2 rows) 417 / 427,
+// 384 x 1248 926 / 1011.
+PairShape pair_shape(const Slot& s, bool corrected) {
+  if (s.ic > 2) return {4, pair_quad_rows(s.n, s.ih, s.iw)};
+  const int forced = knobs().tgv_pair_waves, R2 = pair_split_rows(s.n, s.ih, s.iw);
+  const int sx = (s.iw + tgvstrip::kCols2 - 1) / tgvstrip::kCols2;
+  int waves = 2;
+  if (forced) waves = forced;
+  else if (knobs().tgv_adj_rows > 0) waves = s.ic;
+  else if (R2 == 1) waves = s.ic == 2 ? 4 : ((long long)sx * s.ih * s.n > compute_unit_count() ? 1 : 2);
+  if (waves == 4 && s.ic != 2) waves = 2;
+  if (waves == 1 && corrected) waves = 2;  // (the one-wavefront kernel has no such form)
+  if (waves == 4) return {4, pair_quad_rows(s.n, s.ih, s.iw)};
+  if (waves == 2) return {2, R2};
+  return {1, R2 == 1 && !forced ? 1 : strip_rows(s.n, s.ih, s.iw, tgvstrip::kCols2, knobs().tgv_adj_rows, 8)};
+}
+// Whether the corrected gradient takes two steps per launch.
+bool corrected_pairs() { return knobs().tgv_pair_waves != 1; }
 
-// TRUE_ADJ (the corrected gradient) exists for the two-wavefront kernel only; the caller checks pair_split().
 template <int C, bool BEND, bool TRUE_ADJ>
 void launch_adjoint_pair_strip(const Slot& s, hipStream_t stream, const float* c, const float* b, const float* xa,
                                const float* xb, const float* xc, const float* g05_in, float* g05_out, const float* gxk,
-                               float* gxk_m1, float* gx_final, float tA, float tB) {
+                               float* gxk_m1, float* gx_final, float tA, float tB, PairShape shape) {
   const int i = s.acc_cur, o = 1 - s.acc_cur, ib = s.accb_cur, ob = 1 - s.accb_cur;
-  // two channels: the two steps run in two wavefronts of a workgroup (one strip per 128-thread workgroup);
-  // one channel: both steps fit one wavefront's registers (four strips per 256-thread workgroup)
-  const bool split = pair_split(C);
+  // two wavefronts: one strip per 128-thread workgroup; one: four strips per 256-thread workgroup
+  const bool split = shape.waves == 2;
   auto kern1 = gx_final ? tgvstrip::tgv_adjoint_strip2<C, BEND, true> : tgvstrip::tgv_adjoint_strip2<C, BEND, false>;
-  const int R = split ? pair_split_rows(s.n, s.ih, s.iw)
-                      : strip_rows(s.n, s.ih, s.iw, tgvstrip::kCols2, knobs().tgv_adj_rows, 8);
+  const int R = shape.R;
   const int sx = (s.iw + tgvstrip::kCols2 - 1) / tgvstrip::kCols2, sy = (s.ih + R - 1) / R;
   const long long waves = (long long)sx * sy * s.n;
   const size_t sP = (size_t)s.seg_cur * plane_count(s), sF = (size_t)s.seg_cur * field_count(s);  // this segment's records
@@ -942,7 +962,7 @@ void launch_adjoint_pair_strip(const Slot& s, hipStream_t stream, const float* c
 #undef TGV_PAIR_ARGS
 }
 
-// Rows per strip of the four-wavefront pair kernel (three and four channels).  Its 256-thread workgroups (one strip
+// Rows per strip of the four-wavefront pair kernel (three and four channels, two on small images).  Its 256-thread workgroups (one strip
 // each) are resident two per CU; a strip of R rows takes R + 3 pipeline rows, two intervals of two rows behind and the
 // start-up.
 int pair_quad_rows(int n, int ih, int iw) {
@@ -951,7 +971,7 @@ int pair_quad_rows(int n, int ih, int iw) {
   const long long sx = (iw + tgvstrip::kCols2 - 1) / tgvstrip::kCols2;
   int best = 16;
   long long best_cost = -1;
-  for (int R = 8; R <= 96; R++) {
+  for (int R = 1; R <= 96; R++) {
     const long long wg = sx * ((ih + R - 1) / R) * n;
     const long long cost = ((wg + cap - 1) / cap) * (R + 11);
     if (best_cost < 0 || cost < best_cost) {
@@ -969,7 +989,7 @@ void launch_adjoint_pair_quad(const Slot& s, hipStream_t stream, const float* c,
                               float* gxk_m1, float* gx_final, float tA, float tB) {
   const int i = s.acc_cur, o = 1 - s.acc_cur, ib = s.accb_cur, ob = 1 - s.accb_cur;
   auto kern = gx_final ? tgvstrip::tgv_adjoint_strip4w<CM, C1, BEND, true, TRUE_ADJ> : tgvstrip::tgv_adjoint_strip4w<CM, C1, BEND, false, TRUE_ADJ>;
-  const int R = pair_quad_rows(s.n, s.ih, s.iw);
+  const int R = s.pair.R;
   const int sx = (s.iw + tgvstrip::kCols2 - 1) / tgvstrip::kCols2, sy = (s.ih + R - 1) / R;
   const long long strips = (long long)sx * sy * s.n;
   const size_t sP = (size_t)s.seg_cur * plane_count(s), sF = (size_t)s.seg_cur * field_count(s);  // this segment's records
@@ -986,10 +1006,14 @@ template <bool BEND, bool TRUE_ADJ = false>
 void launch_adjoint_pair(Slot& s, hipStream_t stream, const float* c, const float* b, const float* xa, const float* xb,
                          const float* xc, const float* g05_in, float* g05_out, const float* gxk, float* gxk_m1,
                          float* gx_final, float tA, float tB) {
-  if (s.ic == 1) launch_adjoint_pair_strip<1, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB);
-  else if (s.ic == 3) launch_adjoint_pair_quad<2, 1, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB);
+  if (s.ic == 3) launch_adjoint_pair_quad<2, 1, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB);
   else if (s.ic == 4) launch_adjoint_pair_quad<2, 2, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB);
-  else launch_adjoint_pair_strip<2, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB);
+  else {
+    const PairShape shape = s.pair;
+    if (shape.waves == 4) launch_adjoint_pair_quad<1, 1, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB);
+    else if (s.ic == 1) launch_adjoint_pair_strip<1, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB, shape);
+    else launch_adjoint_pair_strip<2, BEND, TRUE_ADJ>(s, stream, c, b, xa, xb, xc, g05_in, g05_out, gxk, gxk_m1, gx_final, tA, tB, shape);
+  }
   s.acc_cur = 1 - s.acc_cur;
   s.accb_cur = 1 - s.accb_cur;
 }
@@ -1201,7 +1225,7 @@ int tgvinpaint_backward(const float* dx, const float* dy, const float* c, const 
   // The sweep's first step rides on its second when the last segment has at least four iterations (that second step
   // is then an inner step) and one launch holds every channel.  That launch starts from zero accumulators without
   // reading them, and every launch after it reads only what its predecessor wrote in full: nothing to clear.
-  const bool corr_pairs_ok = !corr || pair_split(s.ic);
+  const bool corr_pairs_ok = !corr || corrected_pairs();
   const int nseg_all = (int)s.iterations.size();
   const bool first_two = adjoint_pairs(s) && corr_pairs_ok && s.ic <= kGroup && knobs().tgv_fuse_first &&
                          nseg_all > 0 && 2 * ((its - s.iterations[nseg_all - 1]) / 2) >= 4;
@@ -1224,8 +1248,9 @@ int tgvinpaint_backward(const float* dx, const float* dy, const float* c, const 
   // before it is read and is not made).
   // The kernels store g_x only at the very last step (into gx_final).
   const float* gi_src = s.gx_final;
-  // the corrected gradient has a pair kernel in the two-wavefront form only
-  const bool pairs = adjoint_pairs(s) && (!corr || pair_split(s.ic));
+  // (the corrected gradient has no pair kernel in one wavefront)
+  const bool pairs = adjoint_pairs(s) && (!corr || corrected_pairs());
+  if (pairs) s.pair = pair_shape(s, corr);  // (once: every launch of the sweep has the same)
   int lastIt = its;
   int pp_src = 1;
   const int nseg = (int)s.iterations.size();
