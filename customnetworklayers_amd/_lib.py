@@ -1,5 +1,6 @@
 """Loader of the HIP library behind the layers.  There is no fallback: if the library is missing
 or cannot be loaded the import fails, and the message says how to build it."""
+import contextlib
 import ctypes
 import os
 
@@ -79,7 +80,7 @@ def _load():
     lib.medimax_forward.argtypes = [_f32p] * 2 + [_int] * 4 + [ctypes.c_void_p]
     lib.medimax_backward.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_void_p]
     lib.medimax_forward_saving.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_void_p]
-    lib.medimax_backward_saved.argtypes = [_f32p] * 4 + [_int] * 4 + [ctypes.c_void_p]
+    lib.medimax_backward_saved.argtypes = [_f32p] * 2 + [_int] + [_f32p] * 2 + [_int] * 4 + [ctypes.c_void_p]
     lib.flowaux_last_error.restype = ctypes.c_char_p
     lib.hierarchy_next_level_forward.argtypes = [_f32p] * 5 + [_int] * 4 + [ctypes.c_float, ctypes.c_float, ctypes.c_void_p]
     lib.hierarchy_next_level_backward.argtypes = [_f32p] * 3 + [_int] * 4 + [ctypes.c_float, ctypes.c_void_p]
@@ -90,6 +91,16 @@ def _load():
 
 
 lib = _load()
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def device_of(t):
+    """torch.cuda.device(t.device), without the switch and its cost where that device is current already."""
+    import torch
+
+    return _NO_SWITCH if torch.cuda.current_device() == t.device.index else torch.cuda.device(t.device)
 
 
 # ---- the slots' device memory out of PyTorch's caching allocator (t[g]vinpaint_set_allocator) -------------------

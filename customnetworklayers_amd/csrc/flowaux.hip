@@ -2080,7 +2080,7 @@ __global__ __launch_bounds__(64) void median_backward_stream_kernel(const float*
 template <int VEC>
 __global__ __launch_bounds__(64) void median_backward_saved_kernel(const float* __restrict__ vol, const float* __restrict__ gin,
                                                                    const float* __restrict__ saved, float* __restrict__ gvol,
-                                                                   long long P, long long HW, int D) {
+                                                                   long long P, long long HW, int D, int gin_planes) {
   __shared__ float tile[64][kPitch];
   __shared__ float4 bins[64];  // value in front of the crossing, at it, its bin
   typedef float vec4 __attribute__((ext_vector_type(4)));
@@ -2090,8 +2090,8 @@ __global__ __launch_bounds__(64) void median_backward_saved_kernel(const float* 
   float g0v = 0.f, g1v = 0.f, alpha = 0.f, pmid = 1.f, at = 0.f;
   if (lane < npx) {
     const long long n = p / HW, q = p - n * HW;
-    g0v = gin[n * 2 * HW + q];
-    g1v = gin[n * 2 * HW + HW + q];
+    g0v = gin[n * gin_planes * HW + q];
+    if (gin_planes == 2) g1v = gin[n * 2 * HW + HW + q];
     alpha = saved[p];
     pmid = saved[P + p];
     at = saved[2 * P + p];
@@ -2443,18 +2443,21 @@ int medimax_forward_saving(const float* vol, float* out, float* saved, int n, in
   return 0;
 }
 
-int medimax_backward_saved(const float* vol, const float* gin, const float* saved, float* gvol, int n, int ih, int iw, int num_disp,
-                           void* stream) {
+int medimax_backward_saved(const float* vol, const float* gin, int gin_planes, const float* saved, float* gvol, int n, int ih, int iw,
+                           int num_disp, void* stream) {
   if (!vol || !gin || !saved || !gvol) return fail(INPAINT_ERR_ARG, "medimax_backward_saved: null pointer");
+  if (gin_planes != 1 && gin_planes != 2) return fail(INPAINT_ERR_ARG, "medimax_backward_saved: one or two planes of gradient, not %d", gin_planes);
   if (n < 1 || ih < 1 || iw < 1 || num_disp < 1 || num_disp > kMaxRowBins)
     return fail(INPAINT_ERR_ARG, "medimax_backward_saved: bad shape %dx%dx%dx%d", n, ih, iw, num_disp);
   const long long HW = (long long)ih * iw, P = n * HW;
   const dim3 grid((unsigned)((P + 63) / 64)), block(64);
   g_timer.begin((hipStream_t)stream);
   if (aligned16(gvol) && num_disp >= 4)
-    hipLaunchKernelGGL((median_backward_saved_kernel<4>), grid, block, 0, (hipStream_t)stream, vol, gin, saved, gvol, P, HW, num_disp);
+    hipLaunchKernelGGL((median_backward_saved_kernel<4>), grid, block, 0, (hipStream_t)stream, vol, gin, saved, gvol, P, HW, num_disp,
+                       gin_planes);
   else
-    hipLaunchKernelGGL((median_backward_saved_kernel<1>), grid, block, 0, (hipStream_t)stream, vol, gin, saved, gvol, P, HW, num_disp);
+    hipLaunchKernelGGL((median_backward_saved_kernel<1>), grid, block, 0, (hipStream_t)stream, vol, gin, saved, gvol, P, HW, num_disp,
+                       gin_planes);
   g_timer.end((hipStream_t)stream, 1);
   INPAINT_HIP(hipGetLastError());
   return 0;

@@ -25,6 +25,27 @@ class MedianFunction(Function):
         return outputs[0]
 
 
+class _MedianImage(Function):
+    """The position plane of MedianFunction for one H x W x D volume, as a node of its own: the mass plane, which the module drops,
+    gets no gradient of zeros."""
+
+    @staticmethod
+    def forward(ctx, in_vol):
+        h, w, _ = in_vol.shape
+        if ctx.needs_input_grad[0]:
+            solution, saved = median_cuda_ext.forward_saving(in_vol.unsqueeze(0).contiguous())
+            ctx.save_for_backward(in_vol, saved)
+        else:
+            (solution,) = median_cuda_ext.forward(in_vol.unsqueeze(0).contiguous())
+        return solution.resize_(h, w)  # (the first plane, and not as a view: it may be changed in place)
+
+    @staticmethod
+    def backward(ctx, grad_sol):
+        in_vol, saved = ctx.saved_tensors
+        (gradient,) = median_cuda_ext.backward(grad_sol[None, None].contiguous(), in_vol.unsqueeze(0).contiguous(), saved)
+        return gradient[0]
+
+
 class Median(nn.Module):
     def __init__(self, device):
         super(Median, self).__init__()
@@ -33,6 +54,8 @@ class Median(nn.Module):
     def forward(self, t_vol):
         """t_vol: H x W x D histogram per pixel.  Returns the H x W map of median positions (median.py:69-80
         drops the second output channel, the mass of the median's bin)."""
+        if t_vol.dim() == 3 and t_vol.shape[2] <= median_cuda_ext.MAX_SAVED_BINS:
+            return _MedianImage.apply(t_vol)
         sol = MedianFunction.apply(t_vol.unsqueeze(0))
         return sol.squeeze(0).permute(1, 2, 0)[:, :, 0]
 

@@ -9,7 +9,7 @@ import ctypes
 
 import torch
 
-from .._lib import lib
+from .._lib import device_of, lib
 
 _ERRORS = {1: IndexError, 2: ValueError, 3: ValueError, 4: RuntimeError, 5: RuntimeError}
 
@@ -48,7 +48,7 @@ def forward(in_vol):
     the median's position in bins and the mass of the bin that holds it."""
     n, h, w, d = _check_volume(in_vol)
     solution = torch.empty((n, 2, h, w), dtype=torch.float32, device=in_vol.device)
-    with torch.cuda.device(in_vol.device):
+    with device_of(in_vol):
         rc = lib.medimax_forward(in_vol.data_ptr(), solution.data_ptr(), n, h, w, d, _stream(in_vol))
     if rc:
         raise _ERRORS.get(rc, RuntimeError)("MediMax::forward failed: %s" % _last_error())
@@ -60,7 +60,7 @@ def forward_saving(in_vol):
     n, h, w, d = _check_volume(in_vol)
     solution = torch.empty((n, 2, h, w), dtype=torch.float32, device=in_vol.device)
     saved = torch.empty((3, n, h, w), dtype=torch.float32, device=in_vol.device)
-    with torch.cuda.device(in_vol.device):
+    with device_of(in_vol):
         rc = lib.medimax_forward_saving(in_vol.data_ptr(), solution.data_ptr(), saved.data_ptr(), n, h, w, d, _stream(in_vol))
     if rc:
         raise _ERRORS.get(rc, RuntimeError)("MediMax::forward failed: %s" % _last_error())
@@ -69,10 +69,11 @@ def forward_saving(in_vol):
 
 def backward(d_iGf, in_vol, saved=None):
     """d_iGf: (n,2,h,w) gradient wrt the result.  Returns [gradient wrt in_vol].  `saved`: the second result of
-    forward_saving(in_vol); the gradient is the same without it, at the cost of a second read of the volume."""
+    forward_saving(in_vol); the gradient is the same without it, at the cost of a second read of the volume.  With it d_iGf
+    may be (n,1,h,w): the gradient wrt the position alone."""
     n, h, w, d = _check_volume(in_vol)
     _check_input(d_iGf, "d_iGf")
-    if tuple(d_iGf.shape) != (n, 2, h, w):
+    if tuple(d_iGf.shape) != (n, 2, h, w) and (saved is None or tuple(d_iGf.shape) != (n, 1, h, w)):
         raise ValueError("d_iGf must have shape (%d, 2, %d, %d), got %s" % (n, h, w, tuple(d_iGf.shape)))
     if d_iGf.device != in_vol.device:
         raise RuntimeError("all tensors must live on one device")
@@ -83,12 +84,12 @@ def backward(d_iGf, in_vol, saved=None):
             raise ValueError("saved must have shape (3, %d, %d, %d), got %s" % (n, h, w, tuple(saved.shape)))
         if saved.device != in_vol.device:
             raise RuntimeError("all tensors must live on one device")
-    with torch.cuda.device(in_vol.device):
+    with device_of(in_vol):
         if saved is None:
             rc = lib.medimax_backward(in_vol.data_ptr(), d_iGf.data_ptr(), outGrad.data_ptr(), n, h, w, d, _stream(in_vol))
         else:
-            rc = lib.medimax_backward_saved(in_vol.data_ptr(), d_iGf.data_ptr(), saved.data_ptr(), outGrad.data_ptr(), n, h, w, d,
-                                            _stream(in_vol))
+            rc = lib.medimax_backward_saved(in_vol.data_ptr(), d_iGf.data_ptr(), d_iGf.shape[1], saved.data_ptr(), outGrad.data_ptr(), n, h, w,
+                                            d, _stream(in_vol))
     if rc:
         raise _ERRORS.get(rc, RuntimeError)("MediMax::backward failed: %s" % _last_error())
     return [outGrad]

@@ -11,7 +11,7 @@ import ctypes
 
 import torch
 
-from .._lib import lib
+from .._lib import device_of, lib
 
 _ERRORS = {1: IndexError, 2: ValueError, 3: ValueError, 4: RuntimeError, 5: RuntimeError}
 
@@ -61,7 +61,7 @@ def forward(featureImage0, featureImage1, flow):
     fitted maximum in x and y (to be added to the rounded displaced position) and the fitted score."""
     n, c, h, w = _check_maps(featureImage0, featureImage1, flow)
     flowUpdate = torch.empty((n, 3, h, w), dtype=torch.float32, device=flow.device)
-    with torch.cuda.device(flow.device):
+    with device_of(flow):
         rc = lib.quadfit_forward(featureImage0.data_ptr(), featureImage1.data_ptr(), flow.data_ptr(),
                                  flowUpdate.data_ptr(), n, c, h, w, flow.shape[1], _stream(flow))
     if rc:
@@ -79,7 +79,7 @@ def forward_saving(featureImage0, featureImage1, flow):
     n, c, h, w = _check_maps(featureImage0, featureImage1, flow)
     flowUpdate = torch.empty((n, 3, h, w), dtype=torch.float32, device=flow.device)
     costs = torch.empty((5, n, h, w), dtype=torch.float32, device=flow.device)
-    with torch.cuda.device(flow.device):
+    with device_of(flow):
         rc = lib.quadfit_forward_saving(featureImage0.data_ptr(), featureImage1.data_ptr(), flow.data_ptr(), flowUpdate.data_ptr(),
                                         costs.data_ptr(), n, c, h, w, flow.shape[1], _stream(flow))
     if rc:
@@ -109,7 +109,7 @@ def backward(d_iGf, featureImage0, featureImage1, flow, use_atomics=False, costs
     maps = (featureImage0.data_ptr(), featureImage1.data_ptr(), flow.data_ptr(), d_iGf.data_ptr())
     rest = (d_oFeat0.data_ptr(), d_oFeat1.data_ptr(), n, c, h, w, flow.shape[1], workspace.data_ptr() if ws_bytes else None, ws_bytes,
             _stream(flow))
-    with torch.cuda.device(flow.device):
+    with device_of(flow):
         rc = lib.quadfit_backward(*maps, *rest) if costs is None else lib.quadfit_backward_saved(*maps, costs.data_ptr(), *rest)
     if rc:
         raise _ERRORS.get(rc, RuntimeError)("FlowQuadFitting::backward failed: %s" % _last_error())
@@ -141,7 +141,7 @@ def image_forward(feat0, feat1, flow, want_costs):
     flow, pixel, channel = _flow_strides(flow)
     out = torch.empty((h, w, 3), dtype=torch.float32, device=flow.device)
     costs = torch.empty((5, h, w), dtype=torch.float32, device=flow.device) if want_costs else None
-    with torch.cuda.device(flow.device):
+    with device_of(flow):
         rc = lib.quadfit_image_forward(feat0.data_ptr(), feat1.data_ptr(), flow.data_ptr(), out.data_ptr(),
                                        costs.data_ptr() if want_costs else None, c, h, w, pixel, channel, _stream(flow))
     if rc:
@@ -158,7 +158,7 @@ def image_backward(d_iGf, feat0, feat1, flow, costs):
     g0, g1 = torch.empty_like(feat0), torch.empty_like(feat1)
     ws_bytes = lib.quadfit_backward_workspace_bytes(1, h, w)
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=flow.device)
-    with torch.cuda.device(flow.device):
+    with device_of(flow):
         rc = lib.quadfit_image_backward(feat0.data_ptr(), feat1.data_ptr(), flow.data_ptr(), d_iGf.data_ptr(), costs.data_ptr(),
                                         g0.data_ptr(), g1.data_ptr(), c, h, w, pixel, channel, workspace.data_ptr(), ws_bytes,
                                         _stream(flow))

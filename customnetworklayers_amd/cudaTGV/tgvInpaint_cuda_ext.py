@@ -13,7 +13,7 @@ import os
 
 import torch
 
-from .._lib import last_error, lib, torch_allocator_in_use, use_torch_allocator
+from .._lib import device_of, last_error, lib, torch_allocator_in_use, use_torch_allocator
 
 # The per-id device blocks come out of PyTorch's caching allocator (t[g]vinpaint_set_allocator), so that
 # torch.cuda.memory_allocated() counts them and reset_id() returns them to the pool; INPAINT_TORCH_ALLOCATOR=0 leaves
@@ -57,7 +57,7 @@ def forward(d_x, d_y, d_c, d_b, d_i, its, id, keep=None):  # noqa: A002 - the re
     solution = torch.empty_like(d_i)
     if keep is not None:
         _set_keep(id, keep)
-    with torch.cuda.device(d_b.device):
+    with device_of(d_b):
         rc = lib.tgvinpaint_forward(d_x.data_ptr(), d_y.data_ptr(), d_c.data_ptr(), d_b.data_ptr(), d_i.data_ptr(),
                                     solution.data_ptr(), n, c, h, w, int(its), int(id), _stream(d_b))
     if keep is not None:
@@ -76,7 +76,7 @@ def backward(d_iGf, d_x, d_y, d_c, d_b, its, id):  # noqa: A002
     n, c, h, w = d_b.shape
     d_oGx, d_oGy, d_oGc = torch.empty_like(d_x), torch.empty_like(d_y), torch.empty_like(d_c)
     d_oGb, d_oGi = torch.empty_like(d_b), torch.empty_like(d_iGf)
-    with torch.cuda.device(d_b.device):
+    with device_of(d_b):
         rc = lib.tgvinpaint_backward(d_x.data_ptr(), d_y.data_ptr(), d_c.data_ptr(), d_b.data_ptr(), d_iGf.data_ptr(),
                                      d_oGx.data_ptr(), d_oGy.data_ptr(), d_oGc.data_ptr(), d_oGb.data_ptr(),
                                      d_oGi.data_ptr(), n, c, h, w, int(its), int(id), _stream(d_b))

@@ -5,6 +5,7 @@ import torch
 from torch import nn
 from torch.autograd import Function
 
+from .._image import images, planes, result
 from . import tvInpaint_cuda_ext
 
 
@@ -32,6 +33,24 @@ class TVInpaintingFunction(Function):
         return d_oGx, d_oGy, d_oGc, d_oGb, d_oGi, None, None
 
 
+class _TVInpaintImage(Function):
+    """TVInpaintingFunction of one image with its channels innermost; the permutations are part of the node."""
+
+    @staticmethod
+    def forward(ctx, dx, dy, dc, db, di, its, pid):
+        (sol,) = tvInpaint_cuda_ext.forward(planes(dx), planes(dy), planes(dc), planes(db), planes(di), its, pid,
+                                           keep=None if any(ctx.needs_input_grad[:5]) else 0)
+        ctx.its, ctx.pid = int(its), int(pid)
+        ctx.save_for_backward(dx, dy, dc, db)
+        return result(sol)
+
+    @staticmethod
+    def backward(ctx, grad_sol):
+        dx, dy, dc, db = ctx.saved_tensors
+        gradients = tvInpaint_cuda_ext.backward(planes(grad_sol), planes(dx), planes(dy), planes(dc), planes(db), ctx.its, ctx.pid)
+        return images(gradients, ctx.needs_input_grad) + (None, None)
+
+
 class TVInpaint(nn.Module):
     """Unbatched H x W x C interface of the reference module (cudaTV/TVInpainting.py:32-55)."""
 
@@ -48,14 +67,7 @@ class TVInpaint(nn.Module):
         Yx, Xx, Lx = t_dx.shape  # no batches here
         assert Lx == 1, "diffusion tensors should have 1 channel\n"
 
-        t_dx_in = t_dx.permute(2, 0, 1).unsqueeze(0)  # order is 1,Channel,Height,Width
-        t_dy_in = t_dy.permute(2, 0, 1).unsqueeze(0)
-        t_dc_in = t_dc.permute(2, 0, 1).unsqueeze(0)
-        t_db_in = t_db.permute(2, 0, 1).unsqueeze(0)
-        t_di_in = t_di.permute(2, 0, 1).unsqueeze(0)
-
-        sol = TVInpaintingFunction.apply(t_dx_in, t_dy_in, t_dc_in, t_db_in, t_di_in, self.its, self.id)
-        return sol.squeeze(0).permute(1, 2, 0).contiguous()
+        return _TVInpaintImage.apply(t_dx, t_dy, t_dc, t_db, t_di, self.its, self.id)
 
     def init(self):
         pass

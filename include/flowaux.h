@@ -96,10 +96,11 @@ int medimax_backward(const float* vol, const float* gin, float* gvol, int n, int
  *   saved : 3*n*ih*iw floats, written by medimax_forward_saving and read by medimax_backward_saved
  *   vol   : the volume of the forward pass; the backward pass reads it where a running sum that has reached one half falls
  *           below it again, or is not a number
+ *   gin   : (n,gin_planes,ih,iw), two planes as for medimax_backward, or one: the gradient wrt the position alone
  * num_disp is at most 255.
  */
 int medimax_forward_saving(const float* vol, float* out, float* saved, int n, int ih, int iw, int num_disp, void* stream);
-int medimax_backward_saved(const float* vol, const float* gin, const float* saved, float* gvol, int n, int ih, int iw,
+int medimax_backward_saved(const float* vol, const float* gin, int gin_planes, const float* saved, float* gvol, int n, int ih, int iw,
                            int num_disp, void* stream);
 
 /* Measurement hooks, as tvinpaint_profile / tvinpaint_profile_read: with profiling on, every backward
