@@ -569,8 +569,8 @@ static __global__ __launch_bounds__(256) void guard_tail_decide_many(GuardJobs j
   else guard_tail_decide_body(static_cast<const double*>(jobs.ptr[k]), jobs.n[k], gs, k, run, p, clamp_mean);
 }
 
-static __global__ void guard_clear_kernel(GuardState* gs) {
-  int k = threadIdx.x;
+__device__ __forceinline__ void guard_clear(GuardState* gs) {  // by the first five threads of one block
+  const int k = threadIdx.x;
   if (k < 5) {
     GuardStats z;
     z.sum = 0; z.tail_sum = 0; z.max_bits = 0; z.last_invalid1 = 0; z.num_above = 0; z.num_invalid = 0;
@@ -673,19 +673,9 @@ static __global__ __launch_bounds__(256) void fill_zero_many(ZeroList z) {
     p[i] = 0u;
 }
 
-// Zero the non-finite entries of the caller's upstream gradient in place
-// (TVInpaintFista.cu:1609-1623; TGVInpaintFistaBetas.cu:2690-2701).
-static __global__ __launch_bounds__(256) void scrub_kernel(float* __restrict__ g, long long n) {
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    const float v = g[i];
-    if (!finite_value(v)) g[i] = 0.f;
-  }
-}
-
 // The start of a backward pass in one launch: the buffers of `z` zeroed (blockIdx.y < nz), the non-finite entries of the
-// caller's upstream gradient zeroed in place (blockIdx.y == nz, as scrub_kernel) and the guard's statistics of the
-// previous backward cleared (blockIdx.y == nz + 1, as guard_clear_kernel).  Launch with grid (blocks, nz + 2).
+// caller's upstream gradient zeroed in place (blockIdx.y == nz, TVInpaintFista.cu:1609-1623) and the guard's statistics of the
+// previous backward cleared (blockIdx.y == nz + 1).  Launch with grid (blocks, nz + 2).
 static __global__ __launch_bounds__(256) void backward_prologue_many(ZeroList z, int nz, float* __restrict__ upstream,
                                                                      long long upstream_n, GuardState* gs) {
   const int job = blockIdx.y;
@@ -698,11 +688,8 @@ static __global__ __launch_bounds__(256) void backward_prologue_many(ZeroList z,
       const float v = upstream[i];
       if (!finite_value(v)) upstream[i] = 0.f;
     }
-  } else if (blockIdx.x == 0 && threadIdx.x < 5) {
-    GuardStats zs;
-    zs.sum = 0; zs.tail_sum = 0; zs.max_bits = 0; zs.last_invalid1 = 0; zs.num_above = 0; zs.num_invalid = 0;
-    gs->stats[threadIdx.x] = zs;
-    gs->tickets[threadIdx.x] = 0;
+  } else if (blockIdx.x == 0) {
+    guard_clear(gs);
   }
 }
 
@@ -712,19 +699,6 @@ __device__ inline T guard_limit(T v, const GuardParams& p) {
   if (!finite_value(v)) return T(0);
   if (fabs((double)v) > p.max_tolerance) return p.clamp_to > 0 ? (T)(v > 0 ? p.clamp_to : -p.clamp_to) : T(0);
   return v;
-}
-
-// Gradient wrt the starting point, guarded as a float tensor (TVInpaintFista.cu:1784-1791,1816).
-static __global__ __launch_bounds__(256) void finalize_f32(const float* __restrict__ src, float* __restrict__ out,
-                                                           long long n, const GuardState* __restrict__ gs, int k,
-                                                           GuardParams p) {
-  const double mult = gs->scale[k];
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (long long)gridDim.x * blockDim.x) {
-    float v = guard_limit(src[i], p);
-    if (mult != 1.0) v = (mult == 0.0) ? 0.f : (float)((double)v * mult);
-    out[i] = 0.0f + v;
-  }
 }
 
 // (TGV) every output of a backward pass whose upstream gradient was refused is zero
@@ -744,31 +718,16 @@ struct FinalizeJobs {
   double chain_const[4];
   const double* chain_per_sample[4];
   long long per_sample[4];
-  // optional fifth job (grid.y == 5): a float tensor guarded as finalize_f32 does, with the guard's scale `f32_scale`
+  // optional fifth job (grid.y == 5): the gradient wrt the starting point, guarded as a float tensor (TVInpaintFista.cu:1784-1791,
+  // 1816) with the guard's scale `f32_scale`
   const float* f32_src = nullptr;
   float* f32_out = nullptr;
   long long f32_n = 0;
   int f32_scale = 4;
 };
-static __global__ __launch_bounds__(256) void finalize_many(FinalizeJobs jobs, const GuardState* __restrict__ gs, GuardParams p,
-                                                            float global_mult) {
-  const int k = blockIdx.y;
-  if (gs->upstream_bad) {
-    if (k == 4) finalize_zero(jobs.f32_out, jobs.f32_n);
-    else finalize_zero(jobs.out[k], jobs.n[k]);
-    return;
-  }
-  if (k == 4) {  // (finalize_f32)
-    const double mult = gs->scale[jobs.f32_scale];
-    const float* __restrict__ src = jobs.f32_src;
-    float* __restrict__ out = jobs.f32_out;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < jobs.f32_n; i += (long long)gridDim.x * blockDim.x) {
-      float v = guard_limit(src[i], p);
-      if (mult != 1.0) v = (mult == 0.0) ? 0.f : (float)((double)v * mult);
-      out[i] = 0.0f + v;
-    }
-    return;
-  }
+// job k < 4 (the upstream was not refused)
+__device__ __forceinline__ void finalize_total(const FinalizeJobs& jobs, int k, const GuardState* __restrict__ gs, const GuardParams& p,
+                                               float global_mult) {
   const double mult = gs->scale[k];
   const double* __restrict__ total = jobs.total[k];
   float* __restrict__ out = jobs.out[k];
@@ -783,6 +742,28 @@ static __global__ __launch_bounds__(256) void finalize_many(FinalizeJobs jobs, c
     const double chain = chain_per_sample ? chain_per_sample[i / per_sample] : chain_const;
     out[i] = (chain == 1.0) ? f : (float)(chain * (double)f);
   }
+}
+
+static __global__ __launch_bounds__(256) void finalize_many(FinalizeJobs jobs, const GuardState* __restrict__ gs, GuardParams p,
+                                                            float global_mult) {
+  const int k = blockIdx.y;
+  if (gs->upstream_bad) {
+    if (k == 4) finalize_zero(jobs.f32_out, jobs.f32_n);
+    else finalize_zero(jobs.out[k], jobs.n[k]);
+    return;
+  }
+  if (k == 4) {
+    const double mult = gs->scale[jobs.f32_scale];
+    const float* __restrict__ src = jobs.f32_src;
+    float* __restrict__ out = jobs.f32_out;
+    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < jobs.f32_n; i += (long long)gridDim.x * blockDim.x) {
+      float v = guard_limit(src[i], p);
+      if (mult != 1.0) v = (mult == 0.0) ? 0.f : (float)((double)v * mult);
+      out[i] = 0.0f + v;
+    }
+    return;
+  }
+  finalize_total(jobs, k, gs, p, global_mult);
 }
 
 // Diagnostic: the device guard (the three kernels above, as a backward pass launches them) on one tensor handed over in

@@ -56,62 +56,109 @@ __device__ __forceinline__ float clampT(const float* f, int h, int w, int H, int
 }
 
 // -------------------------------------------------------------------------------------------------
-// Lipschitz bound: TGV.cu:101-148 per pixel, TGV.cu:2516-2527 for the reduction.
-// maxbits[s] must hold the bit pattern of 32.0f (= float(max(12, 8*beta) + 0.000001)) on entry.
+// The start of a pass in two launches.  The first reads the weights for the Lipschitz bounds and, in a backward pass, the upstream
+// gradient for its check, and leaves one word per block; every block of the second reduces the words it needs before it stores its
+// part (scaled weights, or the scrubbed upstream).  Words per block and not atomics on one: there is nothing to clear first.
+// On small images a pass is bound by its launches: with kernels of their own for clearing, filling and using the words a backward
+// pass began with 5 launches and a forward pass with 3, and a backward pass ended with 3 more than now (the guard's statistics
+// cleared, one sample's u block copied, gi stored apart from the other gradients).  Forward + backward of 1 x 1 x 61 x 97, 30
+// iterations: 361 -> 330 us.  At 1 x 1 x 375 x 1241: 16.1 us in the three launches before, 10.5 in these two (tgv_survey 4.9, with a
+// row per wavefront and loads under conditions 8.9).
 // -------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(BX* BY) void tgv_lipschitz_kernel(const float* __restrict__ dx_, const float* __restrict__ dy_,
-                                                               int H, int W, unsigned int* __restrict__ maxbits) {
-  const int w = blockIdx.x * BX + threadIdx.x, h = blockIdx.y * BY + threadIdx.y;
-  const size_t HW = (size_t)H * W;
-  const float* dx = dx_ + (size_t)blockIdx.z * 2 * HW;
-  const float* dy = dy_ + (size_t)blockIdx.z * 2 * HW;
-  const float* betaX = dx + HW;
-  const float* betaY = dy + HW;
-  float v = 0.f;
-  if (w < W && h < H) {
-    const float wx_0 = (w > 0) ? clampT(dx, h, w - 1, H, W) : 0.f;
-    const float wx_1 = (w < W - 1) ? clampT(dx, h, w, H, W) : 0.f;
-    const float wy_0 = (h > 0) ? clampT(dy, h - 1, w, H, W) : 0.f;
-    const float wy_1 = (h < H - 1) ? clampT(dy, h, w, H, W) : 0.f;
-    const float betaTX_1y = (h < H - 1) ? clampT(betaX, h, w, H, W) : 0.f;
-    const float betaTX_1x = (w < W - 1) ? clampT(betaX, h, w, H, W) : 0.f;
-    const float betaTX_0x = (w > 0) ? clampT(betaX, h - 1, w, H, W) : 0.f;  // sic: (w, h-1) under w > 0 (TGV.cu:116)
-    const float betaTX_0y = (h > 0) ? clampT(betaX, h, w - 1, H, W) : 0.f;  // sic: (w-1, h) under h > 0 (TGV.cu:117)
-    const float betaTY_1y = (h < H - 1) ? clampT(betaY, h, w, H, W) : 0.f;
-    const float betaTY_1x = (w < W - 1) ? clampT(betaY, h, w, H, W) : 0.f;
-    const float betaTY_0x = (w > 0) ? clampT(betaY, h - 1, w, H, W) : 0.f;
-    const float betaTY_0y = (h > 0) ? clampT(betaY, h, w - 1, H, W) : 0.f;
-    float weightx = 0.f, weighty1 = 0.f, weighty2 = 0.f;
-    if (h > 0) {
-      weightx += 3 * wy_0;
-      weighty1 += 2 * betaTX_0y;
-      weighty2 += 2 * betaTY_0y;
-    }
-    if (w > 0) {
-      weightx += 3 * wx_0;
-      weighty1 += 2 * betaTX_0x;
-      weighty2 += 2 * betaTY_0x;
-    }
-    weightx += 3 * (wy_1 + wx_1);
-    weighty1 += 2 * betaTX_1x + 2 * betaTX_1y + 3 * wx_1;
-    weighty2 += 2 * betaTY_1x + 2 * betaTY_1y + 3 * wy_1;
-    v = fmaxf(weightx, fmaxf(weighty1, weighty2));
-  }
-  // non-negative floats order like their bit patterns; anything else (negative, NaN) never wins
-  // against the 32.0f start value in the reference's std::max either
-  unsigned int bits = (v > 0.f) ? __float_as_uint(v) : 0u;
+__device__ __forceinline__ unsigned int block_max(unsigned int v) {  // blocks of 256 threads
+  __shared__ unsigned int s_max[4];
   for (int off = 32; off > 0; off >>= 1) {
-    const unsigned int o = __shfl_down(bits, off, 64);
-    bits = o > bits ? o : bits;
+    const unsigned int o = __shfl_xor(v, off, 64);
+    v = o > v ? o : v;
   }
-  if (threadIdx.x == 0 && bits > __float_as_uint(32.0f)) atomicMax(&maxbits[blockIdx.z], bits);
+  if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = v;
+  __syncthreads();
+  const unsigned int a = s_max[0] > s_max[1] ? s_max[0] : s_max[1], b = s_max[2] > s_max[3] ? s_max[2] : s_max[3];
+  return a > b ? a : b;
 }
 
-// (`counts`, when given: the two words of the upstream check that follows, cleared here)
-static __global__ void tgv_lipschitz_init(unsigned int* maxbits, int n, unsigned int* counts) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) maxbits[i] = __float_as_uint((float)(fmax(12., 8. * (double)kBeta) + 0.000001));
-  if (counts && i < 2) counts[i] = 0u;
+// Lipschitz weight of one pixel: TGV.cu:101-148.  dx, dy: the edge weights of its sample, the betas one plane further.
+__device__ __forceinline__ float lipschitz_weight(const float* __restrict__ dx, const float* __restrict__ dy, int h, int w, int H, int W) {
+  const float* betaX = dx + (size_t)H * W;
+  const float* betaY = dy + (size_t)H * W;
+  // (every load on its own, clamped into the image, so that all of them are in flight at once)
+  const float dxl = clampT(dx, h, w - 1, H, W), dxc = clampT(dx, h, w, H, W), dyu = clampT(dy, h - 1, w, H, W), dyc = clampT(dy, h, w, H, W);
+  const float xc = clampT(betaX, h, w, H, W), xu = clampT(betaX, h - 1, w, H, W), xl = clampT(betaX, h, w - 1, H, W);
+  const float yc = clampT(betaY, h, w, H, W), yu = clampT(betaY, h - 1, w, H, W), yl = clampT(betaY, h, w - 1, H, W);
+  const float wx_0 = (w > 0) ? dxl : 0.f;
+  const float wx_1 = (w < W - 1) ? dxc : 0.f;
+  const float wy_0 = (h > 0) ? dyu : 0.f;
+  const float wy_1 = (h < H - 1) ? dyc : 0.f;
+  const float betaTX_1y = (h < H - 1) ? xc : 0.f;
+  const float betaTX_1x = (w < W - 1) ? xc : 0.f;
+  const float betaTX_0x = (w > 0) ? xu : 0.f;  // sic: (w, h-1) under w > 0 (TGV.cu:116)
+  const float betaTX_0y = (h > 0) ? xl : 0.f;  // sic: (w-1, h) under h > 0 (TGV.cu:117)
+  const float betaTY_1y = (h < H - 1) ? yc : 0.f;
+  const float betaTY_1x = (w < W - 1) ? yc : 0.f;
+  const float betaTY_0x = (w > 0) ? yu : 0.f;
+  const float betaTY_0y = (h > 0) ? yl : 0.f;
+  float weightx = 0.f, weighty1 = 0.f, weighty2 = 0.f;
+  if (h > 0) {
+    weightx += 3 * wy_0;
+    weighty1 += 2 * betaTX_0y;
+    weighty2 += 2 * betaTY_0y;
+  }
+  if (w > 0) {
+    weightx += 3 * wx_0;
+    weighty1 += 2 * betaTX_0x;
+    weighty2 += 2 * betaTY_0x;
+  }
+  weightx += 3 * (wy_1 + wx_1);
+  weighty1 += 2 * betaTX_1x + 2 * betaTX_1y + 3 * wx_1;
+  weighty2 += 2 * betaTY_1x + 2 * betaTY_1y + 3 * wy_1;
+  return fmaxf(weightx, fmaxf(weighty1, weighty2));
+}
+
+constexpr unsigned int kBadEntry = 1u, kNonZeroEntry = 2u;
+
+// A block's part of the upstream check (TGV.cu:2686-2703): is there a non-finite entry, a finite one that is not zero?
+__device__ __forceinline__ unsigned int upstream_word(const float* __restrict__ g, long long n, long long block, long long blocks) {
+  typedef float vec4 __attribute__((ext_vector_type(4)));
+  unsigned int word = 0;
+  auto look = [&](float v) { word |= !finite_value(v) ? kBadEntry : v != 0.f ? kNonZeroEntry : 0u; };
+  const long long n4 = ((reinterpret_cast<uintptr_t>(g) & 15) == 0) ? (n >> 2) : 0;  // whole 16-byte groups
+  const vec4* __restrict__ g4 = reinterpret_cast<const vec4*>(g);
+  const long long first = block * 256 + threadIdx.x, step = blocks * 256;
+  for (long long i = first; i < n4; i += step) {
+    const vec4 v = g4[i];
+    look(v.x); look(v.y); look(v.z); look(v.w);
+  }
+  for (long long i = 4 * n4 + first; i < n; i += step) look(g[i]);
+  return (__syncthreads_or((int)(word & kBadEntry)) ? kBadEntry : 0u) | (__syncthreads_or((int)(word & kNonZeroEntry)) ? kNonZeroEntry : 0u);
+}
+
+// First launch: `per_sample` blocks for each of n samples, then the rest of the grid for the upstream's gn entries.
+// maxima[sample * per_sample + block]: the largest weight as float bits (TGV.cu:2516-2523); checks[block]: upstream_word().
+__global__ __launch_bounds__(256) void tgv_survey(const float* __restrict__ dx, const float* __restrict__ dy, int n, int H, int W,
+                                                  int per_sample, unsigned int* __restrict__ maxima, const float* __restrict__ g,
+                                                  long long gn, unsigned int* __restrict__ checks) {
+  const int sample = blockIdx.x / per_sample;
+  if (sample >= n) {
+    const int block = blockIdx.x - n * per_sample;
+    const unsigned int word = upstream_word(g, gn, block, gridDim.x - n * per_sample);
+    if (threadIdx.x == 0) checks[block] = word;
+    return;
+  }
+  const size_t at = (size_t)sample * 2 * H * W;
+  const int across = (W + 63) / 64, tiles = across * ((H + 7) / 8);  // a wavefront two rows of 64 pixels
+  // non-negative floats order like their bit patterns; anything else (negative, NaN) never wins
+  // against the 32.0f start value in the reference's std::max either
+  unsigned int bits = __float_as_uint((float)(fmax(12., 8. * (double)kBeta) + 0.000001));
+  for (int tile = blockIdx.x - sample * per_sample; tile < tiles; tile += per_sample) {
+    const int row = tile / across, w = (tile - row * across) * 64 + (threadIdx.x & 63), h = row * 8 + (threadIdx.x >> 6);
+    const float v0 = lipschitz_weight(dx + at, dy + at, h, w, H, W), v1 = lipschitz_weight(dx + at, dy + at, h + 4, w, H, W);
+    const unsigned int b0 = (w < W && h < H && v0 > 0.f) ? __float_as_uint(v0) : 0u;
+    const unsigned int b1 = (w < W && h + 4 < H && v1 > 0.f) ? __float_as_uint(v1) : 0u;
+    bits = b0 > bits ? b0 : bits;
+    bits = b1 > bits ? b1 : bits;
+  }
+  bits = block_max(bits);
+  if (threadIdx.x == 0) maxima[blockIdx.x] = bits;
 }
 
 __device__ __forceinline__ double lipschitz_from_bits(unsigned int bits) {
@@ -120,21 +167,56 @@ __device__ __forceinline__ double lipschitz_from_bits(unsigned int bits) {
   return (double)oneL;                           // TGV.cu:2527: double L = oneL
 }
 
-// L-scaled private copies of the four weight fields (TGV.cu:2495-2499,2528-2531): (n,H,W) each.
-__global__ __launch_bounds__(256) void tgv_scale_kernel(const float* __restrict__ dx, const float* __restrict__ dy,
-                                                        const unsigned int* __restrict__ maxbits, float* __restrict__ wx,
-                                                        float* __restrict__ wy, float* __restrict__ bx,
-                                                        float* __restrict__ by, double* __restrict__ Ls, long long HW,
-                                                        long long total) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const long long s = i / HW, p = i - s * HW;
-  const double L = lipschitz_from_bits(maxbits[s]);
+// Second launch: `blocks` blocks for each of n samples store the L-scaled private copies of the four weight fields
+// (TGV.cu:2495-2499,2528-2531), (n,H,W) each; the rest of the grid, in a backward pass, decides on the upstream gradient.
+// What the check decides (TGV.cu:2698-2703) is kept on the device: an upstream gradient with a non-finite entry, or zero
+// everywhere, is scrubbed in the caller's tensor; the verdict is latched in the guard's state, where the guard's decision and the
+// kernels that store the outputs read it (zeros out, running means and run count untouched).  The host never learns it and
+// never waits for it.  The guard's statistics of the previous backward pass are cleared on the way.
+__global__ __launch_bounds__(256) void tgv_prepare(const float* __restrict__ dx, const float* __restrict__ dy, int n, long long HW, int blocks,
+                                                   const unsigned int* __restrict__ maxima, int per_sample, float* __restrict__ wx,
+                                                   float* __restrict__ wy, float* __restrict__ bx, float* __restrict__ by,
+                                                   double* __restrict__ Ls, float* __restrict__ g, long long gn,
+                                                   const unsigned int* __restrict__ checks, int nchecks, GuardState* __restrict__ gs) {
+  const int s = blockIdx.x / blocks;
+  if (s >= n) {
+    const long long block = blockIdx.x - n * blocks, nblocks = gridDim.x - n * blocks;
+    unsigned int word = 0;
+    for (int i = threadIdx.x; i < nchecks; i += 256) word |= checks[i];
+    const bool bad = __syncthreads_or((int)(word & kBadEntry)) || !__syncthreads_or((int)(word & kNonZeroEntry));
+    if (block == 0 && threadIdx.x == 0) {
+      gs->upstream_bad = bad ? 1u : 0u;
+      if (bad) gs->skipped += 1u;
+    }
+    if (block == 0) guard_clear(gs);
+    if (!bad) return;
+    for (long long i = block * 256 + threadIdx.x; i < gn; i += nblocks * 256) {
+      const float v = g[i];
+      if (!finite_value(v)) g[i] = 0.f;
+    }
+    return;
+  }
+  const long long p = (long long)(blockIdx.x - s * blocks) * 256 + threadIdx.x, i = s * HW + p;
+  const bool inside = p < HW;
+  float x0 = 0.f, y0 = 0.f, x1 = 0.f, y1 = 0.f;  // (in flight while the maximum is found)
+  if (inside) {
+    const float* __restrict__ sx = dx + s * 2 * HW + p;
+    const float* __restrict__ sy = dy + s * 2 * HW + p;
+    x0 = sx[0]; y0 = sy[0]; x1 = sx[HW]; y1 = sy[HW];
+  }
+  unsigned int bits = 0;
+#pragma unroll 8
+  for (int k = threadIdx.x; k < per_sample; k += 256) {
+    const unsigned int o = maxima[(long long)s * per_sample + k];
+    bits = o > bits ? o : bits;
+  }
+  const double L = lipschitz_from_bits(block_max(bits));
+  if (!inside) return;
   if (p == 0) Ls[s] = L;
-  wx[i] = (float)(L * (double)dx[s * 2 * HW + p]);
-  wy[i] = (float)(L * (double)dy[s * 2 * HW + p]);
-  bx[i] = (float)(L * (double)dx[s * 2 * HW + HW + p]);
-  by[i] = (float)(L * (double)dy[s * 2 * HW + HW + p]);
+  wx[i] = (float)(L * (double)x0);
+  wy[i] = (float)(L * (double)y0);
+  bx[i] = (float)(L * (double)x1);
+  by[i] = (float)(L * (double)y1);
 }
 
 // Prox adjoint + confidence / rhs gradient: TGV.cu:592-612, 1418-1442 (and 166-182 for the first step).
@@ -376,57 +458,6 @@ __global__ __launch_bounds__(BX* BY) void tgv_adjoint_iter0(
   gwy_[smp * 2 * HW + HW + p] = gwy1;
 }
 
-// Upstream check (TGV.cu:2686-2703): counts[0] = non-finite entries, counts[1] != 0 if any finite entry is non-zero.
-// One atomic per block and only for non-finite entries; the non-zero flag is a plain store of the same value from
-// whichever blocks see one (a counter bumped by every block of the launch would queue up at the memory side).
-__global__ __launch_bounds__(256) void tgv_upstream_check(const float* __restrict__ g, long long n,
-                                                          unsigned int* __restrict__ counts) {
-  typedef float vec4 __attribute__((ext_vector_type(4)));
-  unsigned int bad = 0, nz = 0;
-  auto look = [&](float v) {
-    if (!finite_value(v)) bad++;
-    else if (v != 0.f) nz++;
-  };
-  const long long n4 = ((reinterpret_cast<uintptr_t>(g) & 15) == 0) ? (n >> 2) : 0;  // whole 16-byte groups
-  const vec4* __restrict__ g4 = reinterpret_cast<const vec4*>(g);
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (long long)gridDim.x * blockDim.x) {
-    const vec4 v = g4[i];
-    look(v.x); look(v.y); look(v.z); look(v.w);
-  }
-  for (long long i = 4 * n4 + (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    look(g[i]);
-  bad = wave_sum_u(bad);
-  nz = wave_sum_u(nz);
-  __shared__ unsigned int s_bad[4], s_nz[4];
-  if ((threadIdx.x & 63) == 0) { s_bad[threadIdx.x >> 6] = bad; s_nz[threadIdx.x >> 6] = nz; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    bad = s_bad[0] + s_bad[1] + s_bad[2] + s_bad[3];
-    nz = s_nz[0] + s_nz[1] + s_nz[2] + s_nz[3];
-    if (bad) atomicAdd(&counts[0], bad);
-    if (nz) counts[1] = 1u;
-  }
-}
-
-// What the upstream check decides (TGV.cu:2698-2703), kept on the device: an upstream gradient with a non-finite entry,
-// or zero everywhere, is scrubbed in the caller's tensor; the verdict is latched in the guard's state, where the
-// guard's decision and the kernels that store the outputs read it (zeros out, running means and run count untouched).
-// The host never learns it and never waits for it.
-__global__ __launch_bounds__(256) void tgv_upstream_verdict(float* __restrict__ g, long long n,
-                                                            const unsigned int* __restrict__ counts,
-                                                            GuardState* __restrict__ gs) {
-  const bool bad = counts[0] != 0u || counts[1] == 0u;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    gs->upstream_bad = bad ? 1u : 0u;
-    if (bad) gs->skipped += 1u;
-  }
-  if (!bad) return;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const float v = g[i];
-    if (!finite_value(v)) g[i] = 0.f;
-  }
-}
-
 // The guard on the gradient wrt the starting point inspects only the u block (TGV.cu:3014-3021):
 // gather the u blocks of all samples into one contiguous tensor ...
 __global__ __launch_bounds__(256) void tgv_gather_u(const float* __restrict__ src, float* __restrict__ dst,
@@ -437,28 +468,42 @@ __global__ __launch_bounds__(256) void tgv_gather_u(const float* __restrict__ sr
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < CHW; i += (long long)gridDim.x * blockDim.x)
     dp[i] = sp[i];
 }
-// ... and apply its verdict to the u blocks only; v1 / v2 gradients pass through (TGV.cu:3047).
-__global__ __launch_bounds__(256) void tgv_finalize_init(const float* __restrict__ src, float* __restrict__ out,
-                                                         long long CHW, const GuardState* __restrict__ gs, GuardParams p) {
-  // grid (blocks, n, 3): blockIdx.y is the sample, blockIdx.z the variable (0 = u)
-  const long long base = ((long long)blockIdx.y * 3 + blockIdx.z) * CHW;
-  const float* __restrict__ sp = src + base;
-  float* __restrict__ op = out + base;
-  const bool is_u = blockIdx.z == 0;
+// ... and apply its verdict to the u blocks only; v1 / v2 gradients pass through (TGV.cu:3047).  The other four gradients go out in
+// the same launch: grid (blocks, 7), blockIdx.y < 4 as finalize_many, above that a third each of gi's 3 * part entries.
+__global__ __launch_bounds__(256) void tgv_finalize_many(FinalizeJobs jobs, const float* __restrict__ src, float* __restrict__ out,
+                                                         long long part, long long CHW, const GuardState* __restrict__ gs,
+                                                         GuardParams p, float global_mult) {
+  const int k = blockIdx.y;
+  if (k < 4) {
+    if (gs->upstream_bad) finalize_zero(jobs.out[k], jobs.n[k]);
+    else finalize_total(jobs, k, gs, p, global_mult);
+    return;
+  }
+  const long long first = (k - 4) * part;
   if (gs->upstream_bad) {  // a refused upstream gradient: zeros (TGV.cu:2698-2703)
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < CHW; i += (long long)gridDim.x * blockDim.x) op[i] = 0.f;
+    finalize_zero(out + first, part);
     return;
   }
   const double mult = gs->scale[4];
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < CHW; i += (long long)gridDim.x * blockDim.x) {
-    float v = sp[i];
+  const bool small = 3 * part < (1ll << 32);
+  for (long long i = first + (long long)blockIdx.x * blockDim.x + threadIdx.x; i < first + part; i += (long long)gridDim.x * blockDim.x) {
+    float v = src[i];
+    const bool is_u = (small ? (unsigned)i / (unsigned)CHW % 3u : (unsigned)(i / CHW % 3)) == 0u;
     if (is_u) {
       v = guard_limit(v, p);
       if (mult != 1.0) v = (mult == 0.0) ? 0.f : (float)((double)v * mult);
     }
-    op[i] = v;
+    out[i] = v;
   }
 }
+
+// Blocks of tgv_survey: per sample, enough to fill the chip but few enough for every block of tgv_prepare to read their words
+// (with 65535 samples the grid stays below 2^32 threads); for the upstream's entries.
+int survey_blocks(int n, int h, int w) {
+  const long long tiles = (long long)((w + 63) / 64) * ((h + 7) / 8);
+  return (int)std::min<long long>(tiles, std::max(n > 1024 ? 64 : 256, 1024 / n));
+}
+int check_blocks(long long entries) { return std::min(grid_stride(entries / 4 + 1), 1024); }
 
 // -------------------------------------------------------------------------------------------------
 // per-id state (idStructBs, TGVInpaintFista.h:7-50)
@@ -499,8 +544,8 @@ struct Slot {
   // S3 = n*3*ic*ih*iw floats (state), F = n*ic*ih*iw, P = n*ih*iw
   float *wx = nullptr, *wy = nullptr, *bx = nullptr, *by = nullptr;  // L-scaled weights, P each
   double* Ls = nullptr;                                              // per-sample L
-  unsigned int* maxbits = nullptr;                                   // per-sample Lipschitz bound (float bits)
-  unsigned int* counts = nullptr;                                    // upstream check
+  unsigned int* maxima = nullptr;                                    // Lipschitz bounds, per block (float bits)
+  unsigned int* checks = nullptr;                                    // upstream check, per block
   float *ypp[2] = {nullptr, nullptr}, *xpp[2] = {nullptr, nullptr}, *ckpt_y = nullptr, *ckpt_x = nullptr, *x05 = nullptr;
   float *g05[2] = {nullptr, nullptr}, *gxk[2] = {nullptr, nullptr}, *gi_u = nullptr, *gx_final = nullptr;
   // per-segment fp32 accumulators, double-buffered: a strip-kernel step reads one set and writes the other
@@ -573,7 +618,7 @@ int prepare_slot(Slot& s, int n, int ic, int ih, int iw, int its, int keep_mode,
   need += Arena::padded(P, 4) * (4 + 2) + Arena::padded(2 * P, 4) * 4;
   need += Arena::padded(P, 8) + Arena::padded(2 * P, 8) * 2;
   need += Arena::padded(P * nck, 4) + Arena::padded(2 * P * nck, 4) * 2 + Arena::padded(F * nck, 4);
-  need += Arena::padded((size_t)n, 8) + Arena::padded((size_t)n, 4) + Arena::padded(2, 4);
+  need += Arena::padded((size_t)n, 8) + Arena::padded((size_t)n * survey_blocks(n, ih, iw), 4) + Arena::padded(check_blocks(S3), 4);
   need += Arena::padded(std::max(F, 2 * P), 4);  // the field of zeros
   need += Arena::padded(1, sizeof(GuardState));
   rc = s.arena.reserve(need, g_allocator, stream);
@@ -581,8 +626,8 @@ int prepare_slot(Slot& s, int n, int ic, int ih, int iw, int its, int keep_mode,
   Arena& a = s.arena;
   s.wx = a.take<float>(P); s.wy = a.take<float>(P); s.bx = a.take<float>(P); s.by = a.take<float>(P);
   s.Ls = a.take<double>((size_t)n);
-  s.maxbits = a.take<unsigned int>((size_t)n);
-  s.counts = a.take<unsigned int>(2);
+  s.maxima = a.take<unsigned int>((size_t)n * survey_blocks(n, ih, iw));
+  s.checks = a.take<unsigned int>(check_blocks(S3));
   s.ypp[0] = a.take<float>(S3); s.ypp[1] = a.take<float>(S3);
   s.xpp[0] = a.take<float>(S3); s.xpp[1] = a.take<float>(S3);
   s.ckpt_y = a.take<float>(S3 * nck); s.ckpt_x = a.take<float>(S3 * nck);
@@ -640,15 +685,15 @@ int check_common(const void* const* ptrs, int nptrs, int n, int ic, int ih, int 
 }
 
 // Lipschitz reduction + scaled weight copies for the weights of this call (forward and backward both
-// redo it, TGV.cu:2513-2531 and 2667-2679).
-void scale_weights(const Slot& s, hipStream_t stream, const float* dx, const float* dy, bool clear_counts = false) {
-  const long long P = (long long)plane_count(s), HW = (long long)s.ih * s.iw;
-  hipLaunchKernelGGL(tgv_lipschitz_init, dim3((s.n + 255) / 256), dim3(256), 0, stream, s.maxbits, s.n,
-                     clear_counts ? s.counts : nullptr);
-  hipLaunchKernelGGL(tgv_lipschitz_kernel, dim3((s.iw + BX - 1) / BX, (s.ih + BY - 1) / BY, s.n), dim3(BX, BY), 0, stream,
-                     dx, dy, s.ih, s.iw, s.maxbits);
-  hipLaunchKernelGGL(tgv_scale_kernel, dim3(grid1d(P)), dim3(256), 0, stream, dx, dy, s.maxbits, s.wx, s.wy, s.bx, s.by,
-                     s.Ls, HW, P);
+// redo it, TGV.cu:2513-2531 and 2667-2679), and in a backward pass the check of its upstream gradient.
+void scale_weights(const Slot& s, hipStream_t stream, const float* dx, const float* dy, float* gin = nullptr) {
+  const long long HW = (long long)s.ih * s.iw, S3 = (long long)state_count(s);
+  const int per_sample = survey_blocks(s.n, s.ih, s.iw), blocks = (int)((HW + 255) / 256);
+  const int nchecks = gin ? check_blocks(S3) : 0, scrubbers = gin ? std::min(grid_stride(S3), 1024) : 0;
+  hipLaunchKernelGGL(tgv_survey, dim3((unsigned)(s.n * per_sample + nchecks)), dim3(256), 0, stream, dx, dy, s.n, s.ih, s.iw, per_sample,
+                     s.maxima, gin, S3, s.checks);
+  hipLaunchKernelGGL(tgv_prepare, dim3((unsigned)(s.n * blocks + scrubbers)), dim3(256), 0, stream, dx, dy, s.n, HW, blocks, s.maxima,
+                     per_sample, s.wx, s.wy, s.bx, s.by, s.Ls, gin, S3, s.checks, nchecks, s.guard);
 }
 
 // -------------------------------------------------------------------------------------------------
@@ -1199,14 +1244,11 @@ int tgvinpaint_backward(const float* dx, const float* dy, const float* c, const 
   const int gS = grid_stride((long long)S3), gF = grid_stride((long long)F),
             g2P = grid_stride((long long)(2 * P));
 
-  // (the first of its launches also clears the two words of the upstream check)
-  scale_weights(s, stream, dx, dy, true);
   // Upstream check (TGV.cu:2686-2703): any non-finite entry, or an upstream that is zero everywhere, returns
   // all-zero gradients, scrubs the caller's tensor and leaves `run` and the running means alone.  The verdict stays
   // on the device: the sweep below runs either way (on the scrubbed tensor; its kernels address nothing by value),
   // the guard's decision and the kernels that store the outputs read the verdict.  No host wait.
-  hipLaunchKernelGGL(tgv_upstream_check, dim3(std::min(grid_stride((long long)S3 / 4 + 1), 2048)), dim3(256), 0, stream, gin, (long long)S3, s.counts);
-  hipLaunchKernelGGL(tgv_upstream_verdict, dim3(std::min(gS, 1024)), dim3(256), 0, stream, gin, (long long)S3, s.counts, s.guard);
+  scale_weights(s, stream, dx, dy, gin);
   // The strip kernels keep one fp32 record of the accumulators per segment; the records are added into the fp64
   // totals after the last segment, in the reference's order (TGV.cu:2944 flushes after every segment: same bits,
   // but the totals are not read and rewritten once per segment).
@@ -1414,8 +1456,8 @@ int tgvinpaint_backward(const float* dx, const float* dy, const float* c, const 
     hipLaunchKernelGGL(flush_kernel, dim3(g2P), dim3(256), 0, stream, s.acc_gy[a], s.tot_gy, (long long)(2 * P));
   }
   // output guard on the device (TGV.cu:2990-3021), then scale and store (TGV.cu:3024-3050)
-  hipLaunchKernelGGL(guard_clear_kernel, dim3(1), dim3(64), 0, stream, s.guard);
-  {
+  // (one sample's u block lies in one piece already)
+  if (n > 1) {
     const long long CHW = (long long)ic * ih * iw;
     hipLaunchKernelGGL(tgv_gather_u, dim3(std::min(grid_stride(CHW), 1024), n), dim3(256), 0, stream, gi_src, s.gi_u, CHW);
   }
@@ -1424,7 +1466,7 @@ int tgvinpaint_backward(const float* dx, const float* dy, const float* c, const 
   GuardJobs jobs;
   long long longest = 0;
   for (int k = 0; k < 5; k++) {
-    jobs.ptr[k] = k < 4 ? (const void*)tots[k] : (const void*)s.gi_u;
+    jobs.ptr[k] = k < 4 ? (const void*)tots[k] : n > 1 ? (const void*)s.gi_u : (const void*)gi_src;
     jobs.n[k] = cnts[k];
     jobs.is_f32[k] = k == 4;
     longest = std::max(longest, cnts[k]);
@@ -1443,12 +1485,8 @@ int tgvinpaint_backward(const float* dx, const float* dy, const float* c, const 
     fin.chain_per_sample[k] = weights ? (const double*)s.Ls : nullptr;
     fin.per_sample[k] = weights ? HW2 : 1;
   }
-  hipLaunchKernelGGL(finalize_many, dim3(g2P > gF ? g2P : gF, 4), dim3(256), 0, stream, fin, s.guard, kGuard, corr ? 1.f : kGlobalGMult);
-  {
-    const long long CHW = (long long)ic * ih * iw;
-    hipLaunchKernelGGL(tgv_finalize_init, dim3(std::min(grid_stride(CHW), 1024), n, 3), dim3(256), 0, stream, gi_src, gi, CHW,
-                       s.guard, kGuard);
-  }
+  hipLaunchKernelGGL(tgv_finalize_many, dim3(std::max(g2P, gF), 7), dim3(256), 0, stream, fin, gi_src, gi, (long long)F,
+                     (long long)ic * ih * iw, s.guard, kGuard, corr ? 1.f : kGlobalGMult);
   INPAINT_HIP(hipGetLastError());
   if (knobs().stats_every > 0) {  // TGV.cu:2996: run % 75 == 0, with the run count the reference would hold
     unsigned int skipped = 0;
