@@ -1,25 +1,75 @@
 """One H x W x C image as the layers' kernels take it: planes (1,C,H,W).  Used inside the modules' autograd nodes, so that a module
 is one node and not a dozen: around a layer on a small image the nodes of the permutations took as long as the layer's own
 launches (1 x 2 x 64 x 128, 20 iterations, forward + backward: 299 us with them, 243 without)."""
+import ctypes
+
+import torch
+
+from ._lib import device_of, lib
+
+# Three images or more of this many pixels change their layout in one launch.  Setting it up takes some 20 us of host time more than
+# torch's copies, a launch each, and saves 5 to 12 us of GPU time (us, torch's copies / one launch, 20 iterations):
+#   TGV  1 channel  1 x 375 x 1241  inference 105 / 96, training 415 / 390;  320 x 960  84 / 80, 355 / 392;  240 x 640  67 / 71, 346 / 386
+#   TGV  2 channels 1 x 375 x 1241  inference 151 / 138, training 642 / 607;  320 x 960  111 / 104, 485 / 460;  240 x 640  87 / 79, 367 / 402
+#   TV   2 channels (two images)    1 x 375 x 1241  inference 78 / 75, training 340 / 378
+_LAUNCH_PIXELS, _LAUNCH_IMAGES = 1 << 18, 3
+_MAX_IMAGES, _MAX_CHANNELS = 8, 16  # images per launch; more channels than that are left to torch's copies
 
 
-def planes(image):
-    """(H,W,C) -> contiguous (1,C,H,W); no copy for a single channel or a view of planes."""
-    return image.permute(2, 0, 1).unsqueeze(0).contiguous()
+def _move(fn, sources, targets, images):
+    """One launch: sources[i] -> targets[i]; images: the sides of the pairs that are H x W x C."""
+    n, (h, w, _) = len(images), images[0].shape
+    pointers = ctypes.c_void_p * n
+    strides = (ctypes.c_longlong * (3 * n))(*[s for t in images for s in t.stride()])
+    device = images[0].device
+    with device_of(images[0]):
+        rc = fn(pointers(*[t.data_ptr() for t in sources]), pointers(*[t.data_ptr() for t in targets]),
+                (ctypes.c_int * n)(*[t.shape[2] for t in images]), strides, n, h, w,
+                ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream))
+    if rc:
+        raise RuntimeError("layout copy failed: %s" % lib.layout_last_error().decode("utf-8", "replace"))
 
 
-def image(planes):
-    """(1,C,H,W) -> contiguous (H,W,C); no copy for a single channel."""
-    return planes.squeeze(0).permute(1, 2, 0).contiguous()
+def _movable(images):
+    first = images[0]
+    return (first.is_cuda and first.shape[0] * first.shape[1] >= _LAUNCH_PIXELS
+            and all(t.dtype == torch.float32 and t.device == first.device and t.shape[:2] == first.shape[:2]
+                    and 1 <= t.shape[2] <= _MAX_CHANNELS for t in images))
+
+
+def planes(*images):
+    """(H,W,C) images -> contiguous (1,C,H,W) tensors; no copy of a single channel or a view of planes."""
+    views = [t.permute(2, 0, 1).unsqueeze(0) for t in images]
+    if images[0].numel() >= _LAUNCH_PIXELS:
+        todo = [i for i, v in enumerate(views) if not v.is_contiguous()]
+        if _LAUNCH_IMAGES <= len(todo) <= _MAX_IMAGES and _movable([images[i] for i in todo]):
+            for i in todo:
+                views[i] = torch.empty(views[i].shape, dtype=torch.float32, device=images[i].device)
+            _move(lib.layout_to_planes, [images[i] for i in todo], [views[i] for i in todo], [images[i] for i in todo])
+    return [v.contiguous() for v in views]
+
+
+def images(tensors):
+    """(1,C,H,W) planes -> contiguous (H,W,C) images; no copy of a single channel."""
+    views = [t.squeeze(0).permute(1, 2, 0) for t in tensors]
+    if views and views[0].numel() >= _LAUNCH_PIXELS:
+        todo = [i for i, v in enumerate(views) if not v.is_contiguous()]
+        if (_LAUNCH_IMAGES <= len(todo) <= _MAX_IMAGES and _movable([views[i] for i in todo])
+                and all(tensors[i].is_contiguous() for i in todo)):
+            for i in todo:
+                views[i] = torch.empty(views[i].shape, dtype=torch.float32, device=views[i].device)
+            _move(lib.layout_to_images, [tensors[i] for i in todo], [views[i] for i in todo], [views[i] for i in todo])
+    return [v.contiguous() for v in views]
 
 
 def result(planes):
-    """image() of a tensor the caller has just made and gives up: never a view, which autograd would not let a program change in
-    place as the output of a node."""
+    """The image of planes that the caller has just made and gives up: never a view, which autograd would not let a program change
+    in place as the output of a node."""
     _, c, h, w = planes.shape
-    return planes.resize_(h, w, 1) if c == 1 else image(planes)
+    return planes.resize_(h, w, 1) if c == 1 else planes.squeeze(0).permute(1, 2, 0).contiguous()
 
 
-def images(gradients, wanted):
+def gradients(tensors, wanted):
     """The gradients of a node's inputs as images, None for inputs nobody asked one for."""
-    return tuple(image(g) if want else None for g, want in zip(gradients, wanted))
+    done = iter(images([t for t, want in zip(tensors, wanted) if want]))
+    return tuple(next(done) if want else None for _, want in zip(tensors, wanted))

@@ -5,7 +5,7 @@ import torch
 from torch import nn
 from torch.autograd import Function
 
-from .._image import images, planes, result
+from .._image import gradients, planes, result
 from . import tvInpaint_cuda_ext
 
 
@@ -38,8 +38,7 @@ class _TVInpaintImage(Function):
 
     @staticmethod
     def forward(ctx, dx, dy, dc, db, di, its, pid):
-        (sol,) = tvInpaint_cuda_ext.forward(planes(dx), planes(dy), planes(dc), planes(db), planes(di), its, pid,
-                                           keep=None if any(ctx.needs_input_grad[:5]) else 0)
+        (sol,) = tvInpaint_cuda_ext.forward(*planes(dx, dy, dc, db, di), its, pid, keep=None if any(ctx.needs_input_grad[:5]) else 0)
         ctx.its, ctx.pid = int(its), int(pid)
         ctx.save_for_backward(dx, dy, dc, db)
         return result(sol)
@@ -47,8 +46,8 @@ class _TVInpaintImage(Function):
     @staticmethod
     def backward(ctx, grad_sol):
         dx, dy, dc, db = ctx.saved_tensors
-        gradients = tvInpaint_cuda_ext.backward(planes(grad_sol), planes(dx), planes(dy), planes(dc), planes(db), ctx.its, ctx.pid)
-        return images(gradients, ctx.needs_input_grad) + (None, None)
+        outputs = tvInpaint_cuda_ext.backward(*planes(grad_sol, dx, dy, dc, db), ctx.its, ctx.pid)
+        return gradients(outputs, ctx.needs_input_grad) + (None, None)
 
 
 class TVInpaint(nn.Module):
