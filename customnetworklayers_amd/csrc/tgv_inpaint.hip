@@ -62,7 +62,7 @@ __device__ __forceinline__ float clampT(const float* f, int h, int w, int H, int
 // On small images a pass is bound by its launches: with kernels of their own for clearing, filling and using the words a backward
 // pass began with 5 launches and a forward pass with 3, and a backward pass ended with 3 more than now (the guard's statistics
 // cleared, one sample's u block copied, gi stored apart from the other gradients).  Forward + backward of 1 x 1 x 61 x 97, 30
-// iterations: 361 -> 330 us.  At 1 x 1 x 375 x 1241: 16.1 us in the three launches before, 10.5 in these two (tgv_survey 4.9, with a
+// iterations: 361 -> 330 us.  At 1 x 2 x 375 x 1241: 16.1 us in the three launches before, 10.5 in these two (tgv_survey 4.9, with a
 // row per wavefront and loads under conditions 8.9).
 // -------------------------------------------------------------------------------------------------
 __device__ __forceinline__ unsigned int block_max(unsigned int v) {  // blocks of 256 threads

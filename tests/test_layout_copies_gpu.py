@@ -18,7 +18,7 @@ LAYOUTS = ("contiguous", "planes", "wide", "deep", "transposed")
 
 def image(h, w, c, layout, seed):
     g = torch.Generator(device="cuda").manual_seed(seed)
-    t = torch.randn((h, w, c), generator=g, device="cuda")
+    t = torch.randn((h, w, c), generator=g, device="cuda", dtype=torch.float32)
     if layout == "planes":
         return t.permute(2, 0, 1).contiguous().permute(1, 2, 0)
     if layout == "wide":
@@ -49,8 +49,8 @@ def test_images_of_two_values_many_times():
     from customnetworklayers_amd import _image
 
     for k in range(300):
-        a, b = torch.randn(1, 1, 2, device="cuda"), torch.randn(1, 2, 1, device="cuda")
-        c = torch.randn(1, 2, 2, device="cuda")
+        a, b = torch.randn(1, 1, 2, device="cuda", dtype=torch.float32), torch.randn(1, 2, 1, device="cuda", dtype=torch.float32)
+        c = torch.randn(1, 2, 2, device="cuda", dtype=torch.float32)
         for given in ([a], [b], [c], [a, b[:, :1], c[:, :1]]):
             there = _image.planes(*given)
             assert all(torch.equal(t, g.permute(2, 0, 1).unsqueeze(0)) for t, g in zip(there, given))
@@ -61,7 +61,7 @@ def test_result_is_no_view():
     from customnetworklayers_amd import _image
 
     for c in (1, 3):
-        t = torch.randn(1, c, 5, 7, device="cuda")
+        t = torch.randn(1, c, 5, 7, device="cuda", dtype=torch.float32)
         want = t.clone().squeeze(0).permute(1, 2, 0)
         got = _image.result(t)
         assert got._base is None and got.is_contiguous() and torch.equal(got, want)
