@@ -94,4 +94,4 @@ def test_saved_errors(med):
     with pytest.raises(TypeError):
         med.backward(g, v, saved.double())
     with pytest.raises(ValueError):
-        med.forward_saving(torch.zeros(1, 2, 2, 256, device="cuda"))
+        med.forward_saving(torch.zeros(1, 2, 2, 256, dtype=torch.float32, device="cuda"))
