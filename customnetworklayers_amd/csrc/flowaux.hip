@@ -16,11 +16,11 @@
 //    overlaps are served by the vector L1.  HBM sees every feature once: (2C+5) floats per pixel
 //    forward, (5C+5) backward (the scatter reads and writes its target).
 //  * median: the histogram bins are innermost in memory, so a lane that walked its own pixel's bins
-//    would touch a new cache line per step.  Instead a wavefront stages 64 pixels x 32 bins through
-//    LDS with full-line loads (32 lanes x 4 B = one 128-byte line of one pixel), and each lane then
-//    walks its pixel's bins from LDS in the reference's sequential order (row pitch 33 words: no
-//    bank conflicts).  The forward pass stops at the chunk in which the last pixel of the block
-//    found its median.
+//    would touch a new cache line per step.  The histograms of 64 consecutive pixels are one
+//    contiguous run: a wavefront brings it into LDS with full-line loads and each lane walks its
+//    pixel's bins there in the reference's sequential order.  Above 255 bins the run comes in pieces
+//    of 32 bins (row pitch 33 words: no bank conflicts), and the forward pass stops at the piece in
+//    which the last pixel of the block found its median.
 #include <hip/hip_runtime.h>
 
 #include <climits>
