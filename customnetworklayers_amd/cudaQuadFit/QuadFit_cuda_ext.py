@@ -129,10 +129,15 @@ def takes_image(feat0, feat1, flow):
 
 
 def _flow_strides(flow):
-    """flow with its pixels a fixed distance apart, that distance and the one between its channels"""
-    if flow.stride(0) != flow.shape[1] * flow.stride(1) or min(flow.stride()) < 1:
-        flow = flow.contiguous()
-    return flow, flow.stride(1), flow.stride(2)
+    """flow with its pixels a fixed distance apart, that distance and the one between its channels.  (The stride of a dimension of
+    one element says nothing: a single column's pixels lie a row apart, and a contiguous tensor may have any number there.)"""
+    h, w, channels = flow.shape
+    row, pixel, channel = flow.stride()
+    if w == 1:
+        pixel = row
+    if pixel < 1 or channel < 1 or (h > 1 and row != w * pixel):
+        return flow.contiguous(), channels, 1
+    return flow, pixel, channel
 
 
 def image_forward(feat0, feat1, flow, want_costs):

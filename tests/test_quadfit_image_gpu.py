@@ -68,6 +68,22 @@ def test_image_many_sources_per_position(flowaux_oracle, c):
     check(run(*(dev(t) for t in (f0, f1, flow, grad))), expected(flowaux_oracle, f0, f1, flow, grad))
 
 
+@pytest.mark.parametrize("h", [2, 5, 130])
+@pytest.mark.parametrize("layout", ["contiguous", "a batch's only column", "planes", "wider image"])
+def test_one_column(flowaux_oracle, h, layout):
+    print("case", h, layout, flush=True)
+    a = inputs(8, h, 1, 0.7)
+    f0, f1, flow, grad = (dev(t) for t in a)
+    if layout == "a batch's only column":  # (contiguous, with a stride of 3 * h between columns)
+        f0, f1, flow, grad = (t.reshape(1, h, -1).transpose(0, 1) for t in (f0, f1, flow, grad))
+        assert flow.is_contiguous() and flow.stride() == (3, 3 * h, 1)
+    if layout == "planes":
+        flow = flow.permute(2, 0, 1).contiguous().permute(1, 2, 0)
+    if layout == "wider image":
+        flow = torch.cat([flow, flow], 1)[:, :1]
+    check(run(f0.detach(), f1.detach(), flow, grad), expected(flowaux_oracle, *a))
+
+
 @pytest.mark.parametrize("layout", ["flow planes", "flow strided", "maps planes", "one map planes", "maps strided", "maps shifted", "grad strided"])
 def test_layouts_the_module_takes(flowaux_oracle, layout):
     a = inputs(8, 12, 30, 1.0)
