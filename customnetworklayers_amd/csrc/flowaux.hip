@@ -1973,8 +1973,12 @@ __global__ __launch_bounds__(64) void median_forward_run_kernel(const float* __r
       if (slot >= D4) { slot -= D4; px++; }
     }
   } else {
-    for (int i = 0; i < total; i += 256)
-      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + 4 * min((i >> 2) + lane, pieces - 1)), (LdsPtr)(tile + i), 16, 0, kReadOnce);
+    // (a load writes 16 bytes for every lane that takes part: in the last round only those with a piece, the run's end is the tile's)
+    const int whole = pieces & ~63;
+    for (int j = 0; j < whole; j += 64)
+      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + 4 * (j + lane)), (LdsPtr)(tile + 4 * j), 16, 0, kReadOnce);
+    if (whole + lane < pieces)
+      __builtin_amdgcn_global_load_lds((GlobalPtr)(src + 4 * (whole + lane)), (LdsPtr)(tile + 4 * whole), 16, 0, kReadOnce);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (RD != 4 && lane < (total & 3)) tile[4 * pieces + lane] = src[4 * pieces + lane];

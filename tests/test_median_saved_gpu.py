@@ -58,6 +58,16 @@ def test_sums_that_fall_below_one_half_again_or_are_not_numbers(med, flowaux_ora
     check(med, flowaux_oracle, vol, m["grad"])
 
 
+@pytest.mark.parametrize("d", [5, 6, 7, 33, 34, 35])
+def test_many_tiles_side_by_side_on_a_unit(med, flowaux_oracle, d):
+    # some twenty tiles of 64 pixels for every compute unit, as many as its LDS holds at once: a tile whose last load reached past
+    # its own rows would be seen in a neighbour's
+    m = workloads.median_inputs(2, 401, 413, d, seed=d, empty_fraction=0.05)
+    check(med, flowaux_oracle, m["vol"], m["grad"])
+    (plain,) = med.forward(dev(m["vol"]))
+    assert np.array_equal(plain.cpu().numpy(), flowaux_oracle.median_forward(m["vol"]))
+
+
 def test_saved_crossing_without_16_byte_alignment(med, flowaux_oracle):
     m = workloads.median_inputs(1, 9, 14, 21, seed=9)
     flat = torch.zeros(m["vol"].size + 3, dtype=torch.float32, device="cuda")
