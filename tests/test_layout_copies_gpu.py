@@ -1,5 +1,7 @@
 """The copies between an image with its channels innermost and channel planes, several images per launch: torch's permutations, bit
-for bit, at the edges of the launch (one pixel, a block of 256, one more), for every layout of the image, and repeatedly."""
+for bit, at the edges of the launch (one pixel, a block of 256, one more), for every layout of the image, and repeatedly.  planes()
+and images() launch only for views that are not contiguous, which an image of one pixel or one channel never is; launched() hands any
+image to the kernel."""
 import pytest
 import torch
 
@@ -12,6 +14,7 @@ def every_size(monkeypatch):
 
     monkeypatch.setattr(_image, "_LAUNCH_PIXELS", 1)
     monkeypatch.setattr(_image, "_LAUNCH_IMAGES", 1)
+
 
 LAYOUTS = ("contiguous", "planes", "wide", "deep", "transposed")
 
@@ -45,16 +48,36 @@ def test_images_to_planes_and_back(h, w, channels, layout):
         assert t.is_contiguous() and torch.equal(t, g)
 
 
-def test_images_of_two_values_many_times():
+def launched(given):
+    """The images through both kernels, whatever their layout: (planes, images)."""
     from customnetworklayers_amd import _image
+    from customnetworklayers_amd._lib import lib
 
+    there = [torch.full((1, t.shape[2]) + t.shape[:2], float("nan"), device="cuda", dtype=torch.float32) for t in given]
+    _image._move(lib.layout_to_planes, given, there, given)
+    back = [torch.full(t.shape, float("nan"), device="cuda", dtype=torch.float32) for t in given]
+    _image._move(lib.layout_to_images, there, back, back)
+    return there, back
+
+
+@pytest.mark.parametrize("h,w", [(1, 1), (1, 2), (2, 1), (16, 16), (1, 257), (33, 70)])
+@pytest.mark.parametrize("channels", [(1,), (2,), (1, 2, 1), (2, 2, 1, 2, 6), (1, 16, 17)])
+@pytest.mark.parametrize("layout", LAYOUTS)
+def test_kernels_on_every_image(h, w, channels, layout):
+    given = [image(h, w, c, layout, seed=i) for i, c in enumerate(channels)]
+    there, back = launched(given)
+    for t, b, g in zip(there, back, given):
+        assert torch.equal(t, g.permute(2, 0, 1).unsqueeze(0)) and torch.equal(b, g)
+
+
+def test_images_of_two_values_many_times():
     for k in range(300):
         a, b = torch.randn(1, 1, 2, device="cuda", dtype=torch.float32), torch.randn(1, 2, 1, device="cuda", dtype=torch.float32)
         c = torch.randn(1, 2, 2, device="cuda", dtype=torch.float32)
-        for given in ([a], [b], [c], [a, b[:, :1], c[:, :1]]):
-            there = _image.planes(*given)
+        for given in ([a], [b], [c], [b, c[..., :1]]):
+            there, back = launched(given)
             assert all(torch.equal(t, g.permute(2, 0, 1).unsqueeze(0)) for t, g in zip(there, given))
-            assert all(torch.equal(t, g) for t, g in zip(_image.images(there), given))
+            assert all(torch.equal(t, g) for t, g in zip(back, given))
 
 
 def test_result_is_no_view():
