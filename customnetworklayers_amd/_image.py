@@ -33,7 +33,7 @@ def _move(fn, sources, targets, images):
 def _movable(images):
     first = images[0]
     return (first.is_cuda and first.shape[0] * first.shape[1] >= _LAUNCH_PIXELS
-            and all(t.dtype == torch.float32 and t.device == first.device and t.shape[:2] == first.shape[:2]
+            and all(t.dtype == torch.float32 and not t.is_neg() and t.device == first.device and t.shape[:2] == first.shape[:2]
                     and 1 <= t.shape[2] <= _MAX_CHANNELS for t in images))
 
 

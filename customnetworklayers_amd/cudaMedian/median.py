@@ -42,7 +42,7 @@ class _MedianImage(Function):
     @staticmethod
     def backward(ctx, grad_sol):
         in_vol, saved = ctx.saved_tensors
-        (gradient,) = median_cuda_ext.backward(grad_sol[None, None].contiguous(), in_vol.unsqueeze(0).contiguous(), saved)
+        (gradient,) = median_cuda_ext.backward(grad_sol[None, None].contiguous().resolve_neg(), in_vol.unsqueeze(0).contiguous(), saved)
         return gradient[0]
 
 

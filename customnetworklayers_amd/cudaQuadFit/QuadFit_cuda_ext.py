@@ -118,11 +118,11 @@ def backward(d_iGf, featureImage0, featureImage1, flow, use_atomics=False, costs
 
 def takes_image(feat0, feat1, flow):
     """Whether image_forward / image_backward take these H x W x C maps and H x W x 3 flow as they are: both maps contiguous with
-    more than one channel innermost.  (Maps that are views of channel planes, and everything that is to be refused, go through
-    forward / backward.)"""
+    more than one channel innermost.  (Maps that are views of channel planes, views whose sign is still to be applied (is_neg), and
+    everything that is to be refused, go through forward / backward.)"""
     if not (feat0.dim() == 3 and flow.dim() == 3 and feat0.shape == feat1.shape and feat0.shape[:2] == flow.shape[:2]):
         return False
-    if not all(t.is_cuda and t.dtype == torch.float32 and t.device == flow.device for t in (feat0, feat1, flow)):
+    if not all(t.is_cuda and t.dtype == torch.float32 and t.device == flow.device and not t.is_neg() for t in (feat0, feat1, flow)):
         return False
     h, w, c = feat0.shape
     return (feat0.is_contiguous() and feat1.is_contiguous() and c > 1 and h * w > 1 and h * w * c < 2 ** 31)

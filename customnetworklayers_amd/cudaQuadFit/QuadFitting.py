@@ -42,7 +42,7 @@ class _QuadFittingImage(Function):
     @staticmethod
     def backward(ctx, grad_sol):
         feat0, feat1, flow, costs = ctx.saved_tensors
-        d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.image_backward(grad_sol.contiguous(), feat0.contiguous(), feat1.contiguous(), flow,
+        d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.image_backward(grad_sol.contiguous().resolve_neg(), feat0.contiguous(), feat1.contiguous(), flow,
                                                                costs.contiguous())
         return d_oGfeat0, d_oGfeat1, None
 

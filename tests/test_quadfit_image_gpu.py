@@ -48,6 +48,13 @@ def check(got, want):
     assert np.abs(got[2] - want[2]).max() <= SCATTER_TOL * max(np.abs(want[2]).max(), 1e-30)
 
 
+def negative_view(t):
+    """t as a view whose sign is still to be applied: the imaginary part of a conjugate."""
+    view = torch.complex(torch.zeros_like(t), -t).conj().imag
+    assert view.is_neg() and torch.equal(view.nan_to_num(), t.nan_to_num())
+    return view
+
+
 def dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
@@ -84,7 +91,8 @@ def test_one_column(flowaux_oracle, h, layout):
     check(run(f0.detach(), f1.detach(), flow, grad), expected(flowaux_oracle, *a))
 
 
-@pytest.mark.parametrize("layout", ["flow planes", "flow strided", "maps planes", "one map planes", "maps strided", "maps shifted", "grad strided"])
+@pytest.mark.parametrize("layout", ["flow planes", "flow strided", "maps planes", "one map planes", "maps strided", "maps shifted", "grad strided",
+                                    "flow negative", "one map negative", "grad negative"])
 def test_layouts_the_module_takes(flowaux_oracle, layout):
     a = inputs(8, 12, 30, 1.0)
     f0, f1, flow, grad = (dev(t) for t in a)
@@ -102,6 +110,12 @@ def test_layouts_the_module_takes(flowaux_oracle, layout):
         f0, f1 = (torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape) for t in (f0, f1))
     if layout == "grad strided":
         grad = as_planes(grad)
+    if layout == "flow negative":
+        flow = negative_view(flow)
+    if layout == "one map negative":
+        f0 = negative_view(f0)
+    if layout == "grad negative":
+        grad = negative_view(grad)
     check(run(f0.detach(), f1.detach(), flow, grad), expected(flowaux_oracle, *a))
 
 
