@@ -7,12 +7,24 @@ import torch
 
 from ._lib import device_of, lib
 
-# Three images or more of this many pixels change their layout in one launch.  Setting it up takes some 20 us of host time more than
-# torch's copies, a launch each, and saves 5 to 12 us of GPU time (us, torch's copies / one launch, 20 iterations):
-#   TGV  1 channel  1 x 375 x 1241  inference 105 / 96, training 415 / 390;  320 x 960  84 / 80, 355 / 392;  240 x 640  67 / 71, 346 / 386
-#   TGV  2 channels 1 x 375 x 1241  inference 151 / 138, training 642 / 607;  320 x 960  111 / 104, 485 / 460;  240 x 640  87 / 79, 367 / 402
-#   TV   2 channels (two images)    1 x 375 x 1241  inference 78 / 75, training 340 / 378
-_LAUNCH_PIXELS, _LAUNCH_IMAGES = 1 << 18, 3
+# Three or more images change their layout in one launch if they are large: four or more of _LAUNCH_PIXELS, three of twice that.
+# Setting a launch up takes 6 to 13 us of host time more than torch's copies, a launch each, and saves GPU time; it loses where the
+# host is what a pass waits for, which fewer iterations make more likely.  TGV, us, torch's copies / one launch:
+#   channels, pixels   inference 10   training 10   training 16   inference 100   training 100 iterations
+#   1 (three images)
+#     320 x 960            66 / 72     291 / 329                     285 / 280      1160 / 1144
+#     375 x 1241           72 / 69     292 / 328     334 / 371       347 / 340      1484 / 1463
+#     540 x 1280           84 / 77     327 / 339                     405 / 398      1851 / 1834
+#     700 x 1280           99 / 91     408 / 391     543 / 528
+#     768 x 1536          114 / 110    486 / 474                     634 / 628      2871 / 2856
+#   2 (five images, backward four)
+#     320 x 960            78 / 73     310 / 346                     390 / 384      1783 / 1760
+#     384 x 1024           82 / 76     347 / 371     473 / 449
+#     375 x 1241          106 / 93     406 / 376     545 / 511       549 / 534      2396 / 2362
+#     768 x 1536          201 / 187    783 / 754                    1157 / 1143     4876 / 4843
+#   3                      375 x 1241 inference 10 139 / 116, training 10 607 / 557;  384 x 1024 106 / 101, 511 / 494
+# (The TV layer has two such images at most.)
+_LAUNCH_PIXELS, _LAUNCH_IMAGES = 7 << 16, 3
 _MAX_IMAGES, _MAX_CHANNELS = 8, 16  # images per launch; more channels than that are left to torch's copies
 
 
@@ -32,7 +44,9 @@ def _move(fn, sources, targets, images):
 
 def _movable(images):
     first = images[0]
-    return (first.is_cuda and first.shape[0] * first.shape[1] >= _LAUNCH_PIXELS
+    if not _LAUNCH_IMAGES <= len(images) <= _MAX_IMAGES:
+        return False
+    return (first.is_cuda and first.shape[0] * first.shape[1] >= _LAUNCH_PIXELS * (2 if len(images) == 3 else 1)
             and all(t.dtype == torch.float32 and not t.is_neg() and t.device == first.device and t.shape[:2] == first.shape[:2]
                     and 1 <= t.shape[2] <= _MAX_CHANNELS for t in images))
 
@@ -42,7 +56,7 @@ def planes(*images):
     views = [t.permute(2, 0, 1).unsqueeze(0) for t in images]
     if images[0].numel() >= _LAUNCH_PIXELS:
         todo = [i for i, v in enumerate(views) if not v.is_contiguous()]
-        if _LAUNCH_IMAGES <= len(todo) <= _MAX_IMAGES and _movable([images[i] for i in todo]):
+        if todo and _movable([images[i] for i in todo]):
             for i in todo:
                 views[i] = torch.empty(views[i].shape, dtype=torch.float32, device=images[i].device)
             _move(lib.layout_to_planes, [images[i] for i in todo], [views[i] for i in todo], [images[i] for i in todo])
@@ -54,8 +68,7 @@ def images(tensors):
     views = [t.squeeze(0).permute(1, 2, 0) for t in tensors]
     if views and views[0].numel() >= _LAUNCH_PIXELS:
         todo = [i for i, v in enumerate(views) if not v.is_contiguous()]
-        if (_LAUNCH_IMAGES <= len(todo) <= _MAX_IMAGES and _movable([views[i] for i in todo])
-                and all(tensors[i].is_contiguous() for i in todo)):
+        if todo and _movable([views[i] for i in todo]) and all(tensors[i].is_contiguous() for i in todo):
             for i in todo:
                 views[i] = torch.empty(views[i].shape, dtype=torch.float32, device=views[i].device)
             _move(lib.layout_to_images, [tensors[i] for i in todo], [views[i] for i in todo], [views[i] for i in todo])

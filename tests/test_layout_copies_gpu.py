@@ -99,9 +99,10 @@ def test_large_images_as_the_modules_pass_them(monkeypatch):
     calls = []
     move = _image._move
     monkeypatch.setattr(_image, "_move", lambda *a: (calls.append(len(a[3])), move(*a)))
-    for h, w, sent in ((511, 513, []), (512, 512, [3, 3])):
+    three, four = (2, 2, 1, 1, 3), (2, 2, 1, 2, 6)  # the layer's images at one and at two channels; those of one channel are no copy
+    for h, w, channels, sent in ((1023, 896, three, []), (1024, 896, three, [3, 3]), (511, 896, four, []), (512, 896, four, [4, 4])):
         calls.clear()
-        given = [image(h, w, c, "contiguous", seed=c) for c in (2, 2, 1, 1, 3)]
+        given = [image(h, w, c, "contiguous", seed=c) for c in channels]
         there = _image.planes(*given)
         back = _image.images(there)
         assert calls == sent
