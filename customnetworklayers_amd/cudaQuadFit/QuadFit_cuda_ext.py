@@ -116,16 +116,37 @@ def backward(d_iGf, featureImage0, featureImage1, flow, use_atomics=False, costs
     return [d_oFeat0, d_oFeat1]
 
 
+def image_pays(channels, pixels, differentiated):
+    """Whether the kernels on one image with its channels innermost are the faster ones.  With fewer than eight channels they are not on
+    large images: a block's 256 lanes work through 32 channels of 64 pixels whatever the number that exists, the copies into planes and the
+    kernels there move what exists.  Copies and kernels on planes / kernels on the image, us, one image at inference:
+      channels   512 x 1024    600 x 1200    750 x 1300    900 x 1600    1600 x 2560
+          2      45 / 43       44 / 58       44 / 84       56 / 128      129 / 355
+          4      45 / 30       48 / 46       50 / 62       80 / 90       216 / 249
+          5      44 / 47       57 / 70       56 / 93       98 / 135      274 / 379
+          7      44 / 53       80 / 73       76 / 97       145 / 144     412 / 458
+          8      49 / 33       94 / 45       90 / 59       172 / 87      489 / 300
+    (below 2^19 pixels planes wait for the host, 44 us; 384 x 1248 with 2 channels 46 / 40).  Forward and backward 2 channels 241 / 223 at
+    900 x 1600, 295 / 379 at 1200 x 2000; 3 348 / 421, 4 399 / 332, 5 482 / 492, 6 561 / 515 there."""
+    if channels >= 8:
+        return True
+    if differentiated:
+        return pixels < 1 << 21 or channels not in (2, 3, 5)
+    return pixels < (7 << 17 if channels == 4 else 1 << 19)
+
+
 def takes_image(feat0, feat1, flow):
-    """Whether image_forward / image_backward take these H x W x C maps and H x W x 3 flow as they are: both maps contiguous with
-    more than one channel innermost.  (Maps that are views of channel planes, views whose sign is still to be applied (is_neg), and
-    everything that is to be refused, go through forward / backward.)"""
+    """Whether image_forward / image_backward are to take these H x W x C maps and H x W x 3 flow as they are: both maps contiguous with
+    more than one channel innermost, at a size where that pays.  (Maps that are views of channel planes, views whose sign is still to be
+    applied (is_neg), and everything that is to be refused, go through forward / backward.)"""
     if not (feat0.dim() == 3 and flow.dim() == 3 and feat0.shape == feat1.shape and feat0.shape[:2] == flow.shape[:2]):
         return False
     if not all(t.is_cuda and t.dtype == torch.float32 and t.device == flow.device and not t.is_neg() for t in (feat0, feat1, flow)):
         return False
     h, w, c = feat0.shape
-    return (feat0.is_contiguous() and feat1.is_contiguous() and c > 1 and h * w > 1 and h * w * c < 2 ** 31)
+    if not (feat0.is_contiguous() and feat1.is_contiguous() and c > 1 and h * w > 1 and h * w * c < 2 ** 31):
+        return False
+    return image_pays(c, h * w, torch.is_grad_enabled() and (feat0.requires_grad or feat1.requires_grad))
 
 
 def _flow_strides(flow):

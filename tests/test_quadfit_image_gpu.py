@@ -119,6 +119,21 @@ def test_layouts_the_module_takes(flowaux_oracle, layout):
     check(run(f0.detach(), f1.detach(), flow, grad), expected(flowaux_oracle, *a))
 
 
+@pytest.mark.parametrize("c,h,w", [(2, 512, 1023), (2, 512, 1024), (3, 512, 1024), (4, 896, 1023), (4, 896, 1024)])
+def test_few_channels_on_both_sides_of_the_rule(flowaux_oracle, c, h, w):
+    from customnetworklayers_amd import QuadFittingFromFlow
+    from customnetworklayers_amd.cudaQuadFit import QuadFit_cuda_ext as ext
+
+    a = inputs(c, h, w, 0.7)
+    f0, f1, flow, _ = (dev(t) for t in a)
+    assert ext.takes_image(f0, f1, flow) == (h * w < (7 << 17 if c == 4 else 1 << 19))
+    assert ext.takes_image(f0.requires_grad_(True), f1, flow)
+    with torch.no_grad():
+        got = QuadFittingFromFlow(torch.device("cuda:0"))(f0, f1, flow).cpu().numpy()
+    want = flowaux_oracle.quadfit_forward(*(planes(t) for t in a[:3]))[0].transpose(1, 2, 0)
+    assert np.array_equal(got, want)
+
+
 def test_image_refuses_what_the_planes_refuse():
     from customnetworklayers_amd import QuadFittingFromFlow
 
