@@ -2356,7 +2356,8 @@ int quadfit_backward_saved(const float* im0, const float* im1, const float* flow
 static int image_args(const char* name, bool pointers, int ic, int ih, int iw, long long flow_pixel_stride, long long flow_channel_stride) {
   if (!pointers) return fail(INPAINT_ERR_ARG, "%s: null pointer", name);
   if (ic < 1 || ih < 1 || iw < 1) return fail(INPAINT_ERR_ARG, "%s: bad shape %dx%dx%d", name, ih, iw, ic);
-  if ((long long)ih * iw * ic >= (1ll << 31)) return fail(INPAINT_ERR_ARG, "%s: image too large", name);
+  // (offsets into a map are 32 bits wide; a pixel has four threads, and a launch fewer than 2^32 of them)
+  if ((long long)ih * iw * ic >= (1ll << 31) || (long long)ih * iw > (1ll << 30) - 1024) return fail(INPAINT_ERR_ARG, "%s: image too large", name);
   if (flow_pixel_stride < 1 || flow_channel_stride < 1) return fail(INPAINT_ERR_ARG, "%s: bad strides of the flow", name);
   return 0;
 }

@@ -67,7 +67,7 @@ int quadfit_saving_pays(int n, int ic, int ih, int iw);
  *   flow : element (pixel p in row order, channel c) lies at p*flow_pixel_stride + c*flow_channel_stride; two channels are read
  *   costs : 5*ih*iw floats, written by the forward pass (NULL: not wanted) and read by the backward pass
  *   workspace : as for quadfit_backward(1, ih, iw), required
- * ih*iw*ic is below 2^31. */
+ * ih*iw*ic is below 2^31, ih*iw at most 2^30 - 1024. */
 int quadfit_image_forward(const float* im0, const float* im1, const float* flow, float* out, float* costs, int ic, int ih, int iw,
                           long long flow_pixel_stride, long long flow_channel_stride, void* stream);
 int quadfit_image_backward(const float* im0, const float* im1, const float* flow, const float* gin, const float* costs, float* g0,

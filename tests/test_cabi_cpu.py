@@ -73,6 +73,11 @@ def test_flow_layers_reject_bad_arguments_before_any_gpu_work():
     assert lib.medimax_forward(None, None, 1, 4, 4, 8, None) == 2
     assert lib.medimax_backward(None, None, None, 1, 4, 4, 8, None) == 2
     assert b"null pointer" in lib.flowaux_last_error()
+    at = ctypes.c_void_p(64)  # (never read: the sizes are refused first)
+    for ic, ih, iw in ((1, 1 << 15, 1 << 15), (1, 46340, 46340), (2, 1 << 15, 1 << 15), (3, 1 << 15, 1 << 15)):
+        assert lib.quadfit_image_forward(at, at, at, at, None, ic, ih, iw, 3, 1, None) == 2
+        assert lib.quadfit_image_backward(at, at, at, at, at, at, at, ic, ih, iw, 3, 1, at, 1 << 62, None) == 2
+        assert b"too large" in lib.flowaux_last_error()
     assert lib.quadfit_backward_workspace_bytes(4, 384, 1248) >= 4 * 384 * 1248 * 4 * 11
     assert lib.quadfit_backward_workspace_bytes(0, 384, 1248) == 0
 
