@@ -77,9 +77,9 @@ def images(tensors):
 
 def result(planes):
     """The image of planes that the caller has just made and gives up: never a view, which autograd would not let a program change
-    in place as the output of a node."""
+    in place as the output of a node (and not by resize_, after which a trace has lost the value)."""
     _, c, h, w = planes.shape
-    return planes.resize_(h, w, 1) if c == 1 else planes.squeeze(0).permute(1, 2, 0).contiguous()
+    return planes.as_strided_((h, w, 1), (w, 1, 1)) if c == 1 else planes.squeeze(0).permute(1, 2, 0).contiguous()
 
 
 def gradients(tensors, wanted):

@@ -37,7 +37,9 @@ class _MedianImage(Function):
             ctx.save_for_backward(in_vol, saved)
         else:
             (solution,) = median_cuda_ext.forward(in_vol.unsqueeze(0).contiguous())
-        return solution.resize_(h, w)  # (the first plane, and not as a view: it may be changed in place)
+        # (the first plane, not as a view so that it may be changed in place; the second stays behind it in the storage, as it did behind
+        # the view of both planes that the permutations gave)
+        return solution.as_strided_((h, w), (w, 1))
 
     @staticmethod
     def backward(ctx, grad_sol):

@@ -104,3 +104,20 @@ def test_median_module_gives_the_functions_numbers(d):
         assert torch.equal(g, want_grad)
         with torch.no_grad():
             assert torch.equal(Median(DEV)(given), want)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+@pytest.mark.parametrize("kind,c", [("tv", 1), ("tv", 2), ("tgv", 1), ("tgv", 2), ("median", 16), ("median", 256)])
+def test_a_trace_of_a_module_runs_on_other_values(kind, c, grad):
+    if kind == "median":
+        d = median_inputs(1, 11, 19, c, seed=c, empty_fraction=0.1)
+        layer, inputs = Median(DEV), [torch.from_numpy(d["vol"][0]).to(DEV)]
+        others = [inputs[0].flip(0).contiguous()]
+    else:
+        layer, _ = fresh(kind)
+        inputs, _ = problem(kind, c)
+        others = inputs[:3] + [0.5 * t for t in inputs[3:]]
+    traced = torch.jit.trace(layer, tuple(t.clone().requires_grad_(grad) for t in inputs), check_trace=False)
+    with torch.no_grad():
+        assert torch.equal(traced(*inputs), layer(*inputs))
+        assert torch.equal(traced(*others), layer(*others))
