@@ -1,5 +1,6 @@
 """Autograd surface of the median layer: the names, arguments and tensor layouts of the reference's
 cudaMedian/median.py (MedianFunction, Median)."""
+import torch
 from torch import nn
 from torch.autograd import Function
 
@@ -32,19 +33,23 @@ class _MedianImage(Function):
     @staticmethod
     def forward(ctx, in_vol):
         h, w, _ = in_vol.shape
-        if ctx.needs_input_grad[0]:
+        if ctx.needs_input_grad[0] and in_vol.shape[2] <= median_cuda_ext.MAX_SAVED_BINS:
             solution, saved = median_cuda_ext.forward_saving(in_vol.unsqueeze(0).contiguous())
             ctx.save_for_backward(in_vol, saved)
         else:
             (solution,) = median_cuda_ext.forward(in_vol.unsqueeze(0).contiguous())
+            ctx.save_for_backward(in_vol)
         # (the first plane, not as a view so that it may be changed in place; the second stays behind it in the storage, as it did behind
         # the view of both planes that the permutations gave)
         return solution.as_strided_((h, w), (w, 1))
 
     @staticmethod
     def backward(ctx, grad_sol):
-        in_vol, saved = ctx.saved_tensors
-        (gradient,) = median_cuda_ext.backward(grad_sol[None, None].contiguous().resolve_neg(), in_vol.unsqueeze(0).contiguous(), saved)
+        in_vol, *saved = ctx.saved_tensors
+        grad_sol = grad_sol[None, None].contiguous().resolve_neg()
+        if not saved:  # (more bins than a crossing is saved for)
+            grad_sol = torch.cat([grad_sol, torch.zeros_like(grad_sol)], 1)
+        (gradient,) = median_cuda_ext.backward(grad_sol, in_vol.unsqueeze(0).contiguous(), *saved)
         return gradient[0]
 
 
@@ -56,10 +61,7 @@ class Median(nn.Module):
     def forward(self, t_vol):
         """t_vol: H x W x D histogram per pixel.  Returns the H x W map of median positions (median.py:69-80
         drops the second output channel, the mass of the median's bin)."""
-        if t_vol.dim() == 3 and t_vol.shape[2] <= median_cuda_ext.MAX_SAVED_BINS:
-            return _MedianImage.apply(t_vol)
-        sol = MedianFunction.apply(t_vol.unsqueeze(0))
-        return sol.squeeze(0).permute(1, 2, 0)[:, :, 0]
+        return _MedianImage.apply(t_vol)
 
     def init(self):
         pass

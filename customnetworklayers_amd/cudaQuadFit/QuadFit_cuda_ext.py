@@ -154,6 +154,8 @@ def _flow_strides(flow):
     one element says nothing: a single column's pixels lie a row apart, and a contiguous tensor may have any number there.)"""
     h, w, channels = flow.shape
     row, pixel, channel = flow.stride()
+    if flow.is_neg():
+        return flow.contiguous().resolve_neg(), channels, 1
     if w == 1:
         pixel = row
     if pixel < 1 or channel < 1 or (h > 1 and row != w * pixel):
@@ -161,9 +163,22 @@ def _flow_strides(flow):
     return flow, pixel, channel
 
 
+def _check_image(feat0, feat1, flow):
+    for t, name in ((feat0, "featureImage0"), (feat1, "featureImage1")):
+        _check_input(t, name)
+    if feat0.shape != feat1.shape or feat0.dim() != 3 or flow.dim() != 3 or flow.shape[:2] != feat0.shape[:2] or flow.shape[2] < 2:
+        raise ValueError("the maps must be H x W x C, the flow H x W x 2 or more, got %s, %s and %s"
+                         % (tuple(feat0.shape), tuple(feat1.shape), tuple(flow.shape)))
+    if flow.dtype != torch.float32:
+        raise TypeError("Input/Output type to the operator must be single/float (flow is %s)" % flow.dtype)
+    if not feat0.device == feat1.device == flow.device:
+        raise RuntimeError("all tensors must live on one device")
+    return feat0.shape
+
+
 def image_forward(feat0, feat1, flow, want_costs):
-    """The fit of one image, feat0, feat1 H x W x C, flow H x W x 3 (takes_image).  Returns [H x W x 3, costs (5,H,W) or None]."""
-    h, w, c = feat0.shape
+    """The fit of one image, feat0, feat1 H x W x C contiguous, flow H x W x 3 anyhow.  Returns [H x W x 3, costs (5,H,W) or None]."""
+    h, w, c = _check_image(feat0, feat1, flow)
     flow, pixel, channel = _flow_strides(flow)
     out = torch.empty((h, w, 3), dtype=torch.float32, device=flow.device)
     costs = torch.empty((5, h, w), dtype=torch.float32, device=flow.device) if want_costs else None
@@ -177,9 +192,13 @@ def image_forward(feat0, feat1, flow, want_costs):
 
 def image_backward(d_iGf, feat0, feat1, flow, costs):
     """d_iGf: H x W x 3 gradient wrt the result, costs: the second result of image_forward.  Returns the two maps' gradients."""
-    for t, name in ((d_iGf, "d_iGf"), (feat0, "featureImage0"), (feat1, "featureImage1"), (costs, "costs")):
+    h, w, c = _check_image(feat0, feat1, flow)
+    for t, name, shape in ((d_iGf, "d_iGf", (h, w, 3)), (costs, "costs", (5, h, w))):
         _check_input(t, name)
-    h, w, c = feat0.shape
+        if tuple(t.shape) != shape:
+            raise ValueError("%s must have shape %s, got %s" % (name, shape, tuple(t.shape)))
+        if t.device != flow.device:
+            raise RuntimeError("all tensors must live on one device")
     flow, pixel, channel = _flow_strides(flow)
     g0, g1 = torch.empty_like(feat0), torch.empty_like(feat1)
     ws_bytes = lib.quadfit_backward_workspace_bytes(1, h, w)

@@ -31,19 +31,20 @@ class QuadFittingFromFlowFunction(Function):
 
 
 class _QuadFittingImage(Function):
-    """QuadFittingFromFlowFunction of one image with its channels innermost, no permutations around it."""
+    """QuadFittingFromFlowFunction of one image with its channels innermost, no permutations around it.  (A trace calls it with whatever
+    it is given later: other layouts are made contiguous here as they are there.)"""
 
     @staticmethod
     def forward(ctx, feat0, feat1, flow):
-        sol, costs = QuadFit_cuda_ext.image_forward(feat0, feat1, flow, any(ctx.needs_input_grad))
+        sol, costs = QuadFit_cuda_ext.image_forward(feat0.contiguous(), feat1.contiguous(), flow, any(ctx.needs_input_grad))
         ctx.save_for_backward(feat0, feat1, flow, costs)
         return sol
 
     @staticmethod
     def backward(ctx, grad_sol):
         feat0, feat1, flow, costs = ctx.saved_tensors
-        d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.image_backward(grad_sol.contiguous().resolve_neg(), feat0.contiguous(), feat1.contiguous(), flow,
-                                                               costs.contiguous())
+        d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.image_backward(grad_sol.contiguous().resolve_neg(), feat0.contiguous(), feat1.contiguous(),
+                                                               flow, costs.contiguous())
         return d_oGfeat0, d_oGfeat1, None
 
 

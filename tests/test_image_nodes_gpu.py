@@ -121,3 +121,55 @@ def test_a_trace_of_a_module_runs_on_other_values(kind, c, grad):
     with torch.no_grad():
         assert torch.equal(traced(*inputs), layer(*inputs))
         assert torch.equal(traced(*others), layer(*others))
+
+
+def gradient_of(function, t, grad):
+    t = t.detach().requires_grad_(True)
+    (g,) = torch.autograd.grad(function(t), t, grad)
+    return g
+
+
+@pytest.mark.parametrize("layout", ["planes", "wider", "one row for all"])
+def test_a_trace_of_the_fit_takes_other_layouts(layout):
+    from customnetworklayers_amd import QuadFittingFromFlow
+
+    layer = QuadFittingFromFlow(DEV)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    f0, f1, flow, grad = (torch.randn((12, 30, c), generator=g, device="cuda", dtype=torch.float32) for c in (8, 8, 3, 3))
+    traced = torch.jit.trace(layer, (f0, f1, flow), check_trace=False)
+    if layout == "planes":
+        f0, f1, flow = (t.permute(2, 0, 1).contiguous().permute(1, 2, 0) for t in (f0, f1, flow))
+    if layout == "wider":
+        f0, f1, flow = (torch.cat([t, t], 2)[..., :t.shape[2]] for t in (f0, f1, flow))
+    if layout == "one row for all":
+        f0, f1, flow = (t[:1].expand(12, 30, -1) for t in (f0, f1, flow))
+    assert torch.equal(traced(f0, f1, flow), layer(f0, f1, flow))
+    assert torch.equal(gradient_of(lambda t: traced(t, f1, flow), f0, grad), gradient_of(lambda t: layer(t, f1, flow), f0, grad))
+
+
+def test_a_trace_of_the_median_takes_other_numbers_of_bins():
+    vols = [torch.from_numpy(median_inputs(1, 11, 19, d, seed=d, empty_fraction=0.1)["vol"][0]).to(DEV) for d in (16, 256)]
+    grad = torch.randn((11, 19), device="cuda", dtype=torch.float32)
+    for first, second in (vols, vols[::-1]):
+        traced = torch.jit.trace(Median(DEV), (first,), check_trace=False)
+        assert torch.equal(traced(second), Median(DEV)(second))
+        assert torch.equal(gradient_of(traced, second, grad), gradient_of(lambda t: MedianFunction.apply(t.unsqueeze(0))[0, 0], second, grad))
+
+
+def test_the_fits_image_calls_refuse_what_they_cannot_read():
+    from customnetworklayers_amd.cudaQuadFit import QuadFit_cuda_ext as ext
+
+    f0, f1, flow, grad = (torch.ones((4, 6, c), device="cuda", dtype=torch.float32) for c in (8, 8, 3, 3))
+    _, costs = ext.image_forward(f0, f1, flow, True)
+    for bad in ((f0.double(), f1, flow), (f0, f1, flow.double())):
+        with pytest.raises(TypeError):
+            ext.image_forward(*bad, True)
+    for bad in ((f0[..., ::2], f1[..., ::2], flow), (f0, f1.cpu(), flow), (f0, f1, flow.cpu())):
+        with pytest.raises(RuntimeError):
+            ext.image_forward(*bad, True)
+    for bad in ((f0, f1[:3], flow), (f0, f1, flow[:3]), (f0, f1, flow[..., :1]), (f0[None], f1[None], flow[None])):
+        with pytest.raises(ValueError):
+            ext.image_forward(*bad, True)
+    for bad in ((grad[:3], costs), (grad, costs[:4])):
+        with pytest.raises(ValueError):
+            ext.image_backward(bad[0], f0, f1, flow, bad[1])
