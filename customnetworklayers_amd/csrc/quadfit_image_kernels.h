@@ -7,8 +7,10 @@
 //
 // A block owns 64 consecutive pixels.  Same arithmetic, operation by operation, as the kernels on planes.
 // Bound by latency on small images (64 x 96 x 312: forward 7 us, backward 10 + 8 + 5), by memory on large ones.  Module, forward +
-// backward, us, kernels on planes with their copies / these: 64 x 96 x 312 155 / 71 (host time), 32 x 200 x 640 333 / 71, 32 x 448 x
-// 1280 1298 / 126, 64 x 448 x 1280 2439 / 267; with 12 pixels of noise on the flow 4679 / 335; forward alone 1150 / 79.
+// backward, us, kernels on planes with their copies / these: 64 x 96 x 312 232 / 127 and 32 x 200 x 640 334 / 130 (host time), 32 x 448 x
+// 1280 1296 / 134, 64 x 448 x 1280 2443 / 266; with 12 pixels of noise on the flow 4679 / 335; forward alone 1150 / 76.  The forward
+// pass works through whole chunks of 32 channels: with fewer than eight it loses on large images, which are not sent here
+// (image_pays in QuadFit_cuda_ext.py).
 #pragma once
 
 namespace quadfit_image {
