@@ -181,33 +181,37 @@ def bench_flowaux(args, cfg, d):
     if cfg["kind"] == "quadfit":
         from customnetworklayers_amd.cudaQuadFit import QuadFit_cuda_ext as ext
         c = cfg["c"]
-        fwd = lambda: ext.forward(t["feat0"], t["feat1"], t["flow"])  # noqa: E731
-        bwd = lambda: ext.backward(t["grad"], t["feat0"], t["feat1"], t["flow"])  # noqa: E731
-        # floats per pixel: forward reads both feature maps and the flow, writes 3; backward reads both maps,
-        # flow and upstream, writes g0, zero-fills g1 and read-modify-writes it
-        # per-source pass of the backward (the dominant kernel): both maps, flow, upstream in; g0 and 5 coefficients out
-        # per-source pass of the backward: both maps, flow, upstream in; g0 and 5 coefficients out (the inverse map not counted)
-        # gather pass (the dominant kernel): first map, 5 coefficients, list length and up to 4 list entries in; g1 out
-        bpp = dict(forward=4 * (2 * c + 5), backward=4 * (5 * c + 5), kernel=4 * (2 * c + 10), sources=4 * (3 * c + 10))
+        maps = t["feat0"], t["feat1"], t["flow"]
+        saving = ext.saving_pays(t["feat0"])  # as the autograd function decides for a pass in training
+        fwd = lambda: ext.forward_saving(*maps)[1] if saving else ext.forward(*maps) and None  # noqa: E731
+        bwd = lambda costs: ext.backward(t["grad"], *maps, costs=costs)  # noqa: E731
+        # floats per pixel: forward reads both feature maps and the flow, writes 3 (and the five costs); backward: the per-source
+        # pass reads the second map, costs, flow and upstream (without the costs both maps), writes g0 and 5 coefficients (and the
+        # inverse map, not counted); the gather pass (the dominant kernel) reads the first map, 5 coefficients, list length and up to
+        # 4 list entries, writes g1
+        sources = 2 * c + 15 if saving else 3 * c + 10
+        bpp = dict(forward=4 * (2 * c + (10 if saving else 5)), backward=4 * (4 * c + 10 if saving else 5 * c + 5), kernel=4 * (2 * c + 10),
+                   sources=4 * sources)
         kernel = "quadfit_gather_tiles<2> (backward, gather pass)"
+        sources_kernel = "quadfit_ring_tiles<1>" if saving else "quadfit_sources_resident<32,true>"
         shape = "features %dx%dx%d" % (c, h, w)
     else:
         from customnetworklayers_amd.cudaMedian import median_cuda_ext as ext
         dd = cfg["d"]
-        fwd = lambda: ext.forward(t["vol"])  # noqa: E731
-        bwd = lambda: ext.backward(t["grad"], t["vol"])  # noqa: E731
-        # forward reads the histogram once (it may stop early) and writes 2; backward reads it, the upstream and writes it
-        bpp = dict(forward=4 * (dd + 2), backward=4 * (2 * dd + 2), kernel=4 * (2 * dd + 2))
-        kernel = "median_backward_stream_kernel<10> (backward)"
+        fwd = lambda: ext.forward_saving(t["vol"])[1]  # noqa: E731
+        bwd = lambda saved: ext.backward(t["grad"], t["vol"], saved)  # noqa: E731
+        # forward reads the histogram once, writes 2 and the crossing (3); backward reads the crossing and the upstream, writes the gradient
+        bpp = dict(forward=4 * (dd + 5), backward=4 * (dd + 5), kernel=4 * (dd + 5))
+        kernel = "median_backward_saved_kernel<4> (backward)"
         shape = "histograms %dx%dx%d" % (h, w, dd)
     bpp["total"] = bpp["forward"] + bpp["backward"]  # "kernel": the dominant kernel alone
     for _ in range(args.warmup):
-        fwd(), bwd()
+        bwd(fwd())
     torch.cuda.synchronize()
     ev = [[torch.cuda.Event(enable_timing=True) for _ in range(3)] for _ in range(args.steps)]
     t0 = time.perf_counter()
     for e in ev:  # events on the stream the kernels are launched on (torch's current stream)
-        e[0].record(); fwd(); e[1].record(); bwd(); e[2].record()
+        e[0].record(); kept = fwd(); e[1].record(); bwd(kept); e[2].record()
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
     f_ms = sum(e[0].elapsed_time(e[1]) for e in ev) / args.steps
@@ -217,7 +221,7 @@ def bench_flowaux(args, cfg, d):
         """HIP events around one kernel of the backward pass, on the stream it is launched on; steps outside the timed region."""
         lib.flowaux_profile(which)
         for _ in range(args.steps):
-            bwd()
+            bwd(kept)
         torch.cuda.synchronize()
         tot_ms, launches = ctypes.c_double(0), ctypes.c_int(0)
         lib.flowaux_profile_read(ctypes.byref(tot_ms), ctypes.byref(launches))
@@ -244,7 +248,7 @@ def bench_flowaux(args, cfg, d):
     }
     if src_ms is not None:  # the second kernel of the backward pass
         out["roofline"]["per_source_pass"] = physical_roofline(
-            {"kernel": "quadfit_sources_resident<32,true>", "avg_launch_ms": round(src_ms, 5), "bytes_per_launch": bpp["sources"] * px},
+            {"kernel": sources_kernel, "avg_launch_ms": round(src_ms, 5), "bytes_per_launch": bpp["sources"] * px},
             cnt, src_ms, key="sources_traffic_bytes")
         out["roofline"]["per_source_pass"].pop("basis")
     if not args.no_cpu_baseline:
