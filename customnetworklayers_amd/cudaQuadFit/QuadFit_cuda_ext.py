@@ -139,14 +139,19 @@ def takes_image(feat0, feat1, flow):
     """Whether image_forward / image_backward are to take these H x W x C maps and H x W x 3 flow as they are: both maps contiguous with
     more than one channel innermost, at a size where that pays.  (Maps that are views of channel planes, views whose sign is still to be
     applied (is_neg), and everything that is to be refused, go through forward / backward.)"""
-    if not (feat0.dim() == 3 and flow.dim() == 3 and feat0.shape == feat1.shape and feat0.shape[:2] == flow.shape[:2]):
-        return False
-    if not all(t.is_cuda and t.dtype == torch.float32 and t.device == flow.device and not t.is_neg() for t in (feat0, feat1, flow)):
+    if not (_readable(feat0, feat1, flow) and not (feat0.is_neg() or feat1.is_neg() or flow.is_neg())):
         return False
     h, w, c = feat0.shape
-    if not (feat0.is_contiguous() and feat1.is_contiguous() and c > 1 and h * w > 1 and h * w * c < 2 ** 31):
-        return False
-    return image_pays(c, h * w, torch.is_grad_enabled() and (feat0.requires_grad or feat1.requires_grad))
+    return (c > 1 and h * w > 1 and h * w * c < 2 ** 31
+            and image_pays(c, h * w, torch.is_grad_enabled() and (feat0.requires_grad or feat1.requires_grad)))
+
+
+def _readable(feat0, feat1, flow):
+    """Whether the kernels on one image can read these.  (One expression: a call at inference waits for the host.)"""
+    shape, of_flow = feat0.shape, flow.shape
+    return (len(shape) == 3 == len(of_flow) and feat1.shape == shape and of_flow[0] == shape[0] and of_flow[1] == shape[1] and of_flow[2] >= 2
+            and flow.is_cuda and feat0.device == feat1.device == flow.device
+            and feat0.dtype == feat1.dtype == flow.dtype == torch.float32 and feat0.is_contiguous() and feat1.is_contiguous())
 
 
 def _flow_strides(flow):
@@ -154,8 +159,6 @@ def _flow_strides(flow):
     one element says nothing: a single column's pixels lie a row apart, and a contiguous tensor may have any number there.)"""
     h, w, channels = flow.shape
     row, pixel, channel = flow.stride()
-    if flow.is_neg():
-        return flow.contiguous().resolve_neg(), channels, 1
     if w == 1:
         pixel = row
     if pixel < 1 or channel < 1 or (h > 1 and row != w * pixel):
@@ -164,21 +167,28 @@ def _flow_strides(flow):
 
 
 def _check_image(feat0, feat1, flow):
-    for t, name in ((feat0, "featureImage0"), (feat1, "featureImage1")):
+    if _readable(feat0, feat1, flow):
+        return feat0.shape
+    for t, name in ((feat0, "featureImage0"), (feat1, "featureImage1"), (flow.contiguous(), "flow")):
         _check_input(t, name)
-    if feat0.shape != feat1.shape or feat0.dim() != 3 or flow.dim() != 3 or flow.shape[:2] != feat0.shape[:2] or flow.shape[2] < 2:
-        raise ValueError("the maps must be H x W x C, the flow H x W x 2 or more, got %s, %s and %s"
-                         % (tuple(feat0.shape), tuple(feat1.shape), tuple(flow.shape)))
-    if flow.dtype != torch.float32:
-        raise TypeError("Input/Output type to the operator must be single/float (flow is %s)" % flow.dtype)
     if not feat0.device == feat1.device == flow.device:
         raise RuntimeError("all tensors must live on one device")
-    return feat0.shape
+    raise ValueError("the maps must be H x W x C, the flow H x W x 2 or more, got %s, %s and %s"
+                     % (tuple(feat0.shape), tuple(feat1.shape), tuple(flow.shape)))
 
 
-def image_forward(feat0, feat1, flow, want_costs):
-    """The fit of one image, feat0, feat1 H x W x C contiguous, flow H x W x 3 anyhow.  Returns [H x W x 3, costs (5,H,W) or None]."""
-    h, w, c = _check_image(feat0, feat1, flow)
+def _check_beside(t, name, shape, flow):
+    _check_input(t, name)
+    if tuple(t.shape) != shape:
+        raise ValueError("%s must have shape %s, got %s" % (name, shape, tuple(t.shape)))
+    if t.device != flow.device:
+        raise RuntimeError("all tensors must live on one device")
+
+
+def image_forward(feat0, feat1, flow, want_costs, checked=False):
+    """The fit of one image, feat0, feat1 H x W x C contiguous, flow H x W x 3 anyhow.  Returns [H x W x 3, costs (5,H,W) or None].
+    checked: takes_image has just said yes to these."""
+    h, w, c = feat0.shape if checked else _check_image(feat0, feat1, flow)
     flow, pixel, channel = _flow_strides(flow)
     out = torch.empty((h, w, 3), dtype=torch.float32, device=flow.device)
     costs = torch.empty((5, h, w), dtype=torch.float32, device=flow.device) if want_costs else None
@@ -193,12 +203,10 @@ def image_forward(feat0, feat1, flow, want_costs):
 def image_backward(d_iGf, feat0, feat1, flow, costs):
     """d_iGf: H x W x 3 gradient wrt the result, costs: the second result of image_forward.  Returns the two maps' gradients."""
     h, w, c = _check_image(feat0, feat1, flow)
-    for t, name, shape in ((d_iGf, "d_iGf", (h, w, 3)), (costs, "costs", (5, h, w))):
-        _check_input(t, name)
-        if tuple(t.shape) != shape:
-            raise ValueError("%s must have shape %s, got %s" % (name, shape, tuple(t.shape)))
-        if t.device != flow.device:
-            raise RuntimeError("all tensors must live on one device")
+    if not (d_iGf.shape == (h, w, 3) and costs.shape == (5, h, w) and d_iGf.dtype == costs.dtype == torch.float32
+            and d_iGf.device == costs.device == flow.device and d_iGf.is_contiguous() and costs.is_contiguous()):
+        _check_beside(d_iGf, "d_iGf", (h, w, 3), flow)
+        _check_beside(costs, "costs", (5, h, w), flow)
     flow, pixel, channel = _flow_strides(flow)
     g0, g1 = torch.empty_like(feat0), torch.empty_like(feat1)
     ws_bytes = lib.quadfit_backward_workspace_bytes(1, h, w)

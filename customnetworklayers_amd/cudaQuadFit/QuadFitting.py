@@ -31,12 +31,14 @@ class QuadFittingFromFlowFunction(Function):
 
 
 class _QuadFittingImage(Function):
-    """QuadFittingFromFlowFunction of one image with its channels innermost, no permutations around it.  (A trace calls it with whatever
-    it is given later: other layouts are made contiguous here as they are there.)"""
+    """QuadFittingFromFlowFunction of one image with its channels innermost, no permutations around it.  checked: takes_image has just
+    said yes to these tensors; a trace calls the node without it, with whatever it is given later."""
 
     @staticmethod
-    def forward(ctx, feat0, feat1, flow):
-        sol, costs = QuadFit_cuda_ext.image_forward(feat0.contiguous(), feat1.contiguous(), flow, any(ctx.needs_input_grad))
+    def forward(ctx, feat0, feat1, flow, checked):
+        if not checked:
+            feat0, feat1, flow = feat0.contiguous(), feat1.contiguous(), flow.resolve_neg()
+        sol, costs = QuadFit_cuda_ext.image_forward(feat0, feat1, flow, any(ctx.needs_input_grad), checked)
         ctx.save_for_backward(feat0, feat1, flow, costs)
         return sol
 
@@ -45,7 +47,7 @@ class _QuadFittingImage(Function):
         feat0, feat1, flow, costs = ctx.saved_tensors
         d_oGfeat0, d_oGfeat1 = QuadFit_cuda_ext.image_backward(grad_sol.contiguous().resolve_neg(), feat0.contiguous(), feat1.contiguous(),
                                                                flow, costs.contiguous())
-        return d_oGfeat0, d_oGfeat1, None
+        return d_oGfeat0, d_oGfeat1, None, None
 
 
 class QuadFittingFromFlow(nn.Module):
@@ -59,7 +61,7 @@ class QuadFittingFromFlow(nn.Module):
         Yi, Xi, Li = t_flow.shape
         assert Li == 3, "flow should have 3 channels: the displacement in X and Y direction and one more\n"
         if QuadFit_cuda_ext.takes_image(t_feat0, t_feat1, t_flow):
-            return _QuadFittingImage.apply(t_feat0, t_feat1, t_flow)
+            return _QuadFittingImage.apply(t_feat0, t_feat1, t_flow, not torch.jit.is_tracing())
         t_feat0_in = t_feat0.permute(2, 0, 1).unsqueeze(0)
         t_feat1_in = t_feat1.permute(2, 0, 1).unsqueeze(0)
         t_flow_in = t_flow.permute(2, 0, 1).unsqueeze(0)

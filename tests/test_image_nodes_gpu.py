@@ -129,7 +129,7 @@ def gradient_of(function, t, grad):
     return g
 
 
-@pytest.mark.parametrize("layout", ["planes", "wider", "one row for all"])
+@pytest.mark.parametrize("layout", ["planes", "wider", "one row for all", "negative"])
 def test_a_trace_of_the_fit_takes_other_layouts(layout):
     from customnetworklayers_amd import QuadFittingFromFlow
 
@@ -143,6 +143,8 @@ def test_a_trace_of_the_fit_takes_other_layouts(layout):
         f0, f1, flow = (torch.cat([t, t], 2)[..., :t.shape[2]] for t in (f0, f1, flow))
     if layout == "one row for all":
         f0, f1, flow = (t[:1].expand(12, 30, -1) for t in (f0, f1, flow))
+    if layout == "negative":  # views whose sign is still to be applied
+        f0, f1, flow = (torch.complex(torch.zeros_like(t), -t).conj().imag for t in (f0, f1, flow))
     assert torch.equal(traced(f0, f1, flow), layer(f0, f1, flow))
     assert torch.equal(gradient_of(lambda t: traced(t, f1, flow), f0, grad), gradient_of(lambda t: layer(t, f1, flow), f0, grad))
 
@@ -173,3 +175,8 @@ def test_the_fits_image_calls_refuse_what_they_cannot_read():
     for bad in ((grad[:3], costs), (grad, costs[:4])):
         with pytest.raises(ValueError):
             ext.image_backward(bad[0], f0, f1, flow, bad[1])
+    for bad in ((grad.cpu(), costs), (grad, costs.cpu()), (grad.transpose(0, 1), costs)):
+        with pytest.raises(RuntimeError):
+            ext.image_backward(bad[0], f0, f1, flow, bad[1])
+    with pytest.raises(TypeError):
+        ext.image_backward(grad, f0, f1, flow, costs.double())
